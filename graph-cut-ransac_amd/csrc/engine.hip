@@ -531,16 +531,15 @@ struct Container {
 };
 
 // SPRT state of a pair's main loop (preemption_sprt.h:141-190): the random
-// pool, the running pool index and the current history; a_table holds A for
-// delta = k / N at the current epsilon, uploaded to a_dev.
+// pool, the running pool index and the current history; a_dev holds A for
+// delta = k / N at the current epsilon (filled by the walk phase).
 struct SprtHost {
   std::vector<int32_t> pool;
   int64_t pool_idx = 0;
   double eps = 0, delta = 0, A = 0;
   double t_M = 0, m_S = 1;
-  std::vector<double> a_table;
   double* a_dev = nullptr;
-  bool table_dirty = true;
+  bool table_dirty = true;  // the device table is of an earlier epsilon
   // preemption_sprt.h:299-330
   double threshold_A(double epsilon, double d) const {
     const double C = (1 - d) * std::log((1 - d) / (1 - epsilon)) + d * (std::log(d / epsilon));
@@ -553,10 +552,9 @@ struct SprtHost {
     }
     return An;
   }
-  void fill_table(size_t n) {
-    a_table.assign(n + 1, 0.0);
-    for (size_t k = 1; k <= n; ++k) a_table[k] = threshold_A(eps, (double)k / (double)n);
-    table_dirty = true;
+  // A for delta = k / n, k in [k0, k1)
+  void fill_table(double* out, size_t n, size_t k0, size_t k1) const {
+    for (size_t k = k0; k < k1; ++k) out[k] = k == 0 ? 0.0 : threshold_A(eps, (double)k / (double)n);
   }
 };
 
@@ -769,6 +767,8 @@ struct PairRunner {
     it.best_value = best_value;
     it.sp = P.sp_on ? 1 : 0;
     it.best_count = best_count;
+    it.stop = it.last = -1;
+    it.delta_changes = 0;
     return DeviceAwait{&P};
   }
   // the inliers of a model in its space-partitioning cells, in cell order
@@ -1116,7 +1116,7 @@ struct PairRunner {
             // (preemption_sprt.h:259-270)
             P.sprt.eps = (double)stop_count / (double)N;
             P.sprt.A = P.sprt.threshold_A(P.sprt.eps, P.sprt.delta);
-            P.sprt.fill_table(N);
+            P.sprt.table_dirty = true;
             s = Score{stop_count, stop_value};
             sprt_start = P.sp_on ? -1 : stop_start;
             // an accepted model was tested on all its cells' points: its list
@@ -1573,6 +1573,8 @@ struct Workspace {
   // an A table of n + 1 entries; the walk requests' upload / download
   DevBuf<int32_t> d_sprt_pool;
   DevBuf<double> d_sprt_tables;
+  HostBuf<double> h_sprt_tables;  // pinned staging of the tables
+  DevBuf<uint64_t> d_sprt_bits;   // a walk's bit rows (SprtPlan)
   // filtered candidate results (device scratch, pinned records), per
   // estimator: the records are read back after the step's other phases ran
   DevBuf<char> d_filt[4];
@@ -1924,7 +1926,7 @@ struct Engine : Workspace {
         P.sprt.delta = ratio / 10.0;
         P.sprt.eps = ratio;
         P.sprt.A = P.sprt.threshold_A(P.sprt.eps, P.sprt.delta);
-        P.sprt.fill_table(n);
+        P.sprt.table_dirty = true;
       }
       P.est = s.kind;
       // the fundamental-matrix estimator of the drivers and of the template
@@ -2105,7 +2107,6 @@ struct Engine : Workspace {
           if (!P.sprt_on) continue;
           h2d(d_sprt_pool.p + off[(size_t)i], P.sprt.pool.data(), P.sprt.pool.size());
           P.sprt.a_dev = d_sprt_tables.p + t;
-          P.sprt.table_dirty = true;
           t += P.n + 1;
         }
       }
@@ -3014,13 +3015,36 @@ struct Engine : Workspace {
 
   // SPRT walks (k_sprt.hip), one wavefront per pair: the items and their
   // slot lists go up in one copy, the items come back in one copy.
+  static constexpr size_t kTableChunk = 256;             // table entries per host task (~20 us)
+  static constexpr int64_t kSprtBudgetWords = 32 << 20;  // 256 MB of bit rows per window
   PhaseTask exec_sprt(std::vector<PairCtx*> items) {
     const int k = (int)items.size();
+    // the A tables of pairs whose epsilon changed: n + 1 entries of several
+    // logarithms each, filled on the host threads into one pinned block
+    struct Fill {
+      PairCtx* P;
+      size_t off, k0, k1;
+    };
+    std::vector<Fill> fills;
+    size_t tab = 0;
     for (auto* P : items)
       if (P->sprt.table_dirty) {
-        h2d(P->sprt.a_dev, P->sprt.a_table.data(), P->sprt.a_table.size());
-        P->sprt.table_dirty = false;
+        const size_t n1 = (size_t)P->n + 1;
+        for (size_t k0 = 0; k0 < n1; k0 += kTableChunk) fills.push_back(Fill{P, tab, k0, std::min(n1, k0 + kTableChunk)});
+        tab += n1;
       }
+    if (!fills.empty()) {
+      double* const ht = h_sprt_tables.ensure(tab);
+      pool->run(fills.size(), [&](size_t i) {
+        const Fill& f = fills[i];
+        f.P->sprt.fill_table(ht + f.off, (size_t)f.P->n, f.k0, f.k1);
+      });
+      for (const Fill& f : fills)
+        if (f.k0 == 0) {
+          h2d(f.P->sprt.a_dev, ht + f.off, (size_t)f.P->n + 1);
+          f.P->sprt.table_dirty = false;
+        }
+    }
     std::vector<SprtItem> it((size_t)k);
     std::vector<int32_t> slots;
     std::vector<size_t> soff((size_t)k);
@@ -3042,9 +3066,15 @@ struct Engine : Workspace {
     if (!slots.empty()) std::memcpy(h + b_items, slots.data(), 4 * slots.size());
     check_hip(hipMemcpyAsync(d, h, total_b, hipMemcpyHostToDevice, stream), "hipMemcpyAsync H2D");
     const int t0 = prof.start("sprt", 0.0);
-    launch_sprt_walk(stream, reinterpret_cast<SprtItem*>(d), k, d_rpts, d_pair_pt_off.p, d_pair_n.p,
-                     d_pair_sq_thr.p, d_sprt_pool.p, d_sp_pairs.p, d_sp_cells.p, d_sp_perm.p, d_sp_cell_of.p,
-                     d_sp_list.p, sp_max_cells);
+    int max_n = 0, max_slots = 0;
+    for (int i = 0; i < k; ++i) {
+      max_n = std::max(max_n, (int)items[(size_t)i]->n);
+      max_slots = std::max(max_slots, (int)it[(size_t)i].num_slots);
+    }
+    const SprtPlan plan = sprt_plan(k, max_n, max_slots, kSprtBudgetWords);
+    launch_sprt_walk(stream, reinterpret_cast<SprtItem*>(d), k, max_slots, plan, d_sprt_bits.ensure(plan.scratch_words),
+                     d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pair_sq_thr.p, d_sprt_pool.p, d_sp_pairs.p, d_sp_cells.p,
+                     d_sp_perm.p, d_sp_cell_of.p, d_sp_list.p, sp_max_cells);
     prof.stop(t0);
     check_hip(hipMemcpyAsync(h, d, sizeof(SprtItem) * (size_t)k, hipMemcpyDeviceToHost, stream),
               "hipMemcpyAsync D2H");

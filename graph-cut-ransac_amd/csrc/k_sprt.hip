@@ -5,236 +5,712 @@
 // the order of a random pool, starting where the previous model stopped,
 // and multiplies a likelihood ratio point by point until it exceeds the
 // decision threshold A; and the test's parameters (delta, A) change after a
-// rejection that moves the estimated delta by more than 5 %.  One wavefront
-// per pair runs the whole sequence: 64 pool positions at a time it computes
-// residuals and inlier flags in parallel, then steps through them in order
-// (every lane carries the same scalar chain) with the reference's
-// operations: lambda * (delta / epsilon) or lambda * ((1 - delta) /
-// (1 - epsilon)), the test against A, and the score sum of
-// 1 - r^2 / tau^2 over the tested inliers.
+// rejection that moves the estimated delta by more than 5 %.  What does not
+// depend on that order are the inlier decisions themselves, so the walk is
+// split in two kernels:
+//   k_sprt_masks  every listed model against every point of its pair, four
+//                 waves per model: one inlier bit per position of the test
+//                 order (the pool, or the space partitioning cells' order);
+//   k_sprt_walk   one wavefront per pair steps through the models on those
+//                 bits, 64 positions at a time.
+// The models of a walk are taken in windows (a mask and a walk launch each),
+// so a walk that stops early leaves the later models' masks unmade and the
+// mask memory is bounded.
 //
 // A after a delta change comes from a table the host fills for the current
-// epsilon (A for delta = k / N, k = 0..N), so every logarithm is the host C
-// library's.  The walk stops at the first accepted model whose score beats
-// the best value given: the host then makes the reference's epsilon update,
-// the validity check and the best-model update, and continues the walk.
+// epsilon (A for delta = k / N, k = 0..N), so every logarithm that enters a
+// result is the host C library's.  The walk stops at the first accepted model
+// whose score beats the best value given: the host then makes the
+// reference's epsilon update, the validity check and the best-model update,
+// and continues the walk.
+//
+// The ratio's chain on 64 positions at once.  After a inliers and b outliers
+// the reference's running product is f_in^a f_out^b up to a relative error of
+// (a + b) 2^-53, so "the product exceeds A" is a log f_in + b log f_out >
+// log A unless the two sides are within a margin of that rounding and of the
+// logarithms'.  Each lane forms the sum for its own position from a popcount
+// of the bits before it; the first lane above log A is where the reference
+// stops.  A model with a position inside the margin before its stop, or with a
+// non-finite logarithm, is walked again by the reference's chain, one
+// multiplication per position, so every decision is the reference's.  So is a
+// model whose product comes near the subnormal range (a model with many
+// inliers under a small delta: the usual good model), unless the positions
+// left are too few for the ratio to climb back; there the chain ends as soon
+// as the product is zero, from which it never returns.
+//
+// Value of an accepted model: the mask kernel sums every model's terms in
+// parallel, so only a model that can beat the best value (within the two
+// sums' rounding) is summed in the reference's order.
+//
+// What bounds it: the walk is a serial chain of models, one wavefront per
+// pair, so it is bound by the latency of a few dozen dependent scalar and
+// vector instructions per 64 positions (or per cell the walk stops in), plus
+// the divisions and logarithms of a delta change; the masks take 12 us per
+// window.  Measured on MI355X, one call with the API's defaults: the walk
+// that evaluated residuals and stepped position by position took 148.7 ms of
+// a findHomography call's 151.0 ms of kernels (2,000 points, 50 % inliers) and
+// 50.4 of 52.6 ms for a fundamental matrix (3,001 points); this one 7.4 ms
+// and 2.7 ms.
 #include "dev_common.hpp"
 #include "dev_sp.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace gcr {
 
-// The same test after the space partitioning selector
-// (preemption_sprt.h:241-258): a model whose kept cells hold fewer points
-// than the best model's inliers is skipped untested; the others are tested
-// over their kept cells' points in cell order, without the pool.  A
-// rejection leaves only the current cell: the following cells are still
-// tested from the last accepted ratio (the reference's break exits the inner
-// loop only), and their tested inliers count.  Each tested model's inliers
-// are written in test order to list (the last tested model's list is the
-// loop's inlier container).
-__device__ void sprt_walk_sp(SprtItem& it, const double* __restrict__ pts, const SpPair& sp,
-                             const SpCell* __restrict__ cells, const int32_t* __restrict__ perm,
-                             const int32_t* __restrict__ cell_of, const double* __restrict__ a_table, int n,
-                             double sq_thr, uint8_t* keep, int32_t* __restrict__ list) {
-  const int lane = threadIdx.x;
-  double delta = it.delta, A = it.A;
-  const double eps = it.eps;
-  double f_in = delta / eps, f_out = (1 - delta) / (1 - eps);
-  it.stop = -1;
-  it.last = -1;
-  for (int s = 0; s < it.num_slots; ++s) {
-    const double* mp = it.models + 9 * (int64_t)it.slots[s];
-    double M[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) M[k] = mp[k];
-    const int64_t kept = sp_select_wave(M, sp, cells, keep);
-    if (kept < it.best_count) continue;
-    double lambda = 1.0, value = 0.0;
-    int64_t count = 0;
-    bool rejected = false;
-    int broken = -1;  // the cell a rejection left
-    for (int b = 0; b < n; b += 64) {
-      const int e = b + lane;
-      int c = -1;
-      bool kp = false, inl = false;
-      double term = 0.0;
-      int32_t p = 0;
-      if (e < n) {
-        c = cell_of[e];
-        kp = keep[c] != 0;
-        if (kp) {
-          p = perm[e];
-          const double r2 = h_sq_residual(pts + 4 * (int64_t)p, M);
-          inl = r2 < sq_thr;
-          if (inl) term = 1.0 - r2 / sq_thr;
-        }
-      }
-      uint64_t mk = __ballot(kp);
-      const uint64_t mi = __ballot(inl);
-      while (mk) {
-        const int l = __ffsll((unsigned long long)mk) - 1;
-        mk &= mk - 1;
-        const int cl = __shfl(c, l, 64);
-        const double tl = __shfl(term, l, 64);
-        const int32_t pl = __shfl(p, l, 64);
-        if (cl == broken) continue;
-        double lambda_new;
-        if ((mi >> l) & 1ull) {
-          lambda_new = lambda * f_in;
-          value += tl;
-          if (lane == 0) list[count] = pl;
-          ++count;
-        } else {
-          lambda_new = lambda * f_out;
-        }
-        if (lambda_new > A) {
-          rejected = true;
-          broken = cl;
-          continue;
-        }
-        lambda = lambda_new;
-      }
-    }
-    it.last = s;
-    it.last_start = -2;
-    it.last_tested = 0;
-    it.last_count = count;
-    it.last_value = value;
-    it.last_accepted = rejected ? 0 : 1;
-    if (!rejected) {
-      if (value > it.best_value) {
-        it.stop = s;
-        break;
-      }
-    } else {
-      const double de = (double)count / (double)n;
-      if (de > 0 && fabs(delta - de) / delta > 0.05) {
-        delta = de;
-        A = a_table[count];
-        f_in = delta / eps;
-        f_out = (1 - delta) / (1 - eps);
-        ++it.delta_changes;
-      }
-    }
-  }
-  it.delta = delta;
-  it.A = A;
+namespace {
+
+constexpr int kMaskThreads = 256;
+
+// A value that is the same on every lane, held in scalar registers: the walk's
+// control flow stays scalar (measured with it in vector registers: about 200
+// instructions and 1,250 cycles per step of walk_cells).
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t uni(uint64_t v) {
+  return ((uint64_t)(uint32_t)uni((int)(v >> 32)) << 32) | (uint32_t)uni((int)(uint32_t)v);
 }
 
-template <int KIND>
-__device__ void sprt_walk_one(SprtItem& it, const double* __restrict__ pts, const int32_t* __restrict__ pool,
-                              const double* __restrict__ a_table, int n, double sq_thr) {
-  const int lane = threadIdx.x;
-  int64_t idx = it.pool_idx;
-  double delta = it.delta, A = it.A;
-  const double eps = it.eps;
-  double f_in = delta / eps, f_out = (1 - delta) / (1 - eps);
-  it.stop = -1;
-  it.last = -1;
-  for (int s = 0; s < it.num_slots; ++s) {
-    const double* mp = it.models + 9 * (int64_t)it.slots[s];
-    double M[9];
+struct Chain {
+  double f_in, f_out, A;
+  double l_in, l_out, l_A;
+  double hi, lo;  // log A and the margin around it
+  int unit;       // both factors are 1: the product stays at 1
+  int fast;       // the logarithms are finite
+};
+
+// The ratio's factors and their logarithms (lanes 0, 1, 2 take one logarithm
+// each).  Margin of a sum of at most n logarithms: the product's n roundings
+// (n 2^-53) and the logarithms' errors, each with a factor of fifty and more
+// to spare.
+__device__ Chain make_chain(double eps, double delta, double A, int n) {
+  Chain c;
+  c.f_in = delta / eps;
+  c.f_out = (1 - delta) / (1 - eps);
+  c.A = A;
+  const int lane = lane_id();
+  const double l = log(lane == 0 ? c.f_in : (lane == 1 ? c.f_out : A));
+  c.l_in = readlane_f64(l, 0);
+  c.l_out = readlane_f64(l, 1);
+  c.l_A = readlane_f64(l, 2);
+  const double m = 1e-14 * (16.0 + (double)n) + 1e-13 * (double)n * fmax(fabs(c.l_in), fabs(c.l_out));
+  c.hi = c.l_A + m;
+  c.lo = c.l_A - m;
+  c.unit = uni(c.f_in == 1.0 && c.f_out == 1.0);
+  c.fast = uni(fabs(c.l_in) < 1e300 && fabs(c.l_out) < 1e300 && fabs(c.l_A) < 1e300);
+  return c;
+}
+
+// The positions of a word against the threshold (lane l: position l with a
+// inliers and b outliers up to it), as lane masks.
+struct Sides {
+  uint64_t above, open, low;  // above A for certain; undecided; below A with a product near the subnormal range
+};
+__device__ __forceinline__ Sides chain_sides(const Chain& c, int a, int b) {
+  const double L = (double)a * c.l_in + (double)b * c.l_out;
+  Sides s;
+  s.above = ballot64(L > c.hi);
+  const uint64_t below = ballot64(L < c.lo);
+  s.open = ~(s.above | below);
+  s.low = below & ballot64(L < -690.0);
+  return s;
+}
+
+// A product below e^-690 cannot exceed A within `left` more factors: it has at
+// least 690 + log A to climb, and no less if it passes through the subnormal
+// range (the climb from 2^-1022 on is in the normal range).
+__device__ __forceinline__ bool no_return(const Chain& c, int left) {
+  const double up = fmax(fmax(c.l_in, c.l_out), 0.0);
+  return uni((double)left * up * (1.0 + 1e-9) < 680.0 + c.l_A) != 0;
+}
+
+}  // namespace
+
+// One workgroup per (item, slot of the window; live of them used).  Position e of item i's test
+// order is point order[e]; bit e of row (item win + j) is set when that point is
+// an inlier of the window's slot j; inl_count and approx: the number of set bits
+// and the sum of their terms in any order.  Space partitioning items also get the
+// row of kept positions, the kept point count and (once per item) the row of
+// the cells' first positions.
+__global__ void __launch_bounds__(kMaskThreads)
+    k_sprt_masks(const SprtItem* __restrict__ items, int win_base, int win, int live, const double* __restrict__ pts,
+                 const int64_t* __restrict__ pair_pt_off, const int32_t* __restrict__ pair_n,
+                 const double* __restrict__ pair_sq_thr, const int32_t* __restrict__ pools,
+                 const SpPair* __restrict__ sp_pairs, const SpCell* __restrict__ sp_cells,
+                 const int32_t* __restrict__ sp_perm, const int32_t* __restrict__ sp_cell_of, int words,
+                 uint64_t* __restrict__ inl_bits, uint64_t* __restrict__ keep_bits, uint64_t* __restrict__ start_bits,
+                 int32_t* __restrict__ kept_count, int32_t* __restrict__ inl_count,
+                 double* __restrict__ approx) {
+  extern __shared__ uint8_t keep[];
+  __shared__ int32_t part[kMaskThreads / 64];
+  __shared__ double vpart[kMaskThreads / 64];
+  const int item = (int)(blockIdx.x / (unsigned)live), j = (int)(blockIdx.x % (unsigned)live);
+  const SprtItem& it = items[item];
+  const int s = win_base + j;
+  if (it.stop >= 0 || s >= it.num_slots) return;
+  const int pair = it.pair;
+  const int64_t base = pair_pt_off[pair];
+  const int n = pair_n[pair];
+  const double sq = pair_sq_thr[pair];
+  const double* __restrict__ P = pts + 4 * base;
+  const double* __restrict__ mp = it.models + 9 * (int64_t)it.slots[s];
+  double M[9];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) M[k] = mp[k];
-    const int64_t start = idx;
-    double lambda = 1.0, value = 0.0;
-    int64_t count = 0, tested = 0;
-    bool rejected = false;
-    for (int b = 0; b < n && !rejected; b += 64) {
-      const int t = b + lane;
+  for (int k = 0; k < 9; ++k) M[k] = mp[k];
+  const int lane = lane_id(), wave = threadIdx.x >> 6;
+  const int64_t row = ((int64_t)item * win + j) * words;
+  const int nw = (n + 63) >> 6;
+  double value = 0.0;
+  int32_t inliers = 0;
+  if (it.sp) {
+    const SpPair sp = sp_pairs[pair];
+    const SpCell* __restrict__ cells = sp_cells + sp.cell_off;
+    const int32_t* __restrict__ cell_of = sp_cell_of + base;
+    const bool any = !(fabs(sp_det3(M)) < 1e-3);
+    int32_t cnt = 0;
+    for (int c = threadIdx.x; c < sp.ncells; c += kMaskThreads) {
+      const SpCell cell = cells[c];
+      const bool k = any && sp_keep(M, cell, sp);
+      keep[c] = k ? 1 : 0;
+      if (k) cnt += cell.len;
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) cnt += __shfl_xor(cnt, d, 64);
+    if (lane == 0) part[wave] = cnt;
+    __syncthreads();
+    const int32_t kept = part[0] + part[1] + part[2] + part[3];
+    if (threadIdx.x == 0) kept_count[(int64_t)item * win + j] = kept;
+    const bool starts = j == 0;
+    const bool tested = kept >= it.best_count;  // else the walk skips the model
+    if (!tested && !starts) return;
+    for (int w = wave; w < nw; w += kMaskThreads / 64) {
+      const int e = 64 * w + lane;
+      bool kp = false, inl = false, first = false;
+      if (e < n) {
+        const int c = cell_of[e];
+        kp = keep[c] != 0;
+        if (starts) first = e == 0 || cell_of[e - 1] != c;
+        if (kp && tested) {
+          const double r2 = h_sq_residual(P + 4 * (int64_t)sp_perm[base + e], M);
+          inl = r2 < sq;
+          if (inl) value += 1.0 - r2 / sq;
+        }
+      }
+      const uint64_t bk = ballot64(kp), bi = ballot64(inl), bs = ballot64(first);
+      inliers += __popcll(bi);
+      if (lane == 0) {
+        keep_bits[row + w] = bk;
+        inl_bits[row + w] = bi;
+        if (starts) start_bits[(int64_t)item * words + w] = bs;
+      }
+    }
+  } else {
+    const int32_t* __restrict__ order = pools + base;
+    for (int w = wave; w < nw; w += kMaskThreads / 64) {
+      const int e = 64 * w + lane;
       bool inl = false;
-      double term = 0.0;
+      if (e < n) {
+        const double* p = P + 4 * (int64_t)order[e];
+        const double r2 = it.kind == 0 ? h_sq_residual(p, M) : f_sq_sampson(p, M);
+        inl = r2 < sq;
+        if (inl) value += 1.0 - r2 / sq;
+      }
+      const uint64_t b = ballot64(inl);
+      inliers += __popcll(b);
+      if (lane == 0) inl_bits[row + w] = b;
+    }
+  }
+  value = wave_tree64(value);
+  __syncthreads();  // part's readers above
+  if (lane == 0) {
+    vpart[wave] = value;
+    part[wave] = inliers;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    approx[(int64_t)item * win + j] = (vpart[0] + vpart[1]) + (vpart[2] + vpart[3]);
+    inl_count[(int64_t)item * win + j] = part[0] + part[1] + part[2] + part[3];
+  }
+}
+
+namespace {
+
+// Sum over the wave: DPP steps inside the rows of
+// 16, then the four rows' totals.
+__device__ __forceinline__ int wave_sum_i32(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, false);  // row_ror:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x124, 0xF, 0xF, false);  // row_ror:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x122, 0xF, 0xF, false);  // row_ror:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x121, 0xF, 0xF, false);  // row_ror:1
+  return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
+         __builtin_amdgcn_readlane(v, 48);
+}
+
+// A model's rows: lane l holds words l of the first 64 words (4,096
+// positions); later words come from memory.
+struct Rows {
+  uint64_t inl, keep, start;  // this lane's words
+  const uint64_t *g_inl, *g_keep, *g_start;
+  __device__ __forceinline__ uint64_t inl_word(int w) const {
+    return w < 64 ? (uint64_t)readlane_i64((int64_t)inl, w) : g_inl[w];
+  }
+};
+
+struct WalkResult {
+  int count, tested;
+  bool rejected;
+};
+
+// The reference's product over the low cnt positions of m (inlier bits); top:
+// the largest product on the way (at least the first).
+__device__ __forceinline__ double chain_word(const Chain& c, double lambda, uint64_t m, int cnt, double& top) {
+  double x = lambda;
+  top = lambda;
+  if (cnt == 64) {
+#pragma unroll
+    for (int l = 0; l < 64; ++l) {
+      x = x * (((m >> l) & 1ull) ? c.f_in : c.f_out);
+      top = fmax(x, top);
+    }
+  } else {
+    for (int l = 0; l < cnt; ++l) {
+      x = x * (((m >> l) & 1ull) ? c.f_in : c.f_out);
+      top = fmax(x, top);
+    }
+  }
+  return x;
+}
+
+// One model from pool position start (see the file header); total: its
+// inliers among all n points.
+__device__ WalkResult walk_pool(const Rows& R, const Chain& c, int start, int n, int total) {
+  const int lane = lane_id();
+  const uint64_t le = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+  const int nw = (n + 63) >> 6;
+  // 64 bits of the row from position p on (zeros beyond the row)
+  auto window = [&](int p) -> uint64_t {
+    const int w = p >> 6, s = p & 63;
+    uint64_t v = R.inl_word(w) >> s;
+    if (s && w + 1 < nw) v |= R.inl_word(w + 1) << (64 - s);
+    return v;
+  };
+  // inlier bits of the test's positions b .. b + 63
+  auto word = [&](int b) -> uint64_t {
+    int64_t p64 = (int64_t)start + b;
+    if (p64 >= n) p64 -= n;
+    const int p = (int)p64;
+    uint64_t v = window(p);
+    if (n - p < 64) v |= window(0) << (n - p);
+    return n - b < 64 ? v & ((1ull << (n - b)) - 1ull) : v;
+  };
+  if (c.unit) {
+    // the product stays at 1: above A at the first point, or never
+    if (1.0 > c.A) return WalkResult{(int)(word(0) & 1ull), 1, true};
+    return WalkResult{total, n, false};
+  }
+  const WalkResult all{total, n, false};
+  bool exact = !c.fast;
+  int count = 0;
+  for (int b = 0; !exact && b < n; b += 64) {
+    const int t = b + lane;
+    const uint64_t m = word(b);
+    const int a = count + __popcll(m & le);
+    Sides s = chain_sides(c, a, t + 1 - a);
+    const uint64_t live = n - b < 64 ? (1ull << (n - b)) - 1ull : ~0ull;
+    const uint64_t above = s.above & live;
+    const uint64_t upto = above ? ((above & -above) << 1) - 1ull : live;  // through the first stop
+    if ((s.open | s.low) & upto) {
+      if (!(s.open & upto) && no_return(c, n - b)) return all;
+      exact = true;
+      break;
+    }
+    if (above) return WalkResult{count + (int)__popcll(m & upto), b + (int)__ffsll((unsigned long long)above), true};
+    count += __popcll(m);
+  }
+  if (!exact) return all;
+  // the reference's chain; a word whose largest product is not above A has no
+  // stop in it, and a product of zero stays there
+  count = 0;
+  double lambda = 1.0;
+  for (int b = 0; b < n && lambda != 0.0; b += 64) {
+    const uint64_t m = word(b);
+    const int cnt = n - b < 64 ? n - b : 64;
+    double top;
+    const double x = chain_word(c, lambda, m, cnt, top);
+    if (top > c.A) {
+      double y = lambda;
+      for (int l = 0; l < cnt; ++l) {
+        y = y * (((m >> l) & 1ull) ? c.f_in : c.f_out);
+        if (y > c.A) return WalkResult{count + (int)__popcll(m & ((2ull << l) - 1ull)), b + l + 1, true};
+      }
+    }
+    lambda = x;
+    count += __popcll(m);
+  }
+  return all;
+}
+
+// One model over its kept cells (preemption_sprt.h:241-258): a rejection
+// leaves only the current cell, and the following cells are tested from the
+// last accepted ratio.  RECORD: the tested inliers' bits go to rec.
+//
+// When a point's factor exceeds A it is not kept, so the ratio stays where a
+// factor of the same kind exceeds A again while one of the other kind (on the
+// other side of 1) does not.  Every following cell that begins with a point of
+// that kind is therefore left at its first point, and the walk goes straight
+// to the next kept cell that begins with a point of the other kind.
+template <bool RECORD>
+__device__ WalkResult walk_cells(const Rows& R, const Chain& c, int n, int total, uint64_t* rec) {
+  const int lane = lane_id();
+  const uint64_t le = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+  const int nw = (n + 63) >> 6;
+  int count = 0, rejected = 0;
+  int exact = !c.fast || c.unit;
+  if (c.unit && !uni(1.0 > c.A)) {
+    if constexpr (RECORD)
+      for (int w = lane; w < nw; w += 64) rec[w] = w < 64 ? R.inl : R.g_inl[w];
+    return WalkResult{total, n, false};
+  }
+  int A0 = 0, B0 = 0;  // the accepted factors
+  int sunk = 0;        // the ratio cannot climb back to A: only the count is left
+  int left = 0;        // the last cell was left by an outlier (1) or an inlier (2)
+  for (int w0 = 0; w0 < nw && !exact; w0 += 64) {
+    // this block's words, one per lane
+    uint64_t kw = 0, iw = 0, sw = 0, hitw = 0;
+    if (w0 == 0) {
+      kw = R.keep;
+      iw = R.inl;
+      sw = R.start;
+    } else if (w0 + lane < nw) {
+      kw = R.g_keep[w0 + lane];
+      iw = R.g_inl[w0 + lane];
+      sw = R.g_start[w0 + lane];
+    }
+    const uint64_t first = kw & sw;  // the kept cells' first positions
+    const int we = nw - w0 < 64 ? nw - w0 : 64;
+    int w = 0, bit = 0;  // the next position of the block
+    while (w < we) {
+      if (left) {
+        // to the next kept cell that begins with a point of the other kind;
+        // the inliers that the cells before it are left at count
+        const uint64_t from = lane < w ? 0ull : (lane == w ? ~0ull << bit : ~0ull);
+        const uint64_t ev = first & (left == 2 ? ~iw : iw) & from;
+        const uint64_t has = ballot64(ev != 0);
+        const int l = has ? __ffsll((unsigned long long)has) - 1 : 64;
+        const uint64_t evw = has ? uni((uint64_t)readlane_i64((int64_t)ev, l)) : 0ull;
+        if (left == 2) {
+          const uint64_t upto = lane < l ? ~0ull : (lane == l ? (evw & -evw) - 1ull : 0ull);
+          hitw |= first & iw & from & upto;
+        }
+        if (!has) break;
+        left = 0;
+        w = l;
+        bit = __ffsll((unsigned long long)evw) - 1;
+      }
+      const uint64_t k = uni((uint64_t)readlane_i64((int64_t)kw, w)) & (~0ull << bit);
+      const uint64_t in = uni((uint64_t)readlane_i64((int64_t)iw, w)) & k;
+      uint64_t above = 0, upto = k;
+      if (!sunk) {
+        Sides s = chain_sides(c, A0 + __popcll(in & le), B0 + __popcll(k & ~in & le));
+        above = s.above & k;
+        if (above) upto = k & (((above & -above) << 1) - 1ull);
+        if ((s.open | s.low) & upto) {
+          if ((s.open & upto) || !no_return(c, n - 64 * (w0 + w))) {
+            exact = 1;
+            break;
+          }
+          sunk = 1;
+          above = 0;
+          upto = k;
+        }
+      }
+      if (lane == w) hitw |= in & upto;
+      if (above) {
+        const uint64_t at = above & -above, before = at - 1ull;  // the factor that exceeded A is not kept
+        rejected = 1;
+        left = (in & at) ? 2 : 1;
+        A0 += __popcll(in & before);
+        B0 += __popcll(k & ~in & before);
+        bit = __ffsll((unsigned long long)above);
+        w += bit >> 6;
+        bit &= 63;
+      } else {
+        A0 += __popcll(in);
+        B0 += __popcll(k & ~in);
+        bit = 0;
+        ++w;
+      }
+    }
+    if (exact) break;
+    count += wave_sum_i32(__popcll(hitw));
+    if constexpr (RECORD)
+      if (w0 + lane < nw) rec[w0 + lane] = hitw;
+  }
+  if (!exact) return WalkResult{uni(count), n, rejected != 0};
+  // the reference's chain
+  WalkResult r{0, n, false};
+  double lambda = 1.0;
+  bool broken = false;  // the current cell was left
+  for (int w0 = 0; w0 < nw; w0 += 64) {
+    uint64_t kw = 0, iw = 0, sw = 0, hitw = 0;
+    if (w0 == 0) {
+      kw = R.keep;
+      iw = R.inl;
+      sw = R.start;
+    } else if (w0 + lane < nw) {
+      kw = R.g_keep[w0 + lane];
+      iw = R.g_inl[w0 + lane];
+      sw = R.g_start[w0 + lane];
+    }
+    const int we = nw - w0 < 64 ? nw - w0 : 64;
+    for (int w = 0; w < we; ++w) {
+      const uint64_t k = (uint64_t)readlane_i64((int64_t)kw, w), in = (uint64_t)readlane_i64((int64_t)iw, w) & k;
+      const uint64_t st = (uint64_t)readlane_i64((int64_t)sw, w);
+      uint64_t hit = 0, todo = k;
+      if (broken) {
+        // the rest of the cell that was left
+        if (st == 0) continue;
+        todo &= ~((st & -st) - 1ull);
+        broken = false;
+      }
+      if (lambda == 0.0) {
+        hit = in & todo;  // no stop any more
+        todo = 0;
+      }
+      while (todo) {
+        const uint64_t at = todo & -todo;
+        todo &= todo - 1ull;
+        const bool inlier = (in & at) != 0;
+        const double next = lambda * (inlier ? c.f_in : c.f_out);
+        if (inlier) hit |= at;
+        if (next > c.A) {
+          r.rejected = true;
+          const uint64_t later = st & ~(at | (at - 1ull));  // the cells that begin after this point
+          if (later) {
+            todo &= ~((later & -later) - 1ull);
+          } else {
+            todo = 0;
+            broken = true;
+          }
+        } else {
+          lambda = next;
+        }
+      }
+      r.count += __popcll(hit);
+      if (lane == w) hitw = hit;
+    }
+    if constexpr (RECORD)
+      if (w0 + lane < nw) rec[w0 + lane] = hitw;
+  }
+  return r;
+}
+
+// Sum of 1 - r^2 / tau^2 over the set bits of an accepted model in test
+// order from position start; four words' points in flight at a time.
+template <class H, class R>
+__device__ double ordered_value(int n, int64_t start, H has, R residual, double sq) {
+  const int lane = lane_id();
+  double value = 0.0;
+  for (int b = 0; b < n; b += 256) {
+    double term[4];
+    uint64_t m[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int t = b + 64 * u + lane;
+      bool in = false;
+      term[u] = 0.0;
       if (t < n) {
         int64_t pos = start + t;
         if (pos >= n) pos -= n;
-        const double r2 = sq_residual<KIND>(pts + 4 * (int64_t)pool[pos], M);
-        inl = r2 < sq_thr;
-        if (inl) term = 1.0 - r2 / sq_thr;
+        in = has((int)pos);
+        const double r2 = residual((int)pos);
+        if (in) term[u] = 1.0 - r2 / sq;
       }
-      const uint64_t mask = __ballot(inl);
-      const int cnt = n - b < 64 ? n - b : 64;
-      for (int l = 0; l < cnt; ++l) {
-        const bool in = (mask >> l) & 1ull;
-        const double tl = __shfl(term, l, 64);
-        double lambda_new;
-        if (in) {
-          lambda_new = lambda * f_in;
-          ++count;
-          value += tl;
-        } else {
-          lambda_new = lambda * f_out;
-        }
-        ++tested;
-        if (lambda_new > A) {
-          rejected = true;
+      m[u] = ballot64(in);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      while (m[u]) {
+        const int l = __ffsll((unsigned long long)m[u]) - 1;
+        value += readlane_f64(term[u], l);
+        m[u] &= m[u] - 1;
+      }
+  }
+  return value;
+}
+
+}  // namespace
+
+// One wavefront per item: the window's models in order.  A model's words are
+// fetched while the model before it is walked, the models' counts and values
+// 64 models at a time.
+__global__ void __launch_bounds__(64)
+    k_sprt_walk(SprtItem* items, int win_base, int win, const double* __restrict__ pts,
+                const int64_t* __restrict__ pair_pt_off, const int32_t* __restrict__ pair_n,
+                const double* __restrict__ pair_sq_thr, const int32_t* __restrict__ pools,
+                const int32_t* __restrict__ sp_perm, int words, const uint64_t* __restrict__ inl_bits,
+                const uint64_t* __restrict__ keep_bits, const uint64_t* __restrict__ start_bits,
+                const int32_t* __restrict__ kept_count, const int32_t* __restrict__ inl_count,
+                const double* __restrict__ approx, uint64_t* rec_bits, int32_t* __restrict__ sp_list) {
+  SprtItem it = items[blockIdx.x];
+  if (it.stop >= 0 || win_base >= it.num_slots) return;
+  const int lane = threadIdx.x;
+  const int64_t base = pair_pt_off[it.pair];
+  const int n = uni(pair_n[it.pair]);
+  const int is_sp = uni(it.sp);
+  const double sq = pair_sq_thr[it.pair];
+  const double* __restrict__ P = pts + 4 * base;
+  const int32_t* __restrict__ order = is_sp ? sp_perm + base : pools + base;
+  const int nw = (n + 63) >> 6;
+  const int left_slots = uni(it.num_slots) - win_base;
+  const int end = left_slots < win ? left_slots : win;
+  const int64_t row0 = (int64_t)blockIdx.x * win * words, slot0 = (int64_t)blockIdx.x * win;
+  Rows R;
+  R.g_start = start_bits + (int64_t)blockIdx.x * words;
+  R.start = is_sp && lane < nw ? R.g_start[lane] : 0ull;
+  Chain c = make_chain(it.eps, it.delta, it.A, n);
+  Chain c_last = c;  // the chain the last tested model was walked with
+  int last = -1;
+  uint64_t p_inl = 0, p_keep = 0;
+  auto fetch = [&](int j) {
+    p_inl = p_keep = 0;
+    if (j < end && lane < nw) {
+      p_inl = inl_bits[row0 + (int64_t)j * words + lane];
+      if (is_sp) p_keep = keep_bits[row0 + (int64_t)j * words + lane];
+    }
+  };
+  auto take = [&](int j) {
+    R.inl = p_inl;
+    R.keep = p_keep;
+    R.g_inl = inl_bits + row0 + (int64_t)j * words;
+    R.g_keep = keep_bits + row0 + (int64_t)j * words;
+  };
+  // the next model at or after j that is tested
+  int32_t g_count = 0;
+  double g_value = 0.0;
+  uint64_t g_tested = 0;
+  int g0 = -64;
+  auto next_tested = [&](int j) -> int {
+    for (; j < end; j = g0 + 64) {
+      if (j >= g0 + 64) {
+        g0 = j & ~63;
+        const bool live = g0 + lane < end;
+        const int64_t s = slot0 + g0 + lane;
+        const bool tested = live && (!is_sp || kept_count[s] >= it.best_count);
+        g_count = tested ? inl_count[s] : 0;
+        g_value = tested ? approx[s] : 0.0;
+        g_tested = ballot64(tested);
+      }
+      const uint64_t m = g_tested & (~0ull << (j - g0));
+      if (m) return g0 + __ffsll((unsigned long long)m) - 1;
+    }
+    return end;
+  };
+  int j = next_tested(0);
+  fetch(j);
+  while (j < end) {
+    take(j);
+    const int total = __builtin_amdgcn_readlane(g_count, j - g0);
+    const double v = readlane_f64(g_value, j - g0);  // the value, to the rounding of two sums of n terms
+    const int jn = next_tested(j + 1);
+    fetch(jn);
+    const int64_t start = it.pool_idx;
+    const WalkResult r = is_sp ? walk_cells<false>(R, c, n, total, nullptr) : walk_pool(R, c, uni((int)start), n, total);
+    last = j;
+    c_last = c;
+    it.last = win_base + j;
+    if (!is_sp) it.pool_idx = (int)start + r.tested >= n ? start + r.tested - n : start + r.tested;
+    it.last_start = is_sp ? -2 : start;
+    it.last_tested = is_sp ? 0 : r.tested;
+    it.last_count = r.count;
+    it.last_value = 0.0;
+    it.last_accepted = r.rejected ? 0 : 1;
+    if (!r.rejected) {
+      if (v + (1e-12 + 4e-16 * (double)n) * (1.0 + v) > it.best_value) {
+        const double* __restrict__ mp = it.models + 9 * (int64_t)it.slots[win_base + j];
+        double M[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) M[k] = mp[k];
+        const uint64_t* __restrict__ bits = R.g_inl;
+        it.last_value = ordered_value(
+            n, is_sp ? 0 : start, [&](int pos) { return (bits[pos >> 6] >> (pos & 63)) & 1ull; },
+            [&](int pos) {
+              const double* p = P + 4 * (int64_t)order[pos];
+              return it.kind == 0 ? h_sq_residual(p, M) : f_sq_sampson(p, M);
+            },
+            sq);
+        if (it.last_value > it.best_value) {
+          it.stop = win_base + j;
           break;
         }
-        lambda = lambda_new;
-      }
-    }
-    idx = (start + tested) % n;
-    it.last = s;
-    it.last_start = start;
-    it.last_tested = tested;
-    it.last_count = count;
-    it.last_value = value;
-    it.last_accepted = rejected ? 0 : 1;
-    if (!rejected) {
-      if (value > it.best_value) {
-        it.stop = s;
-        break;
       }
     } else {
-      const double de = (double)count / (double)n;
-      if (de > 0 && fabs(delta - de) / delta > 0.05) {
-        delta = de;
-        A = a_table[count];
-        f_in = delta / eps;
-        f_out = (1 - delta) / (1 - eps);
+      const double de = (double)r.count / (double)n;
+      if (de > 0 && fabs(it.delta - de) / it.delta > 0.05) {
+        it.delta = de;
+        it.A = it.a_table[r.count];
         ++it.delta_changes;
+        c = make_chain(it.eps, it.delta, it.A, n);
       }
     }
+    j = jn;
   }
-  it.pool_idx = idx;
-  it.delta = delta;
-  it.A = A;
+  if (is_sp && last >= 0) {
+    // the last tested model's inliers in test order
+    const int32_t total = inl_count[slot0 + last];
+    p_inl = p_keep = 0;
+    fetch(last);
+    take(last);
+    uint64_t* const rec = rec_bits + (int64_t)blockIdx.x * words;
+    walk_cells<true>(R, c_last, n, total, rec);
+    __syncthreads();
+    int32_t* __restrict__ list = sp_list + base;
+    int at = 0;
+    for (int w = 0; w < nw; ++w) {
+      const uint64_t m = rec[w];
+      if ((m >> lane) & 1ull) list[at + __popcll(m & ((1ull << lane) - 1ull))] = order[64 * w + lane];
+      at += __popcll(m);
+    }
+  }
+  if (lane == 0) items[blockIdx.x] = it;
 }
 
-__global__ void __launch_bounds__(64) k_sprt_walk(SprtItem* items, const double* __restrict__ pts,
-                                                  const int64_t* __restrict__ pair_pt_off,
-                                                  const int32_t* __restrict__ pair_n,
-                                                  const double* __restrict__ pair_sq_thr,
-                                                  const int32_t* __restrict__ pools,
-                                                  const SpPair* __restrict__ sp_pairs,
-                                                  const SpCell* __restrict__ sp_cells,
-                                                  const int32_t* __restrict__ sp_perm,
-                                                  const int32_t* __restrict__ sp_cell_of, int32_t* sp_list) {
-  extern __shared__ uint8_t keep[];
-  SprtItem it = items[blockIdx.x];
-  const int64_t base = pair_pt_off[it.pair];
-  const int n = pair_n[it.pair];
-  const double sq = pair_sq_thr[it.pair];
-  it.delta_changes = 0;
-  if (it.sp) {
-    const SpPair sp = sp_pairs[it.pair];
-    sprt_walk_sp(it, pts + 4 * base, sp, sp_cells + sp.cell_off, sp_perm + base, sp_cell_of + base, it.a_table, n,
-                 sq, keep, sp_list + base);
-  } else if (it.kind == 0) {
-    sprt_walk_one<0>(it, pts + 4 * base, pools + base, it.a_table, n, sq);
-  } else {
-    sprt_walk_one<1>(it, pts + 4 * base, pools + base, it.a_table, n, sq);
-  }
-  if (threadIdx.x == 0) items[blockIdx.x] = it;
+SprtPlan sprt_plan(int num_items, int max_n, int max_slots, int64_t budget_words) {
+  SprtPlan p;
+  p.words = (max_n + 63) / 64;
+  const int64_t per_slot = 2 * (int64_t)p.words * std::max(1, num_items);
+  p.max_window = (int)std::min<int64_t>(max_slots, std::max<int64_t>(8, budget_words / per_slot));
+  // inlier and kept rows of a window, the start and record rows, values, kept
+  // and inlier counts
+  p.scratch_words = (size_t)(per_slot * p.max_window) + 2 * (size_t)p.words * (size_t)num_items +
+                    2 * (size_t)p.max_window * (size_t)num_items;
+  return p;
 }
 
-void launch_sprt_walk(hipStream_t st, SprtItem* items, int num_items, const double* pts, const int64_t* pair_pt_off,
-                      const int32_t* pair_n, const double* pair_sq_thr, const int32_t* pools, const SpPair* sp_pairs,
-                      const SpCell* sp_cells, const int32_t* sp_perm, const int32_t* sp_cell_of, int32_t* sp_list,
-                      int max_cells) {
-  if (num_items <= 0) return;
-  hipLaunchKernelGGL(k_sprt_walk, dim3(num_items), dim3(64), (size_t)std::max(1, max_cells), st, items, pts,
-                     pair_pt_off, pair_n, pair_sq_thr, pools, sp_pairs, sp_cells, sp_perm, sp_cell_of, sp_list);
+void launch_sprt_walk(hipStream_t st, SprtItem* items, int num_items, int max_slots, const SprtPlan& plan,
+                      uint64_t* scratch, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
+                      const double* pair_sq_thr, const int32_t* pools, const SpPair* sp_pairs, const SpCell* sp_cells,
+                      const int32_t* sp_perm, const int32_t* sp_cell_of, int32_t* sp_list, int max_cells) {
+  if (num_items <= 0 || max_slots <= 0) return;
+  const int words = plan.words;
+  uint64_t* const start = scratch;
+  uint64_t* const rec = start + (size_t)words * num_items;
+  uint64_t* const inl = rec + (size_t)words * num_items;
+  // windows of 256 models, then twice as many each time up to the plan's: a
+  // walk often stops early (a best model found), a late one runs to the end
+  int win = std::min(256, plan.max_window);
+  for (int b = 0; b < max_slots; b += win, win = std::min(2 * win, plan.max_window)) {
+    uint64_t* const keep = inl + (size_t)words * num_items * win;
+    double* const approx = reinterpret_cast<double*>(keep + (size_t)words * num_items * win);
+    int32_t* const kept = reinterpret_cast<int32_t*>(approx + (size_t)num_items * win);
+    int32_t* const count = kept + (size_t)num_items * win;
+    const int live = std::min(win, max_slots - b);
+    hipLaunchKernelGGL(k_sprt_masks, dim3((unsigned)live * (unsigned)num_items), dim3(kMaskThreads),
+                       (size_t)std::max(1, max_cells), st, items, b, win, live, pts, pair_pt_off, pair_n, pair_sq_thr,
+                       pools, sp_pairs, sp_cells, sp_perm, sp_cell_of, words, inl, keep, start, kept, count, approx);
+    hipLaunchKernelGGL(k_sprt_walk, dim3((unsigned)num_items), dim3(64), 0, st, items, b, win, pts, pair_pt_off, pair_n,
+                       pair_sq_thr, pools, sp_perm, words, inl, keep, start, kept, count, approx, rec, sp_list);
+  }
 }
 
 }  // namespace gcr

@@ -166,12 +166,22 @@ struct SprtItem {
   int32_t sp;              // the models go through the space partitioning selector first
   int64_t best_count;      // so-far-the-best inlier number (the selector's skip rule)
 };
-// sp_list: per point of the batch, the tested inliers of the last model an
-// SP walk tested (in test order, from the pair's base)
-void launch_sprt_walk(hipStream_t st, SprtItem* items, int num_items, const double* pts, const int64_t* pair_pt_off,
-                      const int32_t* pair_n, const double* pair_sq_thr, const int32_t* pools, const SpPair* sp_pairs,
-                      const SpCell* sp_cells, const int32_t* sp_perm, const int32_t* sp_cell_of, int32_t* sp_list,
-                      int max_cells);
+// Memory plan of a walk launch: 64-bit words of a point row, models per
+// window, words of scratch.  max_n / max_slots: the largest pair and the
+// longest slot list of the items; budget_words bounds the bit rows of a window
+// (a window holds at least 8 models).
+struct SprtPlan {
+  int words, max_window;
+  size_t scratch_words;
+};
+SprtPlan sprt_plan(int num_items, int max_n, int max_slots, int64_t budget_words);
+// items come with stop = last = -1.  sp_list: per point of the batch, the
+// tested inliers of the last model an SP walk tested (in test order, from the
+// pair's base)
+void launch_sprt_walk(hipStream_t st, SprtItem* items, int num_items, int max_slots, const SprtPlan& plan,
+                      uint64_t* scratch, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
+                      const double* pair_sq_thr, const int32_t* pools, const SpPair* sp_pairs, const SpCell* sp_cells,
+                      const int32_t* sp_perm, const int32_t* sp_cell_of, int32_t* sp_list, int max_cells);
 
 // Candidate results filtered on the device (k_util.hip): per item (one
 // pair's candidates base .. base + k - 1, S slots each), the model slots

@@ -121,3 +121,36 @@ def test_batch_mixing_sprt_and_full_scoring(oracle):
     for i, ((M, mask), (rc, Mo, mo, so)) in enumerate(zip(res, refs)):
         assert stats[i]["status"] == rc, i
         _same(stats[i], so, M, Mo, mask, mo, rc, atol=1e-14)
+
+
+# Sizes at the edges of the walk's 64-position words, of the 64 words a lane
+# set holds at once (4,096 points) and of the rows kept in LDS (65,536
+# points), with and without the space partitioning cells.
+@pytest.mark.parametrize("n", [8, 63, 64, 65, 129, 4095, 4096, 4097, 65537])
+@pytest.mark.parametrize("sp,sampler", [(False, 0), (True, 1)])
+def test_homography_sprt_walk_sizes_match_oracle(oracle, n, sp, sampler):
+    import pygcransac
+    sc = synthetic.homography_scene(synthetic.scene_seed(15, 300 + n), n=n, inlier_ratio=0.6)
+    print("homography sprt walk n=%d sp=%d" % (n, sp), flush=True)
+    H, mask = pygcransac.findHomography(sc["corr"], 480, 640, 480, 640, None, threshold=3.0, conf=0.99,
+                                        spatial_coherence_weight=0.975, max_iters=1000, min_iters=50,
+                                        use_sprt=True, sampler=sampler, neighborhood=0, neighborhood_size=16.0,
+                                        use_space_partitioning=sp, lo_number=20, seed=n)
+    st = pygcransac.last_stats()
+    p = oracle.params(3.0, 0.99, 0.975, 1000, 50, sampler, 20, 16.0, n, use_sprt=True, use_space_partitioning=sp)
+    rc, Ho, mo, so = oracle.find_homography(sc["corr"], 480, 640, 480, 640, p)
+    _same(st, so, H, Ho, mask, mo, rc, atol=1e-9)
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 4097])
+def test_fundamental_sprt_walk_sizes_match_oracle(oracle, n):
+    import pygcransac
+    sc = synthetic.fundamental_scene(synthetic.scene_seed(15, 400 + n), n=n, inlier_ratio=0.6)
+    F, mask = pygcransac.findFundamentalMatrix(sc["corr"], 480, 640, 480, 640, None, threshold=1.0, conf=0.99,
+                                               spatial_coherence_weight=0.0, max_iters=2000, min_iters=50,
+                                               use_sprt=True, sampler=0, neighborhood=0, neighborhood_size=8.0,
+                                               lo_number=50, seed=n)
+    st = pygcransac.last_stats()
+    p = oracle.params(1.0, 0.99, 0.0, 2000, 50, 0, 50, 8.0, n, use_sprt=True, min_inlier_ratio_for_sprt=1e-5)
+    rc, Fo, mo, so = oracle.find_fundamental(sc["corr"], 480, 640, 480, 640, p)
+    _same(st, so, F, Fo, mask, mo, rc, atol=1e-12)
