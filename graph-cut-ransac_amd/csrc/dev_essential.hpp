@@ -74,7 +74,6 @@ constexpr MulTable make_mul_table(const MonoOrder& o) {
     for (int j = 0; j < 4; ++j) t.m21[4 * i + j] = find_code(o.d3, 20, o.d2[i] + kDeg1Code[j]);
   return t;
 }
-__constant__ MulTable kNisterMul = make_mul_table(kNisterOrder);
 __constant__ MulTable kSteweniusMul = make_mul_table(kSteweniusOrder);
 
 // out += s * (p * q), products added in (i, j) order.
@@ -190,35 +189,6 @@ __device__ inline int null_space_rx9(double* a, int r, double* basis /* (9-r) x 
     for (int s = 0; s < rank; ++s) v[col_of_row[s]] = -a[9 * s + freec[k]];
   }
   return dim;
-}
-
-__device__ inline void lu_partial_solve(double* A, double* B, int n, int m) {
-  for (int k = 0; k < n; ++k) {
-    int p = k;
-    double best = fabs(A[n * k + k]);
-    for (int i = k + 1; i < n; ++i)
-      if (fabs(A[n * i + k]) > best) {
-        best = fabs(A[n * i + k]);
-        p = i;
-      }
-    if (p != k) {
-      for (int j = 0; j < n; ++j) gswap(A[n * k + j], A[n * p + j]);
-      for (int j = 0; j < m; ++j) gswap(B[m * k + j], B[m * p + j]);
-    }
-    const double piv = A[n * k + k];
-    for (int i = k + 1; i < n; ++i) {
-      const double f = A[n * i + k] / piv;
-      A[n * i + k] = f;
-      for (int j = k + 1; j < n; ++j) A[n * i + j] = A[n * i + j] - f * A[n * k + j];
-      for (int j = 0; j < m; ++j) B[m * i + j] = B[m * i + j] - f * B[m * k + j];
-    }
-  }
-  for (int j = 0; j < m; ++j)
-    for (int i = n - 1; i >= 0; --i) {
-      double v = B[m * i + j];
-      for (int k = i + 1; k < n; ++k) v = v - A[n * i + k] * B[m * k + j];
-      B[m * i + j] = v / A[n * i + i];
-    }
 }
 
 __device__ inline void lu_full_solve(double* A, double* B, int n, int m) {
@@ -733,149 +703,125 @@ __device__ inline int motion_from_essential_dev(const double* Erm, const double*
 //
 // Monic polynomial and normalised derivative, the Sturm sequence by
 // pseudo-division with -|leading| scaling, sign changes by the three-term
-// recurrence, bisection isolation (depth <= 30, left half first: an explicit
-// stack replaces recursion), Ridders' method to width 1e-3, then up to ten
-// Newton steps (tolerance 1e-10).
-struct DevSturm10 {
+// recurrence; the caller isolates the roots by bisection (depth <= 30, left
+// half first); Ridders' method to width 1e-3, then up to ten Newton steps
+// (tolerance 1e-10).  Every index is a compile-time constant, so the
+// coefficients stay in registers.
+struct SturmSeq10 {
   static constexpr int N = 10;
-  double f[2 * N + 1];
+  double f[N + 1];  // monic, ascending
+  double d[N];      // derivative / N
   double s[3 * N];
 
-  __device__ double eval(const double* p, int deg, double x) const {
-    double v = x + p[deg - 1];
-    for (int i = deg - 2; i >= 0; --i) v = x * v + p[i];
+  template <int DEG>
+  __device__ static __forceinline__ double eval(const double* p, double x) {
+    double v = x + p[DEG - 1];
+#pragma unroll
+    for (int i = DEG - 2; i >= 0; --i) v = x * v + p[i];
     return v;
   }
 
-  __device__ void build() {
-    double buf[3 * N];
-    double* f1 = buf;
-    double* f2 = f1 + N + 1;
-    double* f3 = f2 + N;
-    for (int i = 0; i < 2 * N + 1; ++i) buf[i] = f[i];
-    for (int i = 0; i < N - 1; ++i) {
-      const double q1 = f1[N - i] * f2[N - 1 - i];
-      const double q0 = f1[N - 1 - i] * f2[N - 1 - i] - f1[N - i] * f2[N - 2 - i];
-      f3[0] = f1[0] - q0 * f2[0];
-      for (int j = 1; j < N - 1 - i; ++j) f3[j] = f1[j] - q1 * f2[j - 1] - q0 * f2[j];
-      const double c = -fabs(f3[N - 2 - i]);
-      const double ci = 1.0 / c;
-      for (int j = 0; j < N - 1 - i; ++j) f3[j] = f3[j] * ci;
-      double* t = f1;
-      f1 = f2;
-      f2 = f3;
-      f3 = t;
-      s[3 * i] = q0;
-      s[3 * i + 1] = q1;
-      s[3 * i + 2] = c;
-    }
-    s[3 * N - 3] = f1[0];
-    s[3 * N - 2] = f1[1];
-    s[3 * N - 1] = f2[0];
+  // one pseudo-division: f3 (N - 1 - I entries) from f1, f2
+  template <int I>
+  __device__ __forceinline__ void divide(const double* f1, const double* f2, double* f3) {
+    const double q1 = f1[N - I] * f2[N - 1 - I];
+    const double q0 = f1[N - 1 - I] * f2[N - 1 - I] - f1[N - I] * f2[N - 2 - I];
+    f3[0] = f1[0] - q0 * f2[0];
+#pragma unroll
+    for (int j = 1; j < N - 1 - I; ++j) f3[j] = f1[j] - q1 * f2[j - 1] - q0 * f2[j];
+    const double c = -fabs(f3[N - 2 - I]);
+    const double ci = 1.0 / c;
+#pragma unroll
+    for (int j = 0; j < N - 1 - I; ++j) f3[j] = f3[j] * ci;
+    s[3 * I] = q0;
+    s[3 * I + 1] = q1;
+    s[3 * I + 2] = c;
   }
 
-  __device__ int sign_changes(double x) const {
-    double g[N + 1];
-    g[N] = s[3 * N - 1];
-    g[N - 1] = s[3 * N - 3] + x * s[3 * N - 2];
-    for (int i = N - 2; i >= 0; --i) g[i] = (s[3 * i] + x * s[3 * i + 1]) * g[i + 1] + s[3 * i + 2] * g[i + 2];
-    int cnt = 0;
-    for (int i = 0; i < N; ++i)
-      if ((g[i] < 0) != (g[i + 1] < 0)) ++cnt;
+  // coefficients ascending (11); false when the leading one is zero
+  __device__ __forceinline__ bool init(const double* coeffs) {
+    if (coeffs[N] == 0.0) return false;
+    const double ci = 1.0 / coeffs[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) f[i] = coeffs[i] * ci;
+    f[N] = 1.0;
+#pragma unroll
+    for (int i = 0; i < N - 1; ++i) d[i] = f[i + 1] * ((i + 1) / static_cast<double>(N));
+    d[N - 1] = 1.0;
+    double f3[9], f4[8], f5[7], f6[6], f7[5], f8[4], f9[3], f10[2], f11[1];
+    divide<0>(f, d, f3);
+    divide<1>(d, f3, f4);
+    divide<2>(f3, f4, f5);
+    divide<3>(f4, f5, f6);
+    divide<4>(f5, f6, f7);
+    divide<5>(f6, f7, f8);
+    divide<6>(f7, f8, f9);
+    divide<7>(f8, f9, f10);
+    divide<8>(f9, f10, f11);
+    s[3 * N - 3] = f10[0];
+    s[3 * N - 2] = f10[1];
+    s[3 * N - 1] = f11[0];
+    return true;
+  }
+
+  // every real root lies within this distance of zero
+  __device__ __forceinline__ double root_bound() const {
+    double mx = 0.0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) mx = fmax(mx, fabs(f[i]));
+    return 1.0 + mx;
+  }
+
+  __device__ __forceinline__ int sign_changes(double x) const {
+    double g2 = s[3 * N - 1];
+    double g1 = s[3 * N - 3] + x * s[3 * N - 2];
+    int cnt = (g1 < 0) != (g2 < 0) ? 1 : 0;
+#pragma unroll
+    for (int i = N - 2; i >= 0; --i) {
+      const double g = (s[3 * i] + x * s[3 * i + 1]) * g1 + s[3 * i + 2] * g2;
+      cnt += (g < 0) != (g1 < 0) ? 1 : 0;
+      g2 = g1;
+      g1 = g;
+    }
     return cnt;
   }
 
-  __device__ void refine(double a, double b, double* roots, int& nr, double tol) const {
-    double fa = eval(f, N, a), fb = eval(f, N, b);
-    if (!((fa < 0) ^ (fb < 0))) return;
+  // the root in (a, b); false when the polynomial has the same sign at both
+  __device__ __forceinline__ bool refine(double a, double b, double tol, double& root) const {
+    double fa = eval<N>(f, a), fb = eval<N>(f, b);
+    if (!((fa < 0) ^ (fb < 0))) return false;
     for (int it = 0; it < 30; ++it) {
       if (fabs(a - b) < 1e-3) break;
       const double c = (a + b) * 0.5;
-      const double fc = eval(f, N, c);
+      const double fc = eval<N>(f, c);
       const double sq = sqrt(fc * fc - fa * fb);
       if (!sq) break;
-      const double d = (fa < fb) ? c + (a - c) * fc / sq : c + (c - a) * fc / sq;
-      const double fd = eval(f, N, d);
-      if (fd >= 0 ? (fc < 0) : (fc > 0)) {
+      const double x = (fa < fb) ? c + (a - c) * fc / sq : c + (c - a) * fc / sq;
+      const double fx = eval<N>(f, x);
+      if (fx >= 0 ? (fc < 0) : (fc > 0)) {
         a = c;
         fa = fc;
-        b = d;
-        fb = fd;
-      } else if (fd >= 0 ? (fa < 0) : (fa > 0)) {
-        b = d;
-        fb = fd;
+        b = x;
+        fb = fx;
+      } else if (fx >= 0 ? (fa < 0) : (fa > 0)) {
+        b = x;
+        fb = fx;
       } else {
-        a = d;
-        fa = fd;
+        a = x;
+        fa = fx;
       }
     }
     double x = (a + b) * 0.5;
     for (int it = 0; it < 10; ++it) {
-      const double fx = eval(f, N, x);
+      const double fx = eval<N>(f, x);
       if (fabs(fx) < tol) break;
-      const double fpx = static_cast<double>(N) * eval(f + N + 1, N - 1, x);
+      const double fpx = static_cast<double>(N) * eval<N - 1>(d, x);
       const double dx = fx / fpx;
       x = x - dx;
       if (fabs(dx) < tol) break;
     }
-    roots[nr++] = x;
-  }
-
-  // coefficients ascending (11); returns the number of roots found
-  __device__ int solve(const double* coeffs, double* roots, double tol = 1e-10) {
-    if (coeffs[N] == 0.0) return 0;
-    for (int i = 0; i <= N; ++i) f[i] = coeffs[i];
-    const double ci = 1.0 / f[N];
-    for (int i = 0; i < N; ++i) f[i] *= ci;
-    f[N] = 1.0;
-    for (int i = 0; i < N - 1; ++i) f[N + 1 + i] = f[i + 1] * ((i + 1) / static_cast<double>(N));
-    f[2 * N] = 1.0;
-    build();
-    double mx = 0.0;
-    for (int i = 0; i < N; ++i) mx = fmax(mx, fabs(f[i]));
-    const double r0 = 1.0 + mx;
-    const int sa0 = sign_changes(-r0), sb0 = sign_changes(r0);
-    if (sa0 - sb0 == 0) return 0;
-    int nr = 0;
-    // depth-first, left half first
-    // at most depth + 2 <= 32 pending intervals (one right sibling per level)
-    constexpr int kStack = 40;
-    double sta[kStack], stb[kStack];
-    int ssa[kStack], ssb[kStack], sdep[kStack];
-    int top = 0;
-    sta[0] = -r0;
-    stb[0] = r0;
-    ssa[0] = sa0;
-    ssb[0] = sb0;
-    sdep[0] = 0;
-    top = 1;
-    while (top > 0) {
-      --top;
-      const double a = sta[top], b = stb[top];
-      const int sa = ssa[top], sb = ssb[top], depth = sdep[top];
-      if (depth > 30) continue;
-      const int n = sa - sb;
-      if (n > 1 && top + 2 <= kStack) {
-        const double c = (a + b) * 0.5;
-        const int sc = sign_changes(c);
-        // push the right half, then the left half (popped first)
-        sta[top] = c;
-        stb[top] = b;
-        ssa[top] = sc;
-        ssb[top] = sb;
-        sdep[top] = depth + 1;
-        ++top;
-        sta[top] = a;
-        stb[top] = c;
-        ssa[top] = sa;
-        ssb[top] = sc;
-        sdep[top] = depth + 1;
-        ++top;
-      } else if (n == 1) {
-        refine(a, b, roots, nr, tol);
-      }
-    }
-    return nr;
+    root = x;
+    return true;
   }
 };
 

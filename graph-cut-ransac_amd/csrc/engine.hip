@@ -1530,6 +1530,7 @@ struct Workspace {
   // together): a chunk's samples and pairs; its per-slot results; the
   // scoring kernel's active-slot list, its counter and block offsets
   DevBuf<char> d_cand_in[4], d_cand_res[4], d_cand_work[4];
+  DevBuf<double> d_e5;                 // five-point solver: the matrices of a slab of samples
   DevBuf<double> d_pair_inv_scale;     // matrix-core scoring: per-pair power-of-two inverse scale
   DevBuf<MxPoint> d_mxp;               // matrix-core scoring: per-point operands and error bounds
   bool mx_on = false;                  // this run scores candidate chunks on the matrix cores
@@ -2559,8 +2560,8 @@ struct Engine : Workspace {
         prof.stop(t0);
       } else {
         const int t0 = prof.start("solve_e5", (double)tot);
-        launch_e5_solve(stream, d_rpts, d_pair_pt_off.p, d_cpair, d_samples, tot, d_cand_models,
-                        d_status, d_nmodels);
+        launch_e5_solve(stream, d_rpts, d_pair_pt_off.p, d_cpair, d_samples, tot, d_cand_models, d_status, d_nmodels,
+                        d_e5.ensure((size_t)e5_slab(tot) * kE5SlabValues));
         prof.stop(t0);
       }
       const int t1 = prof.start(kind == GCR_PROBLEM_ESSENTIAL ? "score_e" : "score_f", 0.0);
@@ -3477,7 +3478,10 @@ void solve_minimal(int kind, const double* pts, int64_t n, const int32_t* sample
     check_hip(hipMemcpyAsync(d_s.p, samples, sizeof(int32_t) * m * c, hipMemcpyHostToDevice, st), "H2D");
     check_hip(hipMemsetAsync(d_m.p, 0, sizeof(double) * 9 * S * c, st), "memset");
     if (kind == GCR_PROBLEM_FUNDAMENTAL) launch_f7_solve(st, d_p.p, d_off.p, d_cp.p, d_s.p, c, d_m.p, d_st.p, d_nm.p);
-    else launch_e5_solve(st, d_p.p, d_off.p, d_cp.p, d_s.p, c, d_m.p, d_st.p, d_nm.p);
+    DevBuf<double> d_e5;
+    if (kind == GCR_PROBLEM_ESSENTIAL)
+      launch_e5_solve(st, d_p.p, d_off.p, d_cp.p, d_s.p, c, d_m.p, d_st.p, d_nm.p,
+                      d_e5.ensure((size_t)e5_slab(c) * kE5SlabValues));
     std::vector<int8_t> s8((size_t)c * S);
     check_hip(hipMemcpyAsync(models, d_m.p, sizeof(double) * 9 * S * c, hipMemcpyDeviceToHost, st), "D2H");
     check_hip(hipMemcpyAsync(s8.data(), d_st.p, (size_t)c * S, hipMemcpyDeviceToHost, st), "D2H");

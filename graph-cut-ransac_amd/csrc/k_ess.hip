@@ -1,11 +1,6 @@
-// Essential-matrix kernels: the five-point minimal solver (one thread per
-// candidate sample), the Stewenius non-minimal fit (one wavefront per fit)
-// and the driver's pose bundle adjustment (one wavefront per pair).
-//
-// Minimal: EssentialMatrixEstimator::estimateModel
-// (essential_estimator.h:152-175) -> EssentialMatrixFivePointNisterSolver
-// (solver_essential_matrix_five_point_nister.h:204-615) on K-normalised
-// coordinates, then the oriented epipolar filter (essential_estimator.h:338-398).
+// Essential-matrix kernels: the Stewenius non-minimal fit (one wavefront per
+// fit) and the driver's pose bundle adjustment (one wavefront per pair).  The
+// five-point minimal solver is in k_e5.hip.
 //
 // Non-minimal: estimateModelNonminimal (essential_estimator.h:308-335) ->
 // EssentialMatrixFivePointSteweniusSolver (…stewenius.h:114-231), then
@@ -24,142 +19,6 @@
 #include "kernels.hpp"
 
 namespace gcr {
-
-// ---------------------------------------------------------------------------
-// Five-point minimal solver
-// ---------------------------------------------------------------------------
-// Up to 10 models of one sample (row-major 3x3 each, in root order); returns
-// their number.
-__device__ int nister_solve_thread(const double* P, const int32_t* s, double* models) {
-  double a[45];
-  for (int i = 0; i < 5; ++i) e_row(P + 4 * (int64_t)s[i], 1.0, a + 9 * i);
-  double N[36];
-  if (null_space_rx9(a, 5, N) != 4) return 0;
-  double ee[3][3][4];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j)
-      for (int k = 0; k < 4; ++k) ee[i][j][k] = N[9 * k + 3 * j + i];
-  double C[200];
-  essential_constraints(ee, kNisterMul, 1.0, C);
-  double L[100], B[100];
-  for (int r = 0; r < 10; ++r)
-    for (int c = 0; c < 10; ++c) {
-      L[10 * r + c] = C[20 * r + c];
-      B[10 * r + c] = C[20 * r + 10 + c];
-    }
-  lu_partial_solve(L, B, 10, 10);
-  double A[3][13];
-  for (int i = 0; i < 3; ++i) {
-    const double* r1 = B + 10 * (4 + 2 * i);
-    const double* r2 = B + 10 * (5 + 2 * i);
-    A[i][0] = 0.0;
-    for (int c = 0; c < 3; ++c) A[i][1 + c] = r1[c];
-    for (int c = 0; c < 3; ++c) A[i][c] = A[i][c] - r2[c];
-    A[i][4] = 0.0;
-    for (int c = 0; c < 3; ++c) A[i][5 + c] = r1[3 + c];
-    for (int c = 0; c < 3; ++c) A[i][4 + c] = A[i][4 + c] - r2[3 + c];
-    A[i][8] = 0.0;
-    for (int c = 0; c < 4; ++c) A[i][9 + c] = r1[6 + c];
-    for (int c = 0; c < 4; ++c) A[i][8 + c] = A[i][8 + c] - r2[6 + c];
-  }
-  double Pp[3][4], Qp[3][4], Rp[3][5];
-  for (int i = 0; i < 3; ++i) {
-    for (int d = 0; d < 4; ++d) {
-      Pp[i][d] = A[i][3 - d];
-      Qp[i][d] = A[i][7 - d];
-    }
-    for (int d = 0; d < 5; ++d) Rp[i][d] = A[i][12 - d];
-  }
-  auto mul = [](const double* u, int du, const double* v, int dv, double* out) {
-    for (int k = 0; k <= du + dv; ++k) out[k] = 0.0;
-    for (int i = 0; i <= du; ++i)
-      for (int j = 0; j <= dv; ++j) out[i + j] = out[i + j] + u[i] * v[j];
-  };
-  double c[11];
-  for (int k = 0; k < 11; ++k) c[k] = 0.0;
-  {
-    double t1[8], t2[8], m7[8], full[11];
-    mul(Qp[1], 3, Rp[2], 4, t1);
-    mul(Qp[2], 3, Rp[1], 4, t2);
-    for (int k = 0; k < 8; ++k) m7[k] = t1[k] - t2[k];
-    mul(Pp[0], 3, m7, 7, full);
-    for (int k = 0; k < 11; ++k) c[k] = c[k] + full[k];
-    mul(Pp[1], 3, Rp[2], 4, t1);
-    mul(Pp[2], 3, Rp[1], 4, t2);
-    for (int k = 0; k < 8; ++k) m7[k] = t1[k] - t2[k];
-    mul(Qp[0], 3, m7, 7, full);
-    for (int k = 0; k < 11; ++k) c[k] = c[k] - full[k];
-    double s1[7], s2[7], m6[7];
-    mul(Pp[1], 3, Qp[2], 3, s1);
-    mul(Pp[2], 3, Qp[1], 3, s2);
-    for (int k = 0; k < 7; ++k) m6[k] = s1[k] - s2[k];
-    mul(Rp[0], 4, m6, 6, full);
-    for (int k = 0; k < 11; ++k) c[k] = c[k] + full[k];
-  }
-  double roots[10];
-  DevSturm10 st;
-  const int nr = st.solve(c, roots);
-  for (int q = 0; q < nr; ++q) {
-    const double z = roots[q];
-    const double z2 = z * z, z3 = z2 * z, z4 = z2 * z2;
-    double b0[3], b1[3], bb[3];
-    for (int i = 0; i < 3; ++i) {
-      b0[i] = A[i][0] * z3 + A[i][1] * z2 + A[i][2] * z + A[i][3];
-      b1[i] = A[i][4] * z3 + A[i][5] * z2 + A[i][6] * z + A[i][7];
-      bb[i] = A[i][8] * z4 + A[i][9] * z3 + A[i][10] * z2 + A[i][11] * z + A[i][12];
-    }
-    const double det = b0[0] * b1[1] - b1[0] * b0[1];
-    const double id = 1.0 / det;
-    double xz[2];
-    xz[0] = (b1[1] * id) * bb[0] + (-b1[0] * id) * bb[1];
-    xz[1] = (-b0[1] * id) * bb[0] + (b0[0] * id) * bb[1];
-    if (fabs(b0[2] * xz[0] + b1[2] * xz[1] - bb[2]) > 1e-6) solve3x2_fullpiv(b0, b1, bb, xz);
-    const double x = -xz[0], y = -xz[1];
-    double e[9];
-    const double sc = 1.0 / sqrt(x * x + y * y + z * z + 1.0);
-    for (int k = 0; k < 9; ++k) e[k] = (N[k] * x + N[9 + k] * y + N[18 + k] * z + N[27 + k]) * sc;
-    double* m = models + 9 * q;
-    for (int r = 0; r < 3; ++r)
-      for (int cc = 0; cc < 3; ++cc) m[3 * r + cc] = e[3 * cc + r];
-  }
-  return nr;
-}
-
-// One thread per candidate; 10 model slots per candidate (status 2 = kept,
-// compacted in root order after the oriented filter).
-__global__ void __launch_bounds__(64) k_e5_solve(const double* __restrict__ pts, const int64_t* __restrict__ pair_pt_off,
-                                                 const int32_t* __restrict__ cand_pair,
-                                                 const int32_t* __restrict__ samples, int64_t num_cand,
-                                                 double* __restrict__ models, int8_t* __restrict__ mstatus,
-                                                 int8_t* __restrict__ nmodels) {
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= num_cand) return;
-  const double* P = pts + 4 * pair_pt_off[cand_pair[c]];
-  const int32_t* s = samples + 5 * c;
-  double* out = models + 90 * c;
-  int kept = 0;
-  if (s[0] >= 0) {
-    const int nr = nister_solve_thread(P, s, out);
-    for (int q = 0; q < nr; ++q) {
-      const double* m = out + 9 * q;
-      if (f_orientation_valid_idx(m, P, s, 5)) {
-        if (kept != q)
-          for (int i = 0; i < 9; ++i) out[9 * kept + i] = m[i];
-        ++kept;
-      }
-    }
-  }
-  for (int k = 0; k < 10; ++k) mstatus[10 * c + k] = k < kept ? 2 : 0;
-  nmodels[c] = (int8_t)kept;
-}
-
-void launch_e5_solve(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* cand_pair,
-                     const int32_t* samples, int64_t num_cand, double* models, int8_t* mstatus, int8_t* nmodels) {
-  if (num_cand <= 0) return;
-  const int64_t grid = (num_cand + 63) / 64;
-  hipLaunchKernelGGL(k_e5_solve, dim3((unsigned)grid), dim3(64), 0, st, pts, pair_pt_off, cand_pair, samples,
-                     num_cand, models, mstatus, nmodels);
-}
 
 // ---------------------------------------------------------------------------
 // Non-minimal fit and bundle adjustment (one wave each)

@@ -246,9 +246,15 @@ void launch_irls_weights(hipStream_t st, int kind, const double* pts, const int6
                          const int32_t* inliers, const int64_t* inl_off, const int32_t* inl_n, double* weights,
                          int num_items, int zero, int max_n);
 
-// essential matrices (k_ess.hip)
+// essential matrices (k_e5.hip, k_ess.hip).  The five-point solver takes the
+// candidates in slabs of at most kE5SlabMax (enough waves to fill the chip);
+// scratch: e5_slab(num_cand) x kE5SlabValues doubles.
+constexpr int64_t kE5SlabMax = 131072;
+constexpr int kE5SlabValues = 296;
+int64_t e5_slab(int64_t num_cand);
 void launch_e5_solve(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* cand_pair,
-                     const int32_t* samples, int64_t num_cand, double* models, int8_t* mstatus, int8_t* nmodels);
+                     const int32_t* samples, int64_t num_cand, double* models, int8_t* mstatus, int8_t* nmodels,
+                     double* scratch);
 void launch_fit_e(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* fit_pair,
                   const int64_t* fit_sample_off, const int32_t* fit_ns, const int32_t* samples, const double* weights,
                   const int64_t* weight_off, int weight_mode, double* scratch, const int64_t* scratch_off,
