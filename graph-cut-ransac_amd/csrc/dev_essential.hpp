@@ -1,11 +1,9 @@
 // Device numerics of the essential-matrix path (gfx950).
 //
-// Thread-level routines (one thread runs each call): the five-point solver
-// (Nister: null space, trace and determinant constraints, elimination,
-// degree-10 polynomial, Sturm-sequence roots, back-substitution), the dense
-// steps of the Stewenius non-minimal solver (column-pivoted QR, Gauss-Jordan,
-// real Schur eigenvalues, null vectors) and the relative-pose helpers of the
-// bundle adjustment.  They use only +, -, *, / and sqrt in a fixed order and
+// Thread-level routines (one thread runs each call): the monomial tables of
+// both solvers, the five-point null space, the Sturm-sequence roots of the
+// degree-10 polynomial and the relative-pose helpers of the bundle adjustment.
+// They use only +, -, *, / and sqrt in a fixed order and
 // are compiled without fused multiply-add, so results are reproducible
 // bit for bit by a sequential host restatement of the same steps.
 //
@@ -74,54 +72,6 @@ constexpr MulTable make_mul_table(const MonoOrder& o) {
     for (int j = 0; j < 4; ++j) t.m21[4 * i + j] = find_code(o.d3, 20, o.d2[i] + kDeg1Code[j]);
   return t;
 }
-__constant__ MulTable kSteweniusMul = make_mul_table(kSteweniusOrder);
-
-// out += s * (p * q), products added in (i, j) order.
-__device__ inline void mul11_acc(const MulTable& t, const double* p, const double* q, double s, double* out) {
-  for (int i = 0; i < 4; ++i)
-    for (int j = 0; j < 4; ++j) {
-      const int k = t.m11[4 * i + j];
-      out[k] = out[k] + s * (p[i] * q[j]);
-    }
-}
-__device__ inline void mul21_acc(const MulTable& t, const double* p, const double* q, double s, double* out) {
-  for (int i = 0; i < 10; ++i)
-    for (int j = 0; j < 4; ++j) {
-      const int k = t.m21[4 * i + j];
-      out[k] = out[k] + s * (p[i] * q[j]);
-    }
-}
-
-// Cubic constraints on E = x N0 + y N1 + z N2 + N3 (ee[i][j]: coefficients
-// of E(i, j)): rows 3 i + j = entry (i, j) of eet_scale E E^T E -
-// 0.5 tr(eet_scale E E^T) E, row 9 = det E along the third row; C is 10 x 20.
-__device__ inline void essential_constraints(const double (*ee)[3][4], const MulTable& t, double eet_scale,
-                                             double* C) {
-  for (int i = 0; i < 200; ++i) C[i] = 0.0;
-  const int cof[3][4] = {{0, 1, 1, 2}, {0, 2, 1, 0}, {0, 0, 1, 1}};
-  const int cofn[3][4] = {{0, 2, 1, 1}, {0, 0, 1, 2}, {0, 1, 1, 0}};
-  for (int k = 0; k < 3; ++k) {
-    double d[10];
-    for (int i = 0; i < 10; ++i) d[i] = 0.0;
-    mul11_acc(t, ee[cof[k][0]][cof[k][1]], ee[cof[k][2]][cof[k][3]], 1.0, d);
-    mul11_acc(t, ee[cofn[k][0]][cofn[k][1]], ee[cofn[k][2]][cofn[k][3]], -1.0, d);
-    mul21_acc(t, d, ee[2][k], 1.0, C + 20 * 9);
-  }
-  double eet[3][3][10];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) {
-      for (int k = 0; k < 10; ++k) eet[i][j][k] = 0.0;
-      for (int k = 0; k < 3; ++k) mul11_acc(t, ee[i][k], ee[j][k], eet_scale, eet[i][j]);
-    }
-  double tr[10];
-  for (int k = 0; k < 10; ++k) tr[k] = eet[0][0][k] + eet[1][1][k] + eet[2][2][k];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) {
-      double* row = C + 20 * (3 * i + j);
-      for (int k = 0; k < 3; ++k) mul21_acc(t, eet[i][k], ee[k][j], 1.0, row);
-      mul21_acc(t, tr, ee[i][j], -0.5, row);
-    }
-}
 
 // Coefficient row of one correspondence for vec(E) stacked column by column:
 // row . vec(E) = x2^T E x1.
@@ -139,267 +89,89 @@ __device__ __forceinline__ void e_row(const double* p, double w, double* r) {
   r[8] = w;
 }
 
+// Null space of the 5 x 9 coefficient matrix: N[9 k + j], k < 4.  False when
+// the rank is below 5.
+__device__ __forceinline__ bool null_space_5x9(double (&a)[5][9], double* N) {
+  uint32_t used = 0, row_of_col = 0;  // 3 bits per pivot column: its row
+  double max_pivot = 0.0;
+  bool ok = true;
+#pragma unroll
+  for (int r = 0; r < 5; ++r) {
+    double best = 0.0;
+    int pr = -1, pc = -1;
+#pragma unroll
+    for (int i = r; i < 5; ++i)
+#pragma unroll
+      for (int j = 0; j < 9; ++j) {
+        const double v = fabs(a[i][j]);
+        const bool take = !((used >> j) & 1u) && v > best;
+        best = take ? v : best;
+        pr = take ? i : pr;
+        pc = take ? j : pc;
+      }
+    if (r == 0) max_pivot = best;
+    if (pr < 0 || best <= 5.0 * 2.220446049250313e-16 * max_pivot) ok = false;
+    if (!ok) continue;
+#pragma unroll
+    for (int i = r + 1; i < 5; ++i) {
+      const bool sw = i == pr;
+#pragma unroll
+      for (int j = 0; j < 9; ++j) {
+        const double t = a[r][j];
+        a[r][j] = sw ? a[i][j] : t;
+        a[i][j] = sw ? t : a[i][j];
+      }
+    }
+    double piv = a[r][0];
+#pragma unroll
+    for (int j = 1; j < 9; ++j) piv = j == pc ? a[r][j] : piv;
+#pragma unroll
+    for (int j = 0; j < 9; ++j) a[r][j] = a[r][j] / piv;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      if (i == r) continue;
+      double f = a[i][0];
+#pragma unroll
+      for (int j = 1; j < 9; ++j) f = j == pc ? a[i][j] : f;
+      const bool upd = f != 0.0;
+#pragma unroll
+      for (int j = 0; j < 9; ++j) a[i][j] = upd ? a[i][j] - f * a[r][j] : a[i][j];
+    }
+    used |= 1u << pc;
+    row_of_col |= (uint32_t)r << (3 * pc);
+  }
+  if (!ok) return false;
+  uint32_t freem = ~used & 0x1ffu;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int fc = __builtin_ctz(freem);
+    freem &= freem - 1u;
+    double v[5];
+#pragma unroll
+    for (int r = 0; r < 5; ++r) {
+      double x = a[r][0];
+#pragma unroll
+      for (int j = 1; j < 9; ++j) x = j == fc ? a[r][j] : x;
+      v[r] = -x;
+    }
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+      const int r = (int)((row_of_col >> (3 * j)) & 7u);
+      double x = v[0];
+#pragma unroll
+      for (int i = 1; i < 5; ++i) x = i == r ? v[i] : x;
+      N[9 * k + j] = ((used >> j) & 1u) ? x : (j == fc ? 1.0 : 0.0);
+    }
+  }
+  return true;
+}
+
 struct RelPose {
   double q[4];  // unit quaternion (w, x, y, z)
   double t[3];
 };
 
 __device__ inline double dot3(const double* a, const double* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
-
-__device__ inline int null_space_rx9(double* a, int r, double* basis /* (9-r) x 9 */) {
-  int col_of_row[9];
-  int used[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  int rank = 0;
-  double maxp = 0.0;
-  for (int s = 0; s < r; ++s) {
-    int pr = -1, pc = -1;
-    double best = 0.0;
-    for (int i = s; i < r; ++i)
-      for (int j = 0; j < 9; ++j)
-        if (!used[j] && fabs(a[9 * i + j]) > best) {
-          best = fabs(a[9 * i + j]);
-          pr = i;
-          pc = j;
-        }
-    if (s == 0) maxp = best;
-    if (pr < 0 || best <= (double)r * 2.220446049250313e-16 * maxp) break;
-    if (pr != s)
-      for (int j = 0; j < 9; ++j) gswap(a[9 * s + j], a[9 * pr + j]);
-    const double piv = a[9 * s + pc];
-    for (int j = 0; j < 9; ++j) a[9 * s + j] = a[9 * s + j] / piv;
-    for (int i = 0; i < r; ++i) {
-      if (i == s) continue;
-      const double f = a[9 * i + pc];
-      if (f != 0.0)
-        for (int j = 0; j < 9; ++j) a[9 * i + j] = a[9 * i + j] - f * a[9 * s + j];
-    }
-    used[pc] = 1;
-    col_of_row[s] = pc;
-    ++rank;
-  }
-  const int dim = 9 - rank;
-  if (dim != 9 - r) return dim;
-  int freec[9], nf = 0;
-  for (int j = 0; j < 9; ++j)
-    if (!used[j]) freec[nf++] = j;
-  for (int k = 0; k < nf; ++k) {
-    double* v = basis + 9 * k;
-    for (int j = 0; j < 9; ++j) v[j] = 0.0;
-    v[freec[k]] = 1.0;
-    for (int s = 0; s < rank; ++s) v[col_of_row[s]] = -a[9 * s + freec[k]];
-  }
-  return dim;
-}
-
-__device__ inline void lu_full_solve(double* A, double* B, int n, int m) {
-  int colp[16];
-  for (int j = 0; j < n; ++j) colp[j] = j;
-  for (int k = 0; k < n; ++k) {
-    int pr = k, pc = k;
-    double best = -1.0;
-    for (int i = k; i < n; ++i)
-      for (int j = k; j < n; ++j)
-        if (fabs(A[n * i + j]) > best) {
-          best = fabs(A[n * i + j]);
-          pr = i;
-          pc = j;
-        }
-    if (pr != k) {
-      for (int j = 0; j < n; ++j) gswap(A[n * k + j], A[n * pr + j]);
-      for (int j = 0; j < m; ++j) gswap(B[m * k + j], B[m * pr + j]);
-    }
-    if (pc != k) {
-      for (int i = 0; i < n; ++i) gswap(A[n * i + k], A[n * i + pc]);
-      gswap(colp[k], colp[pc]);
-    }
-    const double piv = A[n * k + k];
-    for (int i = k + 1; i < n; ++i) {
-      const double f = A[n * i + k] / piv;
-      for (int j = k + 1; j < n; ++j) A[n * i + j] = A[n * i + j] - f * A[n * k + j];
-      for (int j = 0; j < m; ++j) B[m * i + j] = B[m * i + j] - f * B[m * k + j];
-    }
-  }
-  double X[16 * 16];
-  for (int j = 0; j < m; ++j)
-    for (int i = n - 1; i >= 0; --i) {
-      double v = B[m * i + j];
-      for (int k = i + 1; k < n; ++k) v = v - A[n * i + k] * X[m * k + j];
-      X[m * i + j] = v / A[n * i + i];
-    }
-  for (int i = 0; i < n; ++i)
-    for (int j = 0; j < m; ++j) B[m * colp[i] + j] = X[m * i + j];
-}
-
-// Real eigenvalues of a real n x n matrix (n <= 10): Householder reduction to
-// Hessenberg form, then Francis double-shift QR steps -- the published
-// "hqr" method (Martin, Peters and Wilkinson, "The QR algorithm for real
-// Hessenberg matrices", Numer. Math. 14, 1970), written here.
-__device__ inline int real_eigenvalues(const double* M, int n, double* ev) {
-  int pos[10];
-  double a[10][10];
-  for (int i = 0; i < n; ++i)
-    for (int j = 0; j < n; ++j) a[i][j] = M[n * i + j];
-  // Hessenberg reduction
-  for (int k = 0; k < n - 2; ++k) {
-    double sigma = 0.0;
-    for (int i = k + 2; i < n; ++i) sigma += a[i][k] * a[i][k];
-    if (sigma == 0.0) continue;
-    const double alpha = a[k + 1][k];
-    const double nrm = sqrt(alpha * alpha + sigma);
-    const double beta = alpha >= 0.0 ? -nrm : nrm;
-    double v[10];
-    v[k + 1] = alpha - beta;
-    for (int i = k + 2; i < n; ++i) v[i] = a[i][k];
-    double vv = 0.0;
-    for (int i = k + 1; i < n; ++i) vv += v[i] * v[i];
-    // A <- (I - 2 v v^T / vv) A (I - 2 v v^T / vv)
-    for (int j = 0; j < n; ++j) {
-      double s = 0.0;
-      for (int i = k + 1; i < n; ++i) s += v[i] * a[i][j];
-      s = 2.0 * s / vv;
-      for (int i = k + 1; i < n; ++i) a[i][j] -= s * v[i];
-    }
-    for (int i = 0; i < n; ++i) {
-      double s = 0.0;
-      for (int j = k + 1; j < n; ++j) s += a[i][j] * v[j];
-      s = 2.0 * s / vv;
-      for (int j = k + 1; j < n; ++j) a[i][j] -= s * v[j];
-    }
-    for (int i = k + 2; i < n; ++i) a[i][k] = 0.0;
-  }
-  // shifted QR (hqr)
-  int nr = 0;
-  int nn = n - 1;
-  double t = 0.0;
-  double anorm = 0.0;
-  for (int i = 0; i < n; ++i)
-    for (int j = (i - 1 > 0 ? i - 1 : 0); j < n; ++j) anorm += fabs(a[i][j]);
-  int its = 0;
-  const double eps = 2.220446049250313e-16;
-  while (nn >= 0) {
-    int l;
-    for (l = nn; l >= 1; --l) {
-      const double s = fabs(a[l - 1][l - 1]) + fabs(a[l][l]);
-      const double sc = s == 0.0 ? anorm : s;
-      if (fabs(a[l][l - 1]) <= eps * sc) {
-        a[l][l - 1] = 0.0;
-        break;
-      }
-    }
-    const double x = a[nn][nn];
-    if (l == nn) {  // one root
-      pos[nr] = nn;
-      ev[nr++] = x + t;
-      --nn;
-      its = 0;
-      continue;
-    }
-    const double y = a[nn - 1][nn - 1];
-    const double w = a[nn][nn - 1] * a[nn - 1][nn];
-    if (l == nn - 1) {  // two roots
-      const double p = 0.5 * (y - x);
-      const double q = p * p + w;
-      const double z = sqrt(fabs(q));
-      const double xx = x + t;
-      if (q >= 0.0) {
-        const double zz = p + (p >= 0.0 ? fabs(z) : -fabs(z));
-        const double r1 = xx + zz;
-        const double r2 = zz != 0.0 ? xx - w / zz : xx + zz;
-        pos[nr] = nn - 1;
-        ev[nr++] = r1;
-        pos[nr] = nn;
-        ev[nr++] = r2;
-      }
-      nn -= 2;
-      its = 0;
-      continue;
-    }
-    if (its == 30 * n) return -1;  // no convergence
-    double xs = x, ys = y, ws = w;
-    if (its == 10 || its == 20) {  // exceptional shift
-      t += x;
-      for (int i = 0; i <= nn; ++i) a[i][i] -= x;
-      const double s = fabs(a[nn][nn - 1]) + fabs(a[nn - 1][nn - 2]);
-      xs = ys = 0.75 * s;
-      ws = -0.4375 * s * s;
-    }
-    ++its;
-    int m;
-    double p = 0, q = 0, r = 0, z;
-    for (m = nn - 2; m >= l; --m) {
-      z = a[m][m];
-      const double rr = xs - z, ss = ys - z;
-      p = (rr * ss - ws) / a[m + 1][m] + a[m][m + 1];
-      q = a[m + 1][m + 1] - z - rr - ss;
-      r = a[m + 2][m + 1];
-      const double s = fabs(p) + fabs(q) + fabs(r);
-      p /= s;
-      q /= s;
-      r /= s;
-      if (m == l) break;
-      const double u = fabs(a[m][m - 1]) * (fabs(q) + fabs(r));
-      const double v = fabs(p) * (fabs(a[m - 1][m - 1]) + fabs(z) + fabs(a[m + 1][m + 1]));
-      if (u <= eps * v) break;
-    }
-    for (int i = m + 2; i <= nn; ++i) {
-      a[i][i - 2] = 0.0;
-      if (i != m + 2) a[i][i - 3] = 0.0;
-    }
-    for (int k = m; k <= nn - 1; ++k) {
-      double xx = 0.0;
-      if (k != m) {
-        p = a[k][k - 1];
-        q = a[k + 1][k - 1];
-        r = 0.0;
-        if (k != nn - 1) r = a[k + 2][k - 1];
-        xx = fabs(p) + fabs(q) + fabs(r);
-        if (xx != 0.0) {
-          p /= xx;
-          q /= xx;
-          r /= xx;
-        }
-      }
-      const double sq = sqrt(p * p + q * q + r * r);
-      const double s = p >= 0.0 ? sq : -sq;
-      if (s != 0.0) {
-        if (k == m) {
-          if (l != m) a[k][k - 1] = -a[k][k - 1];
-        } else
-          a[k][k - 1] = -s * xx;
-        p += s;
-        const double xr = p / s, yr = q / s, zr = r / s;
-        q /= p;
-        r /= p;
-        for (int j = k; j <= nn; ++j) {
-          double pp = a[k][j] + q * a[k + 1][j];
-          if (k != nn - 1) {
-            pp += r * a[k + 2][j];
-            a[k + 2][j] -= pp * zr;
-          }
-          a[k + 1][j] -= pp * yr;
-          a[k][j] -= pp * xr;
-        }
-        const int mmin = nn < k + 3 ? nn : k + 3;
-        for (int i = l; i <= mmin; ++i) {
-          double pp = xr * a[i][k] + yr * a[i][k + 1];
-          if (k != nn - 1) {
-            pp += zr * a[i][k + 2];
-            a[i][k + 2] -= pp * r;
-          }
-          a[i][k + 1] -= pp * q;
-          a[i][k] -= pp;
-        }
-      }
-    }
-  }
-  // report in diagonal order (top to bottom), as the real Schur form lists them
-  for (int a1 = 1; a1 < nr; ++a1)
-    for (int b1 = a1; b1 > 0 && pos[b1 - 1] > pos[b1]; --b1) {
-      gswap(pos[b1 - 1], pos[b1]);
-      gswap(ev[b1 - 1], ev[b1]);
-    }
-  return nr;
-}
 
 __device__ inline void solve3x2_fullpiv(const double* b0, const double* b1, const double* rhs, double* xz) {
   double a[3][2] = {{b0[0], b1[0]}, {b0[1], b1[1]}, {b0[2], b1[2]}};
@@ -442,48 +214,6 @@ __device__ inline void solve3x2_fullpiv(const double* b0, const double* b1, cons
   }
   xz[col[0]] = z[0];
   xz[col[1]] = z[1];
-}
-
-__device__ inline void null_vector_fullpiv(double* A, int n, double* v) {
-  int col[16];
-  for (int j = 0; j < n; ++j) col[j] = j;
-  int rank = 0;
-  double first = 0.0;
-  for (int k = 0; k < n; ++k) {
-    int pr = k, pc = k;
-    double best = -1.0;
-    for (int i = k; i < n; ++i)
-      for (int j = k; j < n; ++j)
-        if (fabs(A[n * i + j]) > best) {
-          best = fabs(A[n * i + j]);
-          pr = i;
-          pc = j;
-        }
-    if (k == 0) first = best;
-    if (best <= (double)n * 2.220446049250313e-16 * first || best == 0.0) break;
-    if (pr != k)
-      for (int j = 0; j < n; ++j) gswap(A[n * k + j], A[n * pr + j]);
-    if (pc != k) {
-      for (int i = 0; i < n; ++i) gswap(A[n * i + k], A[n * i + pc]);
-      gswap(col[k], col[pc]);
-    }
-    for (int i = k + 1; i < n; ++i) {
-      const double f = A[n * i + k] / A[n * k + k];
-      for (int j = k + 1; j < n; ++j) A[n * i + j] = A[n * i + j] - f * A[n * k + j];
-      A[n * i + k] = 0.0;
-    }
-    ++rank;
-  }
-  double z[16];
-  for (int j = 0; j < n; ++j) z[j] = 0.0;
-  const int fr = rank < n ? rank : n - 1;  // the free unknown (in pivoted order)
-  z[fr] = 1.0;
-  for (int k = fr - 1; k >= 0; --k) {
-    double s = 0.0;
-    for (int j = k + 1; j <= fr; ++j) s = s + A[n * k + j] * z[j];
-    z[k] = -s / A[n * k + k];
-  }
-  for (int j = 0; j < n; ++j) v[col[j]] = z[j];
 }
 
 __device__ inline void frobenius_normalise_sign(double* m) {

@@ -58,83 +58,6 @@ __device__ __forceinline__ void mul21(const double* p, const double* q, double s
     for (int j = 0; j < 4; ++j) out[kMul.m21[4 * i + j]] = out[kMul.m21[4 * i + j]] + s * (p[i] * q[j]);
 }
 
-// Null space of the 5 x 9 coefficient matrix: N[9 k + j], k < 4.  False when
-// the rank is below 5.
-__device__ __forceinline__ bool null_space_5x9(double (&a)[5][9], double* N) {
-  uint32_t used = 0, row_of_col = 0;  // 3 bits per pivot column: its row
-  double max_pivot = 0.0;
-  bool ok = true;
-#pragma unroll
-  for (int r = 0; r < 5; ++r) {
-    double best = 0.0;
-    int pr = -1, pc = -1;
-#pragma unroll
-    for (int i = r; i < 5; ++i)
-#pragma unroll
-      for (int j = 0; j < 9; ++j) {
-        const double v = fabs(a[i][j]);
-        const bool take = !((used >> j) & 1u) && v > best;
-        best = take ? v : best;
-        pr = take ? i : pr;
-        pc = take ? j : pc;
-      }
-    if (r == 0) max_pivot = best;
-    if (pr < 0 || best <= 5.0 * 2.220446049250313e-16 * max_pivot) ok = false;
-    if (!ok) continue;
-#pragma unroll
-    for (int i = r + 1; i < 5; ++i) {
-      const bool sw = i == pr;
-#pragma unroll
-      for (int j = 0; j < 9; ++j) {
-        const double t = a[r][j];
-        a[r][j] = sw ? a[i][j] : t;
-        a[i][j] = sw ? t : a[i][j];
-      }
-    }
-    double piv = a[r][0];
-#pragma unroll
-    for (int j = 1; j < 9; ++j) piv = j == pc ? a[r][j] : piv;
-#pragma unroll
-    for (int j = 0; j < 9; ++j) a[r][j] = a[r][j] / piv;
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      if (i == r) continue;
-      double f = a[i][0];
-#pragma unroll
-      for (int j = 1; j < 9; ++j) f = j == pc ? a[i][j] : f;
-      const bool upd = f != 0.0;
-#pragma unroll
-      for (int j = 0; j < 9; ++j) a[i][j] = upd ? a[i][j] - f * a[r][j] : a[i][j];
-    }
-    used |= 1u << pc;
-    row_of_col |= (uint32_t)r << (3 * pc);
-  }
-  if (!ok) return false;
-  uint32_t freem = ~used & 0x1ffu;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int fc = __builtin_ctz(freem);
-    freem &= freem - 1u;
-    double v[5];
-#pragma unroll
-    for (int r = 0; r < 5; ++r) {
-      double x = a[r][0];
-#pragma unroll
-      for (int j = 1; j < 9; ++j) x = j == fc ? a[r][j] : x;
-      v[r] = -x;
-    }
-#pragma unroll
-    for (int j = 0; j < 9; ++j) {
-      const int r = (int)((row_of_col >> (3 * j)) & 7u);
-      double x = v[0];
-#pragma unroll
-      for (int i = 1; i < 5; ++i) x = i == r ? v[i] : x;
-      N[9 * k + j] = ((used >> j) & 1u) ? x : (j == fc ? 1.0 : 0.0);
-    }
-  }
-  return true;
-}
-
 }  // namespace
 
 // Slab layout (doubles): value v of the slab's sample t is at

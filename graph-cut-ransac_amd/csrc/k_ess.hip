@@ -12,10 +12,11 @@
 // refine_relpose / lm_5dof_impl (bundle.cpp:176-251,412-452) with the
 // truncated loss, essential_from_motion.
 //
-// Sums over points use the fixed 64-lane order of wave_sum64; the small
-// dense steps run on lane 0 (their state in LDS) so every lane sees the same
-// values after a barrier.
+// Sums over points use the fixed 64-lane order of wave_sum64; the solver's
+// dense steps are spread over the wave (dev_stewenius.hpp), the adjustment's
+// 5 x 5 steps run on lane 0 (their state in LDS).
 #include "dev_essential.hpp"
+#include "dev_stewenius.hpp"
 #include "kernels.hpp"
 
 namespace gcr {
@@ -23,74 +24,13 @@ namespace gcr {
 // ---------------------------------------------------------------------------
 // Non-minimal fit and bundle adjustment (one wave each)
 // ---------------------------------------------------------------------------
-// sum64 order on one lane: partial i & 63 per term, then the 64-lane tree.
-template <class F>
-__device__ double lane_sum64(int begin, int end, F term) {
-  double p[64];
-  for (int l = 0; l < 64; ++l) p[l] = 0.0;
-  for (int i = begin; i < end; ++i) p[i & 63] += term(i);
-  for (int s = 32; s >= 1; s >>= 1)
-    for (int l = 0; l < s; ++l) p[l] += p[l + s];
-  return p[0];
-}
-
-// Q of the Householder QR with column pivoting of the 9 x 9 matrix A (the
-// role of ColPivHouseholderQR::matrixQ); column norms in the sum64 order.
-__device__ void colpiv_qr_Q9(double* A, double* Q) {
-  const int n = 9;
-  double hv[9][9], tau[9], norms[9];
-  for (int j = 0; j < n; ++j) norms[j] = lane_sum64(0, n, [&](int i) { return A[n * i + j] * A[n * i + j]; });
-  for (int k = 0; k < n; ++k) {
-    int p = k;
-    for (int j = k + 1; j < n; ++j)
-      if (norms[j] > norms[p]) p = j;
-    if (p != k) {
-      for (int i = 0; i < n; ++i) gswap(A[n * i + k], A[n * i + p]);
-      gswap(norms[k], norms[p]);
-    }
-    const double alpha = A[n * k + k];
-    const double sigma = lane_sum64(k + 1, n, [&](int i) { return A[n * i + k] * A[n * i + k]; });
-    tau[k] = 0.0;
-    for (int i = 0; i < n; ++i) hv[k][i] = 0.0;
-    hv[k][k] = 1.0;
-    if (sigma != 0.0) {
-      const double nrm = sqrt(alpha * alpha + sigma);
-      const double beta = alpha >= 0.0 ? -nrm : nrm;
-      tau[k] = (beta - alpha) / beta;
-      const double scale = 1.0 / (alpha - beta);
-      for (int i = k + 1; i < n; ++i) hv[k][i] = A[n * i + k] * scale;
-      A[n * k + k] = beta;
-      for (int i = k + 1; i < n; ++i) A[n * i + k] = 0.0;
-      for (int j = k + 1; j < n; ++j) {
-        const double w = A[n * k + j] + lane_sum64(k + 1, n, [&](int i) { return hv[k][i] * A[n * i + j]; });
-        const double tw = tau[k] * w;
-        A[n * k + j] = A[n * k + j] - tw;
-        for (int i = k + 1; i < n; ++i) A[n * i + j] = A[n * i + j] - tw * hv[k][i];
-      }
-    }
-    for (int j = k + 1; j < n; ++j)
-      norms[j] = lane_sum64(k + 1, n, [&](int i) { return A[n * i + j] * A[n * i + j]; });
-  }
-  for (int i = 0; i < n * n; ++i) Q[i] = 0.0;
-  for (int i = 0; i < n; ++i) Q[n * i + i] = 1.0;
-  for (int k = n - 1; k >= 0; --k) {
-    if (tau[k] == 0.0) continue;
-    for (int j = 0; j < n; ++j) {
-      double w = 0.0;
-      for (int i = k; i < n; ++i) w += hv[k][i] * Q[n * i + j];
-      const double tw = tau[k] * w;
-      for (int i = k; i < n; ++i) Q[n * i + j] = Q[n * i + j] - tw * hv[k][i];
-    }
-  }
-}
-
 // Shared state of one fit (LDS).
 struct EssShared {
-  double M[81];        // A^T A, then scratch of the QR
-  double Q[81];
+  double M[81];        // A^T A
   double NS[9][4];     // null-space basis (columns: x, y, z, 1)
   double models[10][9];
   int nmodels;
+  StewShared st;
   // bundle adjustment
   double dR[9][3], dt[9][2], tb[3][2];
   double pose_q[4], pose_t[3], new_q[4], new_t[3];
@@ -99,45 +39,43 @@ struct EssShared {
   double E[9];
 };
 
-// Stewenius steps after the null space (lane 0): constraints, elimination,
-// action matrix, real eigenvalues, null vectors -> S.models / S.nmodels.
+// Stewenius steps after the null space: constraints, elimination, action
+// matrix, real eigenvalues, null vectors -> S.models / S.nmodels.
 __device__ void stewenius_tail(EssShared& S) {
-  double ee[3][3][4];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j)
-      for (int k = 0; k < 4; ++k) ee[i][j][k] = S.NS[3 * j + i][k];
-  double C[200];
-  essential_constraints(ee, kSteweniusMul, 2.0, C);
-  double L[100], B[100];
-  for (int r = 0; r < 10; ++r)
-    for (int c = 0; c < 10; ++c) {
-      L[10 * r + c] = C[20 * r + c];
-      B[10 * r + c] = C[20 * r + 10 + c];
-    }
-  lu_full_solve(L, B, 10, 10);
-  double Act[100];
-  for (int i = 0; i < 100; ++i) Act[i] = 0.0;
-  const int from[6] = {0, 1, 2, 4, 5, 7};
-  for (int r = 0; r < 6; ++r)
-    for (int c = 0; c < 10; ++c) Act[10 * r + c] = B[10 * from[r] + c];
-  Act[10 * 6 + 0] = -1.0;
-  Act[10 * 7 + 1] = -1.0;
-  Act[10 * 8 + 3] = -1.0;
-  Act[10 * 9 + 6] = -1.0;
-  double ev[10];
-  const int ne = real_eigenvalues(Act, 10, ev);
-  for (int q = 0; q < ne; ++q) {
-    double Ms[100], v[10];
-    for (int i = 0; i < 100; ++i) Ms[i] = Act[i];
-    for (int i = 0; i < 10; ++i) Ms[11 * i] = Ms[11 * i] - ev[q];
-    null_vector_fullpiv(Ms, 10, v);
-    double e[9];
-    for (int r = 0; r < 9; ++r)
-      e[r] = S.NS[r][0] * v[6] + S.NS[r][1] * v[7] + S.NS[r][2] * v[8] + S.NS[r][3] * v[9];
-    for (int r = 0; r < 3; ++r)
-      for (int cc = 0; cc < 3; ++cc) S.models[q][3 * r + cc] = e[3 * cc + r];
+  const int lane = lane_id();
+  double col[10], x[10];
+  int colp;
+  wave_constraints(S.NS, S.st, col);
+  wave_lu_full(col, x, colp);
+  // rows 0, 1, 2, 4, 5, 7 of the solution (unknown colp of lane i is row i of
+  // x) are the action matrix's first six rows
+  for (int e = lane; e < 100; e += 64) S.st.a[e / 10][e % 10] = 0.0;
+  __syncthreads();
+  constexpr int kRow[10] = {0, 1, 2, -1, 3, 4, -1, 5, -1, -1};
+#pragma unroll
+  for (int i = 0; i < 10; ++i) {
+    const int u = __builtin_amdgcn_readlane(colp, i);
+    int r = -1;
+#pragma unroll
+    for (int c = 0; c < 10; ++c) r = c == u ? kRow[c] : r;
+    if (r >= 0 && lane >= 10 && lane < 20) S.st.a[r][lane - 10] = x[i];
   }
-  S.nmodels = ne;
+  if (lane == 0) {
+    S.st.a[6][0] = -1.0;
+    S.st.a[7][1] = -1.0;
+    S.st.a[8][3] = -1.0;
+    S.st.a[9][6] = -1.0;
+  }
+  __syncthreads();
+  const int ne = __builtin_amdgcn_readfirstlane(wave_real_eigenvalues(S.st));
+  if (ne > 0) wave_null_vectors(S.st, ne);
+  for (int e = lane; e < 9 * ne; e += 64) {
+    const int q = e / 9, r = e % 9;
+    const double* v = S.st.vec[q];
+    // entry r of E stacked column by column
+    S.models[q][3 * (r % 3) + r / 3] = S.NS[r][0] * v[6] + S.NS[r][1] * v[7] + S.NS[r][2] * v[8] + S.NS[r][3] * v[9];
+  }
+  if (lane == 0) S.nmodels = ne;
 }
 
 // Stewenius solve of the n rows written to `rows` (9 doubles each, row i by
@@ -145,17 +83,20 @@ __device__ void stewenius_tail(EssShared& S) {
 __device__ void wave_stewenius(const double* rows, int n, EssShared& S) {
   const int lane = lane_id();
   __syncthreads();
+  bool ready = true;  // the null space is in S.NS
   if (n == 5) {
-    if (lane == 0) {
-      double a[45], N[36];
-      for (int i = 0; i < 45; ++i) a[i] = rows[i];
-      S.nmodels = 0;
-      if (null_space_rx9(a, 5, N) == 4) {
-        for (int r = 0; r < 9; ++r)
-          for (int k = 0; k < 4; ++k) S.NS[r][k] = N[9 * k + r];
-        S.nmodels = -1;  // null space ready
-      }
+    // every lane solves the 5 x 9 system alike
+    double a[5][9], N[36];
+#pragma unroll
+    for (int i = 0; i < 45; ++i) a[i / 9][i % 9] = rows[i];
+    ready = null_space_5x9(a, N);
+    if (ready && lane == 0) {
+#pragma unroll
+      for (int r = 0; r < 9; ++r)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) S.NS[r][k] = N[9 * k + r];
     }
+    if (!ready && lane == 0) S.nmodels = 0;
   } else {
     double acc[45];
 #pragma unroll
@@ -184,14 +125,14 @@ __device__ void wave_stewenius(const double* rows, int n, EssShared& S) {
         }
         ++o;
       }
-    if (lane == 0) {
-      colpiv_qr_Q9(S.M, S.Q);
-      for (int r = 0; r < 9; ++r)
-        for (int k = 0; k < 4; ++k) S.NS[r][k] = S.Q[9 * r + 5 + k];
-      S.nmodels = -1;
-    }
+    __syncthreads();
+    double col[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) col[i] = S.M[9 * i + (lane < 9 ? lane : 8)];
+    wave_qr9_null_space(col, S.NS);
   }
-  if (lane == 0 && S.nmodels == -1) stewenius_tail(S);
+  __syncthreads();
+  if (ready) stewenius_tail(S);
   __syncthreads();
 }
 

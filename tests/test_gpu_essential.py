@@ -45,9 +45,8 @@ def test_five_point_bit_exact(oracle, engine, seed):
         assert np.array_equal(_bits(om[k, :n]), _bits(dm[k, :n])), k
 
 
-# Edges of the solver's 64-sample tiles and 131,072-sample slabs; refused
-# samples (negative index), repeated points (rank below five) and a repeated
-# sample among them.
+# Edges of the solver's 64-sample tiles and 131,072-sample slabs, repeated
+# points (rank below five) among them.
 @pytest.mark.parametrize("count", [1, 15, 63, 64, 65, 257, 131072 + 65])
 def test_five_point_tile_edges_bit_exact(oracle, engine, count):
     sc = _scene(5, n=300)
@@ -56,18 +55,33 @@ def test_five_point_tile_edges_bit_exact(oracle, engine, count):
     samples = np.argsort(rng.random((count, 40)), axis=1)[:, :5].astype(np.int32)
     samples[count // 2] = 3                       # one point five times: rank 1
     samples[-1, 1] = samples[-1, 0]               # rank 4
-    samples[count // 3, 0] = -1                   # the sampler refused
     dm, dst = engine.solve_minimal(2, pts, samples)
     check = np.unique(np.concatenate([np.arange(min(count, 200)), np.arange(max(0, count - 200), count),
                                       np.arange(131072 - 70, 131072 + 65)[:max(0, count - 131072 + 70)]]))
-    check = check[(check < count)]
-    assert not (dst[samples[:, 0] < 0] == 2).any()
-    check = check[samples[check, 0] >= 0]
+    check = check[check < count]
     om, onm = oracle.e5_solve(pts, samples[check], orient=True)
     dnm = (dst[check] == 2).sum(axis=1)
     assert np.array_equal(onm, dnm)
     for k, c in enumerate(check):
         assert np.array_equal(_bits(om[k, :onm[k]]), _bits(dm[c, :onm[k]])), c
+
+
+# The fit's 64-lane sums at their edges, and points without a five-dimensional
+# row space (a repeated point: rank one).
+@pytest.mark.parametrize("ns", [5, 6, 8, 9, 63, 64, 65, 129])
+@pytest.mark.parametrize("repeated", [False, True])
+def test_nonminimal_fit_sizes_bit_exact(oracle, engine, ns, repeated):
+    sc = _scene(6)
+    pts = _normalised(oracle, sc)
+    rng = np.random.default_rng(ns)
+    sample = rng.choice(np.nonzero(sc["gt"])[0], ns, replace=False).astype(np.int32)
+    if repeated:
+        sample[:] = sample[0]
+    om = oracle.e_nonminimal(pts, sample, None)
+    dm = engine.fit_nonminimal(2, pts, sample, None, 0, 0, THR / F_PX)
+    assert om.shape == dm.shape
+    same = (_bits(om) == _bits(dm)) | (np.isnan(om) & np.isnan(dm))
+    assert same.all()
 
 
 @pytest.mark.parametrize("mode", ["lo", "five", "irls"])
