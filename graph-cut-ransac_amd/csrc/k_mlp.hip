@@ -8,9 +8,10 @@
 //                    8-nearest-neighbour features (per-pair grid of cells,
 //                    one thread per query walking rings of cells)
 //   k_mlp_predict    forward pass on the matrix cores
-//   k_mlp_train      forward + backward-data pass of one mini-batch
-//   k_mlp_wgrad      weight gradients (batch as the reduction dimension)
-//   k_mlp_reduce     deterministic sum of the per-chunk partials + Adam
+//   k_mlp_train      forward, backward and weight-gradient pass of one
+//                    mini-batch, a partial gradient per workgroup
+//   k_mlp_reduce     deterministic sum of the partials, Adam and the packed
+//                    weights of the next step
 //
 // Matrix-core formulation.  Activations are kept transposed: a wave owns 32
 // points (the N = 32 columns of a 32x32x8 BF16 MFMA) and computes
@@ -19,11 +20,12 @@
 // 32-neuron tile are the neurons 8*(r/4) + 4*(lane/32) + r%4 of point
 // lane%32 -- exactly the B-operand slots of the next layer's k-blocks, so a
 // layer's output (bias, GELU, BF16 rounding applied in registers) feeds the
-// next layer with no data movement.  The backward-data pass does the same
-// with W^T, and the weight gradients G = D H^T run the batch through the
-// reduction dimension from neuron-major BF16 copies written by the forward
-// pass.  Weights live in LDS with a 132-element row stride (no bank
-// conflicts on the 8-byte A-operand reads).
+// next layer with no data movement.  Weights live in LDS with a 132-element
+// row stride (no bank conflicts on the 8-byte A-operand reads).
+//
+// Training has a few thousand points per step, too few for a wave per 32
+// points to fill the chip, so there the four waves of a workgroup share 32
+// points and own 32 neurons of every layer each (k_mlp_train).
 #include <hip/hip_runtime.h>
 
 #include "mlp_kernels.hpp"
@@ -32,12 +34,12 @@ namespace gcr {
 namespace mlp {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
 constexpr int RS = 132;  // LDS row stride (elements) of the 128-wide matrices
-constexpr int ZL = 64 * 64;  // floats of one layer's pre-activations per wave
 
 struct FwdLds {
   uint16_t w1[HID * IN];
@@ -46,12 +48,22 @@ struct FwdLds {
   float b1[HID], b2[HID], b3[HID], w4[HID];
   float b4, pad_[3];
 };
-struct TrainLds {
-  FwdLds f;
-  uint16_t w2t[HID * RS];
-  uint16_t w3t[HID * RS];
-};
 static_assert(sizeof(FwdLds) % 16 == 0, "LDS layout");
+
+// Training: activations and deltas of a workgroup's 32 points, BF16.
+// Point-major rows (the next layer's B operand, 8 neurons per read) and
+// neuron-major rows (the weight gradient's operands, 8 points per read); row
+// strides of 17 and 5 16-byte units keep both free of bank conflicts.
+constexpr int PS = 136, NS = 40;
+struct TrainLds {
+  uint16_t h1p[32][PS], h2p[32][PS], d3p[32][PS], d2p[32][PS];
+  uint16_t x[16][NS];  // input rows 0 .. 7, row 8: ones (the bias gradient)
+  uint16_t h1[HID][NS], h2[HID][NS];
+  uint16_t d1[HID][NS], d2[HID][NS], d3[HID][NS];
+  float z4[4][32];     // the waves' parts of the logits
+  float b1[HID], b2[HID], b3[HID], w4[HID];
+};
+static_assert(sizeof(TrainLds) % 16 == 0, "LDS layout");
 
 __device__ inline uint16_t f2bf(float f) {
   uint32_t u = __float_as_uint(f);
@@ -60,17 +72,19 @@ __device__ inline uint16_t f2bf(float f) {
 }
 __device__ inline float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
-// GELU (tanh form) and its derivative, operations in the oracle's order
+// GELU (tanh form), operations in the oracle's order
 __device__ inline float gelu_f(float z) {
   const float c = 0.7978845608028654f;
   const float u = c * (z + 0.044715f * (z * z * z));
   return 0.5f * z * (1.0f + tanhf(u));
 }
-__device__ inline float gelu_grad_f(float z) {
+// GELU and its derivative from one tanh
+__device__ inline float gelu_both(float z, float& grad) {
   const float c = 0.7978845608028654f;
   const float z2 = z * z;
   const float t = tanhf(c * (z + 0.044715f * (z2 * z)));
-  return 0.5f * (1.0f + t) + 0.5f * z * ((1.0f - t * t) * (c * (1.0f + 0.134145f * z2)));
+  grad = 0.5f * (1.0f + t) + 0.5f * z * ((1.0f - t * t) * (c * (1.0f + 0.134145f * z2)));
+  return 0.5f * z * (1.0f + t);
 }
 __device__ inline float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ inline float softplus_f(float z) {
@@ -94,6 +108,21 @@ __device__ inline f32x16 zero16() {
 
 __device__ inline f32x16 mfma(const bf16x4& a, const bf16x4& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, c, 0, 0, 0);
+}
+// 16 values of the reduction dimension: lane l holds 8 (l / 32) .. + 7 of row /
+// column l % 32
+__device__ inline f32x16 mfma16(const bf16x8& a, const bf16x8& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+__device__ inline bf16x8 load8(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
+__device__ inline bf16x8 fill8(uint16_t v) {
+  union {
+    uint16_t u[8];
+    bf16x8 b;
+  } x;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x.u[e] = v;
+  return x.b;
 }
 
 // 128 x 128 BF16 matrix (row-major) -> LDS rows of RS elements
@@ -119,28 +148,21 @@ __device__ inline void stage_forward(FwdLds& s, const uint16_t* wpk, const float
 }
 
 // bias + GELU + BF16 of one 32-neuron tile; the rounded activations go to
-// the next layer's B operand (k-blocks 4*MT .. 4*MT+3) and, when training,
-// the pre-activations to the wave's z buffer and the activations to the
-// neuron-major copy used by the weight gradients
-template <int MT, bool TRAIN>
-__device__ __attribute__((always_inline)) inline void epilogue(const f32x16& acc, const float* bias, int half, int lane, bf16x4* hout, float* zl,
-                                uint16_t* arow, int64_t bpad, int64_t col) {
+// the next layer's B operand (k-blocks 4*MT .. 4*MT+3)
+template <int MT>
+__device__ __attribute__((always_inline)) inline void epilogue(const f32x16& acc, const float* bias, int half,
+                                                               bf16x4* hout) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int i = 32 * MT + 8 * (r >> 2) + 4 * half + (r & 3);
     const float z = acc[r] + bias[i];
-    const uint16_t h = f2bf(gelu_f(z));
-    hout[4 * MT + (r >> 2)][r & 3] = (short)h;
-    if (TRAIN) {
-      zl[(16 * MT + r) * 64 + lane] = z;
-      arow[(int64_t)i * bpad + col] = h;
-    }
+    hout[4 * MT + (r >> 2)][r & 3] = (short)f2bf(gelu_f(z));
   }
 }
 
-template <int MT, bool TRAIN>
-__device__ __attribute__((always_inline)) inline void hidden_tile(const uint16_t* w, const float* bias, const bf16x4* hin, int j, int half, int lane,
-                                   bf16x4* hout, float* zl, uint16_t* arow, int64_t bpad, int64_t col) {
+template <int MT>
+__device__ __attribute__((always_inline)) inline void hidden_tile(const uint16_t* w, const float* bias,
+                                                                  const bf16x4* hin, int j, int half, bf16x4* hout) {
   f32x16 acc = zero16();
   const uint16_t* wrow = w + (32 * MT + j) * RS + 4 * half;
 #pragma unroll
@@ -148,7 +170,7 @@ __device__ __attribute__((always_inline)) inline void hidden_tile(const uint16_t
     const bf16x4 a = *reinterpret_cast<const bf16x4*>(wrow + 8 * kb);
     acc = mfma(a, hin[kb], acc);
   }
-  epilogue<MT, TRAIN>(acc, bias, half, lane, hout, zl, arow, bpad, col);
+  epilogue<MT>(acc, bias, half, hout);
 }
 
 // Forward pass of the wave's 32 points (lane % 32 = point, lane / 32 = half
@@ -157,10 +179,8 @@ __device__ __attribute__((always_inline)) inline void hidden_tile(const uint16_t
 // wj: lane % 32 as the weight-row index; the persistent inference loop
 // passes it through an empty asm so the weight reads stay inside the loop
 // (hoisted, the 128 weight registers per layer would spill).
-template <bool TRAIN>
 __device__ __attribute__((always_inline)) inline float forward_wave(const FwdLds& s, const float* fptr, int lane,
-                                                                    int wj, float* zw, uint16_t* act, int64_t bpad,
-                                                                    int64_t col) {
+                                                                    int wj) {
   const int j = wj, half = lane >> 5;
   float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   if (fptr) f = *reinterpret_cast<const float4*>(fptr + 4 * half);
@@ -169,41 +189,27 @@ __device__ __attribute__((always_inline)) inline float forward_wave(const FwdLds
   xb[1] = (short)f2bf(f.y);
   xb[2] = (short)f2bf(f.z);
   xb[3] = (short)f2bf(f.w);
-  if (TRAIN) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) act[(int64_t)(ROW_X + 4 * half + e) * bpad + col] = (uint16_t)xb[e];
-  }
   bf16x4 ha[16], hb[16];
   // layer 1: one k-block (8 inputs)
   {
     const uint16_t* wrow = s.w1 + j * IN + 4 * half;
-    uint16_t* a1 = TRAIN ? act + (int64_t)ROW_H1 * bpad : nullptr;
-    float* z1 = TRAIN ? zw : nullptr;
     f32x16 acc0 = mfma(*reinterpret_cast<const bf16x4*>(wrow), xb, zero16());
-    epilogue<0, TRAIN>(acc0, s.b1, half, lane, ha, z1, a1, bpad, col);
+    epilogue<0>(acc0, s.b1, half, ha);
     f32x16 acc1 = mfma(*reinterpret_cast<const bf16x4*>(wrow + 32 * IN), xb, zero16());
-    epilogue<1, TRAIN>(acc1, s.b1, half, lane, ha, z1, a1, bpad, col);
+    epilogue<1>(acc1, s.b1, half, ha);
     f32x16 acc2 = mfma(*reinterpret_cast<const bf16x4*>(wrow + 64 * IN), xb, zero16());
-    epilogue<2, TRAIN>(acc2, s.b1, half, lane, ha, z1, a1, bpad, col);
+    epilogue<2>(acc2, s.b1, half, ha);
     f32x16 acc3 = mfma(*reinterpret_cast<const bf16x4*>(wrow + 96 * IN), xb, zero16());
-    epilogue<3, TRAIN>(acc3, s.b1, half, lane, ha, z1, a1, bpad, col);
+    epilogue<3>(acc3, s.b1, half, ha);
   }
-  {
-    uint16_t* a2 = TRAIN ? act + (int64_t)ROW_H2 * bpad : nullptr;
-    float* z2 = TRAIN ? zw + ZL : nullptr;
-    hidden_tile<0, TRAIN>(s.w2, s.b2, ha, j, half, lane, hb, z2, a2, bpad, col);
-    hidden_tile<1, TRAIN>(s.w2, s.b2, ha, j, half, lane, hb, z2, a2, bpad, col);
-    hidden_tile<2, TRAIN>(s.w2, s.b2, ha, j, half, lane, hb, z2, a2, bpad, col);
-    hidden_tile<3, TRAIN>(s.w2, s.b2, ha, j, half, lane, hb, z2, a2, bpad, col);
-  }
-  {
-    uint16_t* a3 = TRAIN ? act + (int64_t)ROW_H3 * bpad : nullptr;
-    float* z3 = TRAIN ? zw + 2 * ZL : nullptr;
-    hidden_tile<0, TRAIN>(s.w3, s.b3, hb, j, half, lane, ha, z3, a3, bpad, col);
-    hidden_tile<1, TRAIN>(s.w3, s.b3, hb, j, half, lane, ha, z3, a3, bpad, col);
-    hidden_tile<2, TRAIN>(s.w3, s.b3, hb, j, half, lane, ha, z3, a3, bpad, col);
-    hidden_tile<3, TRAIN>(s.w3, s.b3, hb, j, half, lane, ha, z3, a3, bpad, col);
-  }
+  hidden_tile<0>(s.w2, s.b2, ha, j, half, hb);
+  hidden_tile<1>(s.w2, s.b2, ha, j, half, hb);
+  hidden_tile<2>(s.w2, s.b2, ha, j, half, hb);
+  hidden_tile<3>(s.w2, s.b2, ha, j, half, hb);
+  hidden_tile<0>(s.w3, s.b3, hb, j, half, ha);
+  hidden_tile<1>(s.w3, s.b3, hb, j, half, ha);
+  hidden_tile<2>(s.w3, s.b3, hb, j, half, ha);
+  hidden_tile<3>(s.w3, s.b3, hb, j, half, ha);
   // output unit: this half's 64 neurons in ascending order, then the halves
   float sum = 0.0f;
 #pragma unroll
@@ -213,24 +219,6 @@ __device__ __attribute__((always_inline)) inline float forward_wave(const FwdLds
   }
   const float other = __shfl_xor(sum, 32);
   return (half == 0 ? sum + other : other + sum) + s.b4;
-}
-
-// backward-data tile: D_l = (W^T D_{l+1}) * gelu'(Z_l) for 32 neurons
-template <int MT, bool OUT>
-__device__ __attribute__((always_inline)) inline void backward_tile(const uint16_t* wt, const bf16x4* din, int j, int half, int lane, const float* zl,
-                                     bf16x4* dout, uint16_t* drow, int64_t bpad, int64_t col) {
-  f32x16 acc = zero16();
-  const uint16_t* wrow = wt + (32 * MT + j) * RS + 4 * half;
-#pragma unroll
-  for (int kb = 0; kb < 16; ++kb) acc = mfma(*reinterpret_cast<const bf16x4*>(wrow + 8 * kb), din[kb], acc);
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int i = 32 * MT + 8 * (r >> 2) + 4 * half + (r & 3);
-    const float d = acc[r] * gelu_grad_f(zl[(16 * MT + r) * 64 + lane]);
-    const uint16_t b = f2bf(d);
-    if (OUT) dout[4 * MT + (r >> 2)][r & 3] = (short)b;
-    drow[(int64_t)i * bpad + col] = b;
-  }
 }
 
 }  // namespace
@@ -480,7 +468,7 @@ __global__ __launch_bounds__(256) void k_mlp_predict(const uint16_t* __restrict_
     const bool valid = col < n;
     int wj = lane & 31;
     asm volatile("" : "+v"(wj));
-    const float z = forward_wave<false>(s, valid ? feat + IN * col : nullptr, lane, wj, nullptr, nullptr, 0, 0);
+    const float z = forward_wave(s, valid ? feat + IN * col : nullptr, lane, wj);
     if ((lane >> 5) == 0 && valid) {
       logit[col] = z;
       if (prob) prob[col] = sigmoid_f(z);
@@ -488,142 +476,266 @@ __global__ __launch_bounds__(256) void k_mlp_predict(const uint16_t* __restrict_
   }
 }
 
-__global__ __launch_bounds__(256) void k_mlp_train(const uint16_t* __restrict__ wpk, const float* __restrict__ bias,
-                                                   const float* __restrict__ feat, const float* __restrict__ labels,
-                                                   int64_t batch, int64_t bpad, int64_t sample_n, uint64_t seed,
-                                                   int64_t step, float inv_batch, float* __restrict__ zbuf,
-                                                   uint16_t* __restrict__ act, float* __restrict__ d4out,
-                                                   float* __restrict__ lossv) {
+// One mini-batch: forward, backward and weight gradients.  A workgroup takes
+// tiles of 32 points; wave w owns neurons 32 w .. 32 w + 31 of every hidden
+// layer: its rows of W2, W3 and of their transposes are the A operands, the
+// layers' outputs pass between the waves through LDS, and
+// the tile's deltas and activations are contracted into the workgroup's
+// gradient accumulators (the points are the reduction dimension; the bias
+// gradients are one more column of ones).  One partial gradient per workgroup
+// goes to memory.
+//
+// What bounds it: the latency of one tile's chain of nine dependent layer
+// products and their tanh epilogues, with one wave per SIMD.  A wave per 32
+// points for all 128 neurons, the activations written to memory for a second
+// kernel of 16 workgroups, took 135 + 115 us per step of 8,192 rows on MI355X;
+// this kernel 31.8 us (128 workgroups of two tiles 55 us, with 5.9 us in the
+// reduction against 9.2).
+__global__ __launch_bounds__(256, 1) void k_mlp_train(const uint16_t* __restrict__ wpk, const float* __restrict__ bias,
+                                                      const float* __restrict__ feat,
+                                                      const float* __restrict__ labels, int64_t batch,
+                                                      int64_t sample_n, uint64_t seed, int64_t step, float inv_batch,
+                                                      float* __restrict__ part) {
   extern __shared__ __align__(16) unsigned char mlp_lds_t[];
   TrainLds& s = *reinterpret_cast<TrainLds*>(mlp_lds_t);
-  stage_forward(s.f, wpk, bias);
-  stage_matrix(s.w2t, wpk + PK_W2T);
-  stage_matrix(s.w3t, wpk + PK_W3T);
-  __syncthreads();
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = lane & 31, half = lane >> 5;
-  const int64_t wave_g = (int64_t)blockIdx.x * 4 + w;
-  const int64_t col = wave_g * 32 + j;
-  const bool valid = col < batch;
-  int64_t idx = col;
-  if (valid && sample_n > 0)
-    idx = (int64_t)(mix64(seed ^ mix64((uint64_t)step * 0x100000001B3ull + (uint64_t)col)) % (uint64_t)sample_n);
-  float* zw = zbuf + wave_g * (3 * ZL);
-  const float z4 = forward_wave<true>(s.f, valid ? feat + IN * idx : nullptr, lane, j, zw, act, bpad, col);
-  const float y = valid ? labels[idx] : 0.0f;
-  const float d4 = valid ? (sigmoid_f(z4) - y) * inv_batch : 0.0f;
-  if (half == 0) {
-    d4out[col] = d4;
-    lossv[col] = valid ? (softplus_f(z4) - y * z4) * inv_batch : 0.0f;
+  // this wave's neuron of accumulator slot r
+  auto neuron = [&](int r) { return 32 * w + 8 * (r >> 2) + 4 * half + (r & 3); };
+  // A operand of this wave's rows of a 128 x 128 matrix, fetched (from the L2)
+  // a layer ahead of its use; the empty asm keeps the fetch inside the tile
+  // loop (all four matrices held over it, 128 registers, spilled)
+  auto fetch = [&](bf16x8* A, int matrix) {
+    int at = matrix + (32 * w + j) * HID + 8 * half;
+    asm volatile("" : "+v"(at));
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb) A[kb] = load8(wpk + at + 16 * kb);
+  };
+  for (int i = threadIdx.x; i < HID; i += 256) {
+    s.b1[i] = bias[i];
+    s.b2[i] = bias[HID + i];
+    s.b3[i] = bias[2 * HID + i];
+    s.w4[i] = bf2f(wpk[PK_W4 + i]);
   }
-  // D3 = w4 d4 * gelu'(Z3)
-  bf16x4 da[16], db[16];
-  uint16_t* d3row = act + (int64_t)ROW_D3 * bpad;
+  const float b4 = bias[3 * HID];
+  for (int e = threadIdx.x; e < 16 * NS; e += 256) s.x[e / NS][e % NS] = e / NS == 8 ? (uint16_t)0x3F80 : (uint16_t)0;
+  f32x16 g1 = zero16(), gb2 = zero16(), gb3 = zero16();
+  f32x16 g2[4] = {zero16(), zero16(), zero16(), zero16()}, g3[4] = {zero16(), zero16(), zero16(), zero16()};
+  float gw4[16], gb4 = 0.0f, loss = 0.0f;
 #pragma unroll
-  for (int kb = 0; kb < 16; ++kb) {
+  for (int r = 0; r < 16; ++r) gw4[r] = 0.0f;
+  const bf16x8 ones = fill8(j == 0 ? (uint16_t)0x3F80 : (uint16_t)0);
+  // four neurons of a point at a time, and one by one neuron-major
+  auto put = [&](uint16_t (*pm)[PS], uint16_t (*nm)[NS], const uint16_t* v) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int i = 8 * kb + 4 * half + e;
-      const float d = (s.f.w4[i] * d4) * gelu_grad_f(zw[2 * ZL + (4 * kb + e) * 64 + lane]);
-      const uint16_t b = f2bf(d);
-      da[kb][e] = (short)b;
-      d3row[(int64_t)i * bpad + col] = b;
+    for (int g = 0; g < 4; ++g) {
+      if (pm) {
+        uint2 q;
+        q.x = (uint32_t)v[4 * g] | ((uint32_t)v[4 * g + 1] << 16);
+        q.y = (uint32_t)v[4 * g + 2] | ((uint32_t)v[4 * g + 3] << 16);
+        *reinterpret_cast<uint2*>(&pm[j][32 * w + 8 * g + 4 * half]) = q;
+      }
+      if (nm) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) nm[neuron(4 * g + e)][j] = v[4 * g + e];
+      }
+    }
+  };
+  auto layer = [&](const bf16x8* A, uint16_t (*in)[PS]) {
+    f32x16 acc = zero16();
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb) acc = mfma16(A[kb], load8(&in[j][16 * kb + 8 * half]), acc);
+    return acc;
+  };
+  const int64_t tiles = (batch + 31) / 32;
+  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const int64_t col = 32 * tile + j;
+    const bool valid = col < batch;
+    int64_t idx = col;
+    if (valid && sample_n > 0)
+      idx = (int64_t)(mix64(seed ^ mix64((uint64_t)step * 0x100000001B3ull + (uint64_t)col)) % (uint64_t)sample_n);
+    const float y = valid ? labels[idx] : 0.0f;
+    float gr1[16], gr2[16], gr3[16], h3[16];
+    uint16_t v[16];
+    bf16x8 A1 = fill8(0), Aa[8], Ab[8];
+    if (half == 0) A1 = load8(wpk + PK_W1 + (32 * w + j) * IN);
+    fetch(Aa, PK_W2);
+    __syncthreads();  // the last tile's operands have been read
+    {
+      union {
+        uint16_t u[8];
+        bf16x8 b;
+      } x;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x.u[e] = 0;
+      if (half == 0 && valid) {
+        const float4 f0 = *reinterpret_cast<const float4*>(feat + IN * idx);
+        const float4 f1 = *reinterpret_cast<const float4*>(feat + IN * idx + 4);
+        x.u[0] = f2bf(f0.x);
+        x.u[1] = f2bf(f0.y);
+        x.u[2] = f2bf(f0.z);
+        x.u[3] = f2bf(f0.w);
+        x.u[4] = f2bf(f1.x);
+        x.u[5] = f2bf(f1.y);
+        x.u[6] = f2bf(f1.z);
+        x.u[7] = f2bf(f1.w);
+      }
+      if (w == 0 && half == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s.x[e][j] = x.u[e];
+      }
+      const f32x16 acc = mfma16(A1, x.b, zero16());
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[r] = f2bf(gelu_both(acc[r] + s.b1[neuron(r)], gr1[r]));
+    }
+    put(s.h1p, s.h1, v);
+    __syncthreads();
+    {
+      fetch(Ab, PK_W3);
+      const f32x16 acc = layer(Aa, s.h1p);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[r] = f2bf(gelu_both(acc[r] + s.b2[neuron(r)], gr2[r]));
+    }
+    put(s.h2p, s.h2, v);
+    __syncthreads();
+    {
+      fetch(Aa, PK_W3T);
+      const f32x16 acc = layer(Ab, s.h2p);
+      float sum = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        h3[r] = bf2f(f2bf(gelu_both(acc[r] + s.b3[neuron(r)], gr3[r])));
+        sum = sum + s.w4[neuron(r)] * h3[r];
+      }
+      const float other = __shfl_xor(sum, 32);
+      if (half == 0) s.z4[w][j] = sum + other;
+    }
+    __syncthreads();
+    const float z4 = ((s.z4[0][j] + s.z4[1][j]) + (s.z4[2][j] + s.z4[3][j])) + b4;
+    const float d4 = valid ? (sigmoid_f(z4) - y) * inv_batch : 0.0f;
+    if (w == 0 && half == 0 && valid) {
+      gb4 += d4;
+      loss += (softplus_f(z4) - y * z4) * inv_batch;
+    }
+    // D3 = w4 d4 * gelu'(Z3)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      gw4[r] += d4 * h3[r];
+      v[r] = f2bf((s.w4[neuron(r)] * d4) * gr3[r]);
+    }
+    put(s.d3p, s.d3, v);
+    __syncthreads();
+    {
+      fetch(Ab, PK_W2T);
+      const f32x16 acc = layer(Aa, s.d3p);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[r] = f2bf(acc[r] * gr2[r]);
+    }
+    put(s.d2p, s.d2, v);
+    __syncthreads();
+    {
+      const f32x16 acc = layer(Ab, s.d2p);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[r] = f2bf(acc[r] * gr1[r]);
+    }
+    put(nullptr, s.d1, v);
+    __syncthreads();
+    // G = D H^T over the tile's 32 points
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      const int at = 16 * kb + 8 * half;
+      const bf16x8 a3 = load8(&s.d3[32 * w + j][at]), a2 = load8(&s.d2[32 * w + j][at]);
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) {
+        g3[nt] = mfma16(a3, load8(&s.h2[32 * nt + j][at]), g3[nt]);
+        g2[nt] = mfma16(a2, load8(&s.h1[32 * nt + j][at]), g2[nt]);
+      }
+      gb3 = mfma16(a3, ones, gb3);
+      gb2 = mfma16(a2, ones, gb2);
+      const bf16x8 xb = j < 16 ? load8(&s.x[j & 15][at]) : fill8(0);
+      g1 = mfma16(load8(&s.d1[32 * w + j][at]), xb, g1);
     }
   }
-  uint16_t* d2row = act + (int64_t)ROW_D2 * bpad;
-  backward_tile<0, true>(s.w3t, da, j, half, lane, zw + ZL, db, d2row, bpad, col);
-  backward_tile<1, true>(s.w3t, da, j, half, lane, zw + ZL, db, d2row, bpad, col);
-  backward_tile<2, true>(s.w3t, da, j, half, lane, zw + ZL, db, d2row, bpad, col);
-  backward_tile<3, true>(s.w3t, da, j, half, lane, zw + ZL, db, d2row, bpad, col);
-  uint16_t* d1row = act + (int64_t)ROW_D1 * bpad;
-  backward_tile<0, false>(s.w2t, db, j, half, lane, zw, nullptr, d1row, bpad, col);
-  backward_tile<1, false>(s.w2t, db, j, half, lane, zw, nullptr, d1row, bpad, col);
-  backward_tile<2, false>(s.w2t, db, j, half, lane, zw, nullptr, d1row, bpad, col);
-  backward_tile<3, false>(s.w2t, db, j, half, lane, zw, nullptr, d1row, bpad, col);
-}
-
-// Weight gradients of one chunk of WGRAD_CHUNK batch columns.  Wave w owns
-// output rows 32w .. 32w+31 of each 128 x 128 gradient (four 32x32 tiles);
-// biases, w4, b4 and the loss are sequential column-order sums.
-__global__ __launch_bounds__(256) void k_mlp_wgrad(const uint16_t* __restrict__ act, const float* __restrict__ d4,
-                                                   const float* __restrict__ lossv, int64_t bpad,
-                                                   float* __restrict__ part) {
-  const int c = blockIdx.x;
-  const int64_t p0 = (int64_t)c * WGRAD_CHUNK;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = lane & 31, half = lane >> 5;
-  float* out = part + (int64_t)c * PART_STRIDE;
+  float* out = part + (int64_t)blockIdx.x * PART_STRIDE;
 #pragma unroll
-  for (int job = 0; job < 2; ++job) {
-    const uint16_t* D = act + (int64_t)(job == 0 ? ROW_D3 : ROW_D2) * bpad;
-    const uint16_t* H = act + (int64_t)(job == 0 ? ROW_H2 : ROW_H1) * bpad;
-    const int off = job == 0 ? OFF_W3 : OFF_W2;
-    f32x16 acc[4] = {zero16(), zero16(), zero16(), zero16()};
-    const uint16_t* arow = D + (int64_t)(32 * w + j) * bpad + p0 + 4 * half;
-    const uint16_t* brow = H + (int64_t)j * bpad + p0 + 4 * half;
-    for (int kb = 0; kb < WGRAD_CHUNK / 8; ++kb) {
-      const bf16x4 a = *reinterpret_cast<const bf16x4*>(arow + 8 * kb);
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
-        acc[nt] = mfma(a, *reinterpret_cast<const bf16x4*>(brow + (int64_t)32 * nt * bpad + 8 * kb), acc[nt]);
-    }
+  for (int r = 0; r < 16; ++r) {
+    const int k = neuron(r);
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
+      out[OFF_W3 + k * HID + 32 * nt + j] = g3[nt][r];
+      out[OFF_W2 + k * HID + 32 * nt + j] = g2[nt][r];
+    }
+    if (j < IN) out[OFF_W1 + k * IN + j] = g1[r];
+    if (j == IN) out[OFF_B1 + k] = g1[r];
+    if (j == 0) {
+      out[OFF_B2 + k] = gb2[r];
+      out[OFF_B3 + k] = gb3[r];
+    }
+    float q = gw4[r];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int k = 32 * w + 8 * (r >> 2) + 4 * half + (r & 3);
-        out[off + k * HID + 32 * nt + j] = acc[nt][r];
-      }
-    }
+    for (int d = 16; d >= 1; d >>= 1) q += __shfl_xor(q, d);
+    if (j == 0) out[OFF_W4 + k] = q;
   }
-  {
-    // W1: D1 x X^T, input columns j < 8
-    f32x16 acc = zero16();
-    const uint16_t* arow = act + (int64_t)(ROW_D1 + 32 * w + j) * bpad + p0 + 4 * half;
-    const uint16_t* brow = act + (int64_t)(ROW_X + (j < IN ? j : 0)) * bpad + p0 + 4 * half;
-    bf16x4 zb;
-    zb[0] = zb[1] = zb[2] = zb[3] = 0;
-    for (int kb = 0; kb < WGRAD_CHUNK / 8; ++kb) {
-      const bf16x4 a = *reinterpret_cast<const bf16x4*>(arow + 8 * kb);
-      const bf16x4 b = j < IN ? *reinterpret_cast<const bf16x4*>(brow + 8 * kb) : zb;
-      acc = mfma(a, b, acc);
-    }
-    if (j < IN) {
+  if (w == 0) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int k = 32 * w + 8 * (r >> 2) + 4 * half + (r & 3);
-        out[OFF_W1 + k * IN + j] = acc[r];
-      }
+    for (int d = 16; d >= 1; d >>= 1) {
+      gb4 += __shfl_xor(gb4, d);
+      loss += __shfl_xor(loss, d);
     }
-  }
-  for (int row = threadIdx.x; row < 4 * HID + 2; row += blockDim.x) {
-    float sum = 0.0f;
-    if (row < 3 * HID) {
-      const int layer = row / HID, i = row % HID;
-      const uint16_t* src = act + (int64_t)(ROW_D1 + row) * bpad + p0;
-      for (int t = 0; t < WGRAD_CHUNK; ++t) sum = sum + bf2f(src[t]);
-      out[(layer == 0 ? OFF_B1 : layer == 1 ? OFF_B2 : OFF_B3) + i] = sum;
-    } else if (row < 4 * HID) {
-      const int i = row - 3 * HID;
-      const uint16_t* src = act + (int64_t)(ROW_H3 + i) * bpad + p0;
-      for (int t = 0; t < WGRAD_CHUNK; ++t) sum = sum + d4[p0 + t] * bf2f(src[t]);
-      out[OFF_W4 + i] = sum;
-    } else if (row == 4 * HID) {
-      for (int t = 0; t < WGRAD_CHUNK; ++t) sum = sum + d4[p0 + t];
-      out[OFF_B4] = sum;
-    } else {
-      for (int t = 0; t < WGRAD_CHUNK; ++t) sum = sum + lossv[p0 + t];
-      out[NPARAM] = sum;
+    if (lane == 0) {
+      out[OFF_B4] = gb4;
+      out[NPARAM] = loss;
     }
   }
 }
 
+// Where parameter q goes in the packed weights.
+__device__ inline void pack_param(int q, float p, uint16_t* __restrict__ wpk, float* __restrict__ bias) {
+  if (q < OFF_B1) {
+    wpk[PK_W1 + q] = f2bf(p);
+  } else if (q < OFF_W2) {
+    bias[q - OFF_B1] = p;
+  } else if (q < OFF_B2) {
+    const int t = q - OFF_W2;
+    const uint16_t b = f2bf(p);
+    wpk[PK_W2 + t] = b;
+    wpk[PK_W2T + (t % HID) * HID + t / HID] = b;
+  } else if (q < OFF_W3) {
+    bias[HID + q - OFF_B2] = p;
+  } else if (q < OFF_B3) {
+    const int t = q - OFF_W3;
+    const uint16_t b = f2bf(p);
+    wpk[PK_W3 + t] = b;
+    wpk[PK_W3T + (t % HID) * HID + t / HID] = b;
+  } else if (q < OFF_W4) {
+    bias[2 * HID + q - OFF_B3] = p;
+  } else if (q < OFF_B4) {
+    wpk[PK_W4 + q - OFF_W4] = f2bf(p);
+  } else {
+    bias[3 * HID] = p;
+  }
+}
+
+// Four threads per parameter, each summing a quarter of the partials in
+// workgroup order (the quarters' sums are added in order); the first applies
+// Adam and packs the new weight for the next step.
 __global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ part, int chunks,
                                                     float* __restrict__ grad, float* __restrict__ loss_out, int adam,
                                                     float* __restrict__ params, float* __restrict__ m,
-                                                    float* __restrict__ v, float lr, float c1, float c2) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q > NPARAM) return;
+                                                    float* __restrict__ v, float lr, float c1, float c2,
+                                                    uint16_t* __restrict__ wpk, float* __restrict__ bias) {
+  __shared__ float sums[4][64];
+  const int quarter = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int q = blockIdx.x * 64 + lane;
+  const int lo = chunks * quarter / 4, hi = chunks * (quarter + 1) / 4;
   float g = 0.0f;
-  for (int c = 0; c < chunks; ++c) g = g + part[(int64_t)c * PART_STRIDE + q];
+  if (q <= NPARAM) {
+#pragma unroll 8
+    for (int c = lo; c < hi; ++c) g = g + part[(int64_t)c * PART_STRIDE + q];
+  }
+  sums[quarter][lane] = g;
+  __syncthreads();
+  if (quarter != 0 || q > NPARAM) return;
+  g = ((sums[0][lane] + sums[1][lane]) + sums[2][lane]) + sums[3][lane];
   if (q == NPARAM) {
     if (loss_out) *loss_out = g;
     return;
@@ -636,7 +748,9 @@ __global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ pa
     m[q] = mm;
     v[q] = vv;
     const float mh = mm / c1, vh = vv / c2;
-    params[q] = params[q] - lr * mh / (sqrtf(vh) + eps);
+    const float p = params[q] - lr * mh / (sqrtf(vh) + eps);
+    params[q] = p;
+    pack_param(q, p, wpk, bias);
   }
 }
 
@@ -688,23 +802,21 @@ void launch_predict(hipStream_t st, const uint16_t* wpk, const float* bias, cons
                      logit, prob);
 }
 
-void launch_train_fwd_bwd(hipStream_t st, const uint16_t* wpk, const float* bias, const float* feat,
-                          const float* labels, int64_t batch, int64_t bpad, int64_t sample_n, uint64_t seed,
-                          int64_t step, float inv_batch, float* zbuf, uint16_t* act, float* d4, float* lossv) {
-  hipLaunchKernelGGL(k_mlp_train, dim3((unsigned)(bpad / POINTS_PER_BLOCK)), dim3(256), sizeof(TrainLds), st, wpk,
-                     bias, feat, labels, batch, bpad, sample_n, seed, step, inv_batch, zbuf, act, d4, lossv);
+int train_blocks(int64_t batch) {
+  const int64_t tiles = (batch + 31) / 32;
+  return (int)(tiles < kTrainBlocks ? tiles : kTrainBlocks);
 }
 
-void launch_wgrad(hipStream_t st, const uint16_t* act, const float* d4, const float* lossv, int64_t bpad,
-                  float* part) {
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3((unsigned)(bpad / WGRAD_CHUNK)), dim3(256), 0, st, act, d4, lossv, bpad,
-                     part);
+void launch_train(hipStream_t st, const uint16_t* wpk, const float* bias, const float* feat, const float* labels,
+                  int64_t batch, int64_t sample_n, uint64_t seed, int64_t step, float inv_batch, float* part) {
+  hipLaunchKernelGGL(k_mlp_train, dim3((unsigned)train_blocks(batch)), dim3(256), sizeof(TrainLds), st, wpk, bias,
+                     feat, labels, batch, sample_n, seed, step, inv_batch, part);
 }
 
 void launch_reduce_adam(hipStream_t st, const float* part, int chunks, float* grad, float* loss_out, int adam,
-                        float* params, float* m, float* v, float lr, float c1, float c2) {
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((NPARAM + 1 + 255) / 256), dim3(256), 0, st, part, chunks, grad, loss_out,
-                     adam, params, m, v, lr, c1, c2);
+                        float* params, float* m, float* v, float lr, float c1, float c2, uint16_t* wpk, float* bias) {
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((NPARAM + 1 + 63) / 64), dim3(256), 0, st, part, chunks, grad, loss_out, adam,
+                     params, m, v, lr, c1, c2, wpk, bias);
 }
 
 void launch_local_iota(hipStream_t st, const int64_t* pair_off, int num_pairs, int64_t total, int32_t* out) {

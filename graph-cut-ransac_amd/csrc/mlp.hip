@@ -63,8 +63,8 @@ struct Workspace {
   Buf<double> corr, ratio, sorted;
   Buf<int64_t> off;
   Buf<int32_t> sizes, tile_pair, tile_start, vals, perm;
-  Buf<float> feat, labels, params, m, v, logit, skeys, zbuf, d4, lossv, part, grad, loss;
-  Buf<uint16_t> wpk, act;
+  Buf<float> feat, labels, params, m, v, logit, skeys, part, grad, loss;
+  Buf<uint16_t> wpk;
   Buf<float> bias;
   Buf<unsigned char> tmp;
   Buf<KnnGrid> grids;
@@ -216,16 +216,6 @@ void pack(Workspace& w, const float* params) {
   launch_pack(w.st, w.params.p, w.wpk.p, w.bias.p);
 }
 
-int64_t padded(int64_t batch) { return (batch + WGRAD_CHUNK - 1) / WGRAD_CHUNK * WGRAD_CHUNK; }
-
-void train_buffers(Workspace& w, int64_t bpad) {
-  w.zbuf.ensure((size_t)(bpad / 32) * 3 * 64 * 64);
-  w.act.ensure((size_t)ACT_ROWS * (size_t)bpad);
-  w.d4.ensure((size_t)bpad);
-  w.lossv.ensure((size_t)bpad);
-  w.part.ensure((size_t)(bpad / WGRAD_CHUNK) * PART_STRIDE);
-}
-
 int check_pairs(int32_t num_pairs, const int64_t* offsets, std::vector<int64_t>& rel) {
   if (num_pairs <= 0 || !offsets) return fail(GCR_ERR_INVALID_ARGUMENT, "num_pairs must be positive");
   rel.resize((size_t)num_pairs + 1);
@@ -291,19 +281,17 @@ int32_t gcr_mlp_gradient(const float* params, const float* feat, const float* la
     check_lds(lds_train_bytes());
     Workspace& w = ws();
     pack(w, params);
-    const int64_t bpad = padded(n);
-    train_buffers(w, bpad);
+    const int blocks = train_blocks(n);
+    w.part.ensure((size_t)blocks * PART_STRIDE);
     w.feat.ensure(IN * (size_t)n);
     w.labels.ensure((size_t)n);
     w.grad.ensure(NPARAM);
     w.loss.ensure(1);
     h2d(w, w.feat.p, feat, IN * (size_t)n);
     h2d(w, w.labels.p, labels, (size_t)n);
-    launch_train_fwd_bwd(w.st, w.wpk.p, w.bias.p, w.feat.p, w.labels.p, n, bpad, 0, 0, 0, 1.0f / (float)n, w.zbuf.p,
-                         w.act.p, w.d4.p, w.lossv.p);
-    launch_wgrad(w.st, w.act.p, w.d4.p, w.lossv.p, bpad, w.part.p);
-    launch_reduce_adam(w.st, w.part.p, (int)(bpad / WGRAD_CHUNK), w.grad.p, w.loss.p, 0, nullptr, nullptr, nullptr,
-                       0.0f, 1.0f, 1.0f);
+    launch_train(w.st, w.wpk.p, w.bias.p, w.feat.p, w.labels.p, n, 0, 0, 0, 1.0f / (float)n, w.part.p);
+    launch_reduce_adam(w.st, w.part.p, blocks, w.grad.p, w.loss.p, 0, nullptr, nullptr, nullptr, 0.0f, 1.0f, 1.0f,
+                       nullptr, nullptr);
     hip_ok(hipGetLastError(), "gradient launches");
     d2h(w, grad_out, w.grad.p, NPARAM);
     float loss = 0.0f;
@@ -322,8 +310,8 @@ int32_t gcr_mlp_train(float* params, float* adam_m, float* adam_v, int64_t adam_
   return guarded([&]() -> int32_t {
     check_lds(lds_train_bytes());
     Workspace& w = ws();
-    const int64_t bpad = padded(batch);
-    train_buffers(w, bpad);
+    const int blocks = train_blocks(batch);
+    w.part.ensure((size_t)blocks * PART_STRIDE);
     w.params.ensure(NPARAM);
     w.m.ensure(NPARAM);
     w.v.ensure(NPARAM);
@@ -338,15 +326,13 @@ int32_t gcr_mlp_train(float* params, float* adam_m, float* adam_v, int64_t adam_
     h2d(w, w.feat.p, feat, IN * (size_t)n);
     h2d(w, w.labels.p, labels, (size_t)n);
     const float inv = 1.0f / (float)batch;
+    launch_pack(w.st, w.params.p, w.wpk.p, w.bias.p);  // later steps' weights are packed by the step before
     for (int32_t s = 0; s < steps; ++s) {
       const int64_t t = adam_step + s + 1;
       const float c1 = 1.0f - std::pow(0.9f, (float)t), c2 = 1.0f - std::pow(0.999f, (float)t);
-      launch_pack(w.st, w.params.p, w.wpk.p, w.bias.p);
-      launch_train_fwd_bwd(w.st, w.wpk.p, w.bias.p, w.feat.p, w.labels.p, batch, bpad, n, seed, t, inv, w.zbuf.p,
-                           w.act.p, w.d4.p, w.lossv.p);
-      launch_wgrad(w.st, w.act.p, w.d4.p, w.lossv.p, bpad, w.part.p);
-      launch_reduce_adam(w.st, w.part.p, (int)(bpad / WGRAD_CHUNK), nullptr, w.loss.p + s, 1, w.params.p, w.m.p,
-                         w.v.p, lr, c1, c2);
+      launch_train(w.st, w.wpk.p, w.bias.p, w.feat.p, w.labels.p, batch, n, seed, t, inv, w.part.p);
+      launch_reduce_adam(w.st, w.part.p, blocks, nullptr, w.loss.p + s, 1, w.params.p, w.m.p, w.v.p, lr, c1, c2,
+                         w.wpk.p, w.bias.p);
     }
     hip_ok(hipGetLastError(), "training launches");
     d2h(w, params, w.params.p, NPARAM);

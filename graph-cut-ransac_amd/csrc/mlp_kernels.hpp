@@ -25,7 +25,7 @@ constexpr int OFF_B3 = OFF_W3 + HID * HID;
 constexpr int OFF_W4 = OFF_B3 + HID;
 constexpr int OFF_B4 = OFF_W4 + HID;
 constexpr int NPARAM = OFF_B4 + 1;
-// one row of the per-chunk gradient partials: NPARAM gradients + the loss
+// one row of the workgroups' gradient partials: NPARAM gradients + the loss
 constexpr int PART_STRIDE = NPARAM + 3;  // 34,308: 16-byte rows
 
 // packed BF16 weights (uint16 offsets): W1, W2, W3, W2^T, W3^T, w4
@@ -39,13 +39,9 @@ constexpr int PK_TOTAL = PK_W4 + HID;
 // FP32 biases: b1 | b2 | b3 | b4
 constexpr int PB_TOTAL = 3 * HID + 1;
 
-// training activations, BF16, neuron-major rows of `bpad` columns:
-// X (8 rows) | H1 | H2 | H3 | D1 | D2 | D3 (128 rows each)
-constexpr int ROW_X = 0, ROW_H1 = 8, ROW_H2 = ROW_H1 + HID, ROW_H3 = ROW_H2 + HID, ROW_D1 = ROW_H3 + HID,
-              ROW_D2 = ROW_D1 + HID, ROW_D3 = ROW_D2 + HID, ACT_ROWS = ROW_D3 + HID;
-
 constexpr int POINTS_PER_BLOCK = 128;  // 4 waves x 32 points
-constexpr int WGRAD_CHUNK = 512;       // batch columns per weight-gradient workgroup
+// training workgroups at most, each with one partial gradient
+constexpr int kTrainBlocks = 256;
 
 // dynamic LDS of the kernels (bytes)
 int lds_forward_bytes();
@@ -79,20 +75,17 @@ void launch_pack(hipStream_t st, const float* params, uint16_t* wpk, float* bias
 // logits of n points; prob (nullable) = sigmoid(logit)
 void launch_predict(hipStream_t st, const uint16_t* wpk, const float* bias, const float* feat, int64_t n,
                     float* logit, float* prob);
-// forward + backward-data of `batch` columns padded to `bpad` (a multiple of
-// WGRAD_CHUNK).  Column c < batch reads point idx(c): c itself when
+// Forward and backward pass of `batch` columns: train_blocks(batch) rows of
+// PART_STRIDE partial gradients.  Column c reads point idx(c): c itself when
 // sample_n == 0, else a hash of (seed, step, c) modulo sample_n.
-void launch_train_fwd_bwd(hipStream_t st, const uint16_t* wpk, const float* bias, const float* feat,
-                          const float* labels, int64_t batch, int64_t bpad, int64_t sample_n, uint64_t seed,
-                          int64_t step, float inv_batch, float* zbuf, uint16_t* act, float* d4, float* lossv);
-// per-chunk gradient partials: part[c * PART_STRIDE + q]
-void launch_wgrad(hipStream_t st, const uint16_t* act, const float* d4, const float* lossv, int64_t bpad,
-                  float* part);
-// sums the partials of `chunks` chunks in chunk order; grad (nullable),
-// loss_out (nullable) = the summed loss; adam != 0 applies one Adam step
-// with bias corrections c1 = 1 - b1^t, c2 = 1 - b2^t
+int train_blocks(int64_t batch);
+void launch_train(hipStream_t st, const uint16_t* wpk, const float* bias, const float* feat, const float* labels,
+                  int64_t batch, int64_t sample_n, uint64_t seed, int64_t step, float inv_batch, float* part);
+// sums the `chunks` partials; grad (nullable), loss_out (nullable) = the summed
+// loss; adam != 0 applies one Adam step with bias corrections c1 = 1 - b1^t,
+// c2 = 1 - b2^t and packs the new parameters into wpk / bias
 void launch_reduce_adam(hipStream_t st, const float* part, int chunks, float* grad, float* loss_out, int adam,
-                        float* params, float* m, float* v, float lr, float c1, float c2);
+                        float* params, float* m, float* v, float lr, float c1, float c2, uint16_t* wpk, float* bias);
 // out[k] = k - (first row of k's pair), rows relative to pair_off[0]
 void launch_local_iota(hipStream_t st, const int64_t* pair_off, int num_pairs, int64_t total, int32_t* out);
 // sorted[k] = corr[first row of k's pair + perm[k]] (perm holds local indices)

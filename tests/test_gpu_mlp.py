@@ -129,6 +129,26 @@ def test_gradient_matches_oracle(engine, oracle):
     assert (grad.reshape(-1)[OFF["W1"] + 7:OFF["b1"]:8] == 0).all()
 
 
+# The gradient kernel's 32-point tiles and 256 workgroups at their edges; the
+# bar of test_gradient_matches_oracle (one BF16 rounding boundary crossed per
+# activation at most).
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 257, 256 * 32, 256 * 32 + 33])
+def test_gradient_tile_edges_match_oracle(engine, oracle, n):
+    from pygcransac import guided
+    rng = np.random.default_rng(n)
+    feat = np.zeros((n, 8), np.float32)
+    feat[:, :7] = rng.uniform(-1, 1, (n, 7))
+    labels = (rng.random(n) < 0.4).astype(np.float32)
+    p = _net(5)
+    loss, grad = guided.gradient(p, feat, labels)
+    lo, go = oracle.mlp_loss_grad(p, feat, labels)
+    assert abs(loss - lo) <= 1e-4 * abs(lo) + (1e-2 if n < 32 else 0.0)
+    rel = np.linalg.norm(grad - go) / np.linalg.norm(go)
+    print("n=%d rel %.3g" % (n, rel))
+    assert rel < 2e-2
+    assert (grad.reshape(-1)[OFF["W1"] + 7:OFF["b1"]:8] == 0).all()
+
+
 def _mix64(x):
     m = (1 << 64) - 1
     x = (x + 0x9E3779B97F4A7C15) & m
