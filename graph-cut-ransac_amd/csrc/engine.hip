@@ -2324,49 +2324,58 @@ struct Engine : Workspace {
   // step; one launch pair per problem kind.
   // The filtered read-back of a chunk launch (see Request::filtered):
   // models per candidate, each candidate's last model's count and the
-  // records of the slots above each item's best, packed in item order.
+  // records of the slots above each item's best.
   PhaseTask exec_chunk_filtered(std::vector<PairCtx*>& items, int kind, int m, int S, int64_t tot,
                                 const std::vector<int64_t>& base, const int8_t* d_status, int8_t* d_nmodels,
                                 const int32_t* d_counts, const double* d_values, const int32_t* d_sym,
-                                const int8_t* d_valid, const int8_t* d_degen, const int32_t* d_samples,
+                                const int8_t* d_valid, bool degen, const int32_t* d_samples, const int32_t* d_cpair,
                                 const int64_t* d_ibase, const int32_t* d_incand, const double* d_ibest,
                                 const std::shared_ptr<DevBuf<double>>& cand_models, double* d_cand_models,
                                 double* d_cand_degen_h) {
     const size_t ni = items.size();
     const size_t ns = (size_t)tot * S;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    // device: last counts | record counts | packed records | per-item records
-    const size_t f_rc = al(4 * (size_t)tot), f_pk = f_rc + al(4 * ni), f_rs = f_pk + al(sizeof(SlotRec) * ns),
-                 f_end = f_rs + sizeof(SlotRec) * ns;
-    char* const df = d_filt[kind].ensure(f_end);
-    int32_t* const d_last = reinterpret_cast<int32_t*>(df);
-    int32_t* const d_rc = reinterpret_cast<int32_t*>(df + f_rc);
-    SlotRec* const d_packed = reinterpret_cast<SlotRec*>(df + f_pk);
+    // device: record count | last counts | records
+    char* const df = d_filt[kind].p;
+    uint32_t* const d_rc = reinterpret_cast<uint32_t*>(df);
+    int32_t* const d_last = reinterpret_cast<int32_t*>(df + 256);
+    const size_t f_rs = 256 + al(4 * (size_t)tot);
     SlotRec* const d_recs = reinterpret_cast<SlotRec*>(df + f_rs);
-    launch_chunk_filter(stream, kind == GCR_PROBLEM_HOMOGRAPHY ? 1 : 0, S, (int)ni, d_ibase, d_incand, d_ibest,
-                        d_status, d_nmodels, d_counts, d_values, d_sym, d_valid, d_degen, d_samples, m, d_last, d_recs,
-                        d_rc, d_packed);
-    // host: models per candidate | the block's head (last counts, record
-    // counts and the first `spec` packed records, one copy).  Few slots beat
-    // a pair's best, so the records usually come back with the counts; more
-    // than `spec` of them take a second copy after the counts are known.
+    int64_t max_cand = 0;
+    for (auto* p : items) max_cand = std::max(max_cand, p->req.num_cand);
+    launch_chunk_filter(stream, kind == GCR_PROBLEM_HOMOGRAPHY ? 1 : 0, S, (int)ni, (int)max_cand, d_ibase, d_incand,
+                        d_ibest, d_status, d_nmodels, d_counts, d_values, d_sym, d_valid, d_samples, m, d_last, d_recs,
+                        d_rc);
+    if (degen)
+      launch_degen_records(stream, d_rpts, d_pair_pt_off.p, d_cpair, d_samples, d_cand_models, d_ibase, d_rc, d_recs,
+                           d_cand_degen_h);
+    // host: models per candidate | the block's head (record count, last counts
+    // and the first `spec` records, one copy).  Few slots beat a pair's best, so
+    // the records usually come back with the counts; more than `spec` of them
+    // take a second copy after the count is known.
     const size_t spec = std::min(ns, 16 * ni + 256);
-    const size_t h_blk = al((size_t)tot), head = f_pk + sizeof(SlotRec) * spec;
+    const size_t h_blk = al((size_t)tot), head = f_rs + sizeof(SlotRec) * spec;
     char* const hs = h_cand_res[kind].ensure(h_blk + head);
     d2h(reinterpret_cast<int8_t*>(hs), d_nmodels, (size_t)tot);
     d2h(hs + h_blk, df, head);
     co_await step_sync();
     const int8_t* nm = reinterpret_cast<const int8_t*>(hs);
-    const int32_t* lc = reinterpret_cast<const int32_t*>(hs + h_blk);
-    const int32_t* rc = reinterpret_cast<const int32_t*>(hs + h_blk + f_rc);
-    std::vector<int64_t> roff(ni + 1, 0);
-    for (size_t i = 0; i < ni; ++i) roff[i + 1] = roff[i] + rc[i];
-    const SlotRec* hr = reinterpret_cast<const SlotRec*>(hs + h_blk + f_pk);
-    if ((size_t)roff[ni] > spec) {
-      SlotRec* const all = h_filt_recs[kind].ensure((size_t)roff[ni]);
-      d2h(all, d_packed, (size_t)roff[ni]);
+    const size_t nrec = *reinterpret_cast<const uint32_t*>(hs + h_blk);
+    const int32_t* lc = reinterpret_cast<const int32_t*>(hs + h_blk + 256);
+    const SlotRec* hr = reinterpret_cast<const SlotRec*>(hs + h_blk + f_rs);
+    if (nrec > spec) {
+      SlotRec* const all = h_filt_recs[kind].ensure(nrec);
+      d2h(all, d_recs, nrec);
       co_await step_sync();
       hr = all;
+    }
+    // the records by item, in slot order
+    std::vector<uint32_t> roff(ni + 1, 0), order(nrec);
+    for (size_t k = 0; k < nrec; ++k) ++roff[(size_t)hr[k].item + 1];
+    for (size_t i = 0; i < ni; ++i) roff[i + 1] += roff[i];
+    {
+      std::vector<uint32_t> at(roff.begin(), roff.end() - 1);
+      for (size_t k = 0; k < nrec; ++k) order[at[(size_t)hr[k].item]++] = (uint32_t)k;
     }
     pool->run(ni, [&](size_t i) {
       Request& r = items[i]->req;
@@ -2375,7 +2384,10 @@ struct Engine : Workspace {
       r.filtered = true;
       r.nmodels.assign(nm + b, nm + b + k);
       r.last_count.assign(lc + b, lc + b + k);
-      r.recs.assign(hr + roff[i], hr + roff[i + 1]);
+      std::sort(order.begin() + roff[i], order.begin() + roff[i + 1],
+                [&](uint32_t x, uint32_t y) { return hr[x].slot < hr[y].slot; });
+      r.recs.resize(roff[i + 1] - roff[i]);
+      for (uint32_t q = roff[i]; q < roff[i + 1]; ++q) r.recs[q - roff[i]] = hr[order[q]];
       r.dev_models = d_cand_models + 9 * b * S;
       r.models_hold = cand_models;
       if (items[i]->degensac) r.dev_degen_h = d_cand_degen_h + 9 * b * S;
@@ -2511,8 +2523,10 @@ struct Engine : Workspace {
     int32_t* const d_blk = reinterpret_cast<int32_t*>(dwork + al(4 * ns) + 256);
     check_hip(hipMemcpyAsync(din, hin, in_end, hipMemcpyHostToDevice, stream), "hipMemcpyAsync H2D");
     // each candidate's pair, from the items' first candidates and counts
-    launch_fill_cand_pair(stream, (int)ni, d_ibase, d_incand, reinterpret_cast<const int32_t*>(din + in_ip),
-                          d_cpair);
+    // (and the filtered records' counter, at the head of their block)
+    if (filt) d_filt[kind].ensure(256 + al(4 * (size_t)tot) + sizeof(SlotRec) * ns);
+    launch_fill_cand_pair(stream, (int)ni, d_ibase, d_incand, reinterpret_cast<const int32_t*>(din + in_ip), d_cpair,
+                          filt ? reinterpret_cast<uint32_t*>(d_filt[kind].p) : nullptr);
     if (!dsi.empty()) {
       const int ts = prof.start("sample", (double)tot);
       launch_sample_streams(stream, reinterpret_cast<const DevSampleItem*>(din + in_ds),
@@ -2574,15 +2588,15 @@ struct Engine : Workspace {
                      d_cpair, d_status, (int64_t)ns, d_counts, d_values, nullptr,
                      nullptr, d_sym, true, S, d_work_list, d_work_count);
       prof.stop(t1);
-      if (degen_any) {
+      if (degen_any && !filt) {
         launch_degen_test(stream, d_rpts, d_pair_pt_off.p, d_cpair, d_samples, d_cand_models,
                           d_status, (int64_t)ns, d_degen, d_cand_degen_h);
       }
     }
     if (filt) {
       co_await exec_chunk_filtered(items, kind, m, S, tot, base, d_status, d_nmodels, d_counts, d_values, d_sym,
-                                   d_valid, degen_any ? d_degen : nullptr, d_samples, d_ibase, d_incand, d_ibest,
-                                   cand_models, d_cand_models, d_cand_degen_h);
+                                   d_valid, degen_any, d_samples, d_cpair, d_ibase, d_incand, d_ibest, cand_models,
+                                   d_cand_models, d_cand_degen_h);
       co_return;
     }
     char* const hres = h_cand_res[kind].ensure(r_end);

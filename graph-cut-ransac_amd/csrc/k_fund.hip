@@ -901,26 +901,15 @@ __device__ __forceinline__ void cross3v(const double* u, const double* v, double
 }
 __device__ __forceinline__ double sqnorm3(const double* v) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2]; }
 
-// H-degenerate sample test of every kept seven-point model, one thread per
-// model slot (slot / 3 = candidate).  The epipole e (e_3 = 1) is the largest
+// H-degenerate sample test of a seven-point model F of sample smp, one thread
+// per model slot (slot / 3 = candidate).  The epipole e (e_3 = 1) is the largest
 // cross product of two columns of F (the left null vector), A = [e]x F; each
 // of the five sample triplets defines H = A - e (M^-1 b)^T (M: the triplet's
 // first-image points as rows, b_k = ((x2 x A x1) . (x2 x e)) / |x2 x e|^2),
 // and the sample is H-degenerate when that H maps at least five of the seven
 // points within the homography threshold (squared transfer error < 4).
-// degen[slot] = 1 and degen_h[slot] = the first such H.
-__global__ void k_degen_test(const double* __restrict__ pts, const int64_t* __restrict__ pair_pt_off,
-                             const int32_t* __restrict__ cand_pair, const int32_t* __restrict__ samples,
-                             const double* __restrict__ models, const int8_t* __restrict__ status,
-                             int64_t num_slots, int8_t* __restrict__ degen, double* __restrict__ degen_h) {
-  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (q >= num_slots) return;
-  degen[q] = 0;
-  if (status[q] != 2) return;
-  const int64_t c = q / 3;
-  const double* P = pts + 4 * pair_pt_off[cand_pair[c]];
-  const int32_t* smp = samples + 7 * c;
-  const double* F = models + 9 * q;
+// Returns that and writes the first such H to degen_h.
+__device__ bool degen_sample(const double* P, const int32_t* smp, const double* F, double* degen_h) {
   const double c0[3] = {F[0], F[3], F[6]}, c1[3] = {F[1], F[4], F[7]}, c2[3] = {F[2], F[5], F[8]};
   double e01[3], e02[3], e12[3];
   cross3v(c0, c1, e01);
@@ -964,10 +953,42 @@ __global__ void k_degen_test(const double* __restrict__ pts, const int64_t* __re
       if (h_sq_residual(P + 4 * (int64_t)idx, Hm) < 4.0) ++cnt;
     }
     if (cnt >= 5) {
-      degen[q] = 1;
-      for (int i = 0; i < 9; ++i) degen_h[9 * q + i] = Hm[i];
-      return;
+      for (int i = 0; i < 9; ++i) degen_h[i] = Hm[i];
+      return true;
     }
+  }
+  return false;
+}
+
+// Every kept slot of a chunk.
+__global__ void k_degen_test(const double* __restrict__ pts, const int64_t* __restrict__ pair_pt_off,
+                             const int32_t* __restrict__ cand_pair, const int32_t* __restrict__ samples,
+                             const double* __restrict__ models, const int8_t* __restrict__ status,
+                             int64_t num_slots, int8_t* __restrict__ degen, double* __restrict__ degen_h) {
+  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (q >= num_slots) return;
+  const int64_t c = q / 3;
+  degen[q] = status[q] == 2 && degen_sample(pts + 4 * pair_pt_off[cand_pair[c]], samples + 7 * c, models + 9 * q,
+                                            degen_h + 9 * q)
+                 ? 1
+                 : 0;
+}
+
+// The slots of a filtered chunk's records: the loop asks about no others (the
+// whole chunk took 137 us a launch, 4 % of a fundamental batch's kernels).
+__global__ void k_degen_records(const double* __restrict__ pts, const int64_t* __restrict__ pair_pt_off,
+                                const int32_t* __restrict__ cand_pair, const int32_t* __restrict__ samples,
+                                const double* __restrict__ models, const int64_t* __restrict__ item_base,
+                                const uint32_t* __restrict__ rec_count, SlotRec* __restrict__ recs,
+                                double* __restrict__ degen_h) {
+  const uint32_t n = *rec_count;
+  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+    const int64_t q = 3 * item_base[recs[k].item] + recs[k].slot;
+    const int64_t c = q / 3;
+    recs[k].degen = degen_sample(pts + 4 * pair_pt_off[cand_pair[c]], samples + 7 * c, models + 9 * q,
+                                 degen_h + 9 * q)
+                        ? 1
+                        : 0;
   }
 }
 
@@ -1022,6 +1043,14 @@ void launch_degen_test(hipStream_t st, const double* pts, const int64_t* pair_pt
   if (num_slots <= 0) return;
   hipLaunchKernelGGL(k_degen_test, dim3((unsigned)((num_slots + 255) / 256)), dim3(256), 0, st, pts, pair_pt_off,
                      cand_pair, samples, models, status, num_slots, degen, degen_h);
+}
+
+void launch_degen_records(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* cand_pair,
+                          const int32_t* samples, const double* models, const int64_t* item_base,
+                          const uint32_t* rec_count, SlotRec* recs, double* degen_h) {
+  // the count is on the device; few records in all but a run's first chunks
+  hipLaunchKernelGGL(k_degen_records, dim3(64), dim3(256), 0, st, pts, pair_pt_off, cand_pair, samples, models,
+                     item_base, rec_count, recs, degen_h);
 }
 
 void launch_pp_solve(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* cand_pair,

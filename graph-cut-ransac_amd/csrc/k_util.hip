@@ -92,131 +92,90 @@ void launch_irls_weights(hipStream_t st, int kind, const double* pts, const int6
 }
 
 // ---- candidate results filtered on the device --------------------------------
-// One 256-thread block per item walks its slots in order, 1,024 at a time
-// (thread t takes the 4 consecutive slots 4t .. 4t + 3 of the round): a slot
-// (candidate c, model j) holds a model when j < nmodels[c]; the last model's
-// count goes to last_count[c]; the slots whose value beats the item's best
-// are compacted in slot order (block prefix sum of the per-thread counts)
-// into the item's region of recs.
+// One thread per candidate (blockIdx.y = item): the last model's count goes to
+// last_count[c]; the slots whose value beats the item's best become records,
+// appended in any order (the host puts each item's records back in slot
+// order; few slots beat a pair's best).  One block per item walking its slots
+// in order, 1,024 a round, was a serial chain of up to 160 rounds: 670 us per
+// chunk of essential candidates on MI355X.
 __global__ void __launch_bounds__(256)
     k_chunk_filter(int h, int S, const int64_t* __restrict__ item_base, const int32_t* __restrict__ item_ncand,
                    const double* __restrict__ item_best, const int8_t* __restrict__ status, int8_t* nmodels,
                    const int32_t* __restrict__ counts, const double* __restrict__ values,
-                   const int32_t* __restrict__ sym, const int8_t* __restrict__ valid, const int8_t* __restrict__ degen,
+                   const int32_t* __restrict__ sym, const int8_t* __restrict__ valid,
                    const int32_t* __restrict__ samples, int m, int32_t* __restrict__ last_count,
-                   SlotRec* __restrict__ recs, int32_t* __restrict__ rec_count) {
-  __shared__ int wsum[4];
-  const int it = blockIdx.x;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int64_t b = item_base[it];
-  const int64_t nslots = (int64_t)item_ncand[it] * S;
+                   SlotRec* __restrict__ recs, uint32_t* __restrict__ rec_count, int first_item) {
+  const int it = first_item + (int)blockIdx.y;
+  const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  const bool live = q < item_ncand[it];
+  const int64_t c = item_base[it] + (live ? q : 0);
   const double best = item_best[it];
-  SlotRec* out = recs + b * S;
-  int cnt = 0;
-  for (int64_t q0 = 0; q0 < nslots; q0 += 1024) {
-    SlotRec r[4];
-    bool keep[4];
-    int mine = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int64_t q = q0 + 4 * t + k;
-      keep[k] = false;
-      if (q < nslots) {
-        const int64_t c = b + q / S;
-        const int j = (int)(q % S);
-        const int64_t g = b * S + q;
-        int nm;
-        if (h) {
-          nm = status[g] == 2 ? 1 : 0;
-          nmodels[c] = (int8_t)nm;
-        } else {
-          nm = nmodels[c];
-        }
-        if (j < nm) {
-          if (j == nm - 1) last_count[c] = counts[g];
-          const double v = values[g];
-          if (v > best) {
-            keep[k] = true;
-            r[k].slot = (int32_t)q;
-            r[k].count = counts[g];
-            r[k].value = v;
-            r[k].sym = h ? 0 : sym[g];
-            r[k].valid = h ? valid[c] : 1;
-            r[k].degen = degen ? degen[g] : 0;
-            r[k].pad[0] = r[k].pad[1] = 0;
-            r[k].sample0 = samples[c * m];
-            r[k].pad2 = 0;
-          }
-        }
-      }
-      mine += keep[k] ? 1 : 0;
+  int nm = 0;
+  if (live) {
+    if (h) {
+      nm = status[c] == 2 ? 1 : 0;
+      nmodels[c] = (int8_t)nm;
+    } else {
+      nm = nmodels[c];
     }
-    // inclusive prefix of the per-thread counts inside the wave, then across
-    // the four waves
-    int incl = mine;
-#pragma unroll
-    for (int s = 1; s < 64; s <<= 1) {
-      const int o = __shfl_up(incl, s, 64);
-      if (lane >= s) incl += o;
-    }
-    if (lane == 63) wsum[wv] = incl;
-    __syncthreads();
-    int woff = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      if (w < wv) woff += wsum[w];
-      total += wsum[w];
-    }
-    int pos = cnt + woff + incl - mine;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (keep[k]) out[pos++] = r[k];
-    cnt += total;
-    __syncthreads();
+    if (nm > 0) last_count[c] = counts[c * S + nm - 1];
   }
-  if (t == 0) rec_count[it] = cnt;
+  for (int j = 0; ballot64(j < nm) != 0; ++j) {
+    const int64_t g = c * S + j;
+    const double v = j < nm ? values[g] : 0.0;
+    const bool keep = j < nm && v > best;
+    const uint64_t b = ballot64(keep);
+    if (b == 0) continue;
+    uint32_t at = 0;
+    if (lane_id() == 0) at = atomicAdd(rec_count, (uint32_t)__popcll(b));
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    if (keep) {
+      SlotRec r;
+      r.slot = q * S + j;
+      r.count = counts[g];
+      r.value = v;
+      r.sym = h ? 0 : sym[g];
+      r.valid = h ? valid[c] : 1;
+      r.degen = 0;
+      r.pad[0] = r.pad[1] = 0;
+      r.sample0 = samples[c * m];
+      r.item = it;
+      recs[at + __popcll(b & ((1ull << lane_id()) - 1ull))] = r;
+    }
+  }
 }
 
-// cand_pair[base[i] + c] = pair[i] for c < count[i] (one block per item)
+// cand_pair[base[i] + c] = pair[i] for c < count[i] (one block per item); *zero
+// = 0 when given
 __global__ void __launch_bounds__(256) k_fill_cand_pair(const int64_t* __restrict__ base,
                                                         const int32_t* __restrict__ count,
-                                                        const int32_t* __restrict__ pair, int32_t* __restrict__ cand_pair) {
+                                                        const int32_t* __restrict__ pair, int32_t* __restrict__ cand_pair,
+                                                        uint32_t* __restrict__ zero) {
   const int it = blockIdx.x;
+  if (zero && it == 0 && threadIdx.x == 0) *zero = 0u;
   const int64_t b = base[it];
   const int32_t n = count[it], p = pair[it];
   for (int32_t c = threadIdx.x; c < n; c += 256) cand_pair[b + c] = p;
 }
 
 void launch_fill_cand_pair(hipStream_t st, int num_items, const int64_t* base, const int32_t* count,
-                           const int32_t* pair, int32_t* cand_pair) {
+                           const int32_t* pair, int32_t* cand_pair, uint32_t* zero) {
   if (num_items <= 0) return;
-  hipLaunchKernelGGL(k_fill_cand_pair, dim3(num_items), dim3(256), 0, st, base, count, pair, cand_pair);
+  hipLaunchKernelGGL(k_fill_cand_pair, dim3(num_items), dim3(256), 0, st, base, count, pair, cand_pair, zero);
 }
 
-// Item i's records to packed + (sum of the earlier items' counts).
-__global__ void __launch_bounds__(64) k_chunk_pack(int S, const int64_t* __restrict__ item_base,
-                                                   const int32_t* __restrict__ rec_count,
-                                                   const SlotRec* __restrict__ recs, SlotRec* __restrict__ packed) {
-  const int it = blockIdx.x;
-  const int lane = threadIdx.x;
-  int64_t off = 0;
-  for (int i = lane; i < it; i += 64) off += rec_count[i];
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) off += __shfl_xor(off, s, 64);
-  const SlotRec* src = recs + item_base[it] * S;
-  const int n = rec_count[it];
-  for (int k = lane; k < n; k += 64) packed[off + k] = src[k];
-}
-
-void launch_chunk_filter(hipStream_t st, int h, int S, int num_items, const int64_t* item_base,
+void launch_chunk_filter(hipStream_t st, int h, int S, int num_items, int max_cand, const int64_t* item_base,
                          const int32_t* item_ncand, const double* item_best, const int8_t* status, int8_t* nmodels,
                          const int32_t* counts, const double* values, const int32_t* sym, const int8_t* valid,
-                         const int8_t* degen, const int32_t* samples, int m, int32_t* last_count, SlotRec* recs,
-                         int32_t* rec_count, SlotRec* packed) {
-  if (num_items <= 0) return;
-  hipLaunchKernelGGL(k_chunk_filter, dim3(num_items), dim3(256), 0, st, h, S, item_base, item_ncand, item_best, status,
-                     nmodels, counts, values, sym, valid, degen, samples, m, last_count, recs, rec_count);
-  hipLaunchKernelGGL(k_chunk_pack, dim3(num_items), dim3(64), 0, st, S, item_base, rec_count, recs, packed);
+                         const int32_t* samples, int m, int32_t* last_count, SlotRec* recs, uint32_t* rec_count) {
+  if (num_items <= 0 || max_cand <= 0) return;
+  // blockIdx.y holds at most 65,535 items
+  for (int i = 0; i < num_items; i += 65535) {
+    const int k = std::min(65535, num_items - i);
+    hipLaunchKernelGGL(k_chunk_filter, dim3((unsigned)((max_cand + 255) / 256), (unsigned)k), dim3(256), 0, st, h, S,
+                       item_base, item_ncand, item_best, status, nmodels, counts, values, sym, valid, samples, m,
+                       last_count, recs, rec_count, i);
+  }
 }
 
 }  // namespace gcr

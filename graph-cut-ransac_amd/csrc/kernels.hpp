@@ -183,11 +183,6 @@ void launch_sprt_walk(hipStream_t st, SprtItem* items, int num_items, int max_sl
                       const double* pair_sq_thr, const int32_t* pools, const SpPair* sp_pairs, const SpCell* sp_cells,
                       const int32_t* sp_perm, const int32_t* sp_cell_of, int32_t* sp_list, int max_cells);
 
-// Candidate results filtered on the device (k_util.hip): per item (one
-// pair's candidates base .. base + k - 1, S slots each), the model slots
-// whose value beats the item's best value, in slot order, and each
-// candidate's last model's count.  For homographies (h != 0) a slot holds a
-// model when its status is 2, and nmodels is written here.
 // The uniform sampler's generator state of one pair on the device
 // (std::mt19937's 624 words and the position of the next word, 624: the
 // block is used up).
@@ -221,23 +216,33 @@ void launch_mt_seed(hipStream_t st, const uint32_t* seeds, const int32_t* pairs,
 void launch_sample_streams(hipStream_t st, const DevSampleItem* items, const DevSampleSeg* segs, int num_items,
                            DevMT* states, int32_t* samples);
 
+// Candidate results filtered on the device (k_util.hip): per item (one pair's
+// candidates base .. base + ncand - 1, S slots each; at most max_cand per item)
+// a record for every model slot whose value beats the item's best value, in
+// any order, *rec_count of them (zeroed before), and each candidate's last
+// model's count.  For homographies (h != 0) a slot holds a model when its
+// status is 2, and nmodels is written here.
 struct SlotRec {
   int32_t slot, count;  // slot relative to the item's first candidate
   double value;
   int32_t sym;
   int8_t valid, degen, pad[2];
   int32_t sample0;  // first index of the candidate's sample
-  int32_t pad2;
+  int32_t item;
 };
-void launch_chunk_filter(hipStream_t st, int h, int S, int num_items, const int64_t* item_base,
+void launch_chunk_filter(hipStream_t st, int h, int S, int num_items, int max_cand, const int64_t* item_base,
                          const int32_t* item_ncand, const double* item_best, const int8_t* status, int8_t* nmodels,
                          const int32_t* counts, const double* values, const int32_t* sym, const int8_t* valid,
-                         const int8_t* degen, const int32_t* samples, int m, int32_t* last_count, SlotRec* recs,
-                         int32_t* rec_count, SlotRec* packed);
+                         const int32_t* samples, int m, int32_t* last_count, SlotRec* recs, uint32_t* rec_count);
+// launch_degen_test on the slots of a filtered chunk's records only (3 slots
+// per candidate): rec.degen, and degen_h of the degenerate slots
+void launch_degen_records(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* cand_pair,
+                          const int32_t* samples, const double* models, const int64_t* item_base,
+                          const uint32_t* rec_count, SlotRec* recs, double* degen_h);
 
 // small utilities
 void launch_fill_cand_pair(hipStream_t st, int num_items, const int64_t* base, const int32_t* count,
-                           const int32_t* pair, int32_t* cand_pair);
+                           const int32_t* pair, int32_t* cand_pair, uint32_t* zero);
 void launch_copy_models(hipStream_t st, const double* const* src, double* const* dst, int count);
 // a[off[i] .. off[i] + len[i]) = 0 for i < count
 void launch_zero_ranges(hipStream_t st, double* a, const int64_t* off, const int32_t* len, int count, int max_len);

@@ -61,3 +61,35 @@ def test_batch_repeatable(oracle):
     for (Ma, ma), (Mb, mb) in zip(a, b):
         assert np.array_equal(ma, mb)
         assert np.array_equal(Ma.view(np.uint64), Mb.view(np.uint64))
+
+
+# Iterations (first candidate chunk) around the filter's 256-candidate blocks,
+# with few and with many slots above the starting best value (the second lists
+# more records than the read-back's first copy holds), degenerate samples among
+# them.
+@pytest.mark.parametrize("iters", [1, 255, 256, 257, 700])
+def test_chunk_filter_edges_match_oracle(oracle, iters):
+    import pygcransac
+    probs = []
+    for i, kind in enumerate(("fundamental", "homography", "fundamental")):
+        if kind == "homography":
+            sc = synthetic.homography_scene(synthetic.scene_seed(7, i), n=300, inlier_ratio=0.4)
+        elif i == 0:
+            sc = synthetic.fundamental_scene(synthetic.scene_seed(7, i), n=300, inlier_ratio=0.5)
+        else:
+            sc = synthetic.fundamental_scene(synthetic.scene_seed(7, i), n=300, inlier_ratio=0.6, plane_fraction=0.9)
+        probs.append(dict(kind=kind, correspondences=sc["corr"], h1=480, w1=640, h2=480, w2=640, threshold=1.5,
+                          conf=0.999, spatial_coherence_weight=0.975, max_iters=iters, min_iters=iters, use_sprt=False,
+                          sampler=0, neighborhood=0, neighborhood_size=8.0, lo_number=50, seed=iters + i))
+    res = pygcransac.findBatch(probs)
+    stats = pygcransac.last_batch_stats()
+    for i, pb in enumerate(probs):
+        p = oracle.params(1.5, 0.999, 0.975, iters, iters, 0, 50, 8.0, pb["seed"])
+        find = oracle.find_homography if pb["kind"] == "homography" else oracle.find_fundamental
+        rc, Mo, mo, so = find(pb["correspondences"], 480, 640, 480, 640, p)
+        M, mask = res[i]
+        assert np.array_equal(mask, mo), i
+        for key in ("iteration_number", "local_optimization_number", "graph_cut_number"):
+            assert stats[i][key] == so[key], (i, key)
+        if Mo is not None and M is not None:
+            np.testing.assert_allclose(M, Mo, rtol=1e-12, atol=1e-14)
