@@ -1532,7 +1532,8 @@ struct Workspace {
   DevBuf<char> d_cand_in[4], d_cand_res[4], d_cand_work[4];
   DevBuf<double> d_e5;                 // five-point solver: the matrices of a slab of samples
   DevBuf<double> d_pair_inv_scale;     // matrix-core scoring: per-pair power-of-two inverse scale
-  DevBuf<MxPoint> d_mxp;               // matrix-core scoring: per-point operands and error bounds
+  DevBuf<uint16_t> d_mxp;              // matrix-core scoring: per-point operands and error bounds
+  int64_t mx_total = 0;                // points of the run (d_mxp's planes)
   bool mx_on = false;                  // this run scores candidate chunks on the matrix cores
   int mx_max_n = 0;                    // largest pair of the run (candidate-mask rows)
   DevBuf<uint32_t> d_mx_mask;          // matrix-core scoring: candidate masks of one list segment
@@ -2140,7 +2141,8 @@ struct Engine : Workspace {
       for (int i = 0; i < np; ++i) mx_max_n = std::max(mx_max_n, (int)nn[(size_t)i]);
       d_mx_mask.ensure(mx_mask_words(mx_max_n));
       d_pair_inv_scale.ensure(np);
-      d_mxp.ensure((size_t)total);
+      mx_total = total;
+      d_mxp.ensure((size_t)(kMxPointHalves * total));
       launch_mx_prepare(stream, d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pt_pair.p, np, total, d_pair_inv_scale.p,
                         d_mxp.p);
     }
@@ -2541,7 +2543,7 @@ struct Engine : Workspace {
       const int t1 = prof.start("score_h", 0.0);
       if (mx)
         launch_score_mx(stream, 0, d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pair_sq_thr.p, d_pair_inv_scale.p,
-                        d_mxp.p, d_cand_models, d_cpair, d_status, tot, d_counts, d_values, nullptr, 1,
+                        d_mxp.p, mx_total, d_cand_models, d_cpair, d_status, tot, d_counts, d_values, nullptr, 1,
                         d_work_list, d_work_count, d_blk, mx_max_n, d_mx_mask.p);
       else
         launch_score(stream, 0, d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pair_sq_thr.p, d_cand_models, d_cpair,
@@ -2581,7 +2583,7 @@ struct Engine : Workspace {
       const int t1 = prof.start(kind == GCR_PROBLEM_ESSENTIAL ? "score_e" : "score_f", 0.0);
       if (mx)
         launch_score_mx(stream, 1, d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pair_sq_thr.p, d_pair_inv_scale.p,
-                        d_mxp.p, d_cand_models, d_cpair, d_status, (int64_t)ns, d_counts, d_values, d_sym, S,
+                        d_mxp.p, mx_total, d_cand_models, d_cpair, d_status, (int64_t)ns, d_counts, d_values, d_sym, S,
                         d_work_list, d_work_count, d_blk, mx_max_n, d_mx_mask.p);
       else
         launch_score(stream, 1, d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pair_sq_thr.p, d_cand_models,

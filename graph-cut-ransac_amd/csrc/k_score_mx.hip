@@ -4,13 +4,13 @@
 // MSAC scoring (scoring_function.h:137-233) of a model over a pair's points is
 // a dense contraction: for the Sampson distance (fundamental_estimator.h:
 // 195-222) the numerator is C = x2^T F x1 = vec(F) . z with
-// z = x2 (x) x1 = (x2x1, x2y1, x2, y2x1, y2y1, y2, x1, y1, 1), and the four
-// denominator terms (F x1)_0,1 and (F^T x2)_0,1 are linear in z as well.  For
+// z = x2 (x) x1 = (x2x1, x2y1, x2, y2x1, y2y1, y2, x1, y1, 1), and the
+// denominator is linear in 11 squared terms.  For
 // the homography transfer error (homography_estimator.h:181-199) the
 // quantities P = x2 w - u, Q = y2 w - v and W = w (u, v, w = H x1) are linear
 // in z, with r^2 = (P^2 + Q^2) / W^2.  So one wave scores 32 models x 32
-// points per step as five (Sampson) or three (transfer) 32x32 MFMA tiles
-// whose reduction dimension holds the z terms.
+// points per step as two (Sampson) or three (transfer) 32x32 MFMA tiles
+// whose reduction dimension holds the terms.
 //
 // Precision.  Points are scaled by a per-pair power of two 1/s (exact) so
 // that |x'| <= 1, models to F'' = S F S / m (S = diag(s, s, 1), m = max |.|,
@@ -23,11 +23,15 @@
 // 2^-22 relative each, the dropped lo*lo term 2^-22, FP32 rounding of z
 // 2^-24, FP32 accumulation of 27 exact products 27 * 2^-24, FP16 subnormal
 // spacing 2^-24); with |c_t| <= 1 the kernel uses delta = 2^-17 S + 2^-20,
-// S the sum of |z_t| over the terms the quantity reads (C: (1 + |x1| + |y1|)
-// (1 + |x2| + |y2|); (F x1): 1 + |x1| + |y1|; (F^T x2): 1 + |x2| + |y2|).
+// S the sum of |z_t| over the terms the quantity reads (C, P, Q: (1 + |x1| +
+// |y1|) (1 + |x2| + |y2|); W: 1 + |x1| + |y1|).  The Sampson denominator
+// |(F x1)_01|^2 + |(F^T x2)_01|^2 is a linear form too, in the 11 squared terms
+// (x1^2, x1 y1, y1^2, x1, y1, the same of the second image, 1); a quarter of it,
+// D, has |coefficients| <= 1, and 11 + 10 + 11 products fill the 32 (the lo of
+// the 1 is 0), so its bound is the same with 32 terms: dD = 2^-17 S + 2^-20.
 //
 // A point is dropped for a model only when the bounds prove it an outlier:
-// Sampson (|C| - dC)^2 > tau''^2 (1 + 2^-16) sum (|q| + dq)^2, transfer
+// Sampson (|C| - dC)+^2 > 4 tau''^2 (1 + 2^-16) (D + dD), transfer
 // (|P| - dP)+^2 + (|Q| - dQ)+^2 > tau''^2 (1 + 2^-16) (|W| + dW)^2 (the
 // factor 1 + 2^-16 covers the FP32 rounding of the test itself, about
 // 10 * 2^-24).  Every other point -- all inliers and every point near the
@@ -57,12 +61,21 @@ constexpr int kMxBlocks = 2048;         // persistent grids: at most 8,192 waves
 // kMxSegMax (each segment costs three launches; the masks bound the memory)
 constexpr int64_t kMxSegMin = 65536, kMxSegMax = 1048576;
 constexpr int64_t kMxMaskBudget = 512ll << 20;
-constexpr int kMxSlice = 128;           // points per rejection work item
+// points per rejection work item: as many as leave kMxItems items (a tenth of
+// the model slots hold a model to score at worst), between kMxSliceMin and
+// kMxSliceMax (every item reads its 32 models' operands once)
+constexpr int kMxSliceMin = 128, kMxSliceMax = 1024;
+constexpr int64_t kMxItems = 16384;
+constexpr int64_t kMxPlaneHalves = 16;  // 16-bit words of a point in one operand plane
 constexpr int kNumXcd = 8;
 
 __device__ __forceinline__ f32x16 mfma16(const h8& a, const h8& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
+
+// v with lane `lane` replaced by the scalar x (clang 20 has no builtin for it)
+extern "C" __device__ __attribute__((const)) uint32_t gcr_writelane(uint32_t x, uint32_t lane,
+                                                                    uint32_t v) __asm("llvm.amdgcn.writelane.i32");
 
 __device__ __forceinline__ f32x16 zero16() {
   f32x16 z;
@@ -71,27 +84,11 @@ __device__ __forceinline__ f32x16 zero16() {
   return z;
 }
 
-// Reduction-dimension layout of one quantity (k = 0..31): k < 9 hi*hi of
-// term k, 9..17 hi(coef)*lo(z) of term k-9, 18..26 lo(coef)*hi(z) of term
-// k-18, 27..31 zero.  Lane half hf of MFMA kh holds k = 16 kh + 8 hf + e.
-__device__ __forceinline__ h8 coef_slice(const _Float16* hi, const _Float16* lo, int kh, int hf) {
-  h8 v;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int k0 = 16 * kh + e, k1 = 16 * kh + 8 + e;
-    const _Float16 a0 = k0 < 9 ? hi[k0] : (k0 < 18 ? hi[k0 - 9] : (k0 < 27 ? lo[k0 - 18] : (_Float16)0.0f));
-    const _Float16 a1 = k1 < 9 ? hi[k1] : (k1 < 18 ? hi[k1 - 9] : (k1 < 27 ? lo[k1 - 18] : (_Float16)0.0f));
-    v[e] = hf ? a1 : a0;
-  }
-  return v;
-}
-
-// One model's coefficient vectors over z (row-major 3x3 M): Sampson
-// quantities C, (F x1)_0, (F x1)_1, (F^T x2)_0, (F^T x2)_1; transfer
-// quantities P, Q, W.
+// One model's coefficient vectors over z (row-major 3x3 M): Sampson C;
+// transfer P, Q, W.
 template <int KIND>
 __device__ __forceinline__ void quantity_coefs(const double* F, double c[][9]) {
-  constexpr int NQ = KIND == 1 ? 5 : 3;
+  constexpr int NQ = KIND == 1 ? 1 : 3;
 #pragma unroll
   for (int q = 0; q < NQ; ++q)
 #pragma unroll
@@ -99,14 +96,29 @@ __device__ __forceinline__ void quantity_coefs(const double* F, double c[][9]) {
   if constexpr (KIND == 1) {
 #pragma unroll
     for (int t = 0; t < 9; ++t) c[0][t] = F[t];
-    c[1][6] = F[0]; c[1][7] = F[1]; c[1][8] = F[2];
-    c[2][6] = F[3]; c[2][7] = F[4]; c[2][8] = F[5];
-    c[3][2] = F[0]; c[3][5] = F[3]; c[3][8] = F[6];
-    c[4][2] = F[1]; c[4][5] = F[4]; c[4][8] = F[7];
   } else {
     c[0][0] = F[6]; c[0][1] = F[7]; c[0][2] = F[8]; c[0][6] = -F[0]; c[0][7] = -F[1]; c[0][8] = -F[2];
     c[1][3] = F[6]; c[1][4] = F[7]; c[1][5] = F[8]; c[1][6] = -F[3]; c[1][7] = -F[4]; c[1][8] = -F[5];
     c[2][6] = F[6]; c[2][7] = F[7]; c[2][8] = F[8];
+  }
+}
+
+// A quarter of the Sampson denominator (F x1)_0^2 + (F x1)_1^2 + (F^T x2)_0^2 +
+// (F^T x2)_1^2 as a linear form in d = (x1^2, x1 y1, y1^2, x1, y1, the same of
+// the second image, 1): every coefficient is at most 1 when |F| <= 1.
+__device__ __forceinline__ void denominator_coefs(const double* F, double g[11]) {
+  const double a[2][3] = {{F[0], F[1], F[2]}, {F[3], F[4], F[5]}};
+  const double b[2][3] = {{F[0], F[3], F[6]}, {F[1], F[4], F[7]}};
+  g[10] = 0.0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const double(*r)[3] = h ? b : a;
+    g[5 * h] = 0.25 * (r[0][0] * r[0][0] + r[1][0] * r[1][0]);
+    g[5 * h + 1] = 0.5 * (r[0][0] * r[0][1] + r[1][0] * r[1][1]);
+    g[5 * h + 2] = 0.25 * (r[0][1] * r[0][1] + r[1][1] * r[1][1]);
+    g[5 * h + 3] = 0.5 * (r[0][0] * r[0][2] + r[1][0] * r[1][2]);
+    g[5 * h + 4] = 0.5 * (r[0][1] * r[0][2] + r[1][1] * r[1][2]);
+    g[10] += 0.25 * (r[0][2] * r[0][2] + r[1][2] * r[1][2]);
   }
 }
 
@@ -150,43 +162,69 @@ __global__ void __launch_bounds__(256) k_mx_pair_scale(const double* __restrict_
   }
 }
 
-// Per point: the B-operand slices of both lane halves (k order, FP16) and
-// the three error bounds.
+// k of the reduction dimension of a quantity of T terms -> (hi, lo) element:
+// k < T hi*hi of term k, then hi(coef)*lo(z) of the terms but the last when L is
+// T - 1 (its z is 1, whose lo is 0), then lo(coef)*hi(z), zero beyond.
+template <int T, int L>
+__device__ __forceinline__ _Float16 k_elem(const _Float16* first, const _Float16* second, const _Float16* third,
+                                           int k) {
+  return k < T ? first[k] : (k < T + L ? second[k - T] : (k < 2 * T + L ? third[k - T - L] : (_Float16)0.0f));
+}
+
+// Per point: the B-operand slices of both lane halves (k order, FP16) of z and
+// of the squared terms d, and the error bounds; a plane per MFMA, so that a
+// wave's load of 32 points is one contiguous kilobyte.
 __global__ void __launch_bounds__(256) k_mx_points(const double* __restrict__ pts,
                                                    const int32_t* __restrict__ pt_pair,
                                                    const double* __restrict__ inv_scale, int64_t total,
-                                                   MxPoint* __restrict__ out) {
+                                                   uint16_t* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= total) return;
   const double is = inv_scale[pt_pair[i]];
   const double x1 = pts[4 * i] * is, y1 = pts[4 * i + 1] * is, x2 = pts[4 * i + 2] * is, y2 = pts[4 * i + 3] * is;
   const double zd[9] = {x2 * x1, x2 * y1, x2, y2 * x1, y2 * y1, y2, x1, y1, 1.0};
-  _Float16 hi[9], lo[9];
+  const double dd[11] = {x1 * x1, x1 * y1, y1 * y1, x1, y1, x2 * x2, x2 * y2, y2 * y2, x2, y2, 1.0};
+  h8* const o = reinterpret_cast<h8*>(out);
+  _Float16 hi[11], lo[11];
 #pragma unroll
   for (int t = 0; t < 9; ++t) {
     const float z = (float)zd[t];
     hi[t] = (_Float16)z;
     lo[t] = (_Float16)(z - (float)hi[t]);
   }
-  MxPoint o;
 #pragma unroll
   for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
+      h8 v;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int k = 16 * kh + 8 * hf + e;
-        const _Float16 v = k < 9 ? hi[k] : (k < 18 ? lo[k - 9] : (k < 27 ? hi[k - 18] : (_Float16)0.0f));
-        o.b[kh][hf][e] = __builtin_bit_cast(uint16_t, v);
-      }
+      for (int e = 0; e < 8; ++e) v[e] = k_elem<9, 9>(hi, lo, hi, 16 * kh + 8 * hf + e);
+      o[(kh * total + i) * 2 + hf] = v;
     }
-  const float sa = 1.0f + fabsf((float)x1) + fabsf((float)y1);
-  const float sb = 1.0f + fabsf((float)x2) + fabsf((float)y2);
-  o.d[0] = kDeltaRel * (sa * sb) + kDeltaAbs;
-  o.d[1] = kDeltaRel * sa + kDeltaAbs;
-  o.d[2] = kDeltaRel * sb + kDeltaAbs;
-  o.d[3] = 0.0f;
-  out[i] = o;
+#pragma unroll
+  for (int t = 0; t < 11; ++t) {
+    const float z = (float)dd[t];
+    hi[t] = (_Float16)z;
+    lo[t] = (_Float16)(z - (float)hi[t]);
+  }
+#pragma unroll
+  for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      h8 v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = k_elem<11, 10>(hi, lo, hi, 16 * kh + 8 * hf + e);
+      o[((2 + kh) * total + i) * 2 + hf] = v;
+    }
+  const float ax = fabsf((float)x1), ay = fabsf((float)y1), bx = fabsf((float)x2), by = fabsf((float)y2);
+  const float sa = 1.0f + ax + ay, sb = 1.0f + bx + by;
+  const float sd = 1.0f + ax * sa + ay * (1.0f + ay) + bx * sb + by * (1.0f + by);
+  float4 d;
+  d.x = kDeltaRel * (sa * sb) + kDeltaAbs;
+  d.y = kDeltaRel * sa + kDeltaAbs;
+  d.z = kDeltaRel * sd + kDeltaAbs;
+  d.w = 0.0f;
+  reinterpret_cast<float4*>(out + kMxPlaneHalves * 4 * total)[i] = d;
 }
 
 // ---- ordered compaction of the active model slots ------------------------------
@@ -283,7 +321,7 @@ __global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pai
                                                   const int32_t* __restrict__ list,
                                                   const uint32_t* __restrict__ list_count, int64_t seg_begin,
                                                   int64_t seg_len, h8* __restrict__ coefs, int slots_per) {
-  constexpr int NQ = KIND == 1 ? 5 : 3;
+  constexpr int NQ = KIND == 1 ? 2 : 3;
   const int64_t total = (int64_t)*list_count;
   if (seg_begin >= total) return;
   const int64_t seg_n = total - seg_begin < seg_len ? total - seg_begin : seg_len;
@@ -319,19 +357,42 @@ __global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pai
   const double inv_mx = lp_ok ? 1.0 / mx : 0.0;
 #pragma unroll
   for (int k = 0; k < 9; ++k) Fs[k] = Fs[k] * inv_mx;
-  double cq[NQ][9];
+  double cq[3][9];
   quantity_coefs<KIND>(Fs, cq);
   h8* out = coefs + (e * 2 + hf) * (2 * NQ);
+  _Float16 hi[11], lo[11];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    _Float16 hi[9], lo[9];
+  for (int q = 0; q < (KIND == 1 ? 1 : 3); ++q) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
       hi[k] = (_Float16)cq[q][k];
       lo[k] = (_Float16)(cq[q][k] - (double)hi[k]);
     }
-    out[2 * q] = coef_slice(hi, lo, 0, hf);
-    out[2 * q + 1] = coef_slice(hi, lo, 1, hf);
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      h8 v;
+#pragma unroll
+      for (int x = 0; x < 8; ++x)
+        v[x] = hf ? k_elem<9, 9>(hi, hi, lo, 16 * kh + 8 + x) : k_elem<9, 9>(hi, hi, lo, 16 * kh + x);
+      out[2 * q + kh] = v;
+    }
+  }
+  if constexpr (KIND == 1) {
+    double g[11];
+    denominator_coefs(Fs, g);
+#pragma unroll
+    for (int k = 0; k < 11; ++k) {
+      hi[k] = (_Float16)g[k];
+      lo[k] = (_Float16)(g[k] - (double)hi[k]);
+    }
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      h8 v;
+#pragma unroll
+      for (int x = 0; x < 8; ++x)
+        v[x] = hf ? k_elem<11, 10>(hi, hi, lo, 16 * kh + 8 + x) : k_elem<11, 10>(hi, hi, lo, 16 * kh + x);
+      out[2 + kh] = v;
+    }
   }
 }
 
@@ -339,23 +400,23 @@ __global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pai
 
 // Work item (tile t, slice j): the 32 list entries 32 t .. 32 t + 31 of the
 // segment (slot order, so the entries of one pair are adjacent; a tile that
-// spans pairs is handled pair by pair) against points 128 j .. 128 j + 127 of
-// their pair.  Lane r < 32 owns entry r and writes, per 32-point chunk, the
+// spans pairs is handled pair by pair) against points slice j .. slice j + slice
+// - 1 of their pair.  Lane r < 32 owns entry r and writes, per 32-point chunk, the
 // 32-bit word of its candidate mask (bit b: point base + b must be evaluated
 // in FP64).  Words of points at or beyond the pair's n are not written.
 template <int KIND>
-__global__ void __launch_bounds__(256) k_mx_reject(const int64_t* __restrict__ pair_pt_off,
+__global__ void __launch_bounds__(256, 4) k_mx_reject(const int64_t* __restrict__ pair_pt_off,
                                                    const int32_t* __restrict__ pair_n,
                                                    const double* __restrict__ pair_sq_thr,
                                                    const double* __restrict__ pair_inv_scale,
-                                                   const MxPoint* __restrict__ mxp,
+                                                   const uint16_t* __restrict__ mxp, int64_t mx_total,
                                                    const h8* __restrict__ coefs,
                                                    const int32_t* __restrict__ model_pair,
                                                    const int32_t* __restrict__ list,
                                                    const uint32_t* __restrict__ list_count, int64_t seg_begin,
-                                                   int64_t seg_len, int slices, int words, uint32_t* __restrict__ mask,
+                                                   int64_t seg_len, int slice, int slices, int words, uint32_t* __restrict__ mask,
                                                    int slots_per) {
-  constexpr int NQ = KIND == 1 ? 5 : 3;
+  constexpr int NQ = KIND == 1 ? 2 : 3;
   const int lane = lane_id();
   const int hf = lane >> 5, r = lane & 31;
   const int64_t total = (int64_t)*list_count;
@@ -366,7 +427,7 @@ __global__ void __launch_bounds__(256) k_mx_reject(const int64_t* __restrict__ p
   // which takes a contiguous range of items (adjacent items share a pair)
   const int xcd = (int)(blockIdx.x % kNumXcd);
   const int64_t waves_per_xcd = (int64_t)(gridDim.x / kNumXcd) * 4;
-  const int64_t w = (int64_t)(blockIdx.x / kNumXcd) * 4 + (threadIdx.x >> 6);
+  const int64_t w = (int64_t)(blockIdx.x / kNumXcd) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t lo_u = items * xcd / kNumXcd, hi_u = items * (xcd + 1) / kNumXcd;
   for (int64_t u = lo_u + w; u < hi_u; u += waves_per_xcd) {
     const int64_t t = u / slices;
@@ -382,7 +443,7 @@ __global__ void __launch_bounds__(256) k_mx_reject(const int64_t* __restrict__ p
       const bool mine = r >= done && r < cnt_all && my_pair == p;
       const int sub_end = done + __popcll(ballot64(mine) & 0xffffffffull);
       const int n = pair_n[p];
-      const int first = kMxSlice * j;
+      const int first = slice * j;
       if (first < n) {
         // the sub-tile's A operands (lane: row r, half hf); other rows zero
         h8 A[NQ][2];
@@ -400,49 +461,38 @@ __global__ void __launch_bounds__(256) k_mx_reject(const int64_t* __restrict__ p
           }
         const double is = pair_inv_scale[p];
         const float tau2m = (float)(pair_sq_thr[p] * is * is * kTauMargin);
-        const MxPoint* __restrict__ X = mxp + pair_pt_off[p];
-        const int last = first + kMxSlice < n ? first + kMxSlice : n;
+        const int64_t off = pair_pt_off[p];
+        const h8* __restrict__ Z = reinterpret_cast<const h8*>(mxp) + 2 * off + hf;
+        const float4* __restrict__ D = reinterpret_cast<const float4*>(mxp + kMxPlaneHalves * 4 * mx_total) + off;
+        const int last = first + slice < n ? first + slice : n;
         for (int base = first; base < last; base += 32) {
-          const int i = base + r;
-          h8 b0, b1;
-          float dq0 = 0.0f, dq1 = 0.0f, dq2 = 0.0f;
-          const bool pin = i < n;
-          if (pin) {
-            const MxPoint& x = X[i];
-            b0 = *reinterpret_cast<const h8*>(x.b[0][hf]);
-            b1 = *reinterpret_cast<const h8*>(x.b[1][hf]);
-            dq0 = x.d[0];
-            dq1 = x.d[1];
-            dq2 = x.d[2];
-          } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              b0[e] = (_Float16)0.0f;
-              b1[e] = (_Float16)0.0f;
-            }
-          }
-          // accumulator slot j holds row 8 (j / 4) + 4 hf + (j % 4) of column r
-          uint64_t keep[16];
+          // points beyond the pair read its last one; their bits are cut below
+          const int i = base + r < n ? base + r : n - 1;
+          const h8 b0 = Z[2 * i], b1 = Z[2 * (mx_total + i)];
+          const float4 dq = D[i];
+          // accumulator slot j holds row 8 (j / 4) + 4 hf + (j % 4) of column
+          // r; the ballot's halves are the words of its two rows, which go to
+          // the lanes of those rows
+          const uint32_t live = last - base < 32 ? (1u << (last - base)) - 1u : ~0u;  // uniform
+          uint32_t word = 0;
+          auto put = [&](int jj, bool rej) {
+            const uint64_t k = ballot64(!rej);
+            const int row = 8 * (jj >> 2) + (jj & 3);
+            word = gcr_writelane((uint32_t)k, row, word);
+            word = gcr_writelane((uint32_t)(k >> 32), row + 4, word);
+          };
           if constexpr (KIND == 1) {
-            f32x16 den = zero16();
-#pragma unroll
-            for (int q = 1; q < 5; ++q) {
-              f32x16 a = mfma16(A[q][0], b0, zero16());
-              a = mfma16(A[q][1], b1, a);
-              const float dlt = q < 3 ? dq1 : dq2;
-#pragma unroll
-              for (int jj = 0; jj < 16; ++jj) {
-                const float uu = fabsf(a[jj]) + dlt;
-                den[jj] = __builtin_fmaf(uu, uu, den[jj]);
-              }
-            }
+            const h8 b2 = Z[2 * (2 * mx_total + i)], b3 = Z[2 * (3 * mx_total + i)];
             f32x16 c = mfma16(A[0][0], b0, zero16());
+            f32x16 den = mfma16(A[1][0], b2, zero16());
             c = mfma16(A[0][1], b1, c);
+            den = mfma16(A[1][1], b3, den);
+            const float k1 = 4.0f * tau2m;
+            const float k2 = k1 * dq.z;
 #pragma unroll
             for (int jj = 0; jj < 16; ++jj) {
-              const float cl = fabsf(c[jj]) - dq0;
-              const bool rej = cl > 0.0f && cl * cl > den[jj] * tau2m;
-              keep[jj] = ballot64(pin && !rej);
+              const float cl = fabsf(c[jj]) - dq.x;
+              put(jj, cl * fabsf(cl) > __builtin_fmaf(den[jj], k1, k2));
             }
           } else {
             f32x16 pp = mfma16(A[0][0], b0, zero16());
@@ -453,20 +503,13 @@ __global__ void __launch_bounds__(256) k_mx_reject(const int64_t* __restrict__ p
             ww = mfma16(A[2][1], b1, ww);
 #pragma unroll
             for (int jj = 0; jj < 16; ++jj) {
-              const float pl = fmaxf(fabsf(pp[jj]) - dq0, 0.0f);
-              const float ql = fmaxf(fabsf(qq[jj]) - dq0, 0.0f);
-              const float wu = fabsf(ww[jj]) + dq1;
-              const bool rej = __builtin_fmaf(pl, pl, ql * ql) > wu * wu * tau2m;
-              keep[jj] = ballot64(pin && !rej);
+              const float pl = fmaxf(fabsf(pp[jj]) - dq.x, 0.0f);
+              const float ql = fmaxf(fabsf(qq[jj]) - dq.x, 0.0f);
+              const float wu = fabsf(ww[jj]) + dq.y;
+              put(jj, __builtin_fmaf(pl, pl, ql * ql) > wu * wu * tau2m);
             }
           }
-          // lane r (< 32) stores row r's word: slot j = 4 (r / 8) + r % 4,
-          // bits 32 ((r / 4) % 2) .. +31 of that slot's ballot
-          const int jr = 4 * (r >> 3) + (r & 3), hr = (r >> 2) & 1;
-          uint64_t sel = 0;
-#pragma unroll
-          for (int jj = 0; jj < 16; ++jj) sel = jr == jj ? keep[jj] : sel;
-          if (mine && hf == 0) my_mask[base >> 5] = (uint32_t)(sel >> (32 * hr));
+          if (mine && hf == 0) my_mask[base >> 5] = word & live;
         }
       }
       done = sub_end;
@@ -476,9 +519,10 @@ __global__ void __launch_bounds__(256) k_mx_reject(const int64_t* __restrict__ p
 
 // ---- phase 2: the FP64 decisions and the in-order MSAC sums -----------------------
 
-// One wave per list entry of the segment.  The candidate points (mask bits)
-// are queued in point order and evaluated 64 at a time by the whole wave with
-// the FP64 kernel's operations; inliers are accumulated in point order
+// One wave per list entry of the segment.  The mask row is taken 64 words
+// (2,048 points) at a time, a word per lane: a prefix sum of the bit counts
+// gives every lane its place in the queue of candidate points (point order),
+// which the whole wave evaluates 64 at a time with the FP64 kernel's operations; inliers are accumulated in point order
 // through the scalar unit (value -= r2), as the FP64 kernel does.
 template <int KIND>
 __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts,
@@ -492,7 +536,7 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
                                                   int64_t seg_len, int words, const uint32_t* __restrict__ mask,
                                                   int32_t* __restrict__ counts, double* __restrict__ values,
                                                   int32_t* __restrict__ sym_counts, int slots_per) {
-  __shared__ int32_t queue[4][128];
+  __shared__ int32_t queue[4][64 + 64 * 32];
   const int lane = lane_id();
   int32_t* q = queue[threadIdx.x >> 6];
   const int64_t total = (int64_t)*list_count;
@@ -515,13 +559,13 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
     double acc = 0.0;
     int64_t cnt = 0, scnt = 0;
     int qn = 0;
-    // evaluates the first cnt_flush queued candidates and accumulates the
+    // evaluates the cnt_flush queued candidates from `at` on and accumulates the
     // inliers among them in queue (= point) order
-    auto flush = [&](int cnt_flush) {
+    auto flush = [&](int at, int cnt_flush) {
       bool in = false, sym_in = false;
       double r2 = 0.0;
       if (lane < cnt_flush) {
-        const double* s = P + 4 * (int64_t)q[lane];
+        const double* s = P + 4 * (int64_t)q[at + lane];
         if constexpr (KIND == 1) {
           double num, den;
           f_sampson_parts(s, M, num, den);
@@ -547,39 +591,37 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
       }
     };
     const int nw = (n + 31) >> 5;
-    // the mask row is read 256 words (8,192 points) at a time, 4 words per
-    // lane, coalesced; the walk then takes the words from the lanes that hold
-    // them, so no memory access sits inside the point loop
-    for (int w0 = 0; w0 < nw; w0 += 256) {
-      uint32_t held[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int wi = w0 + 64 * k + lane;
-        held[k] = wi < nw ? mk[wi] : 0u;
+    uint32_t next = lane < nw ? mk[lane] : 0u;
+    for (int w0 = 0; w0 < nw; w0 += 64) {
+      uint32_t bits = next;
+      next = w0 + 64 + lane < nw ? mk[w0 + 64 + lane] : 0u;
+      int before = __popc(bits);
+      const int have = before;
+      // inclusive prefix over the wave: inside the rows of 16 lanes, then the
+      // rows before
+      before += __builtin_amdgcn_update_dpp(0, before, 0x111, 0xF, 0xF, true);  // row_shr:1
+      before += __builtin_amdgcn_update_dpp(0, before, 0x112, 0xF, 0xF, true);  // row_shr:2
+      before += __builtin_amdgcn_update_dpp(0, before, 0x114, 0xF, 0xF, true);  // row_shr:4
+      before += __builtin_amdgcn_update_dpp(0, before, 0x118, 0xF, 0xF, true);  // row_shr:8
+      const int t0 = __builtin_amdgcn_readlane(before, 15), t1 = t0 + __builtin_amdgcn_readlane(before, 31),
+                t2 = t1 + __builtin_amdgcn_readlane(before, 47), t3 = t2 + __builtin_amdgcn_readlane(before, 63);
+      before += lane >= 48 ? t2 : (lane >= 32 ? t1 : (lane >= 16 ? t0 : 0));
+      int at = qn + before - have;
+      while (bits) {
+        q[at++] = 32 * (w0 + lane) + __ffs(bits) - 1;
+        bits &= bits - 1u;
       }
-      const int wend = nw - w0 < 256 ? nw - w0 : 256;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        for (int t = 0; t < 64 && 64 * k + t < wend; t += 2) {
-          const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)held[k], t);
-          const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)held[k], t + 1);
-          const uint64_t bits = lo | (hi << 32);
-          if (bits == 0) continue;
-          const int wi = w0 + 64 * k + t;
-          const bool c = (bits >> lane) & 1ull;
-          if (c) q[qn + __popcll(bits & ((1ull << lane) - 1ull))] = 32 * wi + lane;
-          qn += __popcll(bits);
-          if (qn >= 64) {
-            flush(64);
-            const int rest = qn - 64;
-            const int32_t moved = lane < rest ? q[64 + lane] : 0;
-            if (lane < rest) q[lane] = moved;
-            qn = rest;
-          }
-        }
+      qn += t3;
+      int h = 0;
+      for (; h + 64 <= qn; h += 64) flush(h, 64);
+      if (h > 0) {
+        const int rest = qn - h;
+        const int32_t moved = lane < rest ? q[h + lane] : 0;
+        if (lane < rest) q[lane] = moved;
+        qn = rest;
       }
     }
-    flush(qn);
+    flush(0, qn);
     if (lane == 0) {
       counts[slot] = (int32_t)cnt;
       values[slot] = cnt == 0 ? 0.0 : (acc + (double)cnt * thr) / thr;
@@ -591,7 +633,7 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
 // ---- launchers --------------------------------------------------------------------
 
 void launch_mx_prepare(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
-                       const int32_t* pt_pair, int num_pairs, int64_t total, double* inv_scale, MxPoint* out) {
+                       const int32_t* pt_pair, int num_pairs, int64_t total, double* inv_scale, uint16_t* out) {
   if (num_pairs <= 0 || total <= 0) return;
   hipLaunchKernelGGL(k_mx_pair_scale, dim3((unsigned)num_pairs), dim3(256), 0, st, pts, pair_pt_off, pair_n,
                      num_pairs, inv_scale);
@@ -606,17 +648,18 @@ size_t mx_list_scratch_ints(int64_t num_models) {
 static int64_t mx_segment(int max_n) {
   const int64_t words = (max_n + 31) / 32 + 1;
   const int64_t fit = kMxMaskBudget / (4 * words);
-  return fit < kMxSegMin ? kMxSegMin : (fit > kMxSegMax ? kMxSegMax : fit);
+  // (a multiple of 32: whole tiles, and the operands behind the masks stay aligned)
+  return fit < kMxSegMin ? kMxSegMin : (fit > kMxSegMax ? kMxSegMax : fit & ~(int64_t)31);
 }
 
 size_t mx_mask_words(int max_n) {
-  // the candidate masks, then the segment's A operands (5 x 2 x 2 x 16 B per entry)
+  // the candidate masks, then the segment's A operands (at most 3 x 2 x 2 x 16 B per entry)
   const int64_t seg = mx_segment(max_n);
-  return (size_t)seg * (size_t)((max_n + 31) / 32 + 1) + (size_t)seg * 80;
+  return (size_t)seg * (size_t)((max_n + 31) / 32 + 1) + (size_t)seg * 48;
 }
 
 void launch_score_mx(hipStream_t st, int kind, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
-                     const double* pair_sq_thr, const double* pair_inv_scale, const MxPoint* mxp,
+                     const double* pair_sq_thr, const double* pair_inv_scale, const uint16_t* mxp, int64_t mx_total,
                      const double* models, const int32_t* model_pair, const int8_t* active, int64_t num_models,
                      int32_t* counts, double* values, int32_t* sym_counts, int slots_per, int32_t* work_list,
                      uint32_t* work_count, int32_t* blk_scratch, int max_n, uint32_t* mask) {
@@ -626,7 +669,9 @@ void launch_score_mx(hipStream_t st, int kind, const double* pts, const int64_t*
                      sym_counts, blk_scratch);
   hipLaunchKernelGGL(k_mx_scan, dim3(1), dim3(1024), 0, st, blk_scratch, nblk, work_count);
   hipLaunchKernelGGL(k_mx_write, dim3((unsigned)nblk), dim3(256), 0, st, active, num_models, blk_scratch, work_list);
-  const int slices = (max_n + kMxSlice - 1) / kMxSlice;
+  int slice = kMxSliceMin;
+  while (slice < kMxSliceMax && (num_models / 320 + 1) * ((max_n + 2 * slice - 1) / (2 * slice)) >= kMxItems) slice *= 2;
+  const int slices = (max_n + slice - 1) / slice;
   const int words = (max_n + 31) / 32 + 1;
   const int64_t segment = mx_segment(max_n);
   h8* const coefs = reinterpret_cast<h8*>(mask + (size_t)segment * (size_t)words);
@@ -645,7 +690,7 @@ void launch_score_mx(hipStream_t st, int kind, const double* pts, const int64_t*
       hipLaunchKernelGGL(k_mx_coefs<0>, dim3(bc), dim3(256), 0, st, pair_inv_scale, models, model_pair, work_list,
                          work_count, seg, seg_len, coefs, slots_per);
       hipLaunchKernelGGL(k_mx_reject<0>, dim3((unsigned)b1), dim3(256), 0, st, pair_pt_off, pair_n, pair_sq_thr,
-                         pair_inv_scale, mxp, coefs, model_pair, work_list, work_count, seg, seg_len, slices, words,
+                         pair_inv_scale, mxp, mx_total, coefs, model_pair, work_list, work_count, seg, seg_len, slice, slices, words,
                          mask, slots_per);
       hipLaunchKernelGGL(k_mx_exact<0>, dim3((unsigned)b2), dim3(256), 0, st, pts, pair_pt_off, pair_n, pair_sq_thr,
                          models, model_pair, work_list, work_count, seg, seg_len, words, mask, counts, values,
@@ -654,7 +699,7 @@ void launch_score_mx(hipStream_t st, int kind, const double* pts, const int64_t*
       hipLaunchKernelGGL(k_mx_coefs<1>, dim3(bc), dim3(256), 0, st, pair_inv_scale, models, model_pair, work_list,
                          work_count, seg, seg_len, coefs, slots_per);
       hipLaunchKernelGGL(k_mx_reject<1>, dim3((unsigned)b1), dim3(256), 0, st, pair_pt_off, pair_n, pair_sq_thr,
-                         pair_inv_scale, mxp, coefs, model_pair, work_list, work_count, seg, seg_len, slices, words,
+                         pair_inv_scale, mxp, mx_total, coefs, model_pair, work_list, work_count, seg, seg_len, slice, slices, words,
                          mask, slots_per);
       hipLaunchKernelGGL(k_mx_exact<1>, dim3((unsigned)b2), dim3(256), 0, st, pts, pair_pt_off, pair_n, pair_sq_thr,
                          models, model_pair, work_list, work_count, seg, seg_len, words, mask, counts, values,

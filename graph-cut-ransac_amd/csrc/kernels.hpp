@@ -31,21 +31,18 @@ void launch_score(hipStream_t st, int kind, const double* pts, const int64_t* pa
 
 // Candidate scoring on the matrix cores (FP16 hi/lo MFMA rejection of
 // proven outliers, FP64 in point order for every other point; same results as
-// launch_score).  MxPoint: one point's B-operand slices (FP16 bits, k order,
-// [MFMA][lane half][8]) and error bounds; launch_mx_prepare fills them and
-// the per-pair power-of-two inverse scale once per engine run.
-struct alignas(16) MxPoint {
-  uint16_t b[2][2][8];
-  float d[4];
-};
+// launch_score).  launch_mx_prepare fills the points' B operands and error
+// bounds (kMxPointHalves 16-bit words a point) and the per-pair power-of-two
+// inverse scale once per engine run; mx_total is its `total`.
+constexpr int64_t kMxPointHalves = 72;
 void launch_mx_prepare(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
-                       const int32_t* pt_pair, int num_pairs, int64_t total, double* inv_scale, MxPoint* out);
+                       const int32_t* pt_pair, int num_pairs, int64_t total, double* inv_scale, uint16_t* out);
 // ints of blk_scratch that launch_score_mx needs for num_models slots, and
 // words of its candidate mask for pairs of at most max_n points
 size_t mx_list_scratch_ints(int64_t num_models);
 size_t mx_mask_words(int max_n);
 void launch_score_mx(hipStream_t st, int kind, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
-                     const double* pair_sq_thr, const double* pair_inv_scale, const MxPoint* mxp,
+                     const double* pair_sq_thr, const double* pair_inv_scale, const uint16_t* mxp, int64_t mx_total,
                      const double* models, const int32_t* model_pair, const int8_t* active, int64_t num_models,
                      int32_t* counts, double* values, int32_t* sym_counts, int slots_per, int32_t* work_list,
                      uint32_t* work_count, int32_t* blk_scratch, int max_n, uint32_t* mask);

@@ -84,3 +84,29 @@ def test_matrix_core_scoring_low_inlier_ratio(monkeypatch):
         assert np.array_equal(ma, mb), i
         for key in ("iteration_number", "local_optimization_number", "graph_cut_number", "num_inliers"):
             assert s64[i][key] == smx[i][key], (i, key)
+
+
+# Points around the 32-point chunks, the 2,048-point rows of the mask walk and
+# the rejection's slices; nearly every point an inlier (a full queue) and few.
+@pytest.mark.parametrize("eps", [0.1, 1.0])
+@pytest.mark.parametrize("ns", [(31, 32, 33, 63, 65), (127, 129, 1023, 1025, 2047), (2048, 2049, 4095, 4097, 6145)])
+def test_mask_and_slice_edges_identical_to_fp64(monkeypatch, ns, eps):
+    probs = []
+    for i, n in enumerate(ns):
+        for kind in ("homography", "fundamental", "essential"):
+            seed = synthetic.scene_seed(8, 100 * n + i)
+            base = dict(kind=kind, conf=0.99, spatial_coherence_weight=0.975, max_iters=500, min_iters=500,
+                        use_sprt=False, sampler=0, neighborhood=0, neighborhood_size=8.0, lo_number=20, seed=n)
+            sc = getattr(synthetic, kind + "_scene")(seed, n=n, inlier_ratio=eps)
+            base.update(correspondences=sc["corr"], h1=768, w1=1024, h2=768, w2=1024, threshold=1.0)
+            if kind == "essential":
+                base.update(K1=sc["K1"], K2=sc["K2"])
+            probs.append(base)
+    r64, s64 = _run(monkeypatch, probs, False)
+    rmx, smx = _run(monkeypatch, probs, True)
+    for i, ((Ma, ma), (Mb, mb)) in enumerate(zip(r64, rmx)):
+        assert np.array_equal(ma, mb), i
+        assert (Ma is None) == (Mb is None), i
+        if Ma is not None:
+            assert np.array_equal(Ma.view(np.uint64), Mb.view(np.uint64)), i
+        assert s64[i]["score"] == smx[i]["score"] and s64[i]["models_scored"] == smx[i]["models_scored"], i

@@ -151,3 +151,74 @@ def test_rejection_never_drops_an_inlier():
         rejected_far += int((rej & far).sum())
         total_far += int(far.sum())
     assert rejected_far > 0.95 * total_far
+
+
+def _denominator_coefs(F):
+    """A quarter of |(F x1)_01|^2 + |(F^T x2)_01|^2 over the squared terms."""
+    g = np.zeros((F.shape[0], 11))
+    for h, rows in enumerate((([0, 1, 2], [3, 4, 5]), ([0, 3, 6], [1, 4, 7]))):
+        a, b = F[:, rows[0]], F[:, rows[1]]
+        g[:, 5 * h] = 0.25 * (a[:, 0] ** 2 + b[:, 0] ** 2)
+        g[:, 5 * h + 1] = 0.5 * (a[:, 0] * a[:, 1] + b[:, 0] * b[:, 1])
+        g[:, 5 * h + 2] = 0.25 * (a[:, 1] ** 2 + b[:, 1] ** 2)
+        g[:, 5 * h + 3] = 0.5 * (a[:, 0] * a[:, 2] + b[:, 0] * b[:, 2])
+        g[:, 5 * h + 4] = 0.5 * (a[:, 1] * a[:, 2] + b[:, 1] * b[:, 2])
+        g[:, 10] += 0.25 * (a[:, 2] ** 2 + b[:, 2] ** 2)
+    return g
+
+
+def test_denominator_form_within_kernel_bound():
+    """The Sampson denominator as one linear form of 32 products: within
+    2^-17 S + 2^-20 of a quarter of the sum of squares in every order of
+    accumulation, and the rejection test with it never drops an inlier."""
+    rng = np.random.default_rng(29)
+    worst = 0.0
+    for trial in range(40):
+        nm, npts = 64, 256
+        F = rng.uniform(-1, 1, (nm, 9)) * 10.0 ** rng.uniform(-7, 0, (nm, 9))
+        F[rng.uniform(size=F.shape) < 0.05] = 0.0
+        F /= np.abs(F).max(axis=1, keepdims=True)
+        if trial % 4 == 0:
+            F = np.sign(F)  # every coefficient at its limit
+        P = rng.uniform(-1, 1, (npts, 4)) * (10.0 ** rng.uniform(-6, 0, (npts, 4)))
+        P[: npts // 8] = np.sign(P[: npts // 8]) * 1.0
+        x1, y1, x2, y2 = P.T
+        d = np.stack([x1 * x1, x1 * y1, y1 * y1, x1, y1, x2 * x2, x2 * y2, y2 * y2, x2, y2, np.ones(npts)], -1)
+        g = _denominator_coefs(F)
+        assert np.abs(g).max() <= 1.0
+        z1, z2 = np.c_[P[:, :2], np.ones(npts)], np.c_[P[:, 2:], np.ones(npts)]
+        M = F.reshape(nm, 3, 3)
+        l1 = np.einsum("mij,pj->mpi", M, z1)[..., :2]
+        l2 = np.einsum("mji,pj->mpi", M, z2)[..., :2]
+        exact = 0.25 * ((l1 ** 2).sum(-1) + (l2 ** 2).sum(-1))
+        dh, dl = _split16(d.astype(np.float32))
+        gh, gl = _split16(g)
+        assert (dl[:, 10] == 0).all()
+        f = np.float32
+        prods = np.concatenate([gh.astype(f)[:, None] * dh.astype(f)[None],
+                                gh.astype(f)[:, None, :10] * dl.astype(f)[None, :, :10],
+                                gl.astype(f)[:, None] * dh.astype(f)[None]], axis=-1)
+        assert prods.shape[-1] == 32
+        ax, ay, bx, by = np.abs(P).astype(f).T
+        sa, sb = 1 + ax + ay, 1 + bx + by
+        S = 1 + ax * sa + ay * (1 + ay) + bx * sb + by * (1 + by)
+        assert (np.abs(d).sum(-1) <= S * (1 + 1e-6)).all()
+        dD = f(2.0 ** -17) * S + f(2.0 ** -20)
+        dC = f(2.0 ** -17) * (sa * sb) + f(2.0 ** -20)
+        zh, zl = _split16(_z(x1, y1, x2, y2).astype(f))
+        ch, cl = _split16(F)
+        c32 = (ch.astype(f) @ zh.astype(f).T + ch.astype(f) @ zl.astype(f).T + cl.astype(f) @ zh.astype(f).T).astype(f)
+        C = F @ _z(x1, y1, x2, y2).T
+        for order in range(3):
+            perm = rng.permutation(32) if order else np.arange(32)
+            acc = np.zeros(prods.shape[:2], f)
+            for k in perm:
+                acc = (acc + prods[..., k]).astype(f)
+            worst = max(worst, float((np.abs(acc - exact) / dD[None]).max()))
+            for tau in (1e-4, 2e-3, 0.1):
+                k1 = f(4) * f(tau ** 2 * (1 + 2.0 ** -16))
+                low = np.abs(c32) - dC[None]
+                rej = low * np.abs(low) > acc * k1 + k1 * dD[None]
+                assert not (rej & (C ** 2 < tau ** 2 * 4 * exact)).any(), (trial, order, tau)
+    print("worst denominator error: %.3f of the kernel's bound" % worst)
+    assert worst < 0.5
