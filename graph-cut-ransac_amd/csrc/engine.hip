@@ -2142,9 +2142,9 @@ struct Engine : Workspace {
       d_mx_mask.ensure(mx_mask_words(mx_max_n));
       d_pair_inv_scale.ensure(np);
       mx_total = total;
-      d_mxp.ensure((size_t)(kMxPointHalves * total));
-      launch_mx_prepare(stream, d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pt_pair.p, np, total, d_pair_inv_scale.p,
-                        d_mxp.p);
+      d_mxp.ensure(mx_point_halves(total));
+      launch_mx_prepare(stream, d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pt_pair.p, d_pair_sq_thr.p, np, total,
+                        d_pair_inv_scale.p, d_mxp.p);
     }
     // generator states of the pairs whose uniform sampler draws on the device
     {
@@ -2291,13 +2291,17 @@ struct Engine : Workspace {
     // thresholds / spatial weight of a pair whose loop switched estimator
     // (DEGENSAC's nested run); the sources are the pairs' own fields, which
     // stay unchanged until the step has synchronised
+    bool dirty = false;
     for (auto& P : pairs)
       if (P.params_dirty) {
         P.params_dirty = false;
+        dirty = true;
         h2d(d_pair_sq_thr.p + P.index, &P.sq_thr, 1);
         h2d(d_pair_lo_thr.p + P.index, &P.lo_thr, 1);
         h2d(d_pair_lambda.p + P.index, &P.lambda, 1);
       }
+    if (dirty && mx_on)
+      launch_mx_slack(stream, d_rpts, d_pt_pair.p, d_pair_sq_thr.p, d_pair_inv_scale.p, mx_total, d_mxp.p);
     if (src.empty()) return;
     // two-phase: stage sources first so a slot that is both a source and a
     // destination in this batch is read before it is written

@@ -23,24 +23,43 @@
 // 2^-22 relative each, the dropped lo*lo term 2^-22, FP32 rounding of z
 // 2^-24, FP32 accumulation of 27 exact products 27 * 2^-24, FP16 subnormal
 // spacing 2^-24); with |c_t| <= 1 the kernel uses delta = 2^-17 S + 2^-20,
-// S the sum of |z_t| over the terms the quantity reads (C, P, Q: (1 + |x1| +
-// |y1|) (1 + |x2| + |y2|); W: 1 + |x1| + |y1|).  The Sampson denominator
-// |(F x1)_01|^2 + |(F^T x2)_01|^2 is a linear form too, in the 11 squared terms
-// (x1^2, x1 y1, y1^2, x1, y1, the same of the second image, 1); a quarter of it,
-// D, has |coefficients| <= 1, and 11 + 10 + 11 products fill the 32 (the lo of
-// the 1 is 0), so its bound is the same with 32 terms: dD = 2^-17 S + 2^-20.
+// S the sum of |z_t| over the terms the quantity reads (at most (1 + |x1| +
+// |y1|) (1 + |x2| + |y2|)).  The denominators |(F x1)_01|^2 + |(F^T x2)_01|^2
+// and W^2 are linear forms too, in the 11 squared terms (x1^2, x1 y1, y1^2, x1,
+// y1, the same of the second image, 1); a quarter, D, has |coefficients| <= 1,
+// and 11 + 10 + 11 products fill the 32 (the lo of the 1 is 0), so its bound is
+// the same with 32 terms: dD = 2^-17 S + 2^-20.
 //
-// A point is dropped for a model only when the bounds prove it an outlier:
-// Sampson (|C| - dC)+^2 > 4 tau''^2 (1 + 2^-16) (D + dD), transfer
-// (|P| - dP)+^2 + (|Q| - dQ)+^2 > tau''^2 (1 + 2^-16) (|W| + dW)^2 (the
-// factor 1 + 2^-16 covers the FP32 rounding of the test itself, about
-// 10 * 2^-24).  Every other point -- all inliers and every point near the
-// threshold -- is evaluated by the FP64 routines of the FP64 kernel
+// A point is dropped for a model only when the bounds prove it an outlier.  With
+// X = tau''^2 times the denominator (= 4 tau''^2 D), sqrt(C^2) > sqrt(X) follows
+// from c^2 > (1 + h) X + (1 + 1/h) dC^2 for the computed c, |c - C| <= dC, and
+// any h > 0 (h = 2^-4 here; the transfer error's (P, Q) likewise, where sqrt(2)
+// times the error of each stays below the same dC).  So the test is, with the
+// pair's scales sigma and kappa = 4 tau''^2 (1 + 2^-14) (1 + h) sigma^2 inside
+// the model's operands,
+//   c^2 > d + slack,  slack = (1 + 2^-14) [max(kappa, 1) dD + (1 + 1/h) (sigma dC)^2],
+// c from sigma C, d from kappa D, one slack per point, which is the product's
+// initial accumulator (the factors 1 + 2^-14 cover the FP32 rounding of the
+// slack, of its way through the accumulator, 33 * 2^-23, and of the FP64
+// decision).  The test is one multiply-add whose sign is the answer; no operand
+// is a NaN (models and points that are not finite have zero operands, and a
+// positive slack drops nothing).  Every other point -- all inliers and every
+// point near the threshold -- is evaluated by the FP64 routines of the FP64 kernel
 // (f_sampson_parts with its guard band, f_sq_sampson, f_sq_symmetric,
 // h_sq_residual) and the MSAC value is accumulated in ascending point order
 // on the model's lane.  Counts, values and symmetric counts are therefore the
-// FP64 kernel's bits.  NaN / inf models or points never pass the rejection
-// test, so they reach the FP64 path as before.
+// FP64 kernel's bits.
+//
+// What bounds the two passes: the rejection its vector instructions (a
+// multiply-add and a shift per 64 models x points, beside the matrix units'
+// 128 cycles per 32 x 32) and, near that, the points' operands from the caches
+// (hence 64 models per wave); the exact pass the latency of the queued points'
+// loads and the in-order sums.  Measured on MI355X, 32 essential pairs of
+// 10,000 points, ms per call.  Rejection: 248 with ten products, ballots and
+// selects per tile, 158 with four products and lane writes of ballots (four
+// streams at once); the latter 156 and this form 96 with one stream.  Exact
+// pass: 184 with a walk over single mask bits, 74 with a word per lane (four
+// streams), 48 with one.
 #include "dev_common.hpp"
 #include "kernels.hpp"
 
@@ -51,9 +70,10 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
-constexpr float kDeltaRel = 0x1p-17f;
-constexpr float kDeltaAbs = 0x1p-20f;
-constexpr double kTauMargin = 1.0 + 0x1p-16;
+constexpr double kDeltaRel = 0x1p-17;
+constexpr double kDeltaAbs = 0x1p-20;
+constexpr double kMargin = 1.0 + 0x1p-14;
+constexpr double kEta = 0x1p-4;
 constexpr int kCompactPerBlock = 2048;  // slots per block of the ordered compaction
 constexpr int kMxBlocks = 2048;         // persistent grids: at most 8,192 waves
 // list entries per rejection + exact pass: as many as keep the segment's
@@ -61,21 +81,22 @@ constexpr int kMxBlocks = 2048;         // persistent grids: at most 8,192 waves
 // kMxSegMax (each segment costs three launches; the masks bound the memory)
 constexpr int64_t kMxSegMin = 65536, kMxSegMax = 1048576;
 constexpr int64_t kMxMaskBudget = 512ll << 20;
-// points per rejection work item: as many as leave kMxItems items (a tenth of
-// the model slots hold a model to score at worst), between kMxSliceMin and
-// kMxSliceMax (every item reads its 32 models' operands once)
-constexpr int kMxSliceMin = 128, kMxSliceMax = 1024;
-constexpr int64_t kMxItems = 16384;
+// The rejection's grid: four waves per SIMD are resident (126 VGPRs).  A work item starts
+// with four dependent loads (entry, pair, sizes, operands: about 3,000 cycles
+// against about 500 per 32 points), so the points are cut into only as many
+// slices as one round of the grid's waves takes, by the list's length, which
+// only the device knows; from half as many tiles as waves on, four rounds (their
+// last one is then a small part).  A slice is a multiple of kMxSliceMin points,
+// the four mask words of one store.
+constexpr int kMxRejectBlocks = 1024;
+constexpr int kMxSliceMin = 128;
+constexpr int kMxTile = 64;             // list entries per work item
 constexpr int64_t kMxPlaneHalves = 16;  // 16-bit words of a point in one operand plane
 constexpr int kNumXcd = 8;
 
 __device__ __forceinline__ f32x16 mfma16(const h8& a, const h8& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
-
-// v with lane `lane` replaced by the scalar x (clang 20 has no builtin for it)
-extern "C" __device__ __attribute__((const)) uint32_t gcr_writelane(uint32_t x, uint32_t lane,
-                                                                    uint32_t v) __asm("llvm.amdgcn.writelane.i32");
 
 __device__ __forceinline__ f32x16 zero16() {
   f32x16 z;
@@ -84,11 +105,34 @@ __device__ __forceinline__ f32x16 zero16() {
   return z;
 }
 
+// The scales of one pair's test: the quantities C (P, Q) are taken times sigma
+// and the denominator form D times kappa, so that the test compares numbers
+// near 1: sigma the power of two that brings kappa = 4 tau''^2 (1 + 2^-14)
+// (1 + h) sigma^2 into [1, 4), at most 2^12 (FP16 coefficients).  Thresholds
+// of half the points' range and more, and ones that are no numbers, drop nothing.
+struct MxScale {
+  double sigma, kappa;
+  bool on;
+};
+__device__ __forceinline__ MxScale mx_scale(double sq_thr, double inv_scale) {
+  MxScale r;
+  const double q = 4.0 * (sq_thr * inv_scale * inv_scale) * kMargin * (1.0 + kEta);
+  r.on = q >= 0.0 && q < 1.0;
+  r.sigma = 1.0;
+  r.kappa = r.on ? q : 0.0;
+#pragma unroll 1
+  for (int e = 0; e < 12 && r.kappa < 1.0; ++e) {
+    r.sigma *= 2.0;
+    r.kappa *= 4.0;
+  }
+  return r;
+}
+
 // One model's coefficient vectors over z (row-major 3x3 M): Sampson C;
-// transfer P, Q, W.
+// transfer P, Q.
 template <int KIND>
 __device__ __forceinline__ void quantity_coefs(const double* F, double c[][9]) {
-  constexpr int NQ = KIND == 1 ? 1 : 3;
+  constexpr int NQ = KIND == 1 ? 1 : 2;
 #pragma unroll
   for (int q = 0; q < NQ; ++q)
 #pragma unroll
@@ -99,26 +143,29 @@ __device__ __forceinline__ void quantity_coefs(const double* F, double c[][9]) {
   } else {
     c[0][0] = F[6]; c[0][1] = F[7]; c[0][2] = F[8]; c[0][6] = -F[0]; c[0][7] = -F[1]; c[0][8] = -F[2];
     c[1][3] = F[6]; c[1][4] = F[7]; c[1][5] = F[8]; c[1][6] = -F[3]; c[1][7] = -F[4]; c[1][8] = -F[5];
-    c[2][6] = F[6]; c[2][7] = F[7]; c[2][8] = F[8];
   }
 }
 
-// A quarter of the Sampson denominator (F x1)_0^2 + (F x1)_1^2 + (F^T x2)_0^2 +
-// (F^T x2)_1^2 as a linear form in d = (x1^2, x1 y1, y1^2, x1, y1, the same of
-// the second image, 1): every coefficient is at most 1 when |F| <= 1.
+// A quarter of the denominator as a linear form in d = (x1^2, x1 y1, y1^2, x1,
+// y1, the same of the second image, 1): (F x1)_0^2 + (F x1)_1^2 + (F^T x2)_0^2 +
+// (F^T x2)_1^2, or W^2.  Every coefficient is at most 1 when |F| <= 1.
+template <int KIND>
 __device__ __forceinline__ void denominator_coefs(const double* F, double g[11]) {
-  const double a[2][3] = {{F[0], F[1], F[2]}, {F[3], F[4], F[5]}};
-  const double b[2][3] = {{F[0], F[3], F[6]}, {F[1], F[4], F[7]}};
   g[10] = 0.0;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const double(*r)[3] = h ? b : a;
-    g[5 * h] = 0.25 * (r[0][0] * r[0][0] + r[1][0] * r[1][0]);
-    g[5 * h + 1] = 0.5 * (r[0][0] * r[0][1] + r[1][0] * r[1][1]);
-    g[5 * h + 2] = 0.25 * (r[0][1] * r[0][1] + r[1][1] * r[1][1]);
-    g[5 * h + 3] = 0.5 * (r[0][0] * r[0][2] + r[1][0] * r[1][2]);
-    g[5 * h + 4] = 0.5 * (r[0][1] * r[0][2] + r[1][1] * r[1][2]);
-    g[10] += 0.25 * (r[0][2] * r[0][2] + r[1][2] * r[1][2]);
+    double a[3], b[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      a[k] = KIND == 1 ? (h ? F[3 * k] : F[k]) : (h ? 0.0 : F[6 + k]);
+      b[k] = KIND == 1 ? (h ? F[3 * k + 1] : F[3 + k]) : 0.0;
+    }
+    g[5 * h] = 0.25 * (a[0] * a[0] + b[0] * b[0]);
+    g[5 * h + 1] = 0.5 * (a[0] * a[1] + b[0] * b[1]);
+    g[5 * h + 2] = 0.25 * (a[1] * a[1] + b[1] * b[1]);
+    g[5 * h + 3] = 0.5 * (a[0] * a[2] + b[0] * b[2]);
+    g[5 * h + 4] = 0.5 * (a[1] * a[2] + b[1] * b[2]);
+    g[10] += 0.25 * (a[2] * a[2] + b[2] * b[2]);
   }
 }
 
@@ -171,9 +218,10 @@ __device__ __forceinline__ _Float16 k_elem(const _Float16* first, const _Float16
   return k < T ? first[k] : (k < T + L ? second[k - T] : (k < 2 * T + L ? third[k - T - L] : (_Float16)0.0f));
 }
 
-// Per point: the B-operand slices of both lane halves (k order, FP16) of z and
-// of the squared terms d, and the error bounds; a plane per MFMA, so that a
-// wave's load of 32 points is one contiguous kilobyte.
+// Per point: the operand slices of both lane halves (k order, FP16) of z and of
+// the squared terms d; a plane per MFMA, so that a wave's load of 32 points is
+// one contiguous kilobyte.  A point outside |x'| <= 1 (only where the pair's
+// coordinates are not all finite) gets zeros: nothing is dropped for it.
 __global__ void __launch_bounds__(256) k_mx_points(const double* __restrict__ pts,
                                                    const int32_t* __restrict__ pt_pair,
                                                    const double* __restrict__ inv_scale, int64_t total,
@@ -182,13 +230,14 @@ __global__ void __launch_bounds__(256) k_mx_points(const double* __restrict__ pt
   if (i >= total) return;
   const double is = inv_scale[pt_pair[i]];
   const double x1 = pts[4 * i] * is, y1 = pts[4 * i + 1] * is, x2 = pts[4 * i + 2] * is, y2 = pts[4 * i + 3] * is;
+  const bool ok = fabs(x1) <= 1.0 && fabs(y1) <= 1.0 && fabs(x2) <= 1.0 && fabs(y2) <= 1.0;
   const double zd[9] = {x2 * x1, x2 * y1, x2, y2 * x1, y2 * y1, y2, x1, y1, 1.0};
   const double dd[11] = {x1 * x1, x1 * y1, y1 * y1, x1, y1, x2 * x2, x2 * y2, y2 * y2, x2, y2, 1.0};
   h8* const o = reinterpret_cast<h8*>(out);
   _Float16 hi[11], lo[11];
 #pragma unroll
   for (int t = 0; t < 9; ++t) {
-    const float z = (float)zd[t];
+    const float z = ok ? (float)zd[t] : 0.0f;
     hi[t] = (_Float16)z;
     lo[t] = (_Float16)(z - (float)hi[t]);
   }
@@ -203,7 +252,7 @@ __global__ void __launch_bounds__(256) k_mx_points(const double* __restrict__ pt
     }
 #pragma unroll
   for (int t = 0; t < 11; ++t) {
-    const float z = (float)dd[t];
+    const float z = ok ? (float)dd[t] : 0.0f;
     hi[t] = (_Float16)z;
     lo[t] = (_Float16)(z - (float)hi[t]);
   }
@@ -216,15 +265,27 @@ __global__ void __launch_bounds__(256) k_mx_points(const double* __restrict__ pt
       for (int e = 0; e < 8; ++e) v[e] = k_elem<11, 10>(hi, lo, hi, 16 * kh + 8 * hf + e);
       o[((2 + kh) * total + i) * 2 + hf] = v;
     }
-  const float ax = fabsf((float)x1), ay = fabsf((float)y1), bx = fabsf((float)x2), by = fabsf((float)y2);
-  const float sa = 1.0f + ax + ay, sb = 1.0f + bx + by;
-  const float sd = 1.0f + ax * sa + ay * (1.0f + ay) + bx * sb + by * (1.0f + by);
-  float4 d;
-  d.x = kDeltaRel * (sa * sb) + kDeltaAbs;
-  d.y = kDeltaRel * sa + kDeltaAbs;
-  d.z = kDeltaRel * sd + kDeltaAbs;
-  d.w = 0.0f;
-  reinterpret_cast<float4*>(out + kMxPlaneHalves * 4 * total)[i] = d;
+}
+
+// Per point: the slack of its test under its pair's threshold (the plane
+// behind the operands).
+__global__ void __launch_bounds__(256) k_mx_slack(const double* __restrict__ pts, const int32_t* __restrict__ pt_pair,
+                                                  const double* __restrict__ pair_sq_thr,
+                                                  const double* __restrict__ inv_scale, int64_t total,
+                                                  float* __restrict__ slack) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const int p = pt_pair[i];
+  const double is = inv_scale[p];
+  const MxScale sc = mx_scale(pair_sq_thr[p], is);
+  const double ax = fabs(pts[4 * i] * is), ay = fabs(pts[4 * i + 1] * is), bx = fabs(pts[4 * i + 2] * is),
+               by = fabs(pts[4 * i + 3] * is);
+  const double sa = 1.0 + ax + ay, sb = 1.0 + bx + by;
+  const double sd = 1.0 + ax * sa + ay * (1.0 + ay) + bx * sb + by * (1.0 + by);
+  const double dc = sc.sigma * (kDeltaRel * (sa * sb) + kDeltaAbs);
+  const double dd = (sc.kappa > 1.0 ? sc.kappa : 1.0) * (kDeltaRel * sd + kDeltaAbs);
+  const double k = kMargin * (dd + (1.0 + 1.0 / kEta) * dc * dc);
+  slack[i] = k < 1e30 ? (float)k : 1.0f;
 }
 
 // ---- ordered compaction of the active model slots ------------------------------
@@ -308,14 +369,15 @@ __global__ void __launch_bounds__(256) k_mx_write(const int8_t* __restrict__ act
   }
 }
 
-// ---- per-model A operands -----------------------------------------------------------
+// ---- per-model operands -----------------------------------------------------------
 
 // One thread per (list entry of the segment, lane half): the entry's scaled,
 // normalised coefficient vectors split into FP16 hi / lo and laid out as the
-// MFMA A-operand slices of that lane half (NQ quantities x 2 MFMAs x 8).  A
+// MFMA operand slices of that lane half (NQ quantities x 2 MFMAs x 8).  A
 // zero, inf or NaN model gets zero operands (nothing is rejected for it).
 template <int KIND>
-__global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pair_inv_scale,
+__global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pair_sq_thr,
+                                                  const double* __restrict__ pair_inv_scale,
                                                   const double* __restrict__ models,
                                                   const int32_t* __restrict__ model_pair,
                                                   const int32_t* __restrict__ list,
@@ -353,20 +415,23 @@ __global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pai
   }
 #pragma unroll
   for (int k = 0; k < 9; ++k) mx = fabs(Fs[k]) > mx ? fabs(Fs[k]) : mx;
-  const bool lp_ok = mx > 0.0 && mx <= 1e300;
+  const MxScale ts = mx_scale(pair_sq_thr[p], is);
+  const bool lp_ok = mx > 0.0 && mx <= 1e300 && ts.on;
   const double inv_mx = lp_ok ? 1.0 / mx : 0.0;
 #pragma unroll
   for (int k = 0; k < 9; ++k) Fs[k] = Fs[k] * inv_mx;
-  double cq[3][9];
+  double cq[2][9], dq[11];
   quantity_coefs<KIND>(Fs, cq);
+  denominator_coefs<KIND>(Fs, dq);
   h8* out = coefs + (e * 2 + hf) * (2 * NQ);
   _Float16 hi[11], lo[11];
 #pragma unroll
-  for (int q = 0; q < (KIND == 1 ? 1 : 3); ++q) {
+  for (int q = 0; q + 1 < NQ; ++q) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-      hi[k] = (_Float16)cq[q][k];
-      lo[k] = (_Float16)(cq[q][k] - (double)hi[k]);
+      const double v = cq[q][k] * ts.sigma;
+      hi[k] = (_Float16)v;
+      lo[k] = (_Float16)(v - (double)hi[k]);
     }
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh) {
@@ -377,52 +442,56 @@ __global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pai
       out[2 * q + kh] = v;
     }
   }
-  if constexpr (KIND == 1) {
-    double g[11];
-    denominator_coefs(Fs, g);
 #pragma unroll
-    for (int k = 0; k < 11; ++k) {
-      hi[k] = (_Float16)g[k];
-      lo[k] = (_Float16)(g[k] - (double)hi[k]);
-    }
+  for (int k = 0; k < 11; ++k) {
+    const double v = dq[k] * ts.kappa;
+    hi[k] = (_Float16)v;
+    lo[k] = (_Float16)(v - (double)hi[k]);
+  }
 #pragma unroll
-    for (int kh = 0; kh < 2; ++kh) {
-      h8 v;
+  for (int kh = 0; kh < 2; ++kh) {
+    h8 v;
 #pragma unroll
-      for (int x = 0; x < 8; ++x)
-        v[x] = hf ? k_elem<11, 10>(hi, hi, lo, 16 * kh + 8 + x) : k_elem<11, 10>(hi, hi, lo, 16 * kh + x);
-      out[2 + kh] = v;
-    }
+    for (int x = 0; x < 8; ++x)
+      v[x] = hf ? k_elem<11, 10>(hi, hi, lo, 16 * kh + 8 + x) : k_elem<11, 10>(hi, hi, lo, 16 * kh + x);
+    out[2 * NQ - 2 + kh] = v;
   }
 }
 
 // ---- phase 1: rejection on the matrix cores ---------------------------------------
 
-// Work item (tile t, slice j): the 32 list entries 32 t .. 32 t + 31 of the
+// Work item (tile t, slice j): the 64 list entries 64 t .. 64 t + 63 of the
 // segment (slot order, so the entries of one pair are adjacent; a tile that
 // spans pairs is handled pair by pair) against points slice j .. slice j + slice
-// - 1 of their pair.  Lane r < 32 owns entry r and writes, per 32-point chunk, the
-// 32-bit word of its candidate mask (bit b: point base + b must be evaluated
-// in FP64).  Words of points at or beyond the pair's n are not written.
+// - 1 of their pair.  The points are the products' rows and the models their
+// columns, and row 8 (j / 4) + 4 hf + (j % 4), accumulator slot j of lane half
+// hf, holds point 16 hf + j of the 32: a lane's slots are consecutive points of
+// its own model, the sign of each slot's test is shifted into the lane's mask
+// word, and one exchange of lane halves completes the words of entries e0 + lane
+// (bit b of a word: point base + b must be evaluated in FP64).  The points'
+// slack is the initial accumulator of the denominator.  Words of points at or
+// beyond the pair's n are zero up to the next multiple of four words.
 template <int KIND>
-__global__ void __launch_bounds__(256, 4) k_mx_reject(const int64_t* __restrict__ pair_pt_off,
-                                                   const int32_t* __restrict__ pair_n,
-                                                   const double* __restrict__ pair_sq_thr,
-                                                   const double* __restrict__ pair_inv_scale,
-                                                   const uint16_t* __restrict__ mxp, int64_t mx_total,
-                                                   const h8* __restrict__ coefs,
-                                                   const int32_t* __restrict__ model_pair,
-                                                   const int32_t* __restrict__ list,
-                                                   const uint32_t* __restrict__ list_count, int64_t seg_begin,
-                                                   int64_t seg_len, int slice, int slices, int words, uint32_t* __restrict__ mask,
-                                                   int slots_per) {
+__global__ void __launch_bounds__(256, KIND == 1 ? 4 : 3) k_mx_reject(
+    const int64_t* __restrict__ pair_pt_off, const int32_t* __restrict__ pair_n, const uint16_t* __restrict__ mxp,
+    int64_t mx_total, const h8* __restrict__ coefs, const int32_t* __restrict__ model_pair,
+    const int32_t* __restrict__ list, const uint32_t* __restrict__ list_count, int64_t seg_begin, int64_t seg_len,
+    int max_n, int words, uint32_t* __restrict__ mask, int slots_per) {
   constexpr int NQ = KIND == 1 ? 2 : 3;
+  struct __attribute__((packed, aligned(4))) F4 {
+    float v[4];
+  };
   const int lane = lane_id();
   const int hf = lane >> 5, r = lane & 31;
+  const int row_pt = 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
   const int64_t total = (int64_t)*list_count;
   if (seg_begin >= total) return;
   const int64_t seg_n = total - seg_begin < seg_len ? total - seg_begin : seg_len;
-  const int64_t items = (seg_n + 31) / 32 * slices;
+  const int tiles = (int)((seg_n + kMxTile - 1) / kMxTile), waves = (int)gridDim.x * 4;
+  int slices = 2 * tiles <= waves ? waves / tiles : (4 * waves + tiles - 1) / tiles;
+  const int slice = ((max_n + slices - 1) / slices + kMxSliceMin - 1) / kMxSliceMin * kMxSliceMin;
+  slices = (max_n + slice - 1) / slice;
+  const int64_t items = (int64_t)tiles * slices;
   // gridDim.x is a multiple of kNumXcd: workgroup b runs on XCD b % kNumXcd,
   // which takes a contiguous range of items (adjacent items share a pair)
   const int xcd = (int)(blockIdx.x % kNumXcd);
@@ -431,85 +500,91 @@ __global__ void __launch_bounds__(256, 4) k_mx_reject(const int64_t* __restrict_
   const int64_t lo_u = items * xcd / kNumXcd, hi_u = items * (xcd + 1) / kNumXcd;
   for (int64_t u = lo_u + w; u < hi_u; u += waves_per_xcd) {
     const int64_t t = u / slices;
-    const int j = (int)(u - t * slices);
-    const int64_t e0 = 32 * t;  // within the segment
-    const int cnt_all = (int)(seg_n - e0 < 32 ? seg_n - e0 : 32);
-    const int64_t slot = r < cnt_all ? (int64_t)list[seg_begin + e0 + r] : -1;
+    const int first = slice * (int)(u - t * slices);
+    const int64_t e0 = kMxTile * t;  // within the segment
+    const int cnt_all = (int)(seg_n - e0 < kMxTile ? seg_n - e0 : kMxTile);
+    const int64_t slot = lane < cnt_all ? (int64_t)list[seg_begin + e0 + lane] : -1;
     const int my_pair = slot >= 0 ? model_pair[slots_per == 1 ? slot : slot / slots_per] : -1;
-    uint32_t* __restrict__ my_mask = mask + (e0 + r) * (int64_t)words;
+    uint32_t* __restrict__ my_mask = mask + (e0 + lane) * (int64_t)words;
     int done = 0;
     while (done < cnt_all) {
       const int p = __builtin_amdgcn_readlane(my_pair, done);
-      const bool mine = r >= done && r < cnt_all && my_pair == p;
-      const int sub_end = done + __popcll(ballot64(mine) & 0xffffffffull);
+      const bool mine = lane >= done && my_pair == p;
+      const int sub_end = done + __popcll(ballot64(mine));
       const int n = pair_n[p];
-      const int first = slice * j;
       if (first < n) {
-        // the sub-tile's A operands (lane: row r, half hf); other rows zero
-        h8 A[NQ][2];
-        const h8* __restrict__ my_coefs = coefs + ((e0 + r) * 2 + hf) * (2 * NQ);
+        // the models' operands (columns 32 s + r, half hf); columns of other
+        // pairs compute what nothing reads
+        h8 B[2][NQ][2];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q)
+        for (int s = 0; s < 2; ++s) {
+          const int e = 32 * s + r < cnt_all ? 32 * s + r : cnt_all - 1;
+          const h8* __restrict__ my_coefs = coefs + ((e0 + e) * 2 + hf) * (2 * NQ);
 #pragma unroll
-          for (int kh = 0; kh < 2; ++kh) {
-            if (mine) {
-              A[q][kh] = my_coefs[2 * q + kh];
-            } else {
+          for (int q = 0; q < NQ; ++q)
 #pragma unroll
-              for (int e = 0; e < 8; ++e) A[q][kh][e] = (_Float16)0.0f;
-            }
-          }
-        const double is = pair_inv_scale[p];
-        const float tau2m = (float)(pair_sq_thr[p] * is * is * kTauMargin);
+            for (int kh = 0; kh < 2; ++kh) B[s][q][kh] = my_coefs[2 * q + kh];
+        }
         const int64_t off = pair_pt_off[p];
         const h8* __restrict__ Z = reinterpret_cast<const h8*>(mxp) + 2 * off + hf;
-        const float4* __restrict__ D = reinterpret_cast<const float4*>(mxp + kMxPlaneHalves * 4 * mx_total) + off;
+        const float* __restrict__ K = reinterpret_cast<const float*>(mxp + kMxPlaneHalves * 4 * mx_total) + off;
         const int last = first + slice < n ? first + slice : n;
-        for (int base = first; base < last; base += 32) {
-          // points beyond the pair read its last one; their bits are cut below
-          const int i = base + r < n ? base + r : n - 1;
-          const h8 b0 = Z[2 * i], b1 = Z[2 * (mx_total + i)];
-          const float4 dq = D[i];
-          // accumulator slot j holds row 8 (j / 4) + 4 hf + (j % 4) of column
-          // r; the ballot's halves are the words of its two rows, which go to
-          // the lanes of those rows
-          const uint32_t live = last - base < 32 ? (1u << (last - base)) - 1u : ~0u;  // uniform
-          uint32_t word = 0;
-          auto put = [&](int jj, bool rej) {
-            const uint64_t k = ballot64(!rej);
-            const int row = 8 * (jj >> 2) + (jj & 3);
-            word = gcr_writelane((uint32_t)k, row, word);
-            word = gcr_writelane((uint32_t)(k >> 32), row + 4, word);
-          };
-          if constexpr (KIND == 1) {
-            const h8 b2 = Z[2 * (2 * mx_total + i)], b3 = Z[2 * (3 * mx_total + i)];
-            f32x16 c = mfma16(A[0][0], b0, zero16());
-            f32x16 den = mfma16(A[1][0], b2, zero16());
-            c = mfma16(A[0][1], b1, c);
-            den = mfma16(A[1][1], b3, den);
-            const float k1 = 4.0f * tau2m;
-            const float k2 = k1 * dq.z;
+#pragma unroll 1
+        for (int base = first; base < last; base += 128) {
+          uint32_t wd[4];
+#pragma unroll 1
+          for (int k = 0; k < 4; ++k) {
+            const int b = base + 32 * k;
+            uint32_t word = 0;
+            if (b < last) {
+              // rows beyond the pair read its last point; their bits are cut below
+              const int i = b + row_pt < n ? b + row_pt : n - 1;
+              const h8 z0 = Z[2 * i], z1 = Z[2 * (mx_total + i)], d0 = Z[2 * (2 * mx_total + i)],
+                       d1 = Z[2 * (3 * mx_total + i)];
+              f32x16 slack;
 #pragma unroll
-            for (int jj = 0; jj < 16; ++jj) {
-              const float cl = fabsf(c[jj]) - dq.x;
-              put(jj, cl * fabsf(cl) > __builtin_fmaf(den[jj], k1, k2));
-            }
-          } else {
-            f32x16 pp = mfma16(A[0][0], b0, zero16());
-            pp = mfma16(A[0][1], b1, pp);
-            f32x16 qq = mfma16(A[1][0], b0, zero16());
-            qq = mfma16(A[1][1], b1, qq);
-            f32x16 ww = mfma16(A[2][0], b0, zero16());
-            ww = mfma16(A[2][1], b1, ww);
+              for (int j = 0; j < 16; j += 4) {
+                const F4 v = *reinterpret_cast<const F4*>(K + b + 16 * hf + j);
 #pragma unroll
-            for (int jj = 0; jj < 16; ++jj) {
-              const float pl = fmaxf(fabsf(pp[jj]) - dq.x, 0.0f);
-              const float ql = fmaxf(fabsf(qq[jj]) - dq.x, 0.0f);
-              const float wu = fabsf(ww[jj]) + dq.y;
-              put(jj, __builtin_fmaf(pl, pl, ql * ql) > wu * wu * tau2m);
+                for (int x = 0; x < 4; ++x) slack[j + x] = v.v[x];
+              }
+              uint32_t half[2];
+#pragma unroll
+              for (int s = 0; s < 2; ++s) {
+                f32x16 den = mfma16(d0, B[s][NQ - 1][0], slack);
+                f32x16 c = mfma16(z0, B[s][0][0], zero16());
+                den = mfma16(d1, B[s][NQ - 1][1], den);
+                c = mfma16(z1, B[s][0][1], c);
+                uint32_t bits = 0;
+                if constexpr (KIND == 1) {
+#pragma unroll
+                  for (int j = 15; j >= 0; --j)
+                    bits = __builtin_amdgcn_alignbit(
+                        bits, __builtin_bit_cast(uint32_t, __builtin_fmaf(-c[j], c[j], den[j])), 31);
+                } else {
+                  f32x16 c2 = mfma16(z0, B[s][1][0], zero16());
+                  c2 = mfma16(z1, B[s][1][1], c2);
+#pragma unroll
+                  for (int j = 15; j >= 0; --j)
+                    bits = __builtin_amdgcn_alignbit(
+                        bits,
+                        __builtin_bit_cast(uint32_t,
+                                           __builtin_fmaf(-c2[j], c2[j], __builtin_fmaf(-c[j], c[j], den[j]))),
+                        31);
+                }
+                half[s] = bits;
+              }
+              // lanes < 32: entry r's two halves of points; lanes >= 32: entry 32 + r's
+              const auto x = __builtin_amdgcn_permlane32_swap(half[0], half[1], false, false);
+              const uint32_t live = n - b < 32 ? (1u << (n - b)) - 1u : ~0u;
+              word = ~(x[0] | (x[1] << 16)) & live;
             }
+            wd[0] = wd[1];
+            wd[1] = wd[2];
+            wd[2] = wd[3];
+            wd[3] = word;
           }
-          if (mine && hf == 0) my_mask[base >> 5] = word & live;
+          if (mine) *reinterpret_cast<uint4*>(my_mask + (base >> 5)) = make_uint4(wd[0], wd[1], wd[2], wd[3]);
         }
       }
       done = sub_end;
@@ -632,30 +707,47 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
 
 // ---- launchers --------------------------------------------------------------------
 
+void launch_mx_slack(hipStream_t st, const double* pts, const int32_t* pt_pair, const double* pair_sq_thr,
+                     const double* inv_scale, int64_t total, uint16_t* out) {
+  if (total <= 0) return;
+  hipLaunchKernelGGL(k_mx_slack, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, pts, pt_pair, pair_sq_thr,
+                     inv_scale, total, reinterpret_cast<float*>(out + kMxPlaneHalves * 4 * total));
+}
+
 void launch_mx_prepare(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
-                       const int32_t* pt_pair, int num_pairs, int64_t total, double* inv_scale, uint16_t* out) {
+                       const int32_t* pt_pair, const double* pair_sq_thr, int num_pairs, int64_t total,
+                       double* inv_scale, uint16_t* out) {
   if (num_pairs <= 0 || total <= 0) return;
   hipLaunchKernelGGL(k_mx_pair_scale, dim3((unsigned)num_pairs), dim3(256), 0, st, pts, pair_pt_off, pair_n,
                      num_pairs, inv_scale);
   hipLaunchKernelGGL(k_mx_points, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, pts, pt_pair, inv_scale,
                      total, out);
+  launch_mx_slack(st, pts, pt_pair, pair_sq_thr, inv_scale, total, out);
 }
+
+size_t mx_point_halves(int64_t total) {
+  // four operand planes, the slack, and the slack that the last 32 points' loads run over
+  return (size_t)(4 * kMxPlaneHalves * total + 2 * total + 64);
+}
+
+// 32-bit words of one entry's candidate mask (stored four at a time)
+static int64_t mx_row_words(int max_n) { return (((int64_t)max_n + 31) / 32 + 3) & ~(int64_t)3; }
 
 size_t mx_list_scratch_ints(int64_t num_models) {
   return (size_t)((num_models + kCompactPerBlock - 1) / kCompactPerBlock);
 }
 
 static int64_t mx_segment(int max_n) {
-  const int64_t words = (max_n + 31) / 32 + 1;
+  const int64_t words = mx_row_words(max_n);
   const int64_t fit = kMxMaskBudget / (4 * words);
-  // (a multiple of 32: whole tiles, and the operands behind the masks stay aligned)
-  return fit < kMxSegMin ? kMxSegMin : (fit > kMxSegMax ? kMxSegMax : fit & ~(int64_t)31);
+  // (whole tiles)
+  return fit < kMxSegMin ? kMxSegMin : (fit > kMxSegMax ? kMxSegMax : fit & ~(int64_t)(kMxTile - 1));
 }
 
 size_t mx_mask_words(int max_n) {
-  // the candidate masks, then the segment's A operands (at most 3 x 2 x 2 x 16 B per entry)
+  // the candidate masks, then the segment's operands (at most 3 x 2 x 2 x 16 B per entry)
   const int64_t seg = mx_segment(max_n);
-  return (size_t)seg * (size_t)((max_n + 31) / 32 + 1) + (size_t)seg * 48;
+  return (size_t)seg * (size_t)mx_row_words(max_n) + (size_t)seg * 48;
 }
 
 void launch_score_mx(hipStream_t st, int kind, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
@@ -669,38 +761,34 @@ void launch_score_mx(hipStream_t st, int kind, const double* pts, const int64_t*
                      sym_counts, blk_scratch);
   hipLaunchKernelGGL(k_mx_scan, dim3(1), dim3(1024), 0, st, blk_scratch, nblk, work_count);
   hipLaunchKernelGGL(k_mx_write, dim3((unsigned)nblk), dim3(256), 0, st, active, num_models, blk_scratch, work_list);
-  int slice = kMxSliceMin;
-  while (slice < kMxSliceMax && (num_models / 320 + 1) * ((max_n + 2 * slice - 1) / (2 * slice)) >= kMxItems) slice *= 2;
-  const int slices = (max_n + slice - 1) / slice;
-  const int words = (max_n + 31) / 32 + 1;
+  const int slices = (max_n + kMxSliceMin - 1) / kMxSliceMin;  // at most
+  const int words = (int)mx_row_words(max_n);
   const int64_t segment = mx_segment(max_n);
   h8* const coefs = reinterpret_cast<h8*>(mask + (size_t)segment * (size_t)words);
   // the active count is on the device; segments up to the slot count, and
   // each kernel returns at once past the end of the list
   for (int64_t seg = 0; seg < num_models; seg += segment) {
     const int64_t seg_len = num_models - seg < segment ? num_models - seg : segment;
-    int64_t b1 = ((seg_len + 31) / 32 * slices + 3) / 4;
-    if (b1 > kMxBlocks) b1 = kMxBlocks;
+    int64_t b1 = ((seg_len + kMxTile - 1) / kMxTile * slices + 3) / 4;
+    if (b1 > kMxRejectBlocks) b1 = kMxRejectBlocks;
     b1 = (b1 + kNumXcd - 1) / kNumXcd * kNumXcd;
     int64_t b2 = (seg_len + 3) / 4;
     if (b2 > kMxBlocks) b2 = kMxBlocks;
     b2 = (b2 + kNumXcd - 1) / kNumXcd * kNumXcd;
     const unsigned bc = (unsigned)((2 * seg_len + 255) / 256);
     if (kind == 0) {
-      hipLaunchKernelGGL(k_mx_coefs<0>, dim3(bc), dim3(256), 0, st, pair_inv_scale, models, model_pair, work_list,
-                         work_count, seg, seg_len, coefs, slots_per);
-      hipLaunchKernelGGL(k_mx_reject<0>, dim3((unsigned)b1), dim3(256), 0, st, pair_pt_off, pair_n, pair_sq_thr,
-                         pair_inv_scale, mxp, mx_total, coefs, model_pair, work_list, work_count, seg, seg_len, slice, slices, words,
-                         mask, slots_per);
+      hipLaunchKernelGGL(k_mx_coefs<0>, dim3(bc), dim3(256), 0, st, pair_sq_thr, pair_inv_scale, models,
+                         model_pair, work_list, work_count, seg, seg_len, coefs, slots_per);
+      hipLaunchKernelGGL(k_mx_reject<0>, dim3((unsigned)b1), dim3(256), 0, st, pair_pt_off, pair_n, mxp, mx_total,
+                         coefs, model_pair, work_list, work_count, seg, seg_len, max_n, words, mask, slots_per);
       hipLaunchKernelGGL(k_mx_exact<0>, dim3((unsigned)b2), dim3(256), 0, st, pts, pair_pt_off, pair_n, pair_sq_thr,
                          models, model_pair, work_list, work_count, seg, seg_len, words, mask, counts, values,
                          sym_counts, slots_per);
     } else {
-      hipLaunchKernelGGL(k_mx_coefs<1>, dim3(bc), dim3(256), 0, st, pair_inv_scale, models, model_pair, work_list,
-                         work_count, seg, seg_len, coefs, slots_per);
-      hipLaunchKernelGGL(k_mx_reject<1>, dim3((unsigned)b1), dim3(256), 0, st, pair_pt_off, pair_n, pair_sq_thr,
-                         pair_inv_scale, mxp, mx_total, coefs, model_pair, work_list, work_count, seg, seg_len, slice, slices, words,
-                         mask, slots_per);
+      hipLaunchKernelGGL(k_mx_coefs<1>, dim3(bc), dim3(256), 0, st, pair_sq_thr, pair_inv_scale, models,
+                         model_pair, work_list, work_count, seg, seg_len, coefs, slots_per);
+      hipLaunchKernelGGL(k_mx_reject<1>, dim3((unsigned)b1), dim3(256), 0, st, pair_pt_off, pair_n, mxp, mx_total,
+                         coefs, model_pair, work_list, work_count, seg, seg_len, max_n, words, mask, slots_per);
       hipLaunchKernelGGL(k_mx_exact<1>, dim3((unsigned)b2), dim3(256), 0, st, pts, pair_pt_off, pair_n, pair_sq_thr,
                          models, model_pair, work_list, work_count, seg, seg_len, words, mask, counts, values,
                          sym_counts, slots_per);

@@ -222,3 +222,86 @@ def test_denominator_form_within_kernel_bound():
                 assert not (rej & (C ** 2 < tau ** 2 * 4 * exact)).any(), (trial, order, tau)
     print("worst denominator error: %.3f of the kernel's bound" % worst)
     assert worst < 0.5
+
+
+def test_scaled_test_never_drops_an_inlier():
+    """The kernel's whole test -- operands scaled by sigma and kappa, the slack
+    as the accumulator's first term, the sign of den - c^2 -- on thresholds over
+    the whole range: no point below the threshold is dropped, and most far ones
+    are."""
+    rng = np.random.default_rng(31)
+    f = np.float32
+    h, margin = 2.0 ** -4, 1 + 2.0 ** -14
+    far_n = far_rej = 0
+    for trial in range(60):
+        tau = 10.0 ** rng.uniform(-6, -0.4)
+        transfer = trial % 3 == 2
+        kappa = 4 * tau * tau * margin * (1 + h)
+        assert kappa < 1
+        sigma = 1.0
+        for _ in range(12):
+            if kappa < 1:
+                sigma, kappa = 2 * sigma, 4 * kappa
+        assert kappa < 4 and sigma <= 4096
+        F = rng.uniform(-1, 1, (32, 9)) * 10.0 ** rng.uniform(-3, 0, (32, 9))
+        F /= np.abs(F).max(axis=1, keepdims=True)
+        n = 2048
+        P = rng.uniform(-1, 1, (n, 4))
+        zero = np.zeros(n)
+        for m in range(32):  # near the threshold of some model, from both sides
+            i = np.arange(m, n, 32)
+            p1 = np.c_[P[i, :2], np.ones(len(i))]
+            l = p1 @ F[m].reshape(3, 3).T
+            if transfer:
+                ang = rng.uniform(0, 2 * np.pi, len(i))
+                off = tau * (1 + 10.0 ** rng.uniform(-6, -1, len(i)) * rng.choice([-1, 1], len(i)))
+                P[i, 2:] = l[:, :2] / l[:, 2:3] + off[:, None] * np.c_[np.cos(ang), np.sin(ang)]
+            else:
+                nn = np.maximum(np.linalg.norm(l[:, :2], axis=1), 1e-30)
+                d = (l[:, 0] * P[i, 2] + l[:, 1] * P[i, 3] + l[:, 2]) / nn
+                off = tau * (1 + 10.0 ** rng.uniform(-6, 0, len(i)) * rng.choice([-1, 1], len(i)))
+                P[i, 2:] -= ((d - off) / nn)[:, None] * l[:, :2]
+        P = P[(np.abs(P) <= 1).all(1)]
+        x1, y1, x2, y2 = P.T
+        z, one = _z(x1, y1, x2, y2), np.ones(len(P))
+        d = np.stack([x1 * x1, x1 * y1, y1 * y1, x1, y1, x2 * x2, x2 * y2, y2 * y2, x2, y2, one], -1)
+        if transfer:
+            num_c = _quantities(F)[:, 5:7]
+            g = np.zeros((32, 11))
+            a = F[:, 6:9]
+            g[:, 0], g[:, 1], g[:, 2] = a[:, 0] ** 2 / 4, a[:, 0] * a[:, 1] / 2, a[:, 1] ** 2 / 4
+            g[:, 3], g[:, 4], g[:, 10] = a[:, 0] * a[:, 2] / 2, a[:, 1] * a[:, 2] / 2, a[:, 2] ** 2 / 4
+        else:
+            num_c = F[:, None, :]
+            g = _denominator_coefs(F)
+        exact = ((num_c @ z.T) ** 2).sum(1) / (4 * np.maximum(g @ d.T, 1e-300))
+        sa, sb = 1 + np.abs(x1) + np.abs(y1), 1 + np.abs(x2) + np.abs(y2)
+        sd = 1 + np.abs(x1) * sa + np.abs(y1) * (1 + np.abs(y1)) + np.abs(x2) * sb + np.abs(y2) * (1 + np.abs(y2))
+        dc = sigma * (2.0 ** -17 * sa * sb + 2.0 ** -20)
+        slack = (margin * (max(kappa, 1) * (2.0 ** -17 * sd + 2.0 ** -20) + (1 + 1 / h) * dc * dc)).astype(f)
+        dh, dl = _split16(d.astype(f))
+        zh, zl = _split16(z.astype(f))
+        gh, gl = _split16(g * kappa)
+        prods = np.concatenate([gh.astype(f)[:, None] * dh.astype(f)[None],
+                                gh.astype(f)[:, None, :10] * dl.astype(f)[None, :, :10],
+                                gl.astype(f)[:, None] * dh.astype(f)[None]], axis=-1)
+        t = np.broadcast_to(slack, prods.shape[:2]).astype(f)
+        for k in rng.permutation(32):
+            t = (t + prods[..., k]).astype(f)
+        t = t.astype(np.float64)
+        for q in range(num_c.shape[1]):
+            ch, cl = _split16(num_c[:, q] * sigma)
+            pr = np.concatenate([ch.astype(f)[:, None] * zh.astype(f)[None], ch.astype(f)[:, None] * zl.astype(f)[None],
+                                 cl.astype(f)[:, None] * zh.astype(f)[None]], axis=-1)
+            c = np.zeros(pr.shape[:2], f)
+            for k in rng.permutation(27):
+                c = (c + pr[..., k]).astype(f)
+            t = (t - c.astype(np.float64) ** 2).astype(f).astype(np.float64)
+        rej = t < 0
+        assert not (rej & (exact < tau * tau)).any(), (trial, tau, transfer)
+        if tau > 5e-4:
+            far = exact > 4 * tau * tau
+            far_n += int(far.sum())
+            far_rej += int((rej & far).sum())
+    print("far points dropped: %.3f" % (far_rej / far_n))
+    assert far_rej > 0.9 * far_n
