@@ -659,10 +659,16 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
       uint64_t b = ballot64(in);
       cnt += __popcll(b);
       if (KIND == 1 && sym_counts) scnt += __popcll(ballot64(sym_in));
-      while (b) {
-        const int l = __ffsll((unsigned long long)b) - 1;
-        acc = acc - readlane_f64(r2, l);
-        b &= b - 1;
+      // many inliers: all 64 lanes in order (an outlier's r2 is no term); few:
+      // one by one through the scalar unit (three instructions each)
+      if (__popcll(b) > 20) {
+        acc = wave_chain(acc, in ? r2 : 0.0, -1.0, cnt_flush);
+      } else {
+        while (b) {
+          const int l = __ffsll((unsigned long long)b) - 1;
+          acc = acc - readlane_f64(r2, l);
+          b &= b - 1;
+        }
       }
     };
     const int nw = (n + 31) >> 5;

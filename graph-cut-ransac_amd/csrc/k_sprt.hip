@@ -530,13 +530,9 @@ __device__ double ordered_value(int n, int64_t start, H has, R residual, double 
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      while (m[u]) {
-        const int l = __ffsll((unsigned long long)m[u]) - 1;
-        value += readlane_f64(term[u], l);
-        m[u] &= m[u] - 1;
-      }
+      if (m[u]) value = wave_chain(value, term[u], 1.0, 64 - __builtin_clzll(m[u]));
   }
-  return value;
+  return readlane_f64(value, 0);
 }
 
 }  // namespace

@@ -133,3 +133,29 @@ def test_find_homography_large_scene_matches_oracle(oracle):
     for key in ("iteration_number", "local_optimization_number", "graph_cut_number"):
         assert so[key] == sd[key], key
     np.testing.assert_allclose(Hd, Ho, rtol=1e-12, atol=1e-12)
+
+
+# Inlier counts around the 16 lanes of a row and the 64 of a wave, in the
+# scores' and the normalisations' sums in point order.
+@pytest.mark.parametrize("k", [4, 15, 16, 17, 32, 33, 47, 48, 49, 63, 64, 65, 127, 128, 129, 333])
+def test_ordered_sum_edges_bit_exact(oracle, engine, k):
+    rng = np.random.default_rng(k)
+    for kind, sc in ((0, _scene(5)), (1, synthetic.fundamental_scene(synthetic.scene_seed(1, 5)))):
+        M = sc["H"] if kind == 0 else sc["F"]
+        good = sc["corr"][sc["gt"]][:k]
+        bad = sc["corr"][~sc["gt"]][:70]
+        pts = np.concatenate([good, bad])[rng.permutation(len(good) + len(bad))]
+        models = np.stack([M.ravel(), M.ravel() * 2.0, rng.normal(size=9)])
+        oc, ov, om = oracle.score(kind, pts, models, TAU2_H)
+        dc, dv, dm = engine.score_models(kind, pts, models, TAU2_H, want_masks=True)
+        assert oc[0] >= min(k, len(good))
+        assert np.array_equal(oc, dc) and np.array_equal(om, dm)
+        assert np.array_equal(_bits(ov), _bits(dv))
+        sample = rng.permutation(len(pts))[:max(k, 8)].astype(np.int32)
+        w = rng.uniform(0, 1, len(pts))
+        if kind == 0:
+            _, Ho = oracle.h_nonminimal(pts, sample, w)
+            assert np.array_equal(_bits(Ho.ravel()), _bits(engine.fit_nonminimal(0, pts, sample, w, 1, 1, 3.0)[0]))
+        else:
+            Fo = oracle.fit_nonminimal(1, pts, sample, w, 1, 1, 1.0)
+            assert np.array_equal(_bits(Fo), _bits(engine.fit_nonminimal(1, pts, sample, w, 1, 1, 1.0)))
