@@ -68,33 +68,16 @@ __device__ __forceinline__ double cubic_eval(double a, double b, double c, doubl
   return ((x + a) * x + b) * x + c;
 }
 
-__device__ __forceinline__ double cubic_root_in(double a, double b, double c, double lo, double hi) {
-  double flo = cubic_eval(a, b, c, lo);
-  double x = 0.5 * (lo + hi);
-  for (int it = 0; it < 100; ++it) {
-    const double fx = cubic_eval(a, b, c, x);
-    if (fx == 0.0) return x;
-    if ((fx < 0.0) == (flo < 0.0)) {
-      lo = x;
-      flo = fx;
-    } else
-      hi = x;
-    const double d = (3.0 * x + 2.0 * a) * x + b;
-    double xn = d != 0.0 ? x - fx / d : 0.5 * (lo + hi);
-    if (!(xn > lo && xn < hi)) xn = 0.5 * (lo + hi);
-    if (fabs(xn - x) <= 1e-15 * fabs(x) || hi - lo <= 1e-15 * fabs(x)) return xn;
-    x = xn;
-  }
-  return x;
-}
-
 // Real roots of c0 + c1 x + c2 x^2 + c3 x^3, ascending (c3 != 0), into
 // r0, r1, r2; returns their number.  The critical points split [-bound,
 // bound] into at most three monotone pieces, taken left to right; a piece
 // whose left end is a root contributes that end (unless it repeats the last
-// root), otherwise a sign change is searched by cubic_root_in; the right end
-// of the last piece is a root when the cubic vanishes there.  Written with
-// named slots instead of indexed arrays so everything stays in registers.
+// root), otherwise a sign change is searched by safeguarded Newton steps; the
+// right end of the last piece is a root when the cubic vanishes there.  The
+// searches of a lane's pieces run in one loop, a step of the lane's current
+// piece at a time, so a wave takes as many steps as its slowest lane has in all
+// its pieces; a loop per piece took the slowest lane's steps of each.  Written
+// with named slots instead of indexed arrays so everything stays in registers.
 __device__ __forceinline__ int cubic_real_roots3(const double* c, double& r0, double& r1, double& r2) {
   const double a = c[2] / c[3], b = c[1] / c[3], cc = c[0] / c[3];
   double bound = 1.0;
@@ -111,36 +94,68 @@ __device__ __forceinline__ int cubic_real_roots3(const double* c, double& r0, do
     v1 = s1 > -bound && s1 < bound;
     v2 = s2 > -bound && s2 < bound && s2 > s1;
   }
+  // the pieces: 0 not there or no root, 1 its left end is a root, 2 a search
+  int what[3];
+  double plo[3], v[3];
+  {
+    double lo = -bound;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const bool use = k == 0 ? v1 : (k == 1 ? v2 : true);
+      const double hi = k == 0 ? s1 : (k == 1 ? s2 : bound);
+      const double flo = cubic_eval(a, b, cc, lo), fhi = cubic_eval(a, b, cc, hi);
+      what[k] = !use ? 0 : (flo == 0.0 ? 1 : ((flo < 0.0) != (fhi < 0.0) && fhi != 0.0 ? 2 : 0));
+      plo[k] = lo;
+      v[k] = lo;
+      if (use) lo = hi;
+    }
+  }
+  int k = what[0] == 2 ? 0 : (what[1] == 2 ? 1 : (what[2] == 2 ? 2 : 3));
+  double lo = 0.0, hi = 0.0, flo = 0.0, x = 0.0;
+  int it = -1;  // -1: the piece is not begun
+  while (k < 3) {
+    if (it < 0) {
+      lo = k == 0 ? plo[0] : (k == 1 ? plo[1] : plo[2]);
+      hi = k == 0 ? s1 : (k == 1 ? s2 : bound);
+      flo = cubic_eval(a, b, cc, lo);
+      x = 0.5 * (lo + hi);
+      it = 0;
+    }
+    const double fx = cubic_eval(a, b, cc, x);
+    bool done = fx == 0.0;
+    if (!done) {
+      if ((fx < 0.0) == (flo < 0.0)) {
+        lo = x;
+        flo = fx;
+      } else
+        hi = x;
+      const double d = (3.0 * x + 2.0 * a) * x + b;
+      double xn = d != 0.0 ? x - fx / d : 0.5 * (lo + hi);
+      if (!(xn > lo && xn < hi)) xn = 0.5 * (lo + hi);
+      done = fabs(xn - x) <= 1e-15 * fabs(x) || hi - lo <= 1e-15 * fabs(x) || ++it == 100;
+      x = xn;
+    }
+    if (done) {
+      v[0] = k == 0 ? x : v[0];
+      v[1] = k == 1 ? x : v[1];
+      v[2] = k == 2 ? x : v[2];
+      k = k == 0 ? (what[1] == 2 ? 1 : (what[2] == 2 ? 2 : 3)) : (k == 1 && what[2] == 2 ? 2 : 3);
+      it = -1;
+    }
+  }
   int nr = 0;
   double last = 0.0;
   r0 = r1 = r2 = 0.0;
-  double lo = -bound;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const bool use = k == 0 ? v1 : (k == 1 ? v2 : true);
-    const double hi = k == 0 ? s1 : (k == 1 ? s2 : bound);
-    if (use) {
-      const double flo = cubic_eval(a, b, cc, lo), fhi = cubic_eval(a, b, cc, hi);
-      bool add = false;
-      double v = 0.0;
-      if (flo == 0.0) {
-        if (nr == 0 || last != lo) {
-          add = true;
-          v = lo;
-        }
-      } else if ((flo < 0.0) != (fhi < 0.0) && fhi != 0.0) {
-        add = true;
-        v = cubic_root_in(a, b, cc, lo, hi);
-      }
-      // value selects (not stores through a chosen reference) keep the
-      // roots in registers
-      r0 = (add && nr == 0) ? v : r0;
-      r1 = (add && nr == 1) ? v : r1;
-      r2 = (add && nr >= 2) ? v : r2;
-      last = add ? v : last;
-      nr += add ? 1 : 0;
-      lo = hi;
-    }
+  for (int q = 0; q < 3; ++q) {
+    const bool add = what[q] == 2 || (what[q] == 1 && (nr == 0 || last != plo[q]));
+    // value selects (not stores through a chosen reference) keep the
+    // roots in registers
+    r0 = (add && nr == 0) ? v[q] : r0;
+    r1 = (add && nr == 1) ? v[q] : r1;
+    r2 = (add && nr >= 2) ? v[q] : r2;
+    last = add ? v[q] : last;
+    nr += add ? 1 : 0;
   }
   const double fb = cubic_eval(a, b, cc, bound);
   const bool addb = fb == 0.0 && nr < 3;

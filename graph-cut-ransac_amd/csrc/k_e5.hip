@@ -31,8 +31,8 @@
 // the most bisections.  One thread per sample for the whole solver kept 5,360
 // bytes of matrices per thread in scratch memory.  Measured on MI355X, 32
 // pairs of 10,000 points at 10 % inliers: 1,079 ms of the call's kernels then,
-// 166 ms now (per 131,072 samples 139 + 86 + 118 + 224 us); the call 1,173 ->
-// 614 ms.
+// 166 ms with these kernels (per 131,072 samples 139 + 86 + 118 + 224 us, four
+// streams at once; alone 24 + 37 + 69 + 148); the call 1,173 -> 614 ms.
 #include "dev_essential.hpp"
 #include "kernels.hpp"
 
@@ -399,8 +399,10 @@ __device__ __forceinline__ void poly_det(const double (&A)[3][13], double* c) {
 // private memory.  An interval is pushed only when it holds a root (others
 // are never looked at), so there are at most as many as roots (ten) unless
 // rounding makes the sign counts inconsistent; one right sibling per level
-// of a depth of 30 is the limit then.
-constexpr int kE5Stack = 10, kE5StackMore = 24;
+// of a depth of 30 is the limit then.  Seven in LDS (19.2 KB with the intervals
+// found) let eight waves be resident on a compute unit, a whole slab at once;
+// with ten (23 KB) six were: 206 us per 131,072 samples on MI355X, 148 now.
+constexpr int kE5Stack = 7, kE5StackMore = 27;
 
 __global__ void __launch_bounds__(64) k_e5_roots(const double* __restrict__ pts,
                                                  const int64_t* __restrict__ pair_pt_off,

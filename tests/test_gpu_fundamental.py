@@ -36,6 +36,26 @@ def test_seven_point_bit_exact(oracle, engine, seed):
     assert np.array_equal(_bits(om[ok]), _bits(dm[ok]))
 
 
+# Samples whose cubics have roots at or beside piece ends, repeated or missing:
+# small integer lattices, repeated points, shifted copies, coordinates near 1.
+@pytest.mark.parametrize("what", ["lattice", "shift", "repeat", "unit"])
+def test_seven_point_root_cases_bit_exact(oracle, engine, what):
+    rng = np.random.default_rng(len(what))
+    pts = rng.integers(-3, 4, (400, 4)).astype(np.float64)
+    if what == "shift":
+        pts[:, 2:] = pts[:, :2] + rng.integers(0, 2, (400, 2))
+    elif what == "repeat":
+        pts = pts[rng.integers(0, 12, 400)] + rng.normal(size=(400, 4)) * 1e-3
+    elif what == "unit":
+        pts = rng.uniform(-1, 1, (400, 4))
+    samples = np.stack([rng.choice(len(pts), 7, replace=False) for _ in range(4097)]).astype(np.int32)
+    om, ost = oracle.f7_solve(pts, samples)
+    dm, dst = engine.solve_minimal(1, pts, samples)
+    assert np.array_equal(ost, dst)
+    ok = ost == 2
+    assert np.array_equal(_bits(om[ok]), _bits(dm[ok]))
+
+
 def test_sampson_scoring_bit_exact(oracle, engine):
     sc = _scene(2)
     pts = sc["corr"]
