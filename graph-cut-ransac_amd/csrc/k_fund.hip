@@ -88,7 +88,8 @@ struct FitShared {
   double tau[9];
   int rowt[9];
   double q[9];       // null vector
-  double JtJ[7][7];  // lower triangle
+  double sum[36];    // J^T r (7), then J^T J's lower triangle row by row
+  double quot[2][20];  // quotients of the rotation steps of U and V
   double sol[7];
   double U[9], V[9], sigma;     // current factorisation
   double Un[9], Vn[9], sigman;  // candidate step
@@ -358,8 +359,12 @@ __device__ void rot_update(const double* w, double a, double b, const double* Ui
 
 // Levenberg-Marquardt refinement (25 iterations, truncated loss, scale 1) of
 // the model in Fio (LDS).  The sums over points are wave-parallel; the dense
-// 7 x 7 steps run on lane 0 with their state in S, and every value the whole
-// wave needs is read back from S after a barrier.
+// 7 x 7 steps run on the first wave with their state in S, and every value the
+// whole block needs is read back from S after a barrier.  A batch's inner fits
+// (49 points, 47,750 fits a launch) are bound by instruction issue: about 2,300
+// instructions an iteration, 4.36 ms a launch on MI355X; 4.87 with the sums
+// stored entry by entry, the diagonal and the forward substitution formed on
+// every lane and the rotations' quotients fetched by lane permutes.
 template <int NT>
 __device__ void wave_lm_f(const FitRows& R, FitShared& S, double* Fio, int& jac_passes, int& cost_passes,
                           const BlockRed& B) {
@@ -377,6 +382,9 @@ __device__ void wave_lm_f(const FitRows& R, FitShared& S, double* Fio, int& jac_
   double cost = lm_cost<NT>(R, Fm, B);
   ++cost_passes;
   double Jtr[7];
+  // lane i < 7 keeps the damped diagonal entry of its row
+  const int row = threadIdx.x < 7 ? threadIdx.x : 6;
+  double diag = 0.0;
   bool recompute = true;
   for (int iter = 0; iter < 25; ++iter) {
     if (recompute) {
@@ -462,19 +470,16 @@ __device__ void wave_lm_f(const FitRows& R, FitShared& S, double* Fio, int& jac_
           if (e < 7) return 0.0 + wres * J[e];
           return 0.0 + w * (J[kTi[e]] * J[kTj[e]]);
         };
+        double z[9];
+#pragma unroll
+        for (int g = 0; g < 9; ++g)
+          z[g] = wave_tree64x4(term(4 * g), term(4 * g + 1), term(4 * g + 2), term(4 * g + 3));
+        // the rows' first lanes hold the totals (x4_lane)
         const int lane = lane_id();
+        if ((lane & 15) == 0) {
+          double* o = S.sum + ((lane >> 5) | ((lane >> 3) & 2));
 #pragma unroll
-        for (int g = 0; g < 36; g += 4) {
-          const double z = wave_tree64x4(term(g), term(g + 1), term(g + 2), term(g + 3));
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int e = g + r;
-            if (e < 7) {
-              Jtr[e] = readlane_f64(z, x4_lane(r));
-            } else if (e < 35) {
-              if (lane == x4_lane(r)) S.JtJ[kTi[e]][kTj[e]] = z;
-            }
-          }
+          for (int g = 0; g < 9; ++g) o[4 * g] = z[g];
         }
       } else {
         // the map dF / d(parameters) in registers on every thread, as above
@@ -542,64 +547,42 @@ __device__ void wave_lm_f(const FitRows& R, FitShared& S, double* Fio, int& jac_
           }
         }
         block_tree<NT, 35>(acc, B.red, B.tot);
-        {
-          int o = 0;
-  #pragma unroll
-          for (int i = 0; i < 7; ++i) Jtr[i] = acc[o++];
-  #pragma unroll
-          for (int i = 0; i < 7; ++i)
-  #pragma unroll
-            for (int j = 0; j <= i; ++j) {
-              const double v = acc[o++];
-              if (t0) S.JtJ[i][j] = v;
-            }
-        }
+        if (threadIdx.x < 35) S.sum[threadIdx.x] = B.tot[threadIdx.x];
       }
 #undef PROWS
 #undef DS
 #undef FE
+      __syncthreads();  // the sums, written by the lanes that hold them
+      diag = S.sum[7 + row * (row + 1) / 2 + row];
+#pragma unroll
+      for (int i = 0; i < 7; ++i) Jtr[i] = S.sum[i];
       double gn = 0.0;
       for (int i = 0; i < 7; ++i) gn += Jtr[i] * Jtr[i];
       if (sqrt(gn) < 1e-8) break;
     }
-    __syncthreads();  // JtJ written by the lanes that hold its totals
-    if (t0)
-      for (int k = 0; k < 7; ++k) S.JtJ[k][k] += lambda;  // the LDS copy keeps the reject bookkeeping
-    __syncthreads();
+    diag += lambda;  // (a rejected step takes it off again)
     if (threadIdx.x < 64) {
-      // Cholesky of the damped lower triangle, column by column: every lane
-      // forms the diagonal (the same value everywhere) from row j, lane i > j
-      // forms L[i][j] from its own row i, and the column is broadcast.  The
-      // forward substitution runs beside the factorisation (y[j] once row j
-      // is complete), the back substitution after it, both on every lane
-      // without branches.  Every element keeps the sequential order of its
-      // sums.
+      // Cholesky of the damped lower triangle, column by column: lane i >= j
+      // forms the sum of its own row, whose square root on lane j is L[j][j]
+      // and whose quotient by it on the lanes below is L[i][j]; the column is
+      // broadcast.  Lane 7 holds -J^T r as one more row, so the forward
+      // substitution is its quotients; the back substitution runs on every
+      // lane.  Every element keeps the sequential order of its sums.
       const int l = threadIdx.x;
-      double a[7], Lr[7];
+      double Lr[7], y[7];
+      double L[7][7], sol[7];
 #pragma unroll
       for (int j = 0; j < 7; ++j) {
-        a[j] = (l < 7 && j <= l) ? S.JtJ[l < 7 ? l : 0][j] : 0.0;
-        Lr[j] = 0.0;
-      }
-      double L[7][7], y[7], sol[7];
-#pragma unroll
-      for (int j = 0; j < 7; ++j) {
-        double d = S.JtJ[j][j];
-#pragma unroll
-        for (int k = 0; k < j; ++k) d -= L[j][k] * L[j][k];
-        L[j][j] = sqrt(d);
-        double v = a[j];
+        double v = l == 7 ? -Jtr[j] : (l == j ? diag : S.sum[7 + row * (row + 1) / 2 + (j < row ? j : row)]);
 #pragma unroll
         for (int k = 0; k < j; ++k) v -= Lr[k] * L[j][k];
-        const double lij = v / L[j][j];
-        if (l > j) Lr[j] = lij;
+        L[j][j] = readlane_f64(sqrt(v), j);
+        Lr[j] = v / L[j][j];
 #pragma unroll
         for (int i = j + 1; i < 7; ++i) L[i][j] = readlane_f64(Lr[j], i);
-        double u = -Jtr[j];
-#pragma unroll
-        for (int k = 0; k < j; ++k) u -= L[j][k] * y[k];
-        y[j] = u / L[j][j];
       }
+#pragma unroll
+      for (int j = 0; j < 7; ++j) y[j] = readlane_f64(Lr[j], 7);
 #pragma unroll
       for (int i = 6; i >= 0; --i) {
         double v = y[i];
@@ -620,31 +603,25 @@ __device__ void wave_lm_f(const FitRows& R, FitShared& S, double* Fio, int& jac_
       // the rotation steps of U (lane 0) and V (lane 1) side by side.  The
       // divisions they need, per side 3 axis components w_i / theta and the
       // 17 series quotients of sin / cos theta, are independent: lane
-      // 20 side + j forms division j of that side, and lanes 0 and 1 fetch
-      // their side's 20.
-      const int l = threadIdx.x;
-      double thv[2], kv[2], rv[2], r2v[2];
-#pragma unroll
-      for (int sd = 0; sd < 2; ++sd) {
-        const double w0 = S.sol[3 * sd], w1 = S.sol[3 * sd + 1], w2 = S.sol[3 * sd + 2];
-        thv[sd] = sqrt(w0 * w0 + w1 * w1 + w2 * w2);
-        sct_reduce(thv[sd], kv[sd], rv[sd], r2v[sd]);
-      }
-      const int sd = l >= 20 ? 1 : 0;
-      const int j = l - 20 * sd;
-      const int jc = j < 20 ? j : 19;
-      const double num = jc < 3 ? S.sol[3 * sd + jc] : (sd ? r2v[1] : r2v[0]);
-      const double den = jc < 3 ? (sd ? thv[1] : thv[0]) : sct_denominator(jc - 3);
-      const double qt = num / den;
-      const int src = l < 2 ? 20 * l : 0;
-      double w[3], q[17];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) w[i] = __shfl(qt, src + i, 64);
-#pragma unroll
-      for (int m = 0; m < 17; ++m) q[m] = __shfl(qt, src + 3 + m, 64);
+      // 2 j + side forms division j of that side, and lanes 0 and 1 fetch
+      // their side's 20 through LDS.
+      const int l = threadIdx.x, sd = l & 1;
+      const double* so = S.sol + 3 * sd;
+      const double th = sqrt(so[0] * so[0] + so[1] * so[1] + so[2] * so[2]);
+      double kk, rr, rr2;
+      sct_reduce(th, kk, rr, rr2);
+      const int j = (l >> 1) < 20 ? l >> 1 : 19;
+      const double qt = (j < 3 ? so[j < 3 ? j : 0] : rr2) / (j < 3 ? th : sct_denominator(j - 3));
+      if (l < 40) S.quot[sd][j] = qt;
+      __builtin_amdgcn_wave_barrier();
       if (l < 2) {
+        double w[3], q[17];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) w[i] = S.quot[l][i];
+#pragma unroll
+        for (int m = 0; m < 17; ++m) q[m] = S.quot[l][3 + m];
         double a, b;
-        sct_finish(l == 0 ? kv[0] : kv[1], l == 0 ? rv[0] : rv[1], q, a, b);
+        sct_finish(kk, rr, q, a, b);
         rot_update(w, a, b, l == 0 ? S.U : S.V, l == 0 ? S.Un : S.Vn);
         if (l == 0) S.sigman = S.sigma + S.sol[6];
       }
@@ -655,16 +632,14 @@ __device__ void wave_lm_f(const FitRows& R, FitShared& S, double* Fio, int& jac_
     const double cost_new = lm_cost<NT>(R, Fnm, B);
     ++cost_passes;
     const bool accept = cost_new < cost;
-    if (t0) {
-      if (accept) {
-        for (int i = 0; i < 9; ++i) {
-          S.U[i] = S.Un[i];
-          S.V[i] = S.Vn[i];
-        }
-        S.sigma = S.sigman;
-      } else {
-        for (int k = 0; k < 7; ++k) S.JtJ[k][k] -= lambda;
+    if (accept) {
+      if (threadIdx.x < 9) {
+        S.U[threadIdx.x] = S.Un[threadIdx.x];
+        S.V[threadIdx.x] = S.Vn[threadIdx.x];
       }
+      if (t0) S.sigma = S.sigman;
+    } else {
+      diag -= lambda;
     }
     if (accept) {
       lambda /= 10;
