@@ -1509,7 +1509,7 @@ struct Workspace {
   DevBuf<uint64_t> d_keys, d_skeys;
   DevBuf<int32_t> d_vals, d_svals, d_run_start, d_run_len, d_pos_of;
   DevBuf<int64_t> d_out_deg, d_edge_off;
-  DevBuf<int32_t> d_cell_pair, d_cell_start, d_cell_len, d_num_cells;
+  DevBuf<int32_t> d_cell_pair, d_cell_start, d_cell_len, d_num_cells, d_cell_list;
   DevBuf<char> d_tmp;
   DevBuf<int64_t> d_rf, d_rb, d_node_src, d_node_sink;
   // radius neighbourhood (pairs with neighborhood 1): per-pair flag and
@@ -2236,6 +2236,7 @@ struct Engine : Workspace {
       d2h(&ncell, d_num_cells.p, 1);
       sync();
       num_cells = ncell;
+      if (num_cells > kCellGrid) d_cell_list.ensure((size_t)num_cells + 1);
       std::vector<int32_t> clen(std::max(1, ncell));
       d2h(clen.data(), d_cell_len.p, (size_t)ncell);
       sync();
@@ -2736,7 +2737,7 @@ struct Engine : Workspace {
     const int t1 = prof.start("mincut", 0.0);
     launch_mincut_cells(stream, d_cell_pair.p, d_cell_start.p, d_cell_len.p, num_cells, u_act, d_pair_lambda.p,
                         d_pair_pt_off.p, d_svals.p, d_edge_off.p, d_rf.p, d_rb.p, d_node_src.p, d_node_sink.p, d_h.p,
-                        d_hn.p, d_sink.p, d_failw, max_cell);
+                        d_hn.p, d_sink.p, d_failw, max_cell, d_cell_list.p);
     if (!radius_pairs.empty())
       launch_mincut_radius(stream, d_rpairs.p, (int)radius_pairs.size(), u_act, d_pair_lambda.p, d_pair_pt_off.p,
                            d_pair_n.p, d_adj_off.p, d_adj_arc.p, d_adj_other.p, d_rf.p, d_rb.p, d_node_src.p,

@@ -94,12 +94,14 @@ void launch_lo_caps(hipStream_t st, const int32_t* pt_pair, const int8_t* pair_a
 // ones use gh / ghn (one int32 per point of the batch) and node_src /
 // node_sink in place.  pair_fail[p] = 1 when a cell of pair p did not
 // converge.
+// cell_list: num_cells + 1 int32 of scratch when num_cells > kCellGrid.
 constexpr int kMaxLdsCell = 2048;
+constexpr int kCellGrid = 32768;
 void launch_mincut_cells(hipStream_t st, const int32_t* cell_pair, const int32_t* cell_start, const int32_t* cell_len,
                          int num_cells, const int8_t* pair_active, const double* pair_lambda,
                          const int64_t* pair_pt_off, const int32_t* svals, const int64_t* edge_off, int64_t* rf,
                          int64_t* rb, int64_t* node_src, int64_t* node_sink, int32_t* gh, int32_t* ghn,
-                         uint8_t* sink_out, int32_t* pair_fail, int max_cell);
+                         uint8_t* sink_out, int32_t* pair_fail, int max_cell, int32_t* cell_list);
 // radius neighbourhood (k_radius.hip): tiles of 256 query points of one pair
 void launch_radius_search(hipStream_t st, bool fill, const double* pts, const int32_t* tile_pair,
                           const int32_t* tile_first, int num_tiles, const int64_t* pair_pt_off, const int32_t* pair_n,

@@ -92,3 +92,18 @@ def test_grouped_batch_device_input(monkeypatch):
         assert np.array_equal(masks[offsets[i]:offsets[i + 1]].astype(bool), m), i
         if M is not None:
             assert np.array_equal(models[9 * i:9 * i + 9].view(np.uint64), M.ravel().view(np.uint64)), i
+
+
+def test_listed_cells_identical_to_a_block_per_cell(monkeypatch):
+    """One group of more than 32,768 grid cells (the cells that label are
+    listed) against eight groups of fewer (a block per cell)."""
+    probs = []
+    for i in range(64):
+        kind = "homography" if i % 2 else "fundamental"
+        sc = getattr(synthetic, kind + "_scene")(synthetic.scene_seed(9, i), n=4000, inlier_ratio=0.5)
+        probs.append(dict(kind=kind, correspondences=sc["corr"], h1=480, w1=640, h2=480, w2=640, threshold=1.5,
+                          conf=0.99, spatial_coherence_weight=0.975, max_iters=300 + i, min_iters=50, use_sprt=False,
+                          sampler=0, neighborhood=0, neighborhood_size=8.0, lo_number=20, seed=500 + i))
+    a, sa = _run(monkeypatch, probs, 1)
+    b, sb = _run(monkeypatch, probs, 8)
+    _same(a, b, sa, sb)
