@@ -14,33 +14,27 @@
 // homography residual, one per Sampson residual) and, for high-inlier models,
 // by the in-order accumulation, 65,536 Sampson models on 5,000 points (a third
 // of them near the truth): 1,447 us with the terms through the scalar unit,
-// 891 us with wave_chain; 64 homographies on 1,000 points: 24.7 and 14.7 us.
+// 891 us with wave_chain.
 #include "dev_common.hpp"
 #include "kernels.hpp"
 
 namespace gcr {
 
-// Scores model slot mdl on the calling wave (every lane takes part).
+struct ModelScore {
+  int32_t count, sym;
+  double value;
+};
+
+// Scores the model at Mp over the n points at P on the calling wave (every lane
+// takes part; the result is lane 0's).  qr: 128 doubles of LDS.
 template <int KIND>
-__device__ __forceinline__ void score_model(int64_t mdl, const double* __restrict__ pts,
-                                            const int64_t* __restrict__ pair_pt_off,
-                                            const int32_t* __restrict__ pair_n,
-                                            const double* __restrict__ pair_sq_thr,
-                                            const double* __restrict__ models,
-                                            const int32_t* __restrict__ model_pair, int32_t* __restrict__ counts,
-                                            double* __restrict__ values, uint8_t* __restrict__ masks,
-                                            const int64_t* __restrict__ mask_off, int32_t* __restrict__ sym_counts,
-                                            int slots_per, double* qr) {
+__device__ __forceinline__ ModelScore score_points(const double* __restrict__ P, int n, double thr,
+                                                   const double* __restrict__ Mp, uint8_t* __restrict__ mask,
+                                                   bool sym_counts, double* qr) {
   const int lane = lane_id();
-  // model_pair holds one entry per group of slots_per model slots
-  const int pair = model_pair[slots_per == 1 ? mdl : mdl / slots_per];
-  const double* __restrict__ P = pts + 4 * pair_pt_off[pair];
-  const int n = pair_n[pair];
-  const double thr = pair_sq_thr[pair];
   double M[9];
 #pragma unroll
-  for (int k = 0; k < 9; ++k) M[k] = models[9 * mdl + k];
-  uint8_t* mask = (masks && mask_off[mdl] >= 0) ? masks + mask_off[mdl] : nullptr;
+  for (int k = 0; k < 9; ++k) M[k] = Mp[k];
   double acc = 0.0;
   int64_t cnt = 0, scnt = 0;
   if constexpr (KIND == 1) {
@@ -117,10 +111,49 @@ __device__ __forceinline__ void score_model(int64_t mdl, const double* __restric
     }
     if (qn > 0) acc = wave_chain(acc, lane < qn ? qr[lane] : 0.0, -1.0, qn);
   }
-  if (lane == 0) {
-    counts[mdl] = (int32_t)cnt;
-    values[mdl] = cnt == 0 ? 0.0 : (acc + (double)cnt * thr) / thr;
-    if (sym_counts) sym_counts[mdl] = (int32_t)scnt;
+  return ModelScore{(int32_t)cnt, (int32_t)scnt, cnt == 0 ? 0.0 : (acc + (double)cnt * thr) / thr};
+}
+
+// Scores model slot mdl on the calling wave.
+template <int KIND>
+__device__ __forceinline__ void score_model(int64_t mdl, const double* __restrict__ pts,
+                                            const int64_t* __restrict__ pair_pt_off,
+                                            const int32_t* __restrict__ pair_n,
+                                            const double* __restrict__ pair_sq_thr,
+                                            const double* __restrict__ models,
+                                            const int32_t* __restrict__ model_pair, int32_t* __restrict__ counts,
+                                            double* __restrict__ values, uint8_t* __restrict__ masks,
+                                            const int64_t* __restrict__ mask_off, int32_t* __restrict__ sym_counts,
+                                            int slots_per, double* qr) {
+  // model_pair holds one entry per group of slots_per model slots
+  const int pair = model_pair[slots_per == 1 ? mdl : mdl / slots_per];
+  const ModelScore r = score_points<KIND>(pts + 4 * pair_pt_off[pair], pair_n[pair], pair_sq_thr[pair],
+                                          models + 9 * mdl,
+                                          (masks && mask_off[mdl] >= 0) ? masks + mask_off[mdl] : nullptr,
+                                          sym_counts != nullptr, qr);
+  if (lane_id() == 0) {
+    counts[mdl] = r.count;
+    values[mdl] = r.value;
+    if (sym_counts) sym_counts[mdl] = r.sym;
+  }
+}
+
+// One set of points, 64-bit counts, model m's mask at masks + m n: a single
+// launch with no tables on the device.
+template <int KIND>
+__global__ void __launch_bounds__(256) k_score_direct(const double* __restrict__ pts, int n, double sq_thr,
+                                                      const double* __restrict__ models, int64_t num_models,
+                                                      int64_t* __restrict__ counts, double* __restrict__ values,
+                                                      uint8_t* __restrict__ masks) {
+  __shared__ double queue[4][128];
+  const int w = threadIdx.x >> 6;
+  const int64_t m = (int64_t)blockIdx.x * (blockDim.x / 64) + w;
+  if (m >= num_models) return;
+  const ModelScore r = score_points<KIND>(pts, n, sq_thr, models + 9 * m, masks ? masks + m * (int64_t)n : nullptr,
+                                          false, queue[w]);
+  if (lane_id() == 0) {
+    counts[m] = r.count;
+    values[m] = r.value;
   }
 }
 
@@ -216,6 +249,92 @@ __global__ void __launch_bounds__(256) k_score_list(const double* __restrict__ p
   for (int64_t k = lo + w; k < hi; k += waves_per_xcd)
     score_model<KIND>((int64_t)list[k], pts, pair_pt_off, pair_n, pair_sq_thr, models, model_pair, counts, values,
                       nullptr, nullptr, sym_counts, slots_per, queue[threadIdx.x >> 6]);
+}
+
+// The same for few models: a workgroup per model.  Waves 0 .. 3 evaluate 64
+// points each per round and leave their inliers' residuals in LDS, compacted,
+// in point order; wave 4 adds the round before's.  What bounds a model is then
+// the sequential addition (about 8 cycles an inlier) or, with few inliers, the
+// evaluation of 256 points a round.
+template <int KIND>
+__global__ void __launch_bounds__(320) k_score_split(const double* __restrict__ pts, int n, double thr,
+                                                     const double* __restrict__ models,
+                                                     int64_t* __restrict__ counts, double* __restrict__ values,
+                                                     uint8_t* __restrict__ masks) {
+  __shared__ double res[2][4][64];
+  __shared__ int cnts[2][4];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+  const int64_t m = blockIdx.x;
+  double M[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) M[k] = models[9 * m + k];
+  uint8_t* const mask = masks ? masks + m * (int64_t)n : nullptr;
+  const int rounds = (int)(((int64_t)n + 255) / 256);
+  double acc = 0.0;
+  int64_t cnt = 0;
+  for (int r = 0; r <= rounds; ++r) {
+    if (w < 4) {
+      const int64_t i = 256 * (int64_t)r + 64 * w + lane;
+      bool in = false;
+      double r2 = 0.0;
+      if (i < n) {
+        const double* s = pts + 4 * i;
+        if constexpr (KIND == 1) {
+          double num, den;
+          f_sampson_parts(s, M, num, den);
+          const double t = thr * den;
+          if (num < t * (1.0 - 1e-12)) in = true;
+          else if (!(num > t * (1.0 + 1e-12))) in = (num / den) < thr;
+          if (in) r2 = f_sq_sampson(s, M);
+        } else {
+          r2 = sq_residual<KIND>(s, M);
+          in = r2 < thr;
+        }
+        if (mask) mask[i] = in ? 1 : 0;
+      }
+      const uint64_t b = ballot64(in);
+      if (in) res[r & 1][w][__popcll(b & ((1ull << lane) - 1ull))] = r2;
+      if (lane == 0) cnts[r & 1][w] = __popcll(b);
+    } else if (r > 0) {
+      for (int v = 0; v < 4; ++v) {
+        const int c = __builtin_amdgcn_readfirstlane(cnts[(r - 1) & 1][v]);
+        if (c == 0) continue;
+        acc = wave_chain(acc, lane < c ? res[(r - 1) & 1][v][lane] : 0.0, -1.0, c);
+        cnt += c;
+      }
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 256) {
+    counts[m] = cnt;
+    values[m] = cnt == 0 ? 0.0 : (acc + (double)cnt * thr) / thr;
+  }
+}
+
+// Up to kSplitModels models a workgroup each, beyond that, where the chip is full
+// either way, a wave each.  Measured on MI355X, us per call, a wave against a
+// workgroup: 1,000 points, 64 / 1,024 / 2,048 models 8.8 / 9.1 / 11.2 against
+// 6.3 / 8.0 / 12.9; 5,000 points 43 / 45 / 55 against 23 / 30 / 58.
+constexpr int64_t kSplitModels = 1024;
+
+void launch_score_direct(hipStream_t st, int kind, const double* pts, int n, double sq_thr, const double* models,
+                         int64_t num_models, int64_t* counts, double* values, uint8_t* masks) {
+  if (num_models <= 0) return;
+  if (num_models <= kSplitModels) {
+    const dim3 grid((unsigned)num_models), block(320);
+    if (kind == 0)
+      hipLaunchKernelGGL(k_score_split<0>, grid, block, 0, st, pts, n, sq_thr, models, counts, values, masks);
+    else
+      hipLaunchKernelGGL(k_score_split<1>, grid, block, 0, st, pts, n, sq_thr, models, counts, values, masks);
+    return;
+  }
+  const dim3 grid((unsigned)((num_models + 3) / 4)), block(256);
+  if (kind == 0)
+    hipLaunchKernelGGL(k_score_direct<0>, grid, block, 0, st, pts, n, sq_thr, models, num_models, counts, values,
+                       masks);
+  else
+    hipLaunchKernelGGL(k_score_direct<1>, grid, block, 0, st, pts, n, sq_thr, models, num_models, counts, values,
+                       masks);
 }
 
 void launch_score(hipStream_t st, int kind, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,

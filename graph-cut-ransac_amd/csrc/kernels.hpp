@@ -29,6 +29,11 @@ void launch_score(hipStream_t st, int kind, const double* pts, const int64_t* pa
                   int32_t* sym_counts = nullptr, bool candidates = false, int slots_per = 1,
                   int32_t* work_list = nullptr, uint32_t* work_count = nullptr);
 
+// One set of n points: 64-bit counts, values and (nullable) masks of num_models
+// rows of n bytes, in a single launch.
+void launch_score_direct(hipStream_t st, int kind, const double* pts, int n, double sq_thr, const double* models,
+                         int64_t num_models, int64_t* counts, double* values, uint8_t* masks);
+
 // Candidate scoring on the matrix cores (FP16 hi/lo MFMA rejection of
 // proven outliers, FP64 in point order for every other point; same results as
 // launch_score).  launch_mx_prepare fills the points' operands and their slack

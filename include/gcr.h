@@ -214,11 +214,10 @@ int32_t gcr_score_models(int32_t kind, const double* pts, int64_t n, const doubl
  * hipMalloc).  No counterpart in the reference.  pts (n x 4), models
  * (k x 9), counts (k, int64), values (k) and masks (k x n, nullable) are
  * DEVICE pointers; the work is queued on `stream` (a hipStream_t; NULL = the
- * null stream) and the call returns without waiting.  The scoring kernel's
- * index tables live in a fixed device array of the library (about 1 MiB per
- * GPU, held until the process ends): k is limited to
- * GCR_SCORE_NOALLOC_MAX_MODELS and larger k is refused.  Calls that overlap
- * on one GPU share that array and race; order them on one stream.  No
+ * null stream) and the call returns without waiting.  The call is one kernel
+ * launch on that stream and uses no device memory besides these arguments, so
+ * calls on different streams may overlap.  k is limited to
+ * GCR_SCORE_NOALLOC_MAX_MODELS and larger k is refused.  No
  * hipMalloc, hipFree, memset or host synchronisation is made. */
 #define GCR_SCORE_NOALLOC_MAX_MODELS 65536
 int32_t gcr_score_models_noalloc(int32_t kind, const double* pts, int64_t n, const double* models, int64_t k,

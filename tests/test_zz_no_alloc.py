@@ -75,3 +75,23 @@ def test_noalloc_refuses_too_many_models():
                                     ctypes.c_void_p(16), ctypes.c_void_p(16), None, None)
     assert rc == _native.GCR_ERR_INVALID_ARGUMENT
     assert b"65536" in L.gcr_last_error()
+
+
+# Points around the 256 of a round, models around the line between a workgroup
+# and a wave per model.
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("n,k", [(1, 1), (63, 3), (255, 1023), (256, 1024), (257, 1025), (513, 5), (1999, 64)])
+def test_noalloc_round_and_model_edges(kind, n, k):
+    rng = np.random.default_rng(n)
+    make = synthetic.homography_scene if kind == 0 else synthetic.fundamental_scene
+    sc = make(synthetic.scene_seed(kind, 8))
+    p = np.ascontiguousarray(sc["corr"][:n])
+    M = _models(kind, sc, rng, k)
+    M[k // 2] = np.nan if k > 4 else M[k // 2]
+    c0, v0, m0 = _native.score_models(kind, p, M, 20.25, want_masks=True)
+    for masks in (True, False):
+        c1, v1, m1 = _noalloc(kind, p, M, 20.25, masks)
+        assert np.array_equal(c0, c1)
+        assert np.array_equal(v0.view(np.uint64), v1.view(np.uint64))
+        if masks:
+            assert np.array_equal(m0, m1)
