@@ -142,6 +142,8 @@ def test_gradient_tile_edges_match_oracle(engine, oracle, n):
     p = _net(5)
     loss, grad = guided.gradient(p, feat, labels)
     lo, go = oracle.mlp_loss_grad(p, feat, labels)
+    # |d loss| <= mean |dz|, and one row's |dz| may reach the forward bar (2e-2
+    # + 1e-2 |z|); few rows average little of it away: half the bar's 2e-2
     assert abs(loss - lo) <= 1e-4 * abs(lo) + (1e-2 if n < 32 else 0.0)
     rel = np.linalg.norm(grad - go) / np.linalg.norm(go)
     print("n=%d rel %.3g" % (n, rel))
