@@ -117,7 +117,7 @@ THRESHOLD = {0: 3.0, 1: 1.0, 2: 0.75}
 FLOP_PER_HYP_PT = {0: 18.0, 1: 42.0, 2: 42.0}
 SCORE_FAMILY = {0: "score_h", 1: "score_f", 2: "score_e"}
 SOLVER_FAMILY = {"solve_h4": "k_h4_solve (four-point homography)", "solve_f7": "k_f7_solve (seven-point fundamental)",
-                 "solve_e5": "k_e5_solve (five-point essential, Nister + Sturm)"}
+                 "solve_e5": "k_e5_null_space, _constraints, _eliminate, _roots (five-point essential, Nister + Sturm)"}
 
 
 def make_pairs(name, count, first=0):
