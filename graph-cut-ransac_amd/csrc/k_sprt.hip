@@ -54,6 +54,7 @@
 #include "dev_common.hpp"
 #include "dev_sp.hpp"
 #include "kernels.hpp"
+#include "sprt_rules.hpp"
 
 #include <algorithm>
 
@@ -669,18 +670,6 @@ __global__ void __launch_bounds__(64)
     }
   }
   if (lane == 0) items[blockIdx.x] = it;
-}
-
-SprtPlan sprt_plan(int num_items, int max_n, int max_slots, int64_t budget_words) {
-  SprtPlan p;
-  p.words = (max_n + 63) / 64;
-  const int64_t per_slot = 2 * (int64_t)p.words * std::max(1, num_items);
-  p.max_window = (int)std::min<int64_t>(max_slots, std::max<int64_t>(8, budget_words / per_slot));
-  // inlier and kept rows of a window, the start and record rows, values, kept
-  // and inlier counts
-  p.scratch_words = (size_t)(per_slot * p.max_window) + 2 * (size_t)p.words * (size_t)num_items +
-                    2 * (size_t)p.max_window * (size_t)num_items;
-  return p;
 }
 
 void launch_sprt_walk(hipStream_t st, SprtItem* items, int num_items, int max_slots, const SprtPlan& plan,

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "sprt_rules.hpp"
+
 namespace gcr {
 
 // minimal solvers
@@ -174,15 +176,6 @@ struct SprtItem {
   int32_t sp;              // the models go through the space partitioning selector first
   int64_t best_count;      // so-far-the-best inlier number (the selector's skip rule)
 };
-// Memory plan of a walk launch: 64-bit words of a point row, models per
-// window, words of scratch.  max_n / max_slots: the largest pair and the
-// longest slot list of the items; budget_words bounds the bit rows of a window
-// (a window holds at least 8 models).
-struct SprtPlan {
-  int words, max_window;
-  size_t scratch_words;
-};
-SprtPlan sprt_plan(int num_items, int max_n, int max_slots, int64_t budget_words);
 // items come with stop = last = -1.  sp_list: per point of the batch, the
 // tested inliers of the last model an SP walk tested (in test order, from the
 // pair's base)
