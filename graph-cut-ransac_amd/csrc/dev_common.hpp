@@ -33,6 +33,16 @@ __device__ __forceinline__ int64_t readlane_i64(int64_t v, int l) {
 
 __device__ __forceinline__ uint64_t ballot64(bool p) { return __ballot(p); }
 
+// Between lanes of one wave that hand values over through LDS: what was written
+// before is read after, and what is read before is not yet overwritten.  A
+// wave's LDS operations are in order, so no instruction comes of it; the fences
+// keep the compiler to that order (a wave barrier alone orders no memory).
+__device__ __forceinline__ void wave_lds_handover() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Reduction order used for every sum the engine evaluates in parallel:
 // lane l owns the terms whose index is congruent to l mod 64 (added in
 // ascending order into a partial that starts at 0.0); the 64 partials are

@@ -613,7 +613,7 @@ __device__ void wave_lm_f(const FitRows& R, FitShared& S, double* Fio, int& jac_
       const int j = (l >> 1) < 20 ? l >> 1 : 19;
       const double qt = (j < 3 ? so[j < 3 ? j : 0] : rr2) / (j < 3 ? th : sct_denominator(j - 3));
       if (l < 40) S.quot[sd][j] = qt;
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_handover();
       if (l < 2) {
         double w[3], q[17];
 #pragma unroll

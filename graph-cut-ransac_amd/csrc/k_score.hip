@@ -47,17 +47,19 @@ __device__ __forceinline__ ModelScore score_points(const double* __restrict__ P,
     // as before) and accumulated in queue order.  Same bits, far fewer
     // divisions when most points are outliers.
     int32_t* q = reinterpret_cast<int32_t*>(qr);
-    int qn = 0;
+    int qn = 0, head = 0;  // a ring of 128, head 0 or 64
     auto flush = [&](int cnt_flush) {
+      wave_lds_handover();
       double r2 = 0.0;
       bool sym_in = false;
       if (lane < cnt_flush) {
-        const double* s = P + 4 * (int64_t)q[lane];
+        const double* s = P + 4 * (int64_t)q[head + lane];
         r2 = f_sq_sampson(s, M);
         if (sym_counts) sym_in = f_sq_symmetric(s, M) < thr;
       }
       if (sym_counts) scnt += __popcll(ballot64(sym_in));
       acc = wave_chain(acc, r2, -1.0, cnt_flush);
+      wave_lds_handover();
     };
     const double lo = 1.0 - 1e-12, hi = 1.0 + 1e-12;
     for (int base = 0; base < n; base += 64) {
@@ -72,22 +74,22 @@ __device__ __forceinline__ ModelScore score_points(const double* __restrict__ P,
         if (mask) mask[i] = in ? 1 : 0;
       }
       const uint64_t b = ballot64(in);
-      if (in) q[qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u))] = i;
+      const int at = head + qn;
+      if (in)
+        q[__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, (uint32_t)at)) & 127u] = i;
       qn += __popcll(b);
       cnt += __popcll(b);
       if (qn >= 64) {
         flush(64);
-        const int rest = qn - 64;
-        const int32_t moved = lane < rest ? q[64 + lane] : 0;
-        if (lane < rest) q[lane] = moved;
-        qn = rest;
+        head ^= 64;
+        qn -= 64;
       }
     }
     flush(qn);
   } else {
     // transfer error: the inliers' residuals go to a per-wave queue (point
     // order) and are accumulated 64 at a time
-    int qn = 0;
+    int qn = 0, head = 0;
     for (int base = 0; base < n; base += 64) {
       const int i = base + lane;
       double r2 = 0.0;
@@ -98,18 +100,22 @@ __device__ __forceinline__ ModelScore score_points(const double* __restrict__ P,
         if (mask) mask[i] = in ? 1 : 0;
       }
       const uint64_t b = ballot64(in);
-      if (in) qr[qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u))] = r2;
+      const int at = head + qn;
+      if (in)
+        qr[__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, (uint32_t)at)) & 127u] = r2;
       qn += __popcll(b);
       cnt += __popcll(b);
       if (qn >= 64) {
-        acc = wave_chain(acc, qr[lane], -1.0, 64);
-        const int rest = qn - 64;
-        const double moved = lane < rest ? qr[64 + lane] : 0.0;
-        if (lane < rest) qr[lane] = moved;
-        qn = rest;
+        wave_lds_handover();
+        acc = wave_chain(acc, qr[head + lane], -1.0, 64);
+        wave_lds_handover();
+        head ^= 64;
+        qn -= 64;
       }
     }
-    if (qn > 0) acc = wave_chain(acc, lane < qn ? qr[lane] : 0.0, -1.0, qn);
+    wave_lds_handover();
+    if (qn > 0) acc = wave_chain(acc, lane < qn ? qr[head + lane] : 0.0, -1.0, qn);
+    wave_lds_handover();  // the next model's queue
   }
   return ModelScore{(int32_t)cnt, (int32_t)scnt, cnt == 0 ? 0.0 : (acc + (double)cnt * thr) / thr};
 }

@@ -693,16 +693,20 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
         bits &= bits - 1u;
       }
       qn += t3;
+      wave_lds_handover();
       int h = 0;
       for (; h + 64 <= qn; h += 64) flush(h, 64);
       if (h > 0) {
         const int rest = qn - h;
         const int32_t moved = lane < rest ? q[h + lane] : 0;
+        wave_lds_handover();
         if (lane < rest) q[lane] = moved;
         qn = rest;
       }
     }
+    wave_lds_handover();
     flush(0, qn);
+    wave_lds_handover();  // the next entry's queue
     if (lane == 0) {
       counts[slot] = (int32_t)cnt;
       values[slot] = cnt == 0 ? 0.0 : (acc + (double)cnt * thr) / thr;
