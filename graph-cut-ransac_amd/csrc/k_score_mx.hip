@@ -62,6 +62,7 @@
 // streams), 48 with one.
 #include "dev_common.hpp"
 #include "kernels.hpp"
+#include "mx_rules.hpp"
 
 namespace gcr {
 
@@ -374,7 +375,8 @@ __global__ void __launch_bounds__(256) k_mx_write(const int8_t* __restrict__ act
 // One thread per (list entry of the segment, lane half): the entry's scaled,
 // normalised coefficient vectors split into FP16 hi / lo and laid out as the
 // MFMA operand slices of that lane half (NQ quantities x 2 MFMAs x 8).  A
-// zero, inf or NaN model gets zero operands (nothing is rejected for it).
+// zero, inf or NaN model gets zero operands (mx_normalise; nothing is rejected
+// for it: the sign of a NaN would decide otherwise).
 template <int KIND>
 __global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pair_sq_thr,
                                                   const double* __restrict__ pair_inv_scale,
@@ -398,28 +400,9 @@ __global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pai
   for (int k = 0; k < 9; ++k) M[k] = models[9 * slot + k];
   const double is = pair_inv_scale[p];
   const double s = 1.0 / is;  // a power of two: exact
-  const double sc[3] = {s, s, 1.0};
-  double Fs[9], mx = 0.0;
-  if constexpr (KIND == 1) {
-    // F' = S F S: C, (F x1) and (F^T x2) in the scaled coordinates
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int k = 0; k < 3; ++k) Fs[3 * i + k] = M[3 * i + k] * sc[i] * sc[k];
-  } else {
-    // H' = S^-1 H S maps scaled x1 to scaled x2
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int k = 0; k < 3; ++k) Fs[3 * i + k] = M[3 * i + k] / sc[i] * sc[k];
-  }
-#pragma unroll
-  for (int k = 0; k < 9; ++k) mx = fabs(Fs[k]) > mx ? fabs(Fs[k]) : mx;
   const MxScale ts = mx_scale(pair_sq_thr[p], is);
-  const bool lp_ok = mx > 0.0 && mx <= 1e300 && ts.on;
-  const double inv_mx = lp_ok ? 1.0 / mx : 0.0;
-#pragma unroll
-  for (int k = 0; k < 9; ++k) Fs[k] = Fs[k] * inv_mx;
+  double Fs[9];
+  mx_normalise<KIND>(M, s, ts.on, Fs);
   double cq[2][9], dq[11];
   quantity_coefs<KIND>(Fs, cq);
   denominator_coefs<KIND>(Fs, dq);

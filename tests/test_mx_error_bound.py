@@ -13,7 +13,12 @@ near-threshold cases, tiny and subnormal-range operands, and coordinates at
 the scale limit |x'| = 1.  The measured worst case is reported as a fraction
 of the bound; the bound must hold everywhere.
 """
+import os
+import shutil
+import subprocess
+
 import numpy as np
+import pytest
 
 
 def _split16(v):
@@ -305,3 +310,19 @@ def test_scaled_test_never_drops_an_inlier():
             far_rej += int((rej & far).sum())
     print("far points dropped: %.3f" % (far_rej / far_n))
     assert far_rej > 0.9 * far_n
+
+
+def test_operands_of_any_model_are_numbers(tmp_path):
+    """The kernel's own normalisation (csrc/mx_rules.hpp) on models with inf,
+    NaN, huge and subnormal entries: operands of magnitude at most 1, or all
+    zero, with which nothing is dropped."""
+    gxx = shutil.which("g++")
+    if not gxx:
+        pytest.skip("g++ not available")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = str(tmp_path / "mx_check")
+    subprocess.check_call([gxx, "-std=c++17", "-O2", "-ffp-contract=off", "-Wno-unknown-pragmas", "-o", exe, "-I",
+                           os.path.join(root, "graph-cut-ransac_amd", "csrc"),
+                           os.path.join(root, "tests", "cpp", "mx_check.cpp")])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout
