@@ -142,7 +142,9 @@ __global__ void __launch_bounds__(kMaskThreads)
                  uint64_t* __restrict__ inl_bits, uint64_t* __restrict__ keep_bits, uint64_t* __restrict__ start_bits,
                  int32_t* __restrict__ kept_count, int32_t* __restrict__ inl_count,
                  double* __restrict__ approx) {
-  extern __shared__ uint8_t keep[];
+  // a bit per cell: the 48 bytes beside it leave room for every cell count that
+  // the selector's other kernels hold in LDS, a byte each
+  extern __shared__ uint64_t keep[];
   __shared__ int32_t part[kMaskThreads / 64];
   __shared__ double vpart[kMaskThreads / 64];
   const int item = (int)(blockIdx.x / (unsigned)live), j = (int)(blockIdx.x % (unsigned)live);
@@ -169,11 +171,16 @@ __global__ void __launch_bounds__(kMaskThreads)
     const int32_t* __restrict__ cell_of = sp_cell_of + base;
     const bool any = !(fabs(sp_det3(M)) < 1e-3);
     int32_t cnt = 0;
-    for (int c = threadIdx.x; c < sp.ncells; c += kMaskThreads) {
-      const SpCell cell = cells[c];
-      const bool k = any && sp_keep(M, cell, sp);
-      keep[c] = k ? 1 : 0;
-      if (k) cnt += cell.len;
+    for (int c0 = 64 * wave; c0 < sp.ncells; c0 += kMaskThreads) {
+      const int c = c0 + lane;
+      bool k = false;
+      if (c < sp.ncells) {
+        const SpCell cell = cells[c];
+        k = any && sp_keep(M, cell, sp);
+        if (k) cnt += cell.len;
+      }
+      const uint64_t b = ballot64(k);
+      if (lane == 0) keep[c0 >> 6] = b;
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) cnt += __shfl_xor(cnt, d, 64);
@@ -189,7 +196,7 @@ __global__ void __launch_bounds__(kMaskThreads)
       bool kp = false, inl = false, first = false;
       if (e < n) {
         const int c = cell_of[e];
-        kp = keep[c] != 0;
+        kp = (keep[c >> 6] >> (c & 63)) & 1ull;
         if (starts) first = e == 0 || cell_of[e - 1] != c;
         if (kp && tested) {
           const double r2 = h_sq_residual(P + 4 * (int64_t)sp_perm[base + e], M);
@@ -691,8 +698,9 @@ void launch_sprt_walk(hipStream_t st, SprtItem* items, int num_items, int max_sl
     int32_t* const count = kept + (size_t)num_items * win;
     const int live = std::min(win, max_slots - b);
     hipLaunchKernelGGL(k_sprt_masks, dim3((unsigned)live * (unsigned)num_items), dim3(kMaskThreads),
-                       (size_t)std::max(1, max_cells), st, items, b, win, live, pts, pair_pt_off, pair_n, pair_sq_thr,
-                       pools, sp_pairs, sp_cells, sp_perm, sp_cell_of, words, inl, keep, start, kept, count, approx);
+                       8 * (size_t)std::max(1, (max_cells + 63) / 64), st, items, b, win, live, pts, pair_pt_off,
+                       pair_n, pair_sq_thr, pools, sp_pairs, sp_cells, sp_perm, sp_cell_of, words, inl, keep, start, kept,
+                       count, approx);
     hipLaunchKernelGGL(k_sprt_walk, dim3((unsigned)num_items), dim3(64), 0, st, items, b, win, pts, pair_pt_off, pair_n,
                        pair_sq_thr, pools, sp_perm, words, inl, keep, start, kept, count, approx, rec, sp_list);
   }

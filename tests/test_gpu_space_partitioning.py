@@ -70,3 +70,41 @@ def test_batch_mixing_selector_and_plain_pairs(oracle):
     for i, ((M, mask), (rc, Mo, mo, so)) in enumerate(zip(res, refs)):
         assert stats[i]["status"] == rc, i
         _same(stats[i], so, M, Mo, mask, mo, rc)
+
+
+def test_sprt_on_as_many_cells_as_the_selector_holds(oracle):
+    """A cell per point and 163,820 of them: within 160 KB of LDS at a byte a
+    cell, which is what the selector's scoring and list kernels take, but not
+    beside other shared values (the mask kernel holds a bit a cell)."""
+    import pygcransac
+    n, side = 163820, 405
+    sc = synthetic.homography_scene(synthetic.scene_seed(17, 60), n=1000, inlier_ratio=0.5)
+    H = sc["H"]
+    rng = np.random.default_rng(60)
+    at = rng.permutation(side * side)[:n]
+    H = sc["H"]
+    x1 = np.stack([(at % side + 0.5) * 640 / side, (at // side + 0.5) * 480 / side, np.ones(n)], 1)
+    x2 = x1 @ H.T
+    x2 = x2[:, :2] / x2[:, 2:] + rng.normal(0, 0.5, (n, 2))
+    out = rng.random(n) < 0.4
+    x2[out] = rng.uniform(0, 1, (int(out.sum()), 2)) * [640, 480]
+    x2 = np.clip(x2, 0, [639.9, 479.9])
+    corr = np.ascontiguousarray(np.concatenate([x1[:, :2], x2], 1))
+    div = 410
+    cells = np.floor(corr / (np.array([640, 480, 640, 480]) / div)).astype(np.int64)
+    num = len(np.unique(cells, axis=0))
+    assert 163840 - 48 < num <= 163840
+    print("space partitioning with %d cells" % num, flush=True)
+    M, mask = pygcransac.findHomography(corr, 480, 640, 480, 640, None, threshold=3.0, conf=0.99,
+                                        spatial_coherence_weight=0.975, max_iters=60, min_iters=50, use_sprt=True,
+                                        sampler=0, neighborhood=0, neighborhood_size=float(div),
+                                        use_space_partitioning=True, lo_number=3, seed=2)
+    st = pygcransac.last_stats()
+    p = oracle.params(3.0, 0.99, 0.975, 60, 50, 0, 3, float(div), 2, use_sprt=True, use_space_partitioning=True)
+    rc, Ho, mo, so = oracle.find_homography(corr, 480, 640, 480, 640, p)
+    assert rc > 0.4 * n
+    assert np.array_equal(mask, mo)
+    for key in ("iteration_number", "local_optimization_number", "graph_cut_number"):
+        assert st[key] == so[key], key
+    # sums of 10^5 terms in another order in the normalisation: 10^5 2^-53
+    np.testing.assert_allclose(M, Ho, rtol=1e-9, atol=1e-9)
