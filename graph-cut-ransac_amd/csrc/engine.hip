@@ -2300,17 +2300,31 @@ struct Engine : Workspace {
     // thresholds / spatial weight of a pair whose loop switched estimator
     // (DEGENSAC's nested run); the sources are the pairs' own fields, which
     // stay unchanged until the step has synchronised
-    bool dirty = false;
-    for (auto& P : pairs)
+    int64_t base = 0;
+    std::vector<std::pair<int64_t, int64_t>> changed;  // first point and points of such pairs
+    for (auto& P : pairs) {
       if (P.params_dirty) {
         P.params_dirty = false;
-        dirty = true;
         h2d(d_pair_sq_thr.p + P.index, &P.sq_thr, 1);
         h2d(d_pair_lo_thr.p + P.index, &P.lo_thr, 1);
         h2d(d_pair_lambda.p + P.index, &P.lambda, 1);
+        changed.emplace_back(base, P.n);
       }
-    if (dirty && mx_on)
-      launch_mx_slack(stream, d_rpts, d_pt_pair.p, d_pair_sq_thr.p, d_pair_inv_scale.p, mx_total, d_mxp.p);
+      base += P.n;
+    }
+    if (mx_on && !changed.empty()) {
+      // the changed pairs' slack: a launch each, or one over all from the first
+      // to the last.  A launch takes 3.3 us, and 2 us of a launch over 256,000
+      // points are its traffic.
+      auto slack = [&](int64_t first, int64_t count) {
+        launch_mx_slack(stream, d_rpts, d_pt_pair.p, d_pair_sq_thr.p, d_pair_inv_scale.p, first, count, mx_total,
+                        d_mxp.p);
+      };
+      const int64_t first = changed.front().first, span = changed.back().first + changed.back().second - first;
+      if ((int64_t)(changed.size() - 1) * kSlackLaunchPoints > span) slack(first, span);
+      else
+        for (const auto& [at, count] : changed) slack(at, count);
+    }
     if (src.empty()) return;
     // two-phase: stage sources first so a slot that is both a source and a
     // destination in this batch is read before it is written
@@ -3045,6 +3059,7 @@ struct Engine : Workspace {
 
   // SPRT walks (k_sprt.hip), one wavefront per pair: the items and their
   // slot lists go up in one copy, the items come back in one copy.
+  static constexpr int64_t kSlackLaunchPoints = 400000;  // points whose traffic takes as long as a launch
   static constexpr size_t kTableChunk = 256;             // table entries per host task (~20 us)
   static constexpr int64_t kSprtBudgetWords = 32 << 20;  // 256 MB of bit rows per window
   PhaseTask exec_sprt(std::vector<PairCtx*> items) {

@@ -268,14 +268,15 @@ __global__ void __launch_bounds__(256) k_mx_points(const double* __restrict__ pt
     }
 }
 
-// Per point: the slack of its test under its pair's threshold (the plane
-// behind the operands).
+// Per point of [first, first + count): the slack of its test under its pair's
+// threshold (the plane behind the operands).
 __global__ void __launch_bounds__(256) k_mx_slack(const double* __restrict__ pts, const int32_t* __restrict__ pt_pair,
                                                   const double* __restrict__ pair_sq_thr,
-                                                  const double* __restrict__ inv_scale, int64_t total,
+                                                  const double* __restrict__ inv_scale, int64_t first, int64_t count,
                                                   float* __restrict__ slack) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= count) return;
+  const int64_t i = first + t;
   const int p = pt_pair[i];
   const double is = inv_scale[p];
   const MxScale sc = mx_scale(pair_sq_thr[p], is);
@@ -701,10 +702,10 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
 // ---- launchers --------------------------------------------------------------------
 
 void launch_mx_slack(hipStream_t st, const double* pts, const int32_t* pt_pair, const double* pair_sq_thr,
-                     const double* inv_scale, int64_t total, uint16_t* out) {
-  if (total <= 0) return;
-  hipLaunchKernelGGL(k_mx_slack, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, pts, pt_pair, pair_sq_thr,
-                     inv_scale, total, reinterpret_cast<float*>(out + kMxPlaneHalves * 4 * total));
+                     const double* inv_scale, int64_t first, int64_t count, int64_t total, uint16_t* out) {
+  if (count <= 0) return;
+  hipLaunchKernelGGL(k_mx_slack, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, pts, pt_pair, pair_sq_thr,
+                     inv_scale, first, count, reinterpret_cast<float*>(out + kMxPlaneHalves * 4 * total));
 }
 
 void launch_mx_prepare(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
@@ -715,7 +716,7 @@ void launch_mx_prepare(hipStream_t st, const double* pts, const int64_t* pair_pt
                      num_pairs, inv_scale);
   hipLaunchKernelGGL(k_mx_points, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, pts, pt_pair, inv_scale,
                      total, out);
-  launch_mx_slack(st, pts, pt_pair, pair_sq_thr, inv_scale, total, out);
+  launch_mx_slack(st, pts, pt_pair, pair_sq_thr, inv_scale, 0, total, total, out);
 }
 
 size_t mx_point_halves(int64_t total) {

@@ -41,13 +41,14 @@ void launch_score_direct(hipStream_t st, int kind, const double* pts, int n, dou
 // launch_score).  launch_mx_prepare fills the points' operands and their slack
 // under their pair's threshold (mx_point_halves(total) 16-bit words) and the
 // per-pair power-of-two inverse scale once per engine run; mx_total is its
-// `total`.  launch_mx_slack: the slack again, after a change of thresholds.
+// `total`.  launch_mx_slack: the slack of points [first, first + count) again,
+// after a change of their pair's threshold.
 size_t mx_point_halves(int64_t total);
 void launch_mx_prepare(hipStream_t st, const double* pts, const int64_t* pair_pt_off, const int32_t* pair_n,
                        const int32_t* pt_pair, const double* pair_sq_thr, int num_pairs, int64_t total,
                        double* inv_scale, uint16_t* out);
 void launch_mx_slack(hipStream_t st, const double* pts, const int32_t* pt_pair, const double* pair_sq_thr,
-                     const double* inv_scale, int64_t total, uint16_t* out);
+                     const double* inv_scale, int64_t first, int64_t count, int64_t total, uint16_t* out);
 // ints of blk_scratch that launch_score_mx needs for num_models slots, and
 // words of its candidate mask for pairs of at most max_n points
 size_t mx_list_scratch_ints(int64_t num_models);

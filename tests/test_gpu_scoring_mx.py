@@ -110,3 +110,24 @@ def test_mask_and_slice_edges_identical_to_fp64(monkeypatch, ns, eps):
         if Ma is not None:
             assert np.array_equal(Ma.view(np.uint64), Mb.view(np.uint64)), i
         assert s64[i]["score"] == smx[i]["score"] and s64[i]["models_scored"] == smx[i]["models_scored"], i
+
+
+def test_changed_thresholds_of_some_pairs_identical_to_fp64(monkeypatch):
+    """DEGENSAC's nested run changes its pair's threshold, and with it the
+    points' slack: plane-dominated pairs at the batch's start, middle and end,
+    ragged sizes, the pairs between unchanged."""
+    probs = []
+    for i, (plane, n) in enumerate([(0.9, 1500), (0.0, 1201), (0.0, 977), (0.85, 2049), (0.9, 700), (0.0, 1600),
+                                    (0.95, 1333)]):
+        sc = synthetic.fundamental_scene(synthetic.scene_seed(9, 10 + i), n=n, inlier_ratio=0.5, plane_fraction=plane)
+        probs.append(dict(kind="fundamental", correspondences=sc["corr"], h1=480, w1=640, h2=480, w2=640,
+                          threshold=1.0, conf=0.99, spatial_coherence_weight=0.975, max_iters=3000, min_iters=1000,
+                          use_sprt=False, sampler=0, neighborhood=0, neighborhood_size=8.0, lo_number=20,
+                          seed=70 + i))
+    r64, s64 = _run(monkeypatch, probs, False)
+    rmx, smx = _run(monkeypatch, probs, True)
+    for i, ((Ma, ma), (Mb, mb)) in enumerate(zip(r64, rmx)):
+        assert np.array_equal(ma, mb), i
+        assert np.array_equal(np.asarray(Ma).view(np.uint64), np.asarray(Mb).view(np.uint64)), i
+        for key in ("iteration_number", "graph_cut_number", "models_scored", "score"):
+            assert s64[i][key] == smx[i][key], (i, key)
