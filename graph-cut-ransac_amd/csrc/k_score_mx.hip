@@ -59,7 +59,7 @@
 // selects per tile, 158 with four products and lane writes of ballots (four
 // streams at once); the latter 156 and this form 96 with one stream.  Exact
 // pass: 184 with a walk over single mask bits, 74 with a word per lane (four
-// streams), 48 with one.
+// streams) and 38 with one, 30 with the queue in 16 bits.
 #include "dev_common.hpp"
 #include "kernels.hpp"
 #include "mx_rules.hpp"
@@ -76,7 +76,10 @@ constexpr double kDeltaAbs = 0x1p-20;
 constexpr double kMargin = 1.0 + 0x1p-14;
 constexpr double kEta = 0x1p-4;
 constexpr int kCompactPerBlock = 2048;  // slots per block of the ordered compaction
-constexpr int kMxBlocks = 2048;         // persistent grids: at most 8,192 waves
+// The exact pass's grid: the workgroups that are resident at 70 VGPRs, seven
+// waves per SIMD (2,048 workgroups, an eighth of them alone in a second round,
+// took 74.6 ms where these take 60.4).
+constexpr int kMxExactBlocks = 1792;
 // list entries per rejection + exact pass: as many as keep the segment's
 // candidate masks within kMxMaskBudget bytes, between kMxSegMin and
 // kMxSegMax (each segment costs three launches; the masks bound the memory)
@@ -580,9 +583,15 @@ __global__ void __launch_bounds__(256, KIND == 1 ? 4 : 3) k_mx_reject(
 
 // One wave per list entry of the segment.  The mask row is taken 64 words
 // (2,048 points) at a time, a word per lane: a prefix sum of the bit counts
-// gives every lane its place in the queue of candidate points (point order),
-// which the whole wave evaluates 64 at a time with the FP64 kernel's operations; inliers are accumulated in point order
-// through the scalar unit (value -= r2), as the FP64 kernel does.
+// gives every lane its places in the window's queue of candidate points (point
+// order), which the whole wave evaluates 64 at a time with the FP64 kernel's
+// operations; fewer than 64 wait in registers for the next window's.  Inliers
+// are accumulated in point order (value -= r2), as the FP64 kernel does.  The
+// queue holds 16-bit offsets into the window, 16 KB per workgroup, so that
+// registers (seven waves per SIMD) and not LDS bound the waves in flight: with
+// 33 KB, four waves per SIMD, 48.7 us a launch in an essential batch of 32 pairs
+// of 10,000 points and 58.0 in a fundamental one of 1,024 on MI355X, now 38.8 and
+// 50.6.
 template <int KIND>
 __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts,
                                                   const int64_t* __restrict__ pair_pt_off,
@@ -595,9 +604,9 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
                                                   int64_t seg_len, int words, const uint32_t* __restrict__ mask,
                                                   int32_t* __restrict__ counts, double* __restrict__ values,
                                                   int32_t* __restrict__ sym_counts, int slots_per) {
-  __shared__ int32_t queue[4][64 + 64 * 32];
+  __shared__ uint16_t queue[4][64 * 32];
   const int lane = lane_id();
-  int32_t* q = queue[threadIdx.x >> 6];
+  uint16_t* q = queue[threadIdx.x >> 6];
   const int64_t total = (int64_t)*list_count;
   if (seg_begin >= total) return;
   const int64_t seg_n = total - seg_begin < seg_len ? total - seg_begin : seg_len;
@@ -617,14 +626,15 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
     const uint32_t* __restrict__ mk = mask + e * (int64_t)words;
     double acc = 0.0;
     int64_t cnt = 0, scnt = 0;
-    int qn = 0;
-    // evaluates the cnt_flush queued candidates from `at` on and accumulates the
-    // inliers among them in queue (= point) order
-    auto flush = [&](int at, int cnt_flush) {
+    int kept = 0;     // candidates kept for the next 64, in order, on lanes 0 .. kept - 1
+    int32_t mine = 0;
+    // evaluates the candidates of lanes 0 .. cnt_flush - 1 and accumulates the
+    // inliers among them in lane (= point) order
+    auto flush = [&](int32_t point, int cnt_flush) {
       bool in = false, sym_in = false;
       double r2 = 0.0;
       if (lane < cnt_flush) {
-        const double* s = P + 4 * (int64_t)q[at + lane];
+        const double* s = P + 4 * (int64_t)point;
         if constexpr (KIND == 1) {
           double num, den;
           f_sampson_parts(s, M, num, den);
@@ -671,26 +681,23 @@ __global__ void __launch_bounds__(256) k_mx_exact(const double* __restrict__ pts
       const int t0 = __builtin_amdgcn_readlane(before, 15), t1 = t0 + __builtin_amdgcn_readlane(before, 31),
                 t2 = t1 + __builtin_amdgcn_readlane(before, 47), t3 = t2 + __builtin_amdgcn_readlane(before, 63);
       before += lane >= 48 ? t2 : (lane >= 32 ? t1 : (lane >= 16 ? t0 : 0));
-      int at = qn + before - have;
+      int at = before - have;
       while (bits) {
-        q[at++] = 32 * (w0 + lane) + __ffs(bits) - 1;
+        q[at++] = (uint16_t)(32 * lane + __ffs(bits) - 1);
         bits &= bits - 1u;
       }
-      qn += t3;
       wave_lds_handover();
+      // the kept ones, then the window's
+      const int all = kept + t3;
+      auto point = [&](int k) { return k < kept ? mine : 32 * w0 + (int)q[k - kept]; };
       int h = 0;
-      for (; h + 64 <= qn; h += 64) flush(h, 64);
-      if (h > 0) {
-        const int rest = qn - h;
-        const int32_t moved = lane < rest ? q[h + lane] : 0;
-        wave_lds_handover();
-        if (lane < rest) q[lane] = moved;
-        qn = rest;
-      }
+      for (; h + 64 <= all; h += 64) flush(point(h + lane), 64);
+      const int32_t rest = h + lane < all ? point(h + lane) : 0;
+      mine = rest;
+      kept = all - h;
+      wave_lds_handover();  // the next window's queue
     }
-    wave_lds_handover();
-    flush(0, qn);
-    wave_lds_handover();  // the next entry's queue
+    flush(mine, kept);
     if (lane == 0) {
       counts[slot] = (int32_t)cnt;
       values[slot] = cnt == 0 ? 0.0 : (acc + (double)cnt * thr) / thr;
@@ -767,7 +774,7 @@ void launch_score_mx(hipStream_t st, int kind, const double* pts, const int64_t*
     if (b1 > kMxRejectBlocks) b1 = kMxRejectBlocks;
     b1 = (b1 + kNumXcd - 1) / kNumXcd * kNumXcd;
     int64_t b2 = (seg_len + 3) / 4;
-    if (b2 > kMxBlocks) b2 = kMxBlocks;
+    if (b2 > kMxExactBlocks) b2 = kMxExactBlocks;
     b2 = (b2 + kNumXcd - 1) / kNumXcd * kNumXcd;
     const unsigned bc = (unsigned)((2 * seg_len + 255) / 256);
     if (kind == 0) {
