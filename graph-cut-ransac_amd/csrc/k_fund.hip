@@ -35,6 +35,11 @@ __global__ void __launch_bounds__(256, 3) k_f7_solve(const double* __restrict__ 
   if (c >= num_cand) return;
   const double* P = pts + 4 * pair_pt_off[cand_pair[c]];
   const int32_t* s = samples + 7 * c;
+  if (s[0] < 0) {  // the sampler refused: indices of -1
+    for (int k = 0; k < 3; ++k) mstatus[3 * c + k] = 0;
+    nmodels[c] = 0;
+    return;
+  }
   double F[3][9];
   const int mask = thread_f7(P, s, F);
   // orientation filter, keeping the order of the remaining models

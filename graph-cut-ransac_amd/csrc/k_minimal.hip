@@ -61,7 +61,8 @@ __device__ __forceinline__ void gauss_elimination(double (&m)[S][S + 1], double 
   }
 }
 
-// status: 0 rejected by the sample test, 1 solver failure, 2 model written.
+// status: 0 refused by the sampler or the sample test, 1 solver failure, 2 model
+// written.
 // valid: isValidModel outcome for written models.
 __global__ void __launch_bounds__(256) k_h4_solve(const double* __restrict__ pts, const int64_t* __restrict__ pair_pt_off,
                                                   const int32_t* __restrict__ cand_pair,
@@ -72,6 +73,11 @@ __global__ void __launch_bounds__(256) k_h4_solve(const double* __restrict__ pts
   if (c >= num_cand) return;
   const double* P = pts + 4 * pair_pt_off[cand_pair[c]];
   const int32_t* s = samples + 4 * c;
+  if (s[0] < 0) {  // the sampler refused: indices of -1
+    status[c] = 0;
+    valid[c] = 0;
+    return;
+  }
   double pa[4], pb[4], pc[4], pd[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {

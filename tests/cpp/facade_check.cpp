@@ -19,17 +19,23 @@ thread_local std::string g_error;
 // (uniform_sampler.h:97-115 over uniform_random_generator.h:43-125) restated
 // with std::mt19937 and std::uniform_int_distribution<size_t>, seeded with
 // the low 32 bits of the seed as the engine seeds its own uniform sampler.
-// throw_after > 0: the call after that many samples throws.
+// throw_after > 0: the call after that many samples throws.  skip 1: every third
+// call refuses (returns false); skip 2: it gives one point for the whole sample
+// instead, from which no model comes.  Neither draws.
 class UserUniformSampler : public gcransac::sampler::Sampler<gcransac::Points, size_t> {
  public:
-  UserUniformSampler(const gcransac::Points* container_, uint64_t seed, int64_t throw_after)
-      : Sampler(container_), gen_((uint32_t)(seed & 0xffffffffu)), throw_after_(throw_after) {}
+  UserUniformSampler(const gcransac::Points* container_, uint64_t seed, int64_t throw_after, int skip = 0)
+      : Sampler(container_), gen_((uint32_t)(seed & 0xffffffffu)), throw_after_(throw_after), skip_(skip) {}
   const std::string getName() const override { return "User Uniform Sampler"; }
   void reset() override {}
   bool initialize(const gcransac::Points* const) override { return true; }
   bool sample(const std::vector<size_t>& pool_, size_t* const subset_, size_t sample_size_) override {
     if (throw_after_ > 0 && calls_++ >= throw_after_) throw std::runtime_error("user sampler failure");
     if (sample_size_ > pool_.size() || pool_.empty()) return false;
+    if (skip_ && skips_++ % 3 == 0) {
+      for (size_t k = 0; k < sample_size_; ++k) subset_[k] = pool_[0];
+      return skip_ == 2;
+    }
     if (pool_.size() != range_) {
       dist_ = std::uniform_int_distribution<size_t>(0, pool_.size() - 1);
       range_ = pool_.size();
@@ -49,12 +55,14 @@ class UserUniformSampler : public gcransac::sampler::Sampler<gcransac::Points, s
   std::uniform_int_distribution<size_t> dist_;
   size_t range_ = 0;
   int64_t throw_after_ = 0, calls_ = 0;
+  int skip_ = 0, skips_ = 0;
 };
 
 struct FacadeArgs {
   double threshold, confidence, spatial_coherence_weight;
   int64_t max_iters, min_iters;
-  int32_t sampler;  // 0 uniform, 1 PROSAC, 2 UserUniformSampler, 3 UserUniformSampler that throws
+  int32_t sampler;  // 0 uniform, 1 PROSAC, 2 UserUniformSampler, 3 UserUniformSampler that throws, 4 one that
+                    // refuses some samples, 5 one that gives one point for those
   int32_t lo_number;
   int32_t divisions;
   uint64_t seed;
@@ -78,7 +86,7 @@ int run_typed(const Estimator& estimator, const double* pts_, int64_t n, const d
   sampler::UniformSampler uniform(&points, a.seed);
   sampler::ProsacSampler prosac(&points, Estimator::sampleSize(), a.seed);
   sampler::UniformSampler lo_sampler(&points, a.seed);
-  UserUniformSampler user(&points, a.seed, a.sampler == 3 ? 40 : 0);
+  UserUniformSampler user(&points, a.seed, a.sampler == 3 ? 40 : 0, a.sampler >= 4 ? a.sampler - 3 : 0);
   sampler::SamplerBase* main_sampler = &uniform;
   if (a.sampler == 1) main_sampler = &prosac;
   if (a.sampler >= 2) main_sampler = &user;

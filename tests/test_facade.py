@@ -197,6 +197,37 @@ def test_user_sampler_plugin_matches_builtin_uniform(kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_refused_samples_give_no_model(oracle, kind):
+    # A sampler that refuses every third sample (Sampler::sample's false) runs
+    # as one that gives a single point for all of it: a minimal solver gets no
+    # model from either, and reads no point of a refused sample.
+    K = None
+    if kind == 0:
+        sc = synthetic.homography_scene(synthetic.scene_seed(4, 50), n=1500, inlier_ratio=0.4)
+        pts, grid, cells, thr = sc["corr"], None, _cells(640, 480, 8), 3.0
+    elif kind == 1:
+        sc = synthetic.fundamental_scene(synthetic.scene_seed(4, 51), n=2000, inlier_ratio=0.5)
+        pts, grid, cells, thr = sc["corr"], None, _cells(640, 480, 8), 1.0
+    else:
+        sc = synthetic.essential_scene(synthetic.scene_seed(4, 52), n=1500, inlier_ratio=0.5)
+        K1, K2 = sc["K1"], sc["K2"]
+        pts, K = oracle.normalise_correspondences(sc["corr"], K1, K2), np.concatenate([np.ravel(K1), np.ravel(K2)])
+        grid, cells, thr = sc["corr"], _cells(1024, 768, 8), 0.75 / K1[0, 0]
+    out = []
+    for sampler in (4, 5):
+        args = FacadeArgs(thr, 0.99, 0.975, 100000, 50, sampler, 50, 8, 11, 0, 1, 0, 0, 0.01, 0.0)
+        out.append(facade_run(kind, pts, grid, cells, args, K))
+    (rc0, M0, m0, st0, s0, e0), (rc1, M1, m1, st1, s1, e1) = out
+    assert rc0 > 0.3 * len(pts), e0
+    assert rc1 == rc0, e1
+    assert np.array_equal(m1, m0)
+    assert np.array_equal(st1[:4], st0[:4])
+    assert s1 == s0
+    assert np.array_equal(M1.view(np.int64), M0.view(np.int64))
+
+
+@pytest.mark.gpu
 def test_user_sampler_exception_reaches_the_caller():
     sc = synthetic.homography_scene(synthetic.scene_seed(4, 42), n=800, inlier_ratio=0.4)
     args = FacadeArgs(3.0, 0.99, 0.975, 100000, 50, 3, 50, 8, 11, 0, 1, 0, 0, 0.01, 0.0)
