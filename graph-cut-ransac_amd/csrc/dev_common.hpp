@@ -33,6 +33,24 @@ __device__ __forceinline__ int64_t readlane_i64(int64_t v, int l) {
 
 __device__ __forceinline__ uint64_t ballot64(bool p) { return __ballot(p); }
 
+// A value that is the same on every lane, held in scalar registers, so that the
+// control flow it decides is scalar (in the SPRT walk over cells, with it in
+// vector registers: about 200 instructions and 1,250 cycles per step).
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t uni(uint64_t v) {
+  return ((uint64_t)(uint32_t)uni((int)(v >> 32)) << 32) | (uint32_t)uni((int)(uint32_t)v);
+}
+
+// Sum over the wave, on every lane: DPP steps inside the rows of 16, then the four rows' totals.
+__device__ __forceinline__ int wave_sum_i32(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, false);  // row_ror:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x124, 0xF, 0xF, false);  // row_ror:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x122, 0xF, 0xF, false);  // row_ror:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x121, 0xF, 0xF, false);  // row_ror:1
+  return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
+         __builtin_amdgcn_readlane(v, 48);
+}
+
 // Between lanes of one wave that hand values over through LDS: what was written
 // before is read after, and what is read before is not yet overwritten.  A
 // wave's LDS operations are in order, so no instruction comes of it; the fences

@@ -1,11 +1,56 @@
-// SPRT walk: the memory plan of a walk launch (k_sprt.hip).
+// SPRT walk: the rules that decide without the reference's running product,
+// and the memory plan of a walk launch (k_sprt.hip).  Plain functions of
+// numbers, for the kernels and for host code.
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 
+#if defined(__HIP__)
+#define GCR_HOST_DEVICE __host__ __device__ __forceinline__
+#else
+#define GCR_HOST_DEVICE inline
+#endif
+
 namespace gcr {
+
+// The ratio's factors, their logarithms and log A with the band around it.
+struct Chain {
+  double f_in, f_out, A;
+  double l_in, l_out, l_A;
+  double hi, lo;  // log A and the margin around it
+  int unit;       // both factors are 1: the product stays at 1
+  int fast;       // the logarithms are finite
+};
+
+// The band of a walk over n positions.  Margin of a sum of at most n
+// logarithms: the product's n roundings (n 2^-53) and the logarithms' errors,
+// each with a factor of fifty and more to spare.
+GCR_HOST_DEVICE void chain_band(Chain& c, int n) {
+  const double m = 1e-14 * (16.0 + (double)n) + 1e-13 * (double)n * fmax(fabs(c.l_in), fabs(c.l_out));
+  c.hi = c.l_A + m;
+  c.lo = c.l_A - m;
+  c.unit = c.f_in == 1.0 && c.f_out == 1.0;
+  c.fast = fabs(c.l_in) < 1e300 && fabs(c.l_out) < 1e300 && fabs(c.l_A) < 1e300;
+}
+
+// The logarithm of the ratio after a inliers and b outliers; above A for
+// certain, below A for certain, or neither; a product below e^-690 is near the
+// subnormal range.
+GCR_HOST_DEVICE double chain_log(const Chain& c, int a, int b) { return (double)a * c.l_in + (double)b * c.l_out; }
+GCR_HOST_DEVICE bool chain_above(const Chain& c, double l) { return l > c.hi; }
+GCR_HOST_DEVICE bool chain_below(const Chain& c, double l) { return l < c.lo; }
+GCR_HOST_DEVICE bool chain_low(double l) { return l < -690.0; }
+
+// A product below e^-690 cannot exceed A within `left` more factors: it has at
+// least 690 + log A to climb, and no less if it passes through the subnormal
+// range (the climb from 2^-1022 on is in the normal range).
+GCR_HOST_DEVICE bool chain_no_return(const Chain& c, int left) {
+  const double up = fmax(fmax(c.l_in, c.l_out), 0.0);
+  return (double)left * up * (1.0 + 1e-9) < 680.0 + c.l_A;
+}
 
 // Memory plan of a walk launch: 64-bit words of a point row, models per
 // window, words of scratch.  max_n / max_slots: the largest pair and the

@@ -1,16 +1,17 @@
-"""The SPRT walk's decision rule (csrc/k_sprt.hip, chain_side) against the
-reference's running product, on the host.
+"""The SPRT walk's decision rule (csrc/sprt_rules.hpp, chain_band and
+chain_no_return) against the reference's running product, on the host.
 
 The device compares a log f_in + b log f_out with log A instead of forming the
 product f_in^a f_out^b one factor at a time, and takes the decision only
-outside a margin of 1e-14 (16 + a + b) + 1e-13 (|a log f_in| + |b log f_out|).
-The product of k rounded factors is off by at most k 2^-53 (1 + O(k 2^-53)),
-each logarithm by an ulp or two, so the margin is about fifty times the
-largest difference.  Checked over histories and thresholds from ratios of
-1e-5 to 0.95, thresholds exactly at a product, equal and nearly equal delta
-and epsilon, and products that underflow: every decided position agrees, and
-where the rule says that a product below e^-690 cannot come back (no_return),
-the product never exceeds A again.
+outside a margin of 1e-14 (16 + n) + 1e-13 n max(|log f_in|, |log f_out|), one
+for a walk over n positions.  The product of k <= n rounded factors is off by at
+most k 2^-53 (1 + O(k 2^-53)), each logarithm by an ulp or two, so the margin is
+at least fifty times the largest difference.  Checked over histories and
+thresholds from ratios of 1e-5 to 0.95, thresholds exactly at a product, equal
+and nearly equal delta and epsilon, and products that underflow: every decided
+position agrees, and where the rule says that a product below e^-690 cannot come
+back (the device asks once per 64 positions), the product never exceeds A again.
+The walk that is built on the rule is checked in test_sprt_rules.py.
 """
 import math
 
@@ -32,10 +33,9 @@ def _threshold(eps, delta, m, m_s):
     return an
 
 
-def _side(a, b, l_in, l_out, l_a):
-    x, y = a * l_in, b * l_out
-    big = x + y
-    margin = 1e-14 * (16 + a + b) + 1e-13 * (np.abs(x) + np.abs(y))
+def _side(a, b, l_in, l_out, l_a, n):
+    big = a * l_in + b * l_out
+    margin = 1e-14 * (16 + n) + 1e-13 * n * max(abs(l_in), abs(l_out))
     side = np.where(big > l_a + margin, 1, np.where(big < l_a - margin, 0, 2))
     return np.where((side == 0) & (big < -690.0), 3, side)
 
@@ -58,7 +58,7 @@ def test_decided_positions_match_the_product(seed):
             continue
         a = np.cumsum(bits)
         b = np.arange(1, n + 1) - a
-        side = _side(a.astype(float), b.astype(float), math.log(f_in), math.log(f_out), math.log(thr))
+        side = _side(a.astype(float), b.astype(float), math.log(f_in), math.log(f_out), math.log(thr), n)
         # positions up to the reference's stop are the ones decided in a walk
         stop = int(np.argmax(product > thr)) if (product > thr).any() else n - 1
         low = np.flatnonzero(side[:stop + 1] == 3)
