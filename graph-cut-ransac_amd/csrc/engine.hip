@@ -69,6 +69,13 @@ static bool use_device_sampling() {
   const char* e = std::getenv("GCR_DEVICE_SAMPLING");
   return e && e[0] == '1';
 }
+// Bit rows of an SPRT walk's window in 64-bit words: 256 MB, or
+// GCR_SPRT_WINDOW_WORDS (same results; a window holds at least eight models).
+static int64_t sprt_window_words() {
+  const char* e = std::getenv("GCR_SPRT_WINDOW_WORDS");
+  const long long v = e ? std::atoll(e) : 0;
+  return v > 0 ? v : 32 << 20;
+}
 static bool use_device_prosac() {
   const char* e = std::getenv("GCR_DEVICE_PROSAC");
   return e && e[0] == '1';
@@ -3061,7 +3068,6 @@ struct Engine : Workspace {
   // slot lists go up in one copy, the items come back in one copy.
   static constexpr int64_t kSlackLaunchPoints = 400000;  // points whose traffic takes as long as a launch
   static constexpr size_t kTableChunk = 256;             // table entries per host task (~20 us)
-  static constexpr int64_t kSprtBudgetWords = 32 << 20;  // 256 MB of bit rows per window
   PhaseTask exec_sprt(std::vector<PairCtx*> items) {
     const int k = (int)items.size();
     // the A tables of pairs whose epsilon changed: n + 1 entries of several
@@ -3116,7 +3122,7 @@ struct Engine : Workspace {
       max_n = std::max(max_n, (int)items[(size_t)i]->n);
       max_slots = std::max(max_slots, (int)it[(size_t)i].num_slots);
     }
-    const SprtPlan plan = sprt_plan(k, max_n, max_slots, kSprtBudgetWords);
+    const SprtPlan plan = sprt_plan(k, max_n, max_slots, sprt_window_words());
     launch_sprt_walk(stream, reinterpret_cast<SprtItem*>(d), k, max_slots, plan, d_sprt_bits.ensure(plan.scratch_words),
                      d_rpts, d_pair_pt_off.p, d_pair_n.p, d_pair_sq_thr.p, d_sprt_pool.p, d_sp_pairs.p, d_sp_cells.p,
                      d_sp_perm.p, d_sp_cell_of.p, d_sp_list.p, sp_max_cells);

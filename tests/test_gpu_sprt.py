@@ -123,9 +123,9 @@ def test_batch_mixing_sprt_and_full_scoring(oracle):
         _same(stats[i], so, M, Mo, mask, mo, rc, atol=1e-14)
 
 
-# Sizes at the edges of the walk's 64-position words, of the 64 words a lane
-# set holds at once (4,096 points) and of the rows kept in LDS (65,536
-# points), with and without the space partitioning cells.
+# Sizes at the edges of the walk's 64-position words and of the 64 words that
+# the lanes hold at once (4,096 points), and far beyond (later words come from
+# memory), with and without the space partitioning cells.
 @pytest.mark.parametrize("n", [8, 63, 64, 65, 129, 4095, 4096, 4097, 65537])
 @pytest.mark.parametrize("sp,sampler", [(False, 0), (True, 1)])
 def test_homography_sprt_walk_sizes_match_oracle(oracle, n, sp, sampler):
@@ -154,3 +154,45 @@ def test_fundamental_sprt_walk_sizes_match_oracle(oracle, n):
     p = oracle.params(1.0, 0.99, 0.0, 2000, 50, 0, 50, 8.0, n, use_sprt=True, min_inlier_ratio_for_sprt=1e-5)
     rc, Fo, mo, so = oracle.find_fundamental(sc["corr"], 480, 640, 480, 640, p)
     _same(st, so, F, Fo, mask, mo, rc, atol=1e-12)
+
+
+def test_windows_of_eight_models_match_one_window(monkeypatch):
+    """The models of a walk come in windows bounded by the bit rows' memory; the
+    test's state (delta, A, the pool position, the last tested model and its
+    inlier list) passes from one to the next.  A budget that leaves eight models
+    a window, and one that the longest slot list crosses a few times, against
+    the default: the same bits, with and without space partitioning, SPRT pairs
+    beside a fully scored one."""
+    import pygcransac
+    probs = []
+    for i, (kind, n, eps, sp) in enumerate([("homography", 1500, 0.2, False), ("homography", 2100, 0.25, True),
+                                            ("fundamental", 1800, 0.3, False), ("homography", 700, 0.3, True),
+                                            ("essential", 1200, 0.3, False), ("homography", 900, 0.4, False)]):
+        sc = getattr(synthetic, kind + "_scene")(synthetic.scene_seed(15, 500 + i), n=n, inlier_ratio=eps)
+        pb = dict(kind=kind, correspondences=sc["corr"], h1=768, w1=1024, h2=768, w2=1024, threshold=2.0, conf=0.99,
+                  spatial_coherence_weight=0.5, max_iters=6000, min_iters=3000, use_sprt=i != 5, sampler=i % 2,
+                  neighborhood=0, neighborhood_size=8.0, lo_number=20, seed=60 + i, min_inlier_ratio_for_sprt=0.01)
+        if kind == "homography":
+            pb["use_space_partitioning"] = sp
+        if kind == "essential":
+            pb.update(K1=sc["K1"], K2=sc["K2"])
+        probs.append(pb)
+    runs = []
+    for words in (None, "1", "40000"):
+        if words is None:
+            monkeypatch.delenv("GCR_SPRT_WINDOW_WORDS", raising=False)
+        else:
+            monkeypatch.setenv("GCR_SPRT_WINDOW_WORDS", words)
+        print("sprt window words:", words, flush=True)
+        runs.append((pygcransac.findBatch(probs), pygcransac.last_batch_stats()))
+    (r0, s0) = runs[0]
+    assert sum(int(m.sum()) for _, m in r0) > 500
+    for r, s in runs[1:]:
+        for i, ((Ma, ma), (Mb, mb)) in enumerate(zip(r0, r)):
+            assert np.array_equal(ma, mb), i
+            assert (Ma is None) == (Mb is None), i
+            if Ma is not None:
+                assert np.array_equal(Ma.view(np.uint64), Mb.view(np.uint64)), i
+            for key in ("iteration_number", "local_optimization_number", "graph_cut_number", "num_inliers", "score",
+                        "models_scored"):
+                assert s0[i][key] == s[i][key], (i, key)
