@@ -71,10 +71,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
-constexpr double kDeltaRel = 0x1p-17;
-constexpr double kDeltaAbs = 0x1p-20;
-constexpr double kMargin = 1.0 + 0x1p-14;
-constexpr double kEta = 0x1p-4;
 constexpr int kCompactPerBlock = 2048;  // slots per block of the ordered compaction
 // The exact pass's grid: the workgroups that are resident at 70 VGPRs, seven
 // waves per SIMD (2,048 workgroups, an eighth of them alone in a second round,
@@ -107,70 +103,6 @@ __device__ __forceinline__ f32x16 zero16() {
 #pragma unroll
   for (int j = 0; j < 16; ++j) z[j] = 0.0f;
   return z;
-}
-
-// The scales of one pair's test: the quantities C (P, Q) are taken times sigma
-// and the denominator form D times kappa, so that the test compares numbers
-// near 1: sigma the power of two that brings kappa = 4 tau''^2 (1 + 2^-14)
-// (1 + h) sigma^2 into [1, 4), at most 2^12 (FP16 coefficients).  Thresholds
-// of half the points' range and more, and ones that are no numbers, drop nothing.
-struct MxScale {
-  double sigma, kappa;
-  bool on;
-};
-__device__ __forceinline__ MxScale mx_scale(double sq_thr, double inv_scale) {
-  MxScale r;
-  const double q = 4.0 * (sq_thr * inv_scale * inv_scale) * kMargin * (1.0 + kEta);
-  r.on = q >= 0.0 && q < 1.0;
-  r.sigma = 1.0;
-  r.kappa = r.on ? q : 0.0;
-#pragma unroll 1
-  for (int e = 0; e < 12 && r.kappa < 1.0; ++e) {
-    r.sigma *= 2.0;
-    r.kappa *= 4.0;
-  }
-  return r;
-}
-
-// One model's coefficient vectors over z (row-major 3x3 M): Sampson C;
-// transfer P, Q.
-template <int KIND>
-__device__ __forceinline__ void quantity_coefs(const double* F, double c[][9]) {
-  constexpr int NQ = KIND == 1 ? 1 : 2;
-#pragma unroll
-  for (int q = 0; q < NQ; ++q)
-#pragma unroll
-    for (int t = 0; t < 9; ++t) c[q][t] = 0.0;
-  if constexpr (KIND == 1) {
-#pragma unroll
-    for (int t = 0; t < 9; ++t) c[0][t] = F[t];
-  } else {
-    c[0][0] = F[6]; c[0][1] = F[7]; c[0][2] = F[8]; c[0][6] = -F[0]; c[0][7] = -F[1]; c[0][8] = -F[2];
-    c[1][3] = F[6]; c[1][4] = F[7]; c[1][5] = F[8]; c[1][6] = -F[3]; c[1][7] = -F[4]; c[1][8] = -F[5];
-  }
-}
-
-// A quarter of the denominator as a linear form in d = (x1^2, x1 y1, y1^2, x1,
-// y1, the same of the second image, 1): (F x1)_0^2 + (F x1)_1^2 + (F^T x2)_0^2 +
-// (F^T x2)_1^2, or W^2.  Every coefficient is at most 1 when |F| <= 1.
-template <int KIND>
-__device__ __forceinline__ void denominator_coefs(const double* F, double g[11]) {
-  g[10] = 0.0;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    double a[3], b[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      a[k] = KIND == 1 ? (h ? F[3 * k] : F[k]) : (h ? 0.0 : F[6 + k]);
-      b[k] = KIND == 1 ? (h ? F[3 * k + 1] : F[3 + k]) : 0.0;
-    }
-    g[5 * h] = 0.25 * (a[0] * a[0] + b[0] * b[0]);
-    g[5 * h + 1] = 0.5 * (a[0] * a[1] + b[0] * b[1]);
-    g[5 * h + 2] = 0.25 * (a[1] * a[1] + b[1] * b[1]);
-    g[5 * h + 3] = 0.5 * (a[0] * a[2] + b[0] * b[2]);
-    g[5 * h + 4] = 0.5 * (a[1] * a[2] + b[1] * b[2]);
-    g[10] += 0.25 * (a[2] * a[2] + b[2] * b[2]);
-  }
 }
 
 }  // namespace
@@ -235,8 +167,8 @@ __global__ void __launch_bounds__(256) k_mx_points(const double* __restrict__ pt
   const double is = inv_scale[pt_pair[i]];
   const double x1 = pts[4 * i] * is, y1 = pts[4 * i + 1] * is, x2 = pts[4 * i + 2] * is, y2 = pts[4 * i + 3] * is;
   const bool ok = fabs(x1) <= 1.0 && fabs(y1) <= 1.0 && fabs(x2) <= 1.0 && fabs(y2) <= 1.0;
-  const double zd[9] = {x2 * x1, x2 * y1, x2, y2 * x1, y2 * y1, y2, x1, y1, 1.0};
-  const double dd[11] = {x1 * x1, x1 * y1, y1 * y1, x1, y1, x2 * x2, x2 * y2, y2 * y2, x2, y2, 1.0};
+  double zd[9], dd[11];
+  mx_terms(x1, y1, x2, y2, zd, dd);
   h8* const o = reinterpret_cast<h8*>(out);
   _Float16 hi[11], lo[11];
 #pragma unroll
@@ -283,14 +215,7 @@ __global__ void __launch_bounds__(256) k_mx_slack(const double* __restrict__ pts
   const int p = pt_pair[i];
   const double is = inv_scale[p];
   const MxScale sc = mx_scale(pair_sq_thr[p], is);
-  const double ax = fabs(pts[4 * i] * is), ay = fabs(pts[4 * i + 1] * is), bx = fabs(pts[4 * i + 2] * is),
-               by = fabs(pts[4 * i + 3] * is);
-  const double sa = 1.0 + ax + ay, sb = 1.0 + bx + by;
-  const double sd = 1.0 + ax * sa + ay * (1.0 + ay) + bx * sb + by * (1.0 + by);
-  const double dc = sc.sigma * (kDeltaRel * (sa * sb) + kDeltaAbs);
-  const double dd = (sc.kappa > 1.0 ? sc.kappa : 1.0) * (kDeltaRel * sd + kDeltaAbs);
-  const double k = kMargin * (dd + (1.0 + 1.0 / kEta) * dc * dc);
-  slack[i] = k < 1e30 ? (float)k : 1.0f;
+  slack[i] = mx_slack(sc, pts[4 * i] * is, pts[4 * i + 1] * is, pts[4 * i + 2] * is, pts[4 * i + 3] * is);
 }
 
 // ---- ordered compaction of the active model slots ------------------------------
@@ -408,8 +333,8 @@ __global__ void __launch_bounds__(256) k_mx_coefs(const double* __restrict__ pai
   double Fs[9];
   mx_normalise<KIND>(M, s, ts.on, Fs);
   double cq[2][9], dq[11];
-  quantity_coefs<KIND>(Fs, cq);
-  denominator_coefs<KIND>(Fs, dq);
+  mx_quantities<KIND>(Fs, cq);
+  mx_denominator<KIND>(Fs, dq);
   h8* out = coefs + (e * 2 + hf) * (2 * NQ);
   _Float16 hi[11], lo[11];
 #pragma unroll
