@@ -295,11 +295,10 @@ __device__ __forceinline__ void wave_lu_full(double (&col)[10], double (&x)[10],
 // Real eigenvalues of the 10 x 10 matrix S.a, in diagonal order of the real
 // Schur form, to S.evs; returns their number (-1: no convergence).
 // Householder reduction to Hessenberg form, then Francis double-shift QR steps
-// -- the published "hqr" method (Martin, Peters and Wilkinson, "The QR
-// algorithm for real Hessenberg matrices", Numer. Math. 14, 1970), written
-// here.  The wave works on S.h: column operations with a lane per column, row
-// operations with a lane per row, the searches with a lane per candidate; the
-// scalar steps run on every lane alike.
+// (Martin, Peters and Wilkinson, "The QR algorithm for real Hessenberg matrices",
+// Numer. Math. 14, 1970).  The wave works on S.h: column operations with a lane
+// per column, row operations with a lane per row, the searches with a lane per
+// candidate; the scalar steps run on every lane alike.
 __device__ inline int wave_real_eigenvalues(StewShared& S) {
   constexpr int n = 10;
   const int lane = lane_id();
@@ -357,157 +356,148 @@ __device__ inline int wave_real_eigenvalues(StewShared& S) {
     }
     __syncthreads();
   }
-  int nr = 0, nn = n - 1, its = 0;
-  double t = 0.0, anorm = 0.0;
+  // double-shift QR on the active block, rows top .. bottom
+  double size = 0.0;  // sum of the magnitudes, where a diagonal is all zero
   for (int i = 0; i < n; ++i)
-    for (int j = (i - 1 > 0 ? i - 1 : 0); j < n; ++j) anorm += fabs(a[i][j]);
+    for (int j = (i - 1 > 0 ? i - 1 : 0); j < n; ++j) size += fabs(a[i][j]);
   const double eps = 2.220446049250313e-16;
-  while (nn >= 0) {
-    // the largest l <= nn with a negligible subdiagonal entry, or 0
-    int l;
+  int nr = 0, steps = 0;
+  double moved = 0.0;  // taken off the diagonal so far
+  auto report = [&](int row, double value) {
+    if (lane == 0) {
+      S.pos[nr] = row;
+      S.ev[nr] = value;
+    }
+    ++nr;
+  };
+  for (int bottom = n - 1; bottom >= 0;) {
+    // the block begins below the last negligible subdiagonal entry
+    int top;
     {
       bool small = false;
-      if (lane >= 1 && lane <= nn) {
-        const double s = fabs(a[lane - 1][lane - 1]) + fabs(a[lane][lane]);
-        const double sc = s == 0.0 ? anorm : s;
-        small = fabs(a[lane][lane - 1]) <= eps * sc;
+      if (lane >= 1 && lane <= bottom) {
+        const double around = fabs(a[lane - 1][lane - 1]) + fabs(a[lane][lane]);
+        small = fabs(a[lane][lane - 1]) <= eps * (around == 0.0 ? size : around);
       }
       const uint64_t b = ballot64(small);
-      l = b ? 63 - __clzll((long long)b) : 0;
-      if (b && lane == 0) a[l][l - 1] = 0.0;
+      top = b ? 63 - __clzll((long long)b) : 0;
+      if (b && lane == 0) a[top][top - 1] = 0.0;
     }
     __syncthreads();
-    const double x = a[nn][nn];
-    if (l == nn) {  // one root
-      if (lane == 0) {
-        S.pos[nr] = nn;
-        S.ev[nr] = x + t;
-      }
-      ++nr;
-      --nn;
-      its = 0;
+    const double last = a[bottom][bottom];
+    if (top == bottom) {
+      report(bottom, last + moved);
+      bottom -= 1;
+      steps = 0;
       continue;
     }
-    const double y = a[nn - 1][nn - 1];
-    const double w = a[nn][nn - 1] * a[nn - 1][nn];
-    if (l == nn - 1) {  // two roots
-      const double p = 0.5 * (y - x);
-      const double q = p * p + w;
-      const double z = sqrt(fabs(q));
-      const double xx = x + t;
-      if (q >= 0.0) {
-        const double zz = p + (p >= 0.0 ? fabs(z) : -fabs(z));
-        const double r1 = xx + zz;
-        const double r2 = zz != 0.0 ? xx - w / zz : xx + zz;
-        if (lane == 0) {
-          S.pos[nr] = nn - 1;
-          S.ev[nr] = r1;
-          S.pos[nr + 1] = nn;
-          S.ev[nr + 1] = r2;
-        }
-        nr += 2;
+    // the last 2 x 2 block (prev . ; . last): its product of off-diagonals
+    const double prev = a[bottom - 1][bottom - 1], cross = a[bottom][bottom - 1] * a[bottom - 1][bottom];
+    if (top + 1 == bottom) {
+      const double half = 0.5 * (prev - last), disc = half * half + cross;
+      if (disc >= 0.0) {
+        // the root away from last first, the other by the product of both
+        const double root = sqrt(disc), far = half >= 0.0 ? half + root : half - root, base = last + moved;
+        report(bottom - 1, base + far);
+        report(bottom, far != 0.0 ? base - cross / far : base + far);
       }
-      nn -= 2;
-      its = 0;
+      bottom -= 2;
+      steps = 0;
       continue;
     }
-    if (its == 30 * n) return -1;  // no convergence
-    double xs = x, ys = y, ws = w;
-    if (its == 10 || its == 20) {  // exceptional shift
-      t += x;
+    if (steps == 30 * n) return -1;  // no convergence
+    // the step's two shifts as the diagonal and the cross product of a block:
+    // the last block, or after ten and twenty steps an ad hoc one
+    double sh_last = last, sh_prev = prev, sh_cross = cross;
+    if (steps == 10 || steps == 20) {
+      moved += last;
       __syncthreads();
-      if (lane <= nn) a[lane][lane] -= x;
+      if (lane <= bottom) a[lane][lane] -= last;
       __syncthreads();
-      const double s = fabs(a[nn][nn - 1]) + fabs(a[nn - 1][nn - 2]);
-      xs = ys = 0.75 * s;
-      ws = -0.4375 * s * s;
+      const double off = fabs(a[bottom][bottom - 1]) + fabs(a[bottom - 1][bottom - 2]);
+      sh_last = sh_prev = 0.75 * off;
+      sh_cross = -0.4375 * off * off;
     }
-    ++its;
-    // the largest m with two small consecutive subdiagonal entries, or l
-    int m;
-    double p = 0.0, q = 0.0, r = 0.0;
+    ++steps;
+    // first column of the shifted square, from the lowest row at which the
+    // entries left of it hardly change under the step (a lane per row)
+    int begin;
+    double x0 = 0.0, x1 = 0.0, x2 = 0.0;
     {
-      bool ok = false;
-      if (lane >= l && lane <= nn - 2) {
-        const double z = a[lane][lane];
-        const double rr = xs - z, ss = ys - z;
-        p = (rr * ss - ws) / a[lane + 1][lane] + a[lane][lane + 1];
-        q = a[lane + 1][lane + 1] - z - rr - ss;
-        r = a[lane + 2][lane + 1];
-        const double s = fabs(p) + fabs(q) + fabs(r);
-        p /= s;
-        q /= s;
-        r /= s;
-        if (lane == l) {
-          ok = true;
+      bool fits = false;
+      if (lane >= top && lane <= bottom - 2) {
+        const double at = a[lane][lane], dl = sh_last - at, dp = sh_prev - at;
+        x0 = (dl * dp - sh_cross) / a[lane + 1][lane] + a[lane][lane + 1];
+        x1 = a[lane + 1][lane + 1] - at - dl - dp;
+        x2 = a[lane + 2][lane + 1];
+        const double sum = fabs(x0) + fabs(x1) + fabs(x2);
+        x0 /= sum;
+        x1 /= sum;
+        x2 /= sum;
+        if (lane == top) {
+          fits = true;
         } else {
-          const double u = fabs(a[lane][lane - 1]) * (fabs(q) + fabs(r));
-          const double v = fabs(p) * (fabs(a[lane - 1][lane - 1]) + fabs(z) + fabs(a[lane + 1][lane + 1]));
-          ok = u <= eps * v;
+          const double change = fabs(a[lane][lane - 1]) * (fabs(x1) + fabs(x2));
+          const double diag = fabs(a[lane - 1][lane - 1]) + fabs(at) + fabs(a[lane + 1][lane + 1]);
+          fits = change <= eps * (fabs(x0) * diag);
         }
       }
-      m = 63 - __clzll((long long)ballot64(ok));
-      p = readlane_f64(p, m);
-      q = readlane_f64(q, m);
-      r = readlane_f64(r, m);
+      begin = 63 - __clzll((long long)ballot64(fits));
+      x0 = readlane_f64(x0, begin);
+      x1 = readlane_f64(x1, begin);
+      x2 = readlane_f64(x2, begin);
     }
     __syncthreads();
-    if (lane >= m + 2 && lane <= nn) {
+    if (lane >= begin + 2 && lane <= bottom) {
       a[lane][lane - 2] = 0.0;
-      if (lane != m + 2) a[lane][lane - 3] = 0.0;
+      if (lane > begin + 2) a[lane][lane - 3] = 0.0;
     }
     __syncthreads();
-    for (int k = m; k <= nn - 1; ++k) {
-      double xx = 0.0;
-      if (k != m) {
-        p = a[k][k - 1];
-        q = a[k + 1][k - 1];
-        r = k != nn - 1 ? a[k + 2][k - 1] : 0.0;
-        xx = fabs(p) + fabs(q) + fabs(r);
-        if (xx != 0.0) {
-          p /= xx;
-          q /= xx;
-          r /= xx;
+    // chase: at every row a reflection of three (at the end two) rows and columns
+    for (int row = begin; row < bottom; ++row) {
+      const bool three = row + 1 < bottom;
+      double scale = 0.0;
+      if (row > begin) {
+        x0 = a[row][row - 1];
+        x1 = a[row + 1][row - 1];
+        x2 = three ? a[row + 2][row - 1] : 0.0;
+        scale = fabs(x0) + fabs(x1) + fabs(x2);
+        if (scale != 0.0) {
+          x0 /= scale;
+          x1 /= scale;
+          x2 /= scale;
         }
       }
-      const double sq = sqrt(p * p + q * q + r * r);
-      const double s = p >= 0.0 ? sq : -sq;
-      if (s != 0.0) {
-        if (lane == 0) {
-          if (k == m) {
-            if (l != m) a[k][k - 1] = -a[k][k - 1];
-          } else {
-            a[k][k - 1] = -s * xx;
-          }
-        }
-        p += s;
-        const double xr = p / s, yr = q / s, zr = r / s;
-        q /= p;
-        r /= p;
-        const bool three = k != nn - 1;
-        __syncthreads();
-        if (lane >= k && lane <= nn) {
-          double pp = a[k][lane] + q * a[k + 1][lane];
-          if (three) {
-            pp += r * a[k + 2][lane];
-            a[k + 2][lane] -= pp * zr;
-          }
-          a[k + 1][lane] -= pp * yr;
-          a[k][lane] -= pp * xr;
-        }
-        __syncthreads();
-        const int mmin = nn < k + 3 ? nn : k + 3;
-        if (lane >= l && lane <= mmin) {
-          double pp = xr * a[lane][k] + yr * a[lane][k + 1];
-          if (three) {
-            pp += zr * a[lane][k + 2];
-            a[lane][k + 2] -= pp * r;
-          }
-          a[lane][k + 1] -= pp * q;
-          a[lane][k] -= pp;
-        }
-        __syncthreads();
+      // I - u v^T with v = (1, v1, v2) takes x to (-length, 0, 0)
+      const double norm = sqrt(x0 * x0 + x1 * x1 + x2 * x2), length = x0 >= 0.0 ? norm : -norm;
+      if (length == 0.0) continue;
+      if (lane == 0) {
+        if (row > begin) a[row][row - 1] = -length * scale;
+        else if (row > top) a[row][row - 1] = -a[row][row - 1];
       }
+      const double head = x0 + length;
+      const double u0 = head / length, u1 = x1 / length, u2 = x2 / length, v1 = x1 / head, v2 = x2 / head;
+      __syncthreads();
+      if (lane >= row && lane <= bottom) {
+        double dot = a[row][lane] + v1 * a[row + 1][lane];
+        if (three) {
+          dot += v2 * a[row + 2][lane];
+          a[row + 2][lane] -= dot * u2;
+        }
+        a[row + 1][lane] -= dot * u1;
+        a[row][lane] -= dot * u0;
+      }
+      __syncthreads();
+      if (lane >= top && lane <= (bottom < row + 3 ? bottom : row + 3)) {
+        double dot = u0 * a[lane][row] + u1 * a[lane][row + 1];
+        if (three) {
+          dot += u2 * a[lane][row + 2];
+          a[lane][row + 2] -= dot * v2;
+        }
+        a[lane][row + 1] -= dot * v1;
+        a[lane][row] -= dot;
+      }
+      __syncthreads();
     }
   }
   __syncthreads();

@@ -19,6 +19,8 @@
 // pinned against the reference's own header (tests/golden).
 #pragma once
 
+#include <array>
+
 #include "oracle_core.hpp"
 #include "oracle_fundamental.hpp"
 #include "oracle_gcransac.hpp"
@@ -394,7 +396,7 @@ inline void lu_full_solve(double* A, double* B, int n, int m) {
 }
 
 // Real eigenvalues of a real n x n matrix (n <= 10): Householder reduction to
-// Hessenberg form, then Francis double-shift QR steps -- the "hqr" method of
+// Hessenberg form, then Francis double-shift QR steps -- the method of
 // Martin, Peters and Wilkinson (Numer. Math. 14, 1970) -- (exceptional shifts at
 // iterations 10 and 20, at most 30 per eigenvalue) until the matrix is quasi
 // upper triangular.  1 x 1 blocks and 2 x 2 blocks with real eigenvalues give
@@ -433,128 +435,111 @@ inline int real_eigenvalues(const double* M, int n, double* ev) {
     }
     for (int i = k + 2; i < n; ++i) a[i][k] = 0.0;
   }
-  // shifted QR (hqr)
-  int nr = 0;
-  int nn = n - 1;
-  double t = 0.0;
-  double anorm = 0.0;
+  // double-shift QR on the active block, rows top .. bottom
+  double size = 0.0;  // sum of the magnitudes, where a diagonal is all zero
   for (int i = 0; i < n; ++i)
-    for (int j = std::max(i - 1, 0); j < n; ++j) anorm += std::fabs(a[i][j]);
-  int its = 0;
+    for (int j = std::max(i - 1, 0); j < n; ++j) size += std::fabs(a[i][j]);
   const double eps = std::numeric_limits<double>::epsilon();
-  while (nn >= 0) {
-    int l;
-    for (l = nn; l >= 1; --l) {
-      const double s = std::fabs(a[l - 1][l - 1]) + std::fabs(a[l][l]);
-      const double sc = s == 0.0 ? anorm : s;
-      if (std::fabs(a[l][l - 1]) <= eps * sc) {
-        a[l][l - 1] = 0.0;
+  int nr = 0, steps = 0;
+  double moved = 0.0;  // taken off the diagonal so far
+  auto report = [&](int row, double value) {
+    pos[nr] = row;
+    ev[nr++] = value;
+  };
+  for (int bottom = n - 1; bottom >= 0;) {
+    // the block begins below the last negligible subdiagonal entry
+    int top = bottom;
+    for (; top > 0; --top) {
+      const double around = std::fabs(a[top - 1][top - 1]) + std::fabs(a[top][top]);
+      if (std::fabs(a[top][top - 1]) <= eps * (around == 0.0 ? size : around)) {
+        a[top][top - 1] = 0.0;
         break;
       }
     }
-    const double x = a[nn][nn];
-    if (l == nn) {  // one root
-      pos[nr] = nn;
-      ev[nr++] = x + t;
-      --nn;
-      its = 0;
+    const double last = a[bottom][bottom];
+    if (top == bottom) {
+      report(bottom, last + moved);
+      bottom -= 1;
+      steps = 0;
       continue;
     }
-    const double y = a[nn - 1][nn - 1];
-    const double w = a[nn][nn - 1] * a[nn - 1][nn];
-    if (l == nn - 1) {  // two roots
-      const double p = 0.5 * (y - x);
-      const double q = p * p + w;
-      const double z = std::sqrt(std::fabs(q));
-      const double xx = x + t;
-      if (q >= 0.0) {
-        const double zz = p + (p >= 0.0 ? std::fabs(z) : -std::fabs(z));
-        const double r1 = xx + zz;
-        const double r2 = zz != 0.0 ? xx - w / zz : xx + zz;
-        pos[nr] = nn - 1;
-        ev[nr++] = r1;
-        pos[nr] = nn;
-        ev[nr++] = r2;
+    // the last 2 x 2 block (prev . ; . last): its product of off-diagonals
+    const double prev = a[bottom - 1][bottom - 1], cross = a[bottom][bottom - 1] * a[bottom - 1][bottom];
+    if (top + 1 == bottom) {
+      const double half = 0.5 * (prev - last), disc = half * half + cross;
+      if (disc >= 0.0) {
+        // the root away from last first, the other by the product of both
+        const double root = std::sqrt(disc), far = half >= 0.0 ? half + root : half - root, base = last + moved;
+        report(bottom - 1, base + far);
+        report(bottom, far != 0.0 ? base - cross / far : base + far);
       }
-      nn -= 2;
-      its = 0;
+      bottom -= 2;
+      steps = 0;
       continue;
     }
-    if (its == 30 * n) return -1;  // no convergence
-    double xs = x, ys = y, ws = w;
-    if (its == 10 || its == 20) {  // exceptional shift
-      t += x;
-      for (int i = 0; i <= nn; ++i) a[i][i] -= x;
-      const double s = std::fabs(a[nn][nn - 1]) + std::fabs(a[nn - 1][nn - 2]);
-      xs = ys = 0.75 * s;
-      ws = -0.4375 * s * s;
+    if (steps == 30 * n) return -1;  // no convergence
+    // the step's two shifts as the diagonal and the cross product of a block:
+    // the last block, or after ten and twenty steps an ad hoc one
+    double sh_last = last, sh_prev = prev, sh_cross = cross;
+    if (steps == 10 || steps == 20) {
+      moved += last;
+      for (int i = 0; i <= bottom; ++i) a[i][i] -= last;
+      const double off = std::fabs(a[bottom][bottom - 1]) + std::fabs(a[bottom - 1][bottom - 2]);
+      sh_last = sh_prev = 0.75 * off;
+      sh_cross = -0.4375 * off * off;
     }
-    ++its;
-    int m;
-    double p = 0, q = 0, r = 0, z;
-    for (m = nn - 2; m >= l; --m) {
-      z = a[m][m];
-      const double rr = xs - z, ss = ys - z;
-      p = (rr * ss - ws) / a[m + 1][m] + a[m][m + 1];
-      q = a[m + 1][m + 1] - z - rr - ss;
-      r = a[m + 2][m + 1];
-      const double s = std::fabs(p) + std::fabs(q) + std::fabs(r);
-      p /= s;
-      q /= s;
-      r /= s;
-      if (m == l) break;
-      const double u = std::fabs(a[m][m - 1]) * (std::fabs(q) + std::fabs(r));
-      const double v = std::fabs(p) * (std::fabs(a[m - 1][m - 1]) + std::fabs(z) + std::fabs(a[m + 1][m + 1]));
-      if (u <= eps * v) break;
+    ++steps;
+    // first column of the shifted square, from the lowest row at which the
+    // entries left of it hardly change under the step
+    auto column = [&](int row) {
+      const double at = a[row][row], dl = sh_last - at, dp = sh_prev - at;
+      std::array<double, 3> x = {(dl * dp - sh_cross) / a[row + 1][row] + a[row][row + 1],
+                                 a[row + 1][row + 1] - at - dl - dp, a[row + 2][row + 1]};
+      const double sum = std::fabs(x[0]) + std::fabs(x[1]) + std::fabs(x[2]);
+      for (double& v : x) v /= sum;
+      return x;
+    };
+    int begin = bottom - 2;
+    std::array<double, 3> x = column(begin);
+    for (; begin > top; x = column(--begin)) {
+      const double change = std::fabs(a[begin][begin - 1]) * (std::fabs(x[1]) + std::fabs(x[2]));
+      const double diag = std::fabs(a[begin - 1][begin - 1]) + std::fabs(a[begin][begin]) +
+                          std::fabs(a[begin + 1][begin + 1]);
+      if (change <= eps * (std::fabs(x[0]) * diag)) break;
     }
-    for (int i = m + 2; i <= nn; ++i) {
+    for (int i = begin + 2; i <= bottom; ++i) {
       a[i][i - 2] = 0.0;
-      if (i != m + 2) a[i][i - 3] = 0.0;
+      if (i > begin + 2) a[i][i - 3] = 0.0;
     }
-    for (int k = m; k <= nn - 1; ++k) {
-      double xx = 0.0;
-      if (k != m) {
-        p = a[k][k - 1];
-        q = a[k + 1][k - 1];
-        r = 0.0;
-        if (k != nn - 1) r = a[k + 2][k - 1];
-        xx = std::fabs(p) + std::fabs(q) + std::fabs(r);
-        if (xx != 0.0) {
-          p /= xx;
-          q /= xx;
-          r /= xx;
-        }
+    // chase: at every row a reflection of three (at the end two) rows and columns
+    for (int row = begin; row < bottom; ++row) {
+      const int rows = row + 1 < bottom ? 3 : 2;
+      double scale = 0.0;
+      if (row > begin) {
+        for (int k = 0; k < 3; ++k) x[k] = k < rows ? a[row + k][row - 1] : 0.0;
+        scale = std::fabs(x[0]) + std::fabs(x[1]) + std::fabs(x[2]);
+        if (scale != 0.0)
+          for (double& v : x) v /= scale;
       }
-      const double sq = std::sqrt(p * p + q * q + r * r);
-      const double s = p >= 0.0 ? sq : -sq;
-      if (s != 0.0) {
-        if (k == m) {
-          if (l != m) a[k][k - 1] = -a[k][k - 1];
-        } else
-          a[k][k - 1] = -s * xx;
-        p += s;
-        const double xr = p / s, yr = q / s, zr = r / s;
-        q /= p;
-        r /= p;
-        for (int j = k; j <= nn; ++j) {
-          double pp = a[k][j] + q * a[k + 1][j];
-          if (k != nn - 1) {
-            pp += r * a[k + 2][j];
-            a[k + 2][j] -= pp * zr;
-          }
-          a[k + 1][j] -= pp * yr;
-          a[k][j] -= pp * xr;
-        }
-        const int mmin = nn < k + 3 ? nn : k + 3;
-        for (int i = l; i <= mmin; ++i) {
-          double pp = xr * a[i][k] + yr * a[i][k + 1];
-          if (k != nn - 1) {
-            pp += zr * a[i][k + 2];
-            a[i][k + 2] -= pp * r;
-          }
-          a[i][k + 1] -= pp * q;
-          a[i][k] -= pp;
-        }
+      // I - u v^T with v = (1, v1, v2) takes x to (-length, 0, 0)
+      double length = std::sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
+      if (!(x[0] >= 0.0)) length = -length;
+      if (length == 0.0) continue;
+      if (row > begin) a[row][row - 1] = -length * scale;
+      else if (row > top) a[row][row - 1] = -a[row][row - 1];
+      const double head = x[0] + length;
+      const double u[3] = {head / length, x[1] / length, x[2] / length}, v[3] = {1.0, x[1] / head, x[2] / head};
+      for (int j = row; j <= bottom; ++j) {
+        double dot = a[row][j];
+        for (int k = 1; k < rows; ++k) dot += v[k] * a[row + k][j];
+        for (int k = 0; k < rows; ++k) a[row + k][j] -= dot * u[k];
+      }
+      const int reach = std::min(bottom, row + 3);
+      for (int i = top; i <= reach; ++i) {
+        double dot = u[0] * a[i][row];
+        for (int k = 1; k < rows; ++k) dot += u[k] * a[i][row + k];
+        a[i][row] -= dot;
+        for (int k = 1; k < rows; ++k) a[i][row + k] -= dot * v[k];
       }
     }
   }
