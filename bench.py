@@ -79,14 +79,12 @@ FIT_KERNEL = {0: "k_fit_h", 1: "k_fit_f", 2: "k_fit_e"}
 # pairs per step, batch groups).  The summary with the commands is
 # profiles/pmc_traffic_fit_kernels.md.
 TRAFFIC_KIB = {
-    ("guided", 1024, 2): (2479.6, 44.6),
-    ("guided", 1024, 3): (2022.3, 34.1),
-    ("fundamental", 1024, 2): (8523.2, 149.6),
-    ("fundamental", 1024, 3): (6292.7, 107.6),
-    ("guided", 1024, 4): (1729.1, 28.3),
-    ("fundamental", 1024, 4): (5261.4, 88.5),
-    ("homography", 1024, 2): (8342.1, 171.2),
-    ("homography", 1024, 4): (4776.2, 95.8),
+    ("guided", 1024, 3): (2005.7, 221.9),
+    ("guided", 1024, 4): (1743.6, 28.3),
+    ("fundamental", 1024, 3): (6265.4, 107.6),
+    ("fundamental", 1024, 4): (5276.3, 146.9),
+    ("homography", 1024, 3): (6080.8, 122.8),
+    ("homography", 1024, 4): (4786.8, 95.8),
 }
 # Algorithmic HBM bytes of a non-minimal fit per point: the gathered
 # correspondence (4 doubles) and its index.

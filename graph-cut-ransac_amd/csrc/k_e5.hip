@@ -29,7 +29,9 @@
 // their instruction fetches) and FP64 VALU, in the elimination the selects of
 // the row exchanges, in the root search lanes that wait for the sample with
 // the most bisections.  One thread per sample for the whole solver kept 5,360
-// bytes of matrices per thread in scratch memory.  Measured on MI355X, 32
+// bytes of matrices per thread in scratch memory; here the matrices are in
+// registers, and scratch holds the root search's rarely used deep intervals (560
+// bytes, kE5StackMore) and 28 bytes of spills in the elimination.  Measured on MI355X, 32
 // pairs of 10,000 points at 10 % inliers: 1,079 ms of the call's kernels then,
 // 166 ms with these kernels (per 131,072 samples 139 + 86 + 118 + 224 us, four
 // streams at once; alone 24 + 37 + 69 + 148); the call 1,173 -> 614 ms.
@@ -94,7 +96,7 @@ __global__ void __launch_bounds__(64) k_e5_null_space(const double* __restrict__
   for (int v = 0; v < 36; ++v) o[(kE5N + v) * kTile] = N[v];
 }
 
-// The nine trace constraints in a loop (entry (i, j)'s operands from LDS): 6 KB
+// The nine trace constraints in a loop (entry (i, j)'s operands from LDS): 11 KB
 // of code instead of 35, and the kernel stays in the instruction cache.  Fully
 // unrolled together with the null space (66 KB) every wave fetched its code
 // from the L2 line by line: 242 us per 131,072 samples.
