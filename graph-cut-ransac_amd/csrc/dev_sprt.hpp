@@ -63,7 +63,7 @@ __device__ __forceinline__ double chain_word(const Chain& c, double lambda, uint
   return x;
 }
 
-// One model from pool position start (see the file header); total: its
+// One model from pool position start (k_sprt.hip); total: its
 // inliers among all n points.
 __device__ WalkResult walk_pool(const Rows& R, const Chain& c, int start, int n, int total) {
   const int lane = lane_id();

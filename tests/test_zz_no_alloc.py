@@ -1,7 +1,7 @@
-"""gcr_score_models_noalloc (device buffers in and out, the library's fixed
-device scratch, no allocation) against gcr_score_models on the same inputs:
-identical counts, values and masks, on two calls in a row, the second with
-fewer points and fewer models than the first."""
+"""gcr_score_models_noalloc (device buffers in and out, one launch, no other
+device memory) against gcr_score_models on the same inputs: identical counts,
+values and masks, on two calls in a row, the second with fewer points and fewer
+models than the first."""
 import ctypes
 
 import numpy as np
